@@ -259,7 +259,7 @@ int lbk_swiglu_bwd_bf16(const uint16_t* grad_out, const uint16_t* x, const uint1
 /*
  * lbk_swiglu_bwd_bf16 plus the bias gradients of lbk_swiglu_fwd_bias_bf16 (each optional, fp32):
  * d_b_gate = column sums of dg, d_b_up = of du [d_ff], d_b_down = of grad_out [d_model],
- * summed per 64-row group and the groups in a fixed order (deterministic).  gate_pre_act and
+ * summed per row group and the groups in a fixed order (deterministic).  gate_pre_act and
  * up_output are the forward's biased pre-activations.  Its workspace
  * (lbk_swiglu_bwd_bias_workspace_bytes) adds the column-sum partials when a bias gradient is
  * asked for.
@@ -569,6 +569,12 @@ size_t lbk_block_ell_matmul_bwd_workspace_bytes(int64_t N, int32_t in_features, 
 int lbk_block_ell_matmul_bwd_bf16(const uint16_t* grad_out, const uint16_t* x, int64_t N, int32_t in_features,
                                   const lbk_bell* w, uint16_t* dx, uint16_t* d_values, void* workspace,
                                   size_t workspace_bytes, void* stream);
+/* The same plus d_bias [R*B] fp32 (optional): the column sums of grad_out in a fixed order. */
+size_t lbk_block_ell_matmul_bwd_bias_workspace_bytes(int64_t N, int32_t in_features, const lbk_bell* w);
+int lbk_block_ell_matmul_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t* x, int64_t N,
+                                       int32_t in_features, const lbk_bell* w, uint16_t* dx,
+                                       uint16_t* d_values, float* d_bias, void* workspace,
+                                       size_t workspace_bytes, void* stream);
 
 /* ---- prune-time topology transforms (integer and copy work; alive masks are one byte per slot,
  * nonzero = alive).  Replaces the JAX functions of looped_blockell/opt/compaction.py and

@@ -1111,7 +1111,7 @@ size_t lbk_swiglu_bwd_bias_workspace_bytes(int64_t N, int32_t d_model, const lbk
   const size_t base = lbk_swiglu_bwd_workspace_bytes(N, d_model, gate, up, down);
   if (!base) return 0;
   const int64_t d_ff = (int64_t)gate->R * gate->B;
-  return base + align256(colsum_bytes(N, (int)(d_ff > d_model ? d_ff : d_model)));
+  return base + align256(colsum_bytes(N, 2 * d_ff + d_model));
 }
 
 int lbk_swiglu_bwd_bf16(const uint16_t* grad_out, const uint16_t* x, const uint16_t* gate_pre_act,
@@ -1216,9 +1216,12 @@ int lbk_swiglu_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t* x, const 
   // bias gradients: column sums of dg, du and grad_out (the partials after the tile partials)
   if (want_db) {
     float* cpart = reinterpret_cast<float*>(reinterpret_cast<char*>(part) + align256(poff * 4));
-    if (d_b_gate && launch_colsum(dg, N, (int)d_ff, d_ff, cpart, d_b_gate, s)) return LBK_ERR_LAUNCH;
-    if (d_b_up && launch_colsum(du, N, (int)d_ff, d_ff, cpart, d_b_up, s)) return LBK_ERR_LAUNCH;
-    if (d_b_down && launch_colsum(grad_out, N, d_model, d_model, cpart, d_b_down, s)) return LBK_ERR_LAUNCH;
+    ColsumJob cj[3];
+    int nc = 0;
+    if (d_b_gate) cj[nc++] = ColsumJob{dg, d_ff, (int)d_ff, d_b_gate, nullptr, 0};
+    if (d_b_up) cj[nc++] = ColsumJob{du, d_ff, (int)d_ff, d_b_up, nullptr, 0};
+    if (d_b_down) cj[nc++] = ColsumJob{grad_out, d_model, d_model, d_b_down, nullptr, 0};
+    if (launch_colsum(cj, nc, N, cpart, s)) return LBK_ERR_LAUNCH;
   }
   return LBK_OK;
 }
@@ -1229,9 +1232,21 @@ size_t lbk_block_ell_matmul_bwd_workspace_bytes(int64_t N, int32_t in_features, 
   return tlist_bytes(w, C) + align256(dw_part_floats(N, w, C, (int64_t)w->R * w->B) * 4);
 }
 
+size_t lbk_block_ell_matmul_bwd_bias_workspace_bytes(int64_t N, int32_t in_features, const lbk_bell* w) {
+  const size_t base = lbk_block_ell_matmul_bwd_workspace_bytes(N, in_features, w);
+  return base ? base + align256(colsum_bytes(N, (int64_t)w->R * w->B)) : 0;
+}
+
 int lbk_block_ell_matmul_bwd_bf16(const uint16_t* grad_out, const uint16_t* x, int64_t N, int32_t in_features,
                                   const lbk_bell* w, uint16_t* dx, uint16_t* d_values, void* workspace,
                                   size_t workspace_bytes, void* stream) {
+  return lbk_block_ell_matmul_bwd_bias_bf16(grad_out, x, N, in_features, w, dx, d_values, nullptr, workspace,
+                                            workspace_bytes, stream);
+}
+
+int lbk_block_ell_matmul_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t* x, int64_t N, int32_t in_features,
+                                       const lbk_bell* w, uint16_t* dx, uint16_t* d_values, float* d_bias,
+                                       void* workspace, size_t workspace_bytes, void* stream) {
   int st;
   if ((st = check_bell(w))) return st;
   if (N < 0 || in_features <= 0) return LBK_ERR_ARG;
@@ -1241,11 +1256,12 @@ int lbk_block_ell_matmul_bwd_bf16(const uint16_t* grad_out, const uint16_t* x, i
   const int64_t nt = (int64_t)w->R * w->K, out_f = (int64_t)w->R * B;
   if (d_values && !a16(d_values)) return LBK_ERR_ALIGN;
   if (nt > 0 && !a16(w->values)) return LBK_ERR_ALIGN;
-  if (N > 0 && (dx || d_values)) {
+  if (N > 0 && (dx || d_values || d_bias)) {
     if (!grad_out || (d_values && !x)) return LBK_ERR_NULL;
     if (!a16(grad_out) || (x && !a16(x)) || (dx && !a16(dx)) || in_features % 8) return LBK_ERR_ALIGN;
   }
-  const size_t need = lbk_block_ell_matmul_bwd_workspace_bytes(N, in_features, w);
+  const size_t need = d_bias ? lbk_block_ell_matmul_bwd_bias_workspace_bytes(N, in_features, w)
+                             : lbk_block_ell_matmul_bwd_workspace_bytes(N, in_features, w);
   if (!workspace || workspace_bytes < need) return LBK_ERR_WORKSPACE;
   if (!a16(workspace)) return LBK_ERR_ALIGN;
   hipStream_t s = S(stream);
@@ -1277,6 +1293,13 @@ int lbk_block_ell_matmul_bwd_bf16(const uint16_t* grad_out, const uint16_t* x, i
     DWJob dj{x, in_features, grad_out, out_f, w->col_idx, w->R, w->K, C, part, d_values,
              lists ? lj.cnt : nullptr, lists ? lj.list : nullptr, 0, 0};
     if (launch_dw(B, &dj, 1, N, s)) return LBK_ERR_LAUNCH;
+  }
+  if (d_bias && out_f > 0) {
+    // the column-sum partials follow the tile partials
+    float* cpart = reinterpret_cast<float*>(reinterpret_cast<char*>(part) +
+                                            align256(dw_part_floats(N, w, C, out_f) * 4));
+    const ColsumJob cj{grad_out, out_f, (int)out_f, d_bias, nullptr, 0};
+    if (launch_colsum(&cj, 1, N, cpart, s)) return LBK_ERR_LAUNCH;
   }
   return LBK_OK;
 }

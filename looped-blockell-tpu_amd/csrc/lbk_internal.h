@@ -166,9 +166,25 @@ int launch_rmsnorm(const uint16_t* x, int64_t N, int d, const float* scale, floa
 int launch_rmsnorm_f32(const float* x, int64_t N, int d, const float* scale, float eps, uint16_t* out,
                        hipStream_t st);
 size_t rmsnorm_bwd_bytes(int64_t N, int d);   // fp32 dscale partials of the workgroups
-// fp32 column sums out[C] of a bf16 [N, C] matrix (deterministic: per-64-row partials in part)
-size_t colsum_bytes(int64_t N, int C);
-int launch_colsum(const uint16_t* a, int64_t N, int C, int64_t lda, float* part, float* out, hipStream_t st);
+// fp32 column sums out[C] of up to three bf16 [N, C] matrices (C % 8 == 0, 16-byte aligned rows);
+// part: colsum_bytes(N, the sum of their C), 4-byte aligned
+struct ColsumJob {
+  const uint16_t* a;
+  int64_t lda;
+  int C;
+  float* out;
+  float* part;               // set by launch_colsum
+  int nchunk;
+};
+struct ColsumJobs {
+  static constexpr int kMax = 3;
+  ColsumJob job[kMax];
+  int first[kMax], rfirst[kMax];   // first workgroup of each job in the two launches
+  int n, rows;
+  int64_t N;
+};
+size_t colsum_bytes(int64_t N, int64_t C);
+int launch_colsum(const ColsumJob* jobs, int n, int64_t N, float* part, hipStream_t st);
 int launch_rmsnorm_bwd(const uint16_t* x, const uint16_t* dy, int64_t N, int d, const float* scale, float eps,
                        uint16_t* dx, float* dscale, float* part, hipStream_t st);
 int launch_injection(const uint16_t* h, const uint16_t* e, const float* log_A, const float* log_dt, int64_t N,

@@ -266,27 +266,40 @@ at::Tensor block_ell_matmul_prepacked(const at::Tensor& x_, const at::Tensor& pa
   return y;
 }
 
-// backward of block_ell_matmul (bias gradient excluded): (dx, d_values)
-std::tuple<at::Tensor, at::Tensor> block_ell_matmul_bwd(const at::Tensor& dy_, const at::Tensor& x_,
-                                                        const at::Tensor& v_, const at::Tensor& c_) {
-  const char* op = "block_ell_matmul_bwd";
-  at::Tensor v = v_, c = c_;
+// backward of block_ell_matmul: dx, d_values and, when asked for, the fp32 bias gradient
+std::vector<at::Tensor> matmul_bwd_impl(const at::Tensor& dy_, const at::Tensor& x_, at::Tensor v, at::Tensor c,
+                                        bool want_bias, const char* op) {
   at::Tensor x = check_x2d(x_, op);
   const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
   lbk_bell w = make_bell(v, c, op, "weight");
-  TORCH_CHECK(x.size(1) % w.B == 0, "titan::block_ell_matmul_bwd: in_features ", x.size(1),
-              " not a multiple of B=", w.B);
+  TORCH_CHECK(x.size(1) % w.B == 0, "titan::", op, ": in_features ", x.size(1), " not a multiple of B=", w.B);
   const int64_t N = x.size(0), out_f = (int64_t)w.R * w.B;
   at::Tensor dy = check_x2d(dy_, op);
-  TORCH_CHECK(dy.size(0) == N && dy.size(1) == out_f, "titan::block_ell_matmul_bwd: grad_out must be [", N, ", ",
-              out_f, "], got ", dy.sizes());
+  TORCH_CHECK(dy.size(0) == N && dy.size(1) == out_f, "titan::", op, ": grad_out must be [", N, ", ", out_f,
+              "], got ", dy.sizes());
   at::Tensor dx = at::empty({N, x.size(1)}, x.options());
   at::Tensor dv = at::empty_like(v);
-  const size_t wsb = lbk_block_ell_matmul_bwd_workspace_bytes(N, (int32_t)x.size(1), &w);
+  at::Tensor db = want_bias ? at::empty({out_f}, x.options().dtype(at::kFloat)) : at::Tensor();
+  const size_t wsb = want_bias ? lbk_block_ell_matmul_bwd_bias_workspace_bytes(N, (int32_t)x.size(1), &w)
+                               : lbk_block_ell_matmul_bwd_workspace_bytes(N, (int32_t)x.size(1), &w);
   at::Tensor ws = workspace(wsb, x);
-  LBK_CALL("block_ell_matmul_bwd", lbk_block_ell_matmul_bwd_bf16(bf(dy), bf(x), N, (int32_t)x.size(1), &w, bfm(dx),
-                                                                 bfm(dv), ws.data_ptr(), wsb, cur_stream(x)));
-  return {dx, dv};
+  LBK_CALL("block_ell_matmul_bwd",
+           lbk_block_ell_matmul_bwd_bias_bf16(bf(dy), bf(x), N, (int32_t)x.size(1), &w, bfm(dx), bfm(dv),
+                                              want_bias ? db.data_ptr<float>() : nullptr, ws.data_ptr(), wsb,
+                                              cur_stream(x)));
+  return {dx, dv, db};
+}
+
+std::tuple<at::Tensor, at::Tensor> block_ell_matmul_bwd(const at::Tensor& dy, const at::Tensor& x,
+                                                        const at::Tensor& v, const at::Tensor& c) {
+  auto r = matmul_bwd_impl(dy, x, v, c, false, "block_ell_matmul_bwd");
+  return {r[0], r[1]};
+}
+
+std::tuple<at::Tensor, at::Tensor, at::Tensor> block_ell_matmul_bwd_bias(const at::Tensor& dy, const at::Tensor& x,
+                                                                         const at::Tensor& v, const at::Tensor& c) {
+  auto r = matmul_bwd_impl(dy, x, v, c, true, "block_ell_matmul_bwd_bias");
+  return {r[0], r[1], r[2]};
 }
 
 // ------------------------------------------------------------------ norm / loop
@@ -829,6 +842,8 @@ TORCH_LIBRARY(titan, m) {
   // ops beyond the reference's set
   m.def("block_ell_matmul(Tensor x, Tensor values, Tensor col_indices, Tensor? bias=None) -> Tensor");
   m.def("block_ell_matmul_bwd(Tensor grad_out, Tensor x, Tensor values, Tensor col_indices) -> (Tensor, Tensor)");
+  m.def("block_ell_matmul_bwd_bias(Tensor grad_out, Tensor x, Tensor values, Tensor col_indices) "
+        "-> (Tensor, Tensor, Tensor)");
   m.def("block_ell_matmul_prepack(Tensor values, Tensor col_indices, int in_features) -> Tensor");
   m.def("block_ell_matmul_prepacked(Tensor x, Tensor packed, Tensor values, Tensor col_indices, Tensor? bias=None) "
         "-> Tensor");
@@ -900,6 +915,7 @@ TORCH_LIBRARY_IMPL(titan, CUDA, m) {
   m.impl("persistent_mlp_step", &persistent_mlp_step);
   m.impl("block_ell_matmul", &block_ell_matmul);
   m.impl("block_ell_matmul_bwd", &block_ell_matmul_bwd);
+  m.impl("block_ell_matmul_bwd_bias", &block_ell_matmul_bwd_bias);
   m.impl("block_ell_matmul_prepack", &block_ell_matmul_prepack);
   m.impl("block_ell_matmul_prepacked", &block_ell_matmul_prepacked);
   m.impl("looped_swiglu", &looped_swiglu);
@@ -931,7 +947,8 @@ TORCH_LIBRARY_IMPL(titan, CompositeExplicitAutograd, m) { m.impl("unpin_weights_
 TORCH_LIBRARY_IMPL(titan, Autograd, m) {
   for (const char* name :
        {"block_ell_swiglu_fwd", "block_ell_swiglu_fwd_with_intermediate", "block_ell_swiglu_bwd",
-        "persistent_mlp_step", "block_ell_matmul", "block_ell_matmul_bwd", "block_ell_swiglu_bwd_ex",
+        "persistent_mlp_step", "block_ell_matmul", "block_ell_matmul_bwd", "block_ell_matmul_bwd_bias",
+        "block_ell_swiglu_bwd_ex",
         "block_ell_matmul_prepack", "block_ell_matmul_prepacked",
         "looped_swiglu", "looped_swiglu_persistent", "looped_swiglu_launches", "looped_core", "rmsnorm",
         "rmsnorm_bwd",
@@ -1010,6 +1027,11 @@ TORCH_LIBRARY_IMPL(titan, Meta, m) {
   });
   m.impl("block_ell_matmul_bwd", [](const at::Tensor&, const at::Tensor& x, const at::Tensor& v, const at::Tensor&) {
     return std::make_tuple(at::empty_like(x), at::empty_like(v));
+  });
+  m.impl("block_ell_matmul_bwd_bias", [](const at::Tensor&, const at::Tensor& x, const at::Tensor& v,
+                                         const at::Tensor&) {
+    return std::make_tuple(at::empty_like(x), at::empty_like(v),
+                           at::empty({v.size(0) * v.size(2)}, x.options().dtype(at::kFloat)));
   });
   m.impl("looped_swiglu", [](const at::Tensor& h, const at::Tensor&, const at::Tensor&, const at::Tensor&,
                              const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&, int64_t,

@@ -59,8 +59,8 @@ def block_ell_matmul_bwd(grad_out, x, values, col_indices):
 
 class _BlockELLMatmulFunction(torch.autograd.Function):
     """Differentiable Block-ELL product: the backward is ``titan::block_ell_matmul_bwd`` (dx and
-    the tile gradients) plus the bias gradient (the column sums of grad_out); the column
-    indices get no gradient."""
+    the tile gradients), or ``..._bwd_bias`` with the bias gradient (the column sums of
+    grad_out); the column indices get no gradient."""
 
     @staticmethod
     def forward(ctx, x2, values, col_indices, bias):
@@ -74,9 +74,11 @@ class _BlockELLMatmulFunction(torch.autograd.Function):
     def backward(ctx, gy):
         x2, values, col_indices = ctx.saved_tensors
         dy = gy.to(torch.bfloat16).contiguous()
+        if ctx.has_bias and ctx.needs_input_grad[3]:
+            dx, dv, db = ops().block_ell_matmul_bwd_bias(dy, x2, values, col_indices)
+            return dx, dv, None, db.to(ctx.bias_dtype)
         dx, dv = ops().block_ell_matmul_bwd(dy, x2, values, col_indices)
-        db = gy.float().sum(0).to(ctx.bias_dtype) if ctx.has_bias and ctx.needs_input_grad[3] else None
-        return dx, dv, None, db
+        return dx, dv, None, None
 
 
 def block_ell_matmul(x: torch.Tensor, values: torch.Tensor, col_indices: torch.Tensor,
