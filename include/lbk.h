@@ -286,7 +286,7 @@ int lbk_rmsnorm_bf16(const uint16_t* x, int64_t N, int32_t d, const float* scale
  * Backward of lbk_rmsnorm_bf16 for an output gradient dy [N, d] (bf16):
  *   dx     [N, d] bf16 = rs * scale * dy - x * rs^3 * mean(scale * dy * x)
  *   dscale [d] fp32    = sum over rows of dy * x * rs,   rs = 1 / sqrt(mean(x^2) + eps)
- * fp32 arithmetic; dscale is summed per 64-row group into the workspace
+ * fp32 arithmetic; dscale is summed per row group into the workspace
  * (lbk_rmsnorm_bwd_workspace_bytes) and the groups in a fixed order: deterministic.
  * The reference differentiates its Flax RMSNorm with JAX autodiff
  * (looped_blockell/layers/norms.py:8-15).

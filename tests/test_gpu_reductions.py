@@ -69,3 +69,55 @@ def test_swiglu_bias_gradients_three_sums(gpu, case):
                               (d[0].astype(np.float64), d[1]))
     for got, want, tol in zip(db, ref, (1e-2, 1e-2, 1e-5)):   # dg, du are summed from bf16; dy is exact
         assert T.rel_err(T.to_np(got), want)[0] <= tol
+
+
+# row widths of the register form (one lane group, two, four; a part of the last) and of the general
+# form (no multiple of 8, wider than 2048, rows off 16-byte alignment)
+@pytest.mark.parametrize("d", [8, 96, 512, 520, 1024, 2040, 2048, 2056, 513])
+@pytest.mark.parametrize("N", [1, 5, 8, 9, 2049, 16385])
+def test_rmsnorm_forward_backward_widths(gpu, N, d):
+    from looped_blockell import kernels
+    if N * d > 2 ** 23:
+        N = 4100
+    rng = np.random.default_rng(N + d)
+    x, dy = T.to_gpu_bf16(T.act(rng, N, d)), T.to_gpu_bf16(T.act(rng, N, d))
+    s = T.to_gpu((1 + 0.2 * rng.standard_normal(d)).astype(np.float32))
+    xd, gd, sd = x.double(), dy.double(), s.double()
+    rs = 1 / torch.sqrt(xd.pow(2).mean(-1, keepdim=True) + 1e-5)
+    # bf16 results: half an ulp, 2^-9 of the value, plus the fp32 arithmetic before the rounding
+    y = kernels.rmsnorm(x, s)
+    ref = xd * rs * sd
+    assert ((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5).all()
+    dx, ds = kernels.rmsnorm_bwd(dy, x, s, 1e-5)
+    t1, t2 = rs * sd * gd, xd * rs.pow(3) * (sd * gd * xd).mean(-1, keepdim=True)
+    assert ((dx.double() - (t1 - t2)).abs() <= 2.0 ** -8 * (t1 - t2).abs() + 1e-5 * (1 + t1.abs() + t2.abs())).all()
+    terms = gd * xd * rs
+    # each term carries about 8 roundings of its own beside those of the sum
+    assert ((ds.double() - terms.sum(0)).abs() <= (_sum_tol(N) + (d / 64 + 16) * 2.0 ** -24) * terms.abs().sum(0) + 1e-30).all()
+
+
+def test_rmsnorm_backward_unaligned_rows(gpu):
+    """Rows that start off 16-byte alignment take the general form and give the same result."""
+    from looped_blockell import abi as A
+    rng = np.random.default_rng(3)
+    N, d = 70, 256
+    s = T.to_gpu((1 + 0.2 * rng.standard_normal(d)).astype(np.float32))
+    x, dy = T.to_gpu_bf16(T.act(rng, N, d)), T.to_gpu_bf16(T.act(rng, N, d))
+    lib = A.load()
+    wsb = lib.lbk_rmsnorm_bwd_workspace_bytes(N, d)
+    outs = []
+    for off in (0, 1):
+        bufs = []
+        for t in (x, dy, None):
+            b = torch.zeros(N * d + 8, dtype=torch.bfloat16, device="cuda")
+            v = b[off:off + N * d]
+            if t is not None:
+                v.copy_(t.reshape(-1))
+            bufs.append(v)
+        ds = torch.empty(d, dtype=torch.float32, device="cuda")
+        ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+        A.check(lib.lbk_rmsnorm_bwd_bf16(T.ptr(bufs[0]), T.ptr(bufs[1]), N, d, T.ptr(s), 1e-5, T.ptr(bufs[2]),
+                                         T.ptr(ds), T.ptr(ws), wsb, T.stream()), "rmsnorm_bwd")
+        outs.append((bufs[2].clone(), ds))
+    assert T.rel_err(T.to_np(outs[1][0]), T.to_np(outs[0][0]))[0] <= 2.0 ** -8
+    assert T.rel_err(T.to_np(outs[1][1]), T.to_np(outs[0][1]))[0] <= 1e-5
