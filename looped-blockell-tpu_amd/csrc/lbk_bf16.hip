@@ -570,6 +570,10 @@ static int launch_rowblock_t(const RowblockLaunch& a, hipStream_t st) {
 
 int launch_rowblock(int B, int mode, const RowblockLaunch& a, hipStream_t st) {
   if (a.N == 0 || a.R == 0) return 0;
+  if (B == 64) {
+    const int rc = launch_t64(mode, a, st);
+    if (rc != -2) return rc;
+  }
   if (a.R > 65535 || (a.N + 63) / 64 > 0x7fffffff) return -3;  // grid limits
 #define LBK_RB(BB)                                                         \
   if (B == BB) {                                                           \

@@ -23,6 +23,13 @@ struct RowblockLaunch {
   uint16_t* aux0; uint16_t* aux1; int64_t ldaux;    // MODE 1 optional pre-activations
 };
 
+// B = 64 products of more tokens than the decode kernels take (lbk_tile64.hip); -2: an operand's
+// alignment or stride does not fit (the row-block kernel takes those)
+struct T64Args : RowblockLaunch {
+  int tg;   // token groups of the XCDs (set by the launcher)
+};
+int launch_t64(int mode, const RowblockLaunch& a, hipStream_t st);
+
 // mode: 0 = product (+bias), 1 = gate/up with SiLU*mul, 2 = down (+residual)
 int launch_rowblock(int B, int mode, const RowblockLaunch& a, hipStream_t st);
 

@@ -1,0 +1,89 @@
+"""The B = 64 product kernels (more tokens than the decode kernels take) against float64 dense
+products: token blocks of 64, 128 and 256 with remainders, block rows that are and are not a
+multiple of 8, slot lists past one 64-entry window, dead slots, rows without a live slot."""
+
+import numpy as np
+import pytest
+import torch
+
+import lbk_testlib as T
+
+pytestmark = pytest.mark.gpu
+# bf16 results of fp32 sums: half an ulp (2^-9 of the value) and the sums' own rounding, with room
+# for the bf16 hidden state's rounding carried through the down product (2^-9 of a norm)
+REL = 6e-3
+
+
+def _dense(v, c, C):
+    """[R, K, B_in, B_out] tiles -> float64 dense [out, in]."""
+    R, K, B, _ = v.shape
+    w = torch.zeros(R, C, B, B, dtype=torch.float64, device=v.device)
+    for k in range(K):
+        col = c[:, k].long()
+        ok = (col >= 0) & (col < C)
+        w[torch.arange(R, device=v.device)[ok], col[ok]] += v[ok, k].double().transpose(-1, -2)
+    return w.permute(0, 2, 1, 3).reshape(R * B, C * B)
+
+
+def _weight(rng, R, C, K, dead=0.0, dead_row=None):
+    vals, col = T.bell_weight(rng, R, C, K, 64)
+    if dead:
+        col[rng.random(col.shape) < dead] = -1
+    if dead_row is not None:
+        col[dead_row] = -1
+    return T.gpu_weight((vals, col))
+
+
+def _close(got, want):
+    return (got.double() - want).norm() <= REL * want.norm() + 1e-12
+
+
+# (N, block rows, input blocks, slots): grids that take token blocks of 64, 128 and 256
+@pytest.mark.parametrize("N,R,C,K", [(1, 3, 2, 1), (64, 8, 4, 2), (65, 5, 6, 6), (127, 8, 3, 3), (700, 16, 80, 80),
+                                     (16385, 3, 4, 2), (8191, 8, 5, 3), (32770, 4, 2, 2)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_product(gpu, N, R, C, K, bias):
+    from looped_blockell import kernels
+    rng = np.random.default_rng(N + K)
+    v, c = _weight(rng, R, C, K, dead=0.2, dead_row=R - 1)
+    x = T.to_gpu_bf16(T.act(rng, N, C * 64))
+    b = T.to_gpu(rng.standard_normal(R * 64).astype(np.float32)) if bias else None
+    y = kernels.block_ell_matmul(x, v, c, b)
+    ref = x.double() @ _dense(v, c, C).T + (b.double() if bias else 0.0)
+    assert _close(y, ref)
+    rows = (y.double() - ref).abs().amax(0)            # a wrong column cannot hide in the norm
+    assert (rows <= 2.0 ** -7 * ref.abs().amax(0) + 1e-5).all()
+
+
+@pytest.mark.parametrize("N", [65, 130, 512, 4099])
+@pytest.mark.parametrize("geo", [(256, 896, 4, 7), (512, 2048, 3, 9), (576, 1024, 9, 16)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_swiglu_and_intermediates(gpu, N, geo, shared):
+    from looped_blockell import kernels
+    d, ff, K, Kd = geo
+    rng = np.random.default_rng(N + d)
+    g = _weight(rng, ff // 64, d // 64, K, dead=0.1, dead_row=1)
+    u = (g[0].flip(0).contiguous(), g[1]) if shared else _weight(rng, ff // 64, d // 64, K, dead=0.1, dead_row=2)
+    dn = _weight(rng, d // 64, ff // 64, Kd, dead=0.1)
+    bs = [T.to_gpu((0.1 * rng.standard_normal(n)).astype(np.float32)) for n in (ff, ff, d)]
+    x = T.to_gpu_bf16(T.act(rng, N, d))
+    wg, wu, wd = (_dense(*w, C) for w, C in ((g, d // 64), (u, d // 64), (dn, ff // 64)))
+    G, U = x.double() @ wg.T + bs[0].double(), x.double() @ wu.T + bs[1].double()
+    H = torch.nn.functional.silu(G) * U
+    out, h, gp, uo = kernels.ops().block_ell_swiglu_fwd_bias(x, *g, bs[0], *u, bs[1], *dn, bs[2], True, True)
+    for got, want in ((gp, G), (uo, U), (h, H), (out, H @ wd.T + bs[2].double() + x.double())):
+        assert _close(got, want)
+    plain = kernels.ops().block_ell_swiglu_fwd_bias(x, *g, bs[0], *u, bs[1], *dn, bs[2], True, False)[0]
+    assert torch.equal(plain, out)
+
+
+def test_unaligned_tiles_take_the_rowblock_kernel(gpu):
+    """Tiles 8 bytes off a 16-byte boundary: the same product from the general kernel."""
+    from looped_blockell import kernels
+    rng = np.random.default_rng(9)
+    v, c = _weight(rng, 4, 6, 3)
+    buf = torch.empty(v.numel() + 8, dtype=torch.bfloat16, device="cuda")
+    off = buf[4:4 + v.numel()].view(v.shape)
+    off.copy_(v)
+    x = T.to_gpu_bf16(T.act(rng, 200, 6 * 64))
+    assert _close(kernels.block_ell_matmul(x, off, c), x.double() @ _dense(v, c, 6).T)
