@@ -275,6 +275,28 @@ int lbk_swiglu_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t* x, const 
                              void* stream);
 
 /*
+ * The training pair for fp32 master tiles.  lbk_swiglu_fwd_train rounds v_* [R, K, B, B] (fp32,
+ * 16-byte aligned) to the bf16 copies vb_* that the backward reads (all tiles, dead slots too) and
+ * runs lbk_swiglu_fwd_bias_bf16 on them with all intermediates; gate/up/down give R, K, B and
+ * col_idx (their values are not read).  Workspace: lbk_swiglu_workspace_bytes with
+ * want_intermediates.  lbk_swiglu_bwd_train is lbk_swiglu_bwd_bias_bf16 with the tile gradients in
+ * fp32, as summed; its workspace is lbk_swiglu_bwd_bias_workspace_bytes, or
+ * lbk_swiglu_bwd_workspace_bytes when no bias gradient is asked for.
+ */
+int lbk_swiglu_fwd_train(const uint16_t* x, int64_t N, int32_t d_model, const lbk_bell* gate,
+                         const lbk_bell* up, const lbk_bell* down, const float* v_gate, const float* v_up,
+                         const float* v_down, uint16_t* vb_gate, uint16_t* vb_up, uint16_t* vb_down,
+                         const float* b_gate, const float* b_up, const float* b_down, int add_residual,
+                         uint16_t* out, uint16_t* h_out, uint16_t* gate_pre_out, uint16_t* up_out,
+                         void* workspace, size_t workspace_bytes, void* stream);
+int lbk_swiglu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint16_t* gate_pre_act,
+                         const uint16_t* up_output, const uint16_t* h, int64_t N, int32_t d_model,
+                         const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down, int add_residual,
+                         uint16_t* dx, float* d_gate_values, float* d_up_values, float* d_down_values,
+                         float* d_b_gate, float* d_b_up, float* d_b_down, void* workspace,
+                         size_t workspace_bytes, void* stream);
+
+/*
  * out = x / sqrt(mean(x^2) + eps) * scale, rows of length d (bf16 in/out, fp32 math).
  * Replaces rmsnorm_cuda (reference csrc/loop/persistent_core.cuh:76-92) with the
  * layer-API semantics of looped_blockell/layers/norms.py:14-15.

@@ -186,7 +186,7 @@ static int matmul_impl(const uint16_t* x, int64_t N, int32_t in_features, const 
     if (!a16(workspace)) return LBK_ERR_ALIGN;
     const int C_in = in_features / w->B;
     PackJob job{w->values, w->col_idx, (int64_t)w->R * w->K, C_in, static_cast<uint32_t*>(workspace), 0,
-                path == MM_LIN ? 1 : 0};
+                path == MM_LIN ? 1 : 0, nullptr, nullptr};
     if (launch_pack_bf16_multi(&job, 1, w->B, s) != 0) return LBK_ERR_LAUNCH;
     pk = workspace;
   }
@@ -226,7 +226,7 @@ int lbk_block_ell_matmul_prepack_bf16(int32_t in_features, const lbk_bell* w, vo
   if (!packed || packed_bytes < lbk_block_ell_matmul_prepacked_bytes(in_features, w)) return LBK_ERR_WORKSPACE;
   if (!a16(packed)) return LBK_ERR_ALIGN;
   PackJob job{w->values, w->col_idx, (int64_t)w->R * w->K, in_features / w->B, static_cast<uint32_t*>(packed), 0,
-              path == MM_LIN ? 1 : 0};
+              path == MM_LIN ? 1 : 0, nullptr, nullptr};
   return launch_pack_bf16_multi(&job, 1, w->B, S(stream)) == 0 ? LBK_OK : LBK_ERR_LAUNCH;
 }
 
@@ -255,8 +255,14 @@ static size_t packed_ffn_bytes(const lbk_bell* gate, const lbk_bell* up, const l
          align256(packed_bf16_bytes((int64_t)down->R * down->K, B));
 }
 
+// fp32 master tiles of gate, up and down and the buffers of their bf16 copies
+struct MasterFFN {
+  const float* v[3];
+  uint16_t* raw[3];
+};
+
 static int pack_ffn(const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down, char* ws, PackedFFN* out,
-                    hipStream_t st) {
+                    hipStream_t st, const MasterFFN* master = nullptr) {
   const int B = gate->B;
   char* p = ws;
   const lbk_bell* ws3[3] = {gate, up, down};
@@ -266,7 +272,8 @@ static int pack_ffn(const lbk_bell* gate, const lbk_bell* up, const lbk_bell* do
   for (int t = 0; t < 3; ++t) {
     const int64_t nt = (int64_t)ws3[t]->R * ws3[t]->K;
     *dst[t] = p;
-    jobs[t] = PackJob{ws3[t]->values, ws3[t]->col_idx, nt, cols[t], reinterpret_cast<uint32_t*>(p), 0, t < 2};
+    jobs[t] = PackJob{ws3[t]->values, ws3[t]->col_idx, nt, cols[t], reinterpret_cast<uint32_t*>(p), 0, t < 2,
+                      master ? master->v[t] : nullptr, master ? master->raw[t] : nullptr};
     p += align256(packed_bf16_bytes(nt, B));
   }
   out->bytes = (size_t)(p - ws);
@@ -335,7 +342,8 @@ int lbk_swiglu_fwd_bf16(const uint16_t* x, int64_t N, int32_t d_model, const lbk
 static int swiglu_fwd_impl(const uint16_t* x, int64_t N, int32_t d_model, const lbk_bell* gate, const lbk_bell* up,
                            const lbk_bell* down, const char* prepacked, size_t prepacked_bytes, Biases bs,
                            int add_residual, uint16_t* out, uint16_t* h_out, uint16_t* gate_pre_out,
-                           uint16_t* up_out, void* workspace, size_t workspace_bytes, hipStream_t s) {
+                           uint16_t* up_out, void* workspace, size_t workspace_bytes, hipStream_t s,
+                           const MasterFFN* master = nullptr) {
   int st;
   if ((st = check_bell(gate)) || (st = check_bell(up)) || (st = check_bell(down))) return st;
   int64_t d_ff = 0;
@@ -390,7 +398,7 @@ static int swiglu_fwd_impl(const uint16_t* x, int64_t N, int32_t d_model, const 
       pk.u = prepacked + align256(packed_bf16_bytes((int64_t)gate->R * gate->K, B));
       pk.d = static_cast<const char*>(pk.u) + align256(packed_bf16_bytes((int64_t)up->R * up->K, B));
       pk.bytes = pbytes;
-    } else if ((st = pack_ffn(gate, up, down, ws, &pk, s))) {
+    } else if ((st = pack_ffn(gate, up, down, ws, &pk, s, master))) {
       return st;
     }
     return swiglu_split(x, nullptr, nullptr, 0.f, N, d_model, gate, up, down, pk, add_residual ? x : nullptr,
@@ -398,6 +406,49 @@ static int swiglu_fwd_impl(const uint16_t* x, int64_t N, int32_t d_model, const 
   }
   return swiglu_general(x, N, d_model, gate, up, down, add_residual ? x : nullptr, out, h, gate_pre_out, up_out, s,
                         bs);
+}
+
+// a bf16 copy of fp32 tiles without a packed form (the geometries that read the raw tiles)
+static int cast_ffn(const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down, const MasterFFN& m,
+                    hipStream_t s) {
+  const lbk_bell* w3[3] = {gate, up, down};
+  PackJob jobs[3];
+  int n = 0;
+  for (int t = 0; t < 3; ++t) {
+    const int64_t nt = (int64_t)w3[t]->R * w3[t]->K;
+    if (nt > 0) jobs[n++] = PackJob{nullptr, w3[t]->col_idx, nt, 0, nullptr, 0, 0, m.v[t], m.raw[t]};
+  }
+  return n == 0 || launch_pack_bf16_multi(jobs, n, gate->B, s) == 0 ? LBK_OK : LBK_ERR_LAUNCH;
+}
+
+int lbk_swiglu_fwd_train(const uint16_t* x, int64_t N, int32_t d_model, const lbk_bell* gate, const lbk_bell* up,
+                         const lbk_bell* down, const float* v_gate, const float* v_up, const float* v_down,
+                         uint16_t* vb_gate, uint16_t* vb_up, uint16_t* vb_down, const float* b_gate,
+                         const float* b_up, const float* b_down, int add_residual, uint16_t* out, uint16_t* h_out,
+                         uint16_t* gate_pre_out, uint16_t* up_out, void* workspace, size_t workspace_bytes,
+                         void* stream) {
+  if (!gate || !up || !down) return LBK_ERR_NULL;
+  const MasterFFN m{{v_gate, v_up, v_down}, {vb_gate, vb_up, vb_down}};
+  lbk_bell w3[3] = {*gate, *up, *down};
+  int st;
+  for (int t = 0; t < 3; ++t) {
+    w3[t].values = m.raw[t];
+    if ((st = check_bell(&w3[t]))) return st;
+    if ((int64_t)w3[t].R * w3[t].K > 0) {
+      if (!m.v[t]) return LBK_ERR_NULL;
+      if (!a16(m.v[t]) || !a16(m.raw[t])) return LBK_ERR_ALIGN;
+    }
+  }
+  int64_t d_ff = 0;
+  if ((st = check_ffn(&w3[0], &w3[1], &w3[2], d_model, &d_ff))) return st;
+  if (N < 0) return LBK_ERR_ARG;
+  if (N > 0 && (!h_out || !gate_pre_out || !up_out)) return LBK_ERR_NULL;
+  // without a packed form (or without tokens) only the copies are written, before the products read them
+  if (N == 0 || !use_split(&w3[0], &w3[1], &w3[2], d_model)) {
+    if ((st = cast_ffn(&w3[0], &w3[1], &w3[2], m, S(stream)))) return st;
+  }
+  return swiglu_fwd_impl(x, N, d_model, &w3[0], &w3[1], &w3[2], nullptr, 0, Biases{b_gate, b_up, b_down}, add_residual,
+                         out, h_out, gate_pre_out, up_out, workspace, workspace_bytes, S(stream), &m);
 }
 
 int lbk_swiglu_fwd_bias_bf16(const uint16_t* x, int64_t N, int32_t d_model, const lbk_bell* gate,
@@ -1124,12 +1175,18 @@ int lbk_swiglu_bwd_bf16(const uint16_t* grad_out, const uint16_t* x, const uint1
                                   workspace, workspace_bytes, stream);
 }
 
-int lbk_swiglu_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t* x, const uint16_t* gate_pre_act,
-                             const uint16_t* up_output, const uint16_t* h, int64_t N, int32_t d_model,
-                             const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down, int add_residual,
-                             uint16_t* dx, uint16_t* d_gate_values, uint16_t* d_up_values,
-                             uint16_t* d_down_values, float* d_b_gate, float* d_b_up, float* d_b_down,
-                             void* workspace, size_t workspace_bytes, void* stream) {
+// outputs of the backward: tile gradients in bf16 (dv) or fp32 (dv32), for gate, up and down
+struct BwdGrads {
+  uint16_t* dv[3];
+  float* dv32[3];
+  const void* any(int t) const { return dv32[t] ? static_cast<const void*>(dv32[t]) : dv[t]; }
+};
+
+static int swiglu_bwd_impl(const uint16_t* grad_out, const uint16_t* x, const uint16_t* gate_pre_act,
+                           const uint16_t* up_output, const uint16_t* h, int64_t N, int32_t d_model,
+                           const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down, int add_residual,
+                           uint16_t* dx, const BwdGrads& dw, float* d_b_gate, float* d_b_up, float* d_b_down,
+                           void* workspace, size_t workspace_bytes, void* stream) {
   const bool want_db = d_b_gate || d_b_up || d_b_down;
   int st;
   if ((st = check_bell(gate)) || (st = check_bell(up)) || (st = check_bell(down))) return st;
@@ -1138,9 +1195,9 @@ int lbk_swiglu_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t* x, const 
   if (N < 0) return LBK_ERR_ARG;
   const int B = gate->B;
   const int64_t tg = (int64_t)gate->R * gate->K, tu = (int64_t)up->R * up->K, td = (int64_t)down->R * down->K;
-  if ((tg && !d_gate_values) || (tu && !d_up_values) || (td && !d_down_values)) return LBK_ERR_NULL;
-  for (const void* p : {(const void*)d_gate_values, (const void*)d_up_values, (const void*)d_down_values})
-    if (p && !a16(p)) return LBK_ERR_ALIGN;
+  if ((tg && !dw.any(0)) || (tu && !dw.any(1)) || (td && !dw.any(2))) return LBK_ERR_NULL;
+  for (int t = 0; t < 3; ++t)
+    if (dw.any(t) && !a16(dw.any(t))) return LBK_ERR_ALIGN;
   if (N > 0) {
     if (!grad_out || !x || !gate_pre_act || !up_output || !h || !dx) return LBK_ERR_NULL;
     for (const void* p : {(const void*)grad_out, (const void*)x, (const void*)gate_pre_act, (const void*)up_output,
@@ -1201,17 +1258,17 @@ int lbk_swiglu_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t* x, const 
   int nj = 0;
   size_t poff = 0;
   auto add = [&](const uint16_t* xx, int64_t ldx, const uint16_t* gy, int64_t ldg, const lbk_bell* w, int C,
-                 uint16_t* out, const TListJob* tl) {
+                 int t, const TListJob* tl) {
     const int64_t nt = (int64_t)w->R * w->K;
     if (nt == 0) return;
-    dj[nj++] = DWJob{xx, ldx, gy, ldg, w->col_idx, w->R, w->K, C, part + poff, out, tl ? tl->cnt : nullptr,
-                     tl ? tl->list : nullptr, 0, 0};
+    dj[nj++] = DWJob{xx, ldx, gy, ldg, w->col_idx, w->R, w->K, C, part + poff, dw.dv[t], dw.dv32[t],
+                     tl ? tl->cnt : nullptr, tl ? tl->list : nullptr, 0, 0};
     poff += dw_part_floats(N, w, C, ldg);
   };
-  add(x, d_model, dg, d_ff, gate, C_in, d_gate_values, nullptr);
-  add(x, d_model, du, d_ff, up, C_in, d_up_values, nullptr);
+  add(x, d_model, dg, d_ff, gate, C_in, 0, nullptr);
+  add(x, d_model, du, d_ff, up, C_in, 1, nullptr);
   // the down weight's transposed lists (built above when N > 0) serve its tile gradients too
-  add(h, d_ff, grad_out, d_model, down, C_d, d_down_values, N > 0 ? &lj[0] : nullptr);
+  add(h, d_ff, grad_out, d_model, down, C_d, 2, N > 0 ? &lj[0] : nullptr);
   if (nj && launch_dw(B, dj, nj, N, s)) return LBK_ERR_LAUNCH;
   // bias gradients: column sums of dg, du and grad_out (the partials after the tile partials)
   if (want_db) {
@@ -1224,6 +1281,28 @@ int lbk_swiglu_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t* x, const 
     if (launch_colsum(cj, nc, N, cpart, s)) return LBK_ERR_LAUNCH;
   }
   return LBK_OK;
+}
+
+int lbk_swiglu_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t* x, const uint16_t* gate_pre_act,
+                             const uint16_t* up_output, const uint16_t* h, int64_t N, int32_t d_model,
+                             const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down, int add_residual,
+                             uint16_t* dx, uint16_t* d_gate_values, uint16_t* d_up_values,
+                             uint16_t* d_down_values, float* d_b_gate, float* d_b_up, float* d_b_down,
+                             void* workspace, size_t workspace_bytes, void* stream) {
+  return swiglu_bwd_impl(grad_out, x, gate_pre_act, up_output, h, N, d_model, gate, up, down, add_residual, dx,
+                         BwdGrads{{d_gate_values, d_up_values, d_down_values}, {}}, d_b_gate, d_b_up, d_b_down,
+                         workspace, workspace_bytes, stream);
+}
+
+int lbk_swiglu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint16_t* gate_pre_act,
+                         const uint16_t* up_output, const uint16_t* h, int64_t N, int32_t d_model,
+                         const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down, int add_residual,
+                         uint16_t* dx, float* d_gate_values, float* d_up_values, float* d_down_values,
+                         float* d_b_gate, float* d_b_up, float* d_b_down, void* workspace, size_t workspace_bytes,
+                         void* stream) {
+  return swiglu_bwd_impl(grad_out, x, gate_pre_act, up_output, h, N, d_model, gate, up, down, add_residual, dx,
+                         BwdGrads{{}, {d_gate_values, d_up_values, d_down_values}}, d_b_gate, d_b_up, d_b_down,
+                         workspace, workspace_bytes, stream);
 }
 
 size_t lbk_block_ell_matmul_bwd_workspace_bytes(int64_t N, int32_t in_features, const lbk_bell* w) {
@@ -1290,7 +1369,7 @@ int lbk_block_ell_matmul_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t*
   if (d_values && nt > 0) {
     // the transposed lists exist when dx was computed above
     const bool lists = dx && N > 0;
-    DWJob dj{x, in_features, grad_out, out_f, w->col_idx, w->R, w->K, C, part, d_values,
+    DWJob dj{x, in_features, grad_out, out_f, w->col_idx, w->R, w->K, C, part, d_values, nullptr,
              lists ? lj.cnt : nullptr, lists ? lj.list : nullptr, 0, 0};
     if (launch_dw(B, &dj, 1, N, s)) return LBK_ERR_LAUNCH;
   }

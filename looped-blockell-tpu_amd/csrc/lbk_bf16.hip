@@ -683,7 +683,10 @@ __global__ __launch_bounds__(256) void pack_bf16_kernel(const uint16_t* __restri
 // several weights in one launch, one wave per tile (the R*K tiles of weight t and its zero
 // tile are workgroups [first[t], first[t + 1])): the raw tile is read with 16-byte loads into
 // LDS, then each lane gathers its fragment dwords from there and writes them as 16-byte chunks
-// (chunk index (ks, m) is 64 consecutive u32x4 across the wave)
+// (chunk index (ks, m) is 64 consecutive u32x4 across the wave).  With fp32 master tiles (training:
+// the weights change every step) the same pass rounds them and writes the bf16 copy, where a cast
+// of each weight and then the pack read and wrote the tiles twice in four launches (three weights
+// [128, 8, 32, 32] and the down: 3 x 4.9 + 5.4 us, 7.8 us in one).
 template <int B>
 __global__ __launch_bounds__(64) void pack_bf16_multi_kernel(PackJobs jobs) {
   constexpr int CW = TileShape<B>::CW, NKS = TileShape<B>::NKS;
@@ -699,11 +702,24 @@ __global__ __launch_bounds__(64) void pack_bf16_multi_kernel(PackJobs jobs) {
   const int lane = threadIdx.x;
   u32x4* out = reinterpret_cast<u32x4*>(J.packed) + tile * U32X4;
   const int c0 = tile < J.ntiles ? J.col[tile] : -1;
-  if (c0 < 0 || c0 >= J.C) {                         // dead slot or the appended zero tile
+  const bool dead = c0 < 0 || c0 >= J.C;             // dead slot or the appended zero tile
+  if (J.src32 && tile < J.ntiles) {
+    const f32x4* src = reinterpret_cast<const f32x4*>(J.src32 + tile * B * B);
+    u32x4* raw = reinterpret_cast<u32x4*>(J.raw + tile * B * B);
+    for (int q = lane; q < RAW; q += 64) {
+      const f32x4 a = src[2 * q], b = src[2 * q + 1];
+      const u32x4 v = {pack2_bf16(a[0], a[1]), pack2_bf16(a[2], a[3]), pack2_bf16(b[0], b[1]), pack2_bf16(b[2], b[3])};
+      raw[q] = v;
+      reinterpret_cast<u32x4*>(s)[q] = v;
+    }
+    if (!J.packed) return;
+  }
+  if (dead) {
     for (int q = lane; q < U32X4; q += 64) out[q] = u32x4{0, 0, 0, 0};
     return;
   }
-  if ((reinterpret_cast<uintptr_t>(J.values) & 15u) == 0) {
+  if (J.src32) {
+  } else if ((reinterpret_cast<uintptr_t>(J.values) & 15u) == 0) {
     const u32x4* src = reinterpret_cast<const u32x4*>(J.values + tile * B * B);
     for (int q = lane; q < RAW; q += 64) reinterpret_cast<u32x4*>(s)[q] = src[q];
   } else {                                           // 8-byte aligned values (the ABI's minimum)
@@ -747,7 +763,7 @@ int launch_pack_bf16_multi(const PackJob* jobs, int n, int B, hipStream_t st) {
     J.job[t] = jobs[t];
     J.job[t].ndw = (int64_t)(packed_bf16_bytes(jobs[t].ntiles, B) / 4);
     J.first[t] = blocks;
-    blocks += jobs[t].ntiles + 1;                    // one wave per tile, plus the zero tile
+    blocks += jobs[t].ntiles + (jobs[t].packed ? 1 : 0);   // one wave per tile, plus the zero tile
   }
   if (blocks == 0 || blocks > 0x7fffffff) return -2;
   const dim3 grid((unsigned)blocks);

@@ -1820,7 +1820,7 @@ __global__ __launch_bounds__(1024, 1) void dwt16_kernel(DWJobs jobs) {
   }
 }
 
-// dW[e] = sum over chunks of the partial tiles (fixed order), bf16; dead slots -> 0.  Four
+// dW[e] = sum over chunks of the partial tiles (fixed order), bf16 or fp32; dead slots -> 0.  Four
 // consecutive elements of one tile per thread (16-byte partial loads, four chunks in flight)
 __global__ __launch_bounds__(256) void dw_reduce_kernel(DWJobs jobs, int B) {
   int jt = 0;
@@ -1853,8 +1853,12 @@ __global__ __launch_bounds__(256) void dw_reduce_kernel(DWJobs jobs, int B) {
       for (int m = 0; m < 4; ++m) s[m] += v[m];
     }
   }
-  const float o[4] = {s[0], s[1], s[2], s[3]};
-  store_bf16<4>(J.dw + idx, o);
+  if (J.dw32) {
+    *reinterpret_cast<f32x4*>(J.dw32 + idx) = s;
+  } else {
+    const float o[4] = {s[0], s[1], s[2], s[3]};
+    store_bf16<4>(J.dw + idx, o);
+  }
 }
 
 // the transposed-list kernels: column blocks per workgroup, and whether a weight's shape fits

@@ -54,6 +54,9 @@ inline int set_lds_limit_once(const void* kern, int bytes, std::atomic<uint64_t>
 struct PackJob {
   const uint16_t* values; const int32_t* col; int64_t ntiles; int C; uint32_t* packed; int64_t ndw;
   int gu_layout;   // 1: column order of the gate/up kernel's swapped product (B = 32)
+  // optional fp32 master tiles [ntiles, B, B] (16-byte aligned), read in place of values: every
+  // tile's bf16 copy goes to raw, and from there to packed (null: no packed copy)
+  const float* src32; uint16_t* raw;
 };
 struct PackJobs {
   static constexpr int kMax = 3;
@@ -311,6 +314,7 @@ struct DWJob {
   const int32_t* col; int R, K, C;
   float* part;                       // [nchunk, R*K, B, B]
   uint16_t* dw;                      // [R, K, B, B] bf16
+  float* dw32;                       // the same in fp32, unrounded (one of the two)
   // optional transposed topology of launch_tlist (per column block c: tcnt[c] slots e at
   // tlist[c * R * K ..]); lets a weight with wide input rows and narrow output rows (the down
   // projection) stage its G rows whole and walk the slots of each input column block

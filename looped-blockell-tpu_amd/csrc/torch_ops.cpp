@@ -801,6 +801,95 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tenso
   return {dx, dvg, dvu, dvd, dbg, dbu, dbd};
 }
 
+// ------------------------------------------------------------------ training from fp32 master tiles
+// fp32 values [R,K,B,B] + col_idx [R,K] int32: the bell (its values are filled in by the caller)
+lbk_bell make_master(at::Tensor& v, at::Tensor& c, const char* op, const char* name) {
+  check_gpu(v, op, name);
+  check_gpu(c, op, name);
+  TORCH_CHECK(v.scalar_type() == at::kFloat, "titan::", op, ": ", name, " values must be fp32");
+  TORCH_CHECK(c.scalar_type() == at::kInt, "titan::", op, ": ", name, " col_indices must be int32");
+  TORCH_CHECK(v.dim() == 4 && v.size(2) == v.size(3), "titan::", op, ": ", name,
+              " values must be [R, K, B, B], got ", v.sizes());
+  TORCH_CHECK(c.dim() == 2 && c.size(0) == v.size(0) && c.size(1) == v.size(1), "titan::", op, ": ", name,
+              " col_indices must be [R, K] matching values, got ", c.sizes());
+  v = v.contiguous();
+  if (reinterpret_cast<uintptr_t>(v.data_ptr()) & 15u) v = v.clone();   // a view off 16-byte alignment
+  c = c.contiguous();
+  return lbk_bell{nullptr, c.data_ptr<int32_t>(), (int32_t)v.size(0), (int32_t)v.size(1), (int32_t)v.size(2)};
+}
+
+// (out, h, gate_pre_act, up_out, and the bf16 copies of the three weights that the backward reads)
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor> swiglu_fwd_train(
+    const at::Tensor& x_, const at::Tensor& vg_, const at::Tensor& cg_, const c10::optional<at::Tensor>& bg_,
+    const at::Tensor& vu_, const at::Tensor& cu_, const c10::optional<at::Tensor>& bu_, const at::Tensor& vd_,
+    const at::Tensor& cd_, const c10::optional<at::Tensor>& bd_, bool add_residual) {
+  const char* op = "block_ell_swiglu_fwd_train";
+  at::Tensor vg = vg_, cg = cg_, vu = vu_, cu = cu_, vd = vd_, cd = cd_;
+  at::Tensor x = check_x2d(x_, op);
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
+  lbk_bell g = make_master(vg, cg, op, "gate"), u = make_master(vu, cu, op, "up"),
+           d = make_master(vd, cd, op, "down");
+  const int64_t N = x.size(0), d_model = x.size(1);
+  TORCH_CHECK((int64_t)d.R * d.B == d_model, "titan::", op, ": values_down R_model=", d.R,
+              " inconsistent with d_model=", d_model);
+  TORCH_CHECK(g.R == u.R, "titan::", op, ": gate and up must have same R_ff");
+  const int64_t d_ff = (int64_t)g.R * g.B;
+  const at::Tensor bg = opt_bias(bg_, d_ff, x, op, "b_gate"), bu = opt_bias(bu_, d_ff, x, op, "b_up"),
+                   bd = opt_bias(bd_, d_model, x, op, "b_down");
+  at::Tensor out = at::empty({N, d_model}, x.options()), h = at::empty({N, d_ff}, x.options()),
+             gp = at::empty({N, d_ff}, x.options()), uo = at::empty({N, d_ff}, x.options());
+  at::Tensor wg = at::empty(vg.sizes(), x.options()), wu = at::empty(vu.sizes(), x.options()),
+             wd = at::empty(vd.sizes(), x.options());
+  g.values = bf(wg);
+  u.values = bf(wu);
+  d.values = bf(wd);
+  const size_t wsb = lbk_swiglu_workspace_bytes(N, (int32_t)d_model, &g, &u, &d, 1);
+  at::Tensor ws = wsb ? workspace(wsb, x) : at::Tensor();
+  LBK_CALL("block_ell_swiglu_fwd_train",
+           lbk_swiglu_fwd_train(bf(x), N, (int32_t)d_model, &g, &u, &d, vg.data_ptr<float>(), vu.data_ptr<float>(),
+                                vd.data_ptr<float>(), bfm(wg), bfm(wu), bfm(wd), fptr(bg), fptr(bu), fptr(bd),
+                                add_residual ? 1 : 0, bfm(out), bfm(h), bfm(gp), bfm(uo),
+                                wsb ? ws.data_ptr() : nullptr, wsb, cur_stream(x)));
+  return {out, h, gp, uo, wg, wu, wd};
+}
+
+// (dx, fp32 tile gradients of gate, up, down, fp32 bias gradients; the last three empty without biases)
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor> swiglu_bwd_train(
+    const at::Tensor& dy_, const at::Tensor& x_, const at::Tensor& gp_, const at::Tensor& uo_, const at::Tensor& h_,
+    const at::Tensor& wg_, const at::Tensor& cg_, const at::Tensor& wu_, const at::Tensor& cu_, const at::Tensor& wd_,
+    const at::Tensor& cd_, bool add_residual, bool biases) {
+  const char* op = "block_ell_swiglu_bwd_train";
+  at::Tensor vg = wg_, cg = cg_, vu = wu_, cu = cu_, vd = wd_, cd = cd_;
+  at::Tensor x = check_x2d(x_, op);
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
+  lbk_bell g = make_bell(vg, cg, op, "gate"), u = make_bell(vu, cu, op, "up"), d = make_bell(vd, cd, op, "down");
+  const int64_t N = x.size(0), d_model = x.size(1);
+  const int64_t d_ff = (int64_t)g.R * g.B;
+  auto act = [&](const at::Tensor& t, int64_t cols, const char* name) {
+    check_gpu(t, op, name);
+    TORCH_CHECK(t.scalar_type() == at::kBFloat16, "titan::", op, ": ", name, " must be bf16");
+    TORCH_CHECK(t.dim() == 2 && t.size(0) == N && t.size(1) == cols, "titan::", op, ": ", name, " must be [", N,
+                ", ", cols, "], got ", t.sizes());
+    return t.contiguous();
+  };
+  at::Tensor dy = act(dy_, d_model, "grad_out"), gp = act(gp_, d_ff, "gate_pre_act"),
+             uo = act(uo_, d_ff, "up_output"), h = act(h_, d_ff, "h");
+  const auto f32 = x.options().dtype(at::kFloat);
+  at::Tensor dx = at::empty({N, d_model}, x.options());
+  at::Tensor dvg = at::empty(vg.sizes(), f32), dvu = at::empty(vu.sizes(), f32), dvd = at::empty(vd.sizes(), f32);
+  at::Tensor dbg = at::empty({biases ? d_ff : 0}, f32), dbu = at::empty({biases ? d_ff : 0}, f32),
+             dbd = at::empty({biases ? d_model : 0}, f32);
+  auto fp = [&](at::Tensor& t) { return biases ? t.data_ptr<float>() : nullptr; };
+  const size_t wsb = biases ? lbk_swiglu_bwd_bias_workspace_bytes(N, (int32_t)d_model, &g, &u, &d)
+                            : lbk_swiglu_bwd_workspace_bytes(N, (int32_t)d_model, &g, &u, &d);
+  at::Tensor ws = workspace(wsb, x);
+  LBK_CALL("block_ell_swiglu_bwd_train",
+           lbk_swiglu_bwd_train(bf(dy), bf(x), bf(gp), bf(uo), bf(h), N, (int32_t)d_model, &g, &u, &d,
+                                add_residual ? 1 : 0, bfm(dx), dvg.data_ptr<float>(), dvu.data_ptr<float>(),
+                                dvd.data_ptr<float>(), fp(dbg), fp(dbu), fp(dbd), ws.data_ptr(), wsb, cur_stream(x)));
+  return {dx, dvg, dvu, dvd, dbg, dbu, dbd};
+}
+
 // the reference operator: dx always includes grad_out (the forward's residual)
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> swiglu_bwd(
     const at::Tensor& dy, const at::Tensor& x, const at::Tensor& gp, const at::Tensor& uo, const at::Tensor& h,
@@ -861,6 +950,13 @@ TORCH_LIBRARY(titan, m) {
   m.def("looped_swiglu_bias(Tensor h, Tensor norm_scale, Tensor v_gate, Tensor ci_gate, Tensor? b_gate, "
         "Tensor v_up, Tensor ci_up, Tensor? b_up, Tensor v_down, Tensor ci_down, Tensor? b_down, int L, "
         "float eps=1e-05) -> Tensor");
+  m.def("block_ell_swiglu_fwd_train(Tensor x, Tensor values_gate, Tensor col_indices_gate, Tensor? b_gate, "
+        "Tensor values_up, Tensor col_indices_up, Tensor? b_up, Tensor values_down, Tensor col_indices_down, "
+        "Tensor? b_down, bool add_residual) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
+  m.def("block_ell_swiglu_bwd_train(Tensor grad_out, Tensor x, Tensor gate_pre_act, Tensor up_out, Tensor h, "
+        "Tensor values_gate, Tensor col_indices_gate, Tensor values_up, Tensor col_indices_up, Tensor values_down, "
+        "Tensor col_indices_down, bool add_residual, bool biases) "
+        "-> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
   m.def("block_ell_swiglu_bwd_ex(Tensor grad_out, Tensor x, Tensor gate_pre_act, Tensor up_out, Tensor h, "
         "Tensor v_gate, Tensor ci_gate, Tensor v_up, Tensor ci_up, Tensor v_down, Tensor ci_down, "
         "bool add_residual) -> (Tensor, Tensor, Tensor, Tensor)");
@@ -916,6 +1012,8 @@ TORCH_LIBRARY_IMPL(titan, CUDA, m) {
   m.impl("block_ell_matmul", &block_ell_matmul);
   m.impl("block_ell_matmul_bwd", &block_ell_matmul_bwd);
   m.impl("block_ell_matmul_bwd_bias", &block_ell_matmul_bwd_bias);
+  m.impl("block_ell_swiglu_fwd_train", &swiglu_fwd_train);
+  m.impl("block_ell_swiglu_bwd_train", &swiglu_bwd_train);
   m.impl("block_ell_matmul_prepack", &block_ell_matmul_prepack);
   m.impl("block_ell_matmul_prepacked", &block_ell_matmul_prepacked);
   m.impl("looped_swiglu", &looped_swiglu);
@@ -948,6 +1046,7 @@ TORCH_LIBRARY_IMPL(titan, Autograd, m) {
   for (const char* name :
        {"block_ell_swiglu_fwd", "block_ell_swiglu_fwd_with_intermediate", "block_ell_swiglu_bwd",
         "persistent_mlp_step", "block_ell_matmul", "block_ell_matmul_bwd", "block_ell_matmul_bwd_bias",
+        "block_ell_swiglu_fwd_train", "block_ell_swiglu_bwd_train",
         "block_ell_swiglu_bwd_ex",
         "block_ell_matmul_prepack", "block_ell_matmul_prepacked",
         "looped_swiglu", "looped_swiglu_persistent", "looped_swiglu_launches", "looped_core", "rmsnorm",
@@ -1028,6 +1127,24 @@ TORCH_LIBRARY_IMPL(titan, Meta, m) {
   m.impl("block_ell_matmul_bwd", [](const at::Tensor&, const at::Tensor& x, const at::Tensor& v, const at::Tensor&) {
     return std::make_tuple(at::empty_like(x), at::empty_like(v));
   });
+  m.impl("block_ell_swiglu_fwd_train",
+         [](const at::Tensor& x, const at::Tensor& vg, const at::Tensor&, const c10::optional<at::Tensor>&,
+            const at::Tensor& vu, const at::Tensor&, const c10::optional<at::Tensor>&, const at::Tensor& vd,
+            const at::Tensor&, const c10::optional<at::Tensor>&, bool) {
+           auto act = [&]() { return at::empty({x.size(0), vg.size(0) * vg.size(2)}, x.options()); };
+           return std::make_tuple(at::empty_like(x), act(), act(), act(), at::empty(vg.sizes(), x.options()),
+                                  at::empty(vu.sizes(), x.options()), at::empty(vd.sizes(), x.options()));
+         });
+  m.impl("block_ell_swiglu_bwd_train",
+         [](const at::Tensor&, const at::Tensor& x, const at::Tensor&, const at::Tensor&, const at::Tensor&,
+            const at::Tensor& wg, const at::Tensor&, const at::Tensor& wu, const at::Tensor&, const at::Tensor& wd,
+            const at::Tensor&, bool, bool biases) {
+           const auto f = x.options().dtype(at::kFloat);
+           const int64_t d_ff = biases ? wg.size(0) * wg.size(2) : 0, d = biases ? x.size(1) : 0;
+           return std::make_tuple(at::empty_like(x), at::empty(wg.sizes(), f), at::empty(wu.sizes(), f),
+                                  at::empty(wd.sizes(), f), at::empty({d_ff}, f), at::empty({d_ff}, f),
+                                  at::empty({d}, f));
+         });
   m.impl("block_ell_matmul_bwd_bias", [](const at::Tensor&, const at::Tensor& x, const at::Tensor& v,
                                          const at::Tensor&) {
     return std::make_tuple(at::empty_like(x), at::empty_like(v),

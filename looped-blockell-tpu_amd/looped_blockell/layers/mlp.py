@@ -139,8 +139,8 @@ class MLPBlock(nn.Module):
             self.fc2 = BlockELLLinear(d_model, d_ff, **kw)
         self._frozen = None
 
-    def swiglu_weights(self):
-        """(v_gate, ci_gate, v_up, ci_up, v_down, ci_down) in kernel form.
+    def swiglu_columns(self):
+        """(ci_gate, ci_up, ci_down) in kernel form.
 
         When gate and up have the same topology (as initialised: both are seeded from the
         same hash, reference ``mlp.py:94``) the same index tensor is passed for both, which
@@ -150,10 +150,22 @@ class MLPBlock(nn.Module):
         key = (self.w_gate._eff_cache[0], self.w_up._eff_cache[0])   # (pointer, version) of both
         if getattr(self, "_shared_key", None) != key:
             self._shared_key, self._shared = key, bool(torch.equal(cg, cu))
-        if self._shared:
-            cu = cg
-        return (self.w_gate.kernel_values(), cg, self.w_up.kernel_values(), cu,
-                self.w_down.kernel_values(), self.w_down.effective_col_indices())
+        return cg, (cg if self._shared else cu), self.w_down.effective_col_indices()
+
+    def swiglu_weights(self):
+        """(v_gate, ci_gate, v_up, ci_up, v_down, ci_down) in kernel form."""
+        cg, cu, cd = self.swiglu_columns()
+        return (self.w_gate.kernel_values(), cg, self.w_up.kernel_values(), cu, self.w_down.kernel_values(), cd)
+
+    def _swiglu_grad(self, x2, bg, bu, bd):
+        """The differentiable forward: fp32 values go to the kernels as they are, rounded there."""
+        lins = (self.w_gate, self.w_up, self.w_down)
+        if all(lin.values.dtype == torch.float32 and type(lin).kernel_values is BlockELLLinear.kernel_values
+               for lin in lins):
+            cg, cu, cd = self.swiglu_columns()
+            return kernels.swiglu_train(x2, self.w_gate.values, cg, self.w_up.values, cu, self.w_down.values, cd,
+                                        add_residual=False, b_gate=bg, b_up=bu, b_down=bd)
+        return kernels.swiglu(x2, *self.swiglu_weights(), add_residual=False, b_gate=bg, b_up=bu, b_down=bd)
 
     def _frozen_swiglu(self):
         """(kernel-form weights, packed copy), rebuilt when any weight's version changes."""
@@ -181,7 +193,7 @@ class MLPBlock(nn.Module):
             bg, bu, bd = self.swiglu_biases()
             grad = torch.is_grad_enabled() and (x2.requires_grad or any(p.requires_grad for p in self.parameters()))
             if grad:
-                out = kernels.swiglu(x2, *self.swiglu_weights(), add_residual=False, b_gate=bg, b_up=bu, b_down=bd)
+                out = self._swiglu_grad(x2, bg, bu, bd)
             else:
                 w, packed = self._frozen_swiglu()
                 out = kernels.swiglu_fwd_prepacked(x2, packed, *w, add_residual=False, b_gate=bg, b_up=bu, b_down=bd)

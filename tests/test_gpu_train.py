@@ -1,0 +1,77 @@
+"""The training operators on fp32 master tiles against the bf16 operators they fuse the casts of."""
+
+import numpy as np
+import pytest
+import torch
+
+import lbk_testlib as T
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(rng, d, ff, B, dens, dead):
+    ws = []
+    for w in T.ffn_weights(rng, d, ff, B, dens, sentinel_frac=dead):
+        v, c = T.gpu_weight(w)
+        ws += [v.float() + 1e-5 * torch.randn(v.shape, device="cuda"), c]     # not bf16 numbers
+    return ws
+
+
+# packed geometries (B = 16, 32), unpacked ones (B = 64, more than 2048 wide), one and several token chunks
+@pytest.mark.parametrize("case", [(256, 512, 16, 0.5, 1, 0.1), (256, 1024, 32, 0.25, 70, 0.2), (512, 1024, 64, 0.25, 100, 0.1),
+                                  (256, 512, 32, 0.5, 2100, 0.0), (128, 256, 64, 1.0, 2049, 0.3), (2080, 64, 32, 0.1, 5, 0.0),
+                                  (128, 256, 16, 1.0, 0, 0.0)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_train_operators_equal_cast_and_bf16_operators(gpu, case, bias):
+    from looped_blockell import kernels
+    d, ff, B, dens, N, dead = case
+    rng = np.random.default_rng(N + d + B)
+    vg, cg, vu, cu, vd, cd = _weights(rng, d, ff, B, dens, dead)
+    bs = [T.to_gpu((0.1 * rng.standard_normal(n)).astype(np.float32)) if bias else None for n in (ff, ff, d)]
+    x, dy = T.to_gpu_bf16(T.act(rng, N, d)), T.to_gpu_bf16(T.act(rng, N, d))
+    out, h, gp, uo, wg, wu, wd = kernels.ops().block_ell_swiglu_fwd_train(x, vg, cg, bs[0], vu, cu, bs[1], vd, cd, bs[2],
+                                                                          False)
+    for w, v in ((wg, vg), (wu, vu), (wd, vd)):
+        assert torch.equal(w, v.to(torch.bfloat16))
+    ref = kernels.ops().block_ell_swiglu_fwd_bias(x, wg, cg, bs[0], wu, cu, bs[1], wd, cd, bs[2], False, True)
+    assert all(torch.equal(a, b) for a, b in zip((out, h, gp, uo), ref))
+    got = kernels.ops().block_ell_swiglu_bwd_train(dy, x, gp, uo, h, wg, cg, wu, cu, wd, cd, False, bias)
+    want = kernels.ops().block_ell_swiglu_bwd_bias(dy, x, gp, uo, h, wg, cg, wu, cu, wd, cd, False)
+    assert torch.equal(got[0], want[0])
+    for a, b in zip(got[1:4], want[1:4]):
+        assert a.dtype == torch.float32 and torch.equal(a.to(torch.bfloat16), b)
+    if bias:
+        assert all(torch.equal(a, b) for a, b in zip(got[4:], want[4:]))
+
+
+def test_train_values_off_alignment(gpu):
+    """fp32 tiles 4 bytes off a 16-byte boundary (views of one flat buffer) give the same step."""
+    from looped_blockell import kernels
+    rng = np.random.default_rng(2)
+    vg, cg, vu, cu, vd, cd = _weights(rng, 128, 256, 32, 0.5, 0.1)
+    flat = torch.empty(vg.numel() + 1, device="cuda")
+    off = flat[1:].view(vg.shape)
+    off.copy_(vg)
+    x = T.to_gpu_bf16(T.act(rng, 40, 128))
+    a = kernels.ops().block_ell_swiglu_fwd_train(x, vg, cg, None, vu, cu, None, vd, cd, None, True)
+    b = kernels.ops().block_ell_swiglu_fwd_train(x, off, cg, None, vu, cu, None, vd, cd, None, True)
+    assert all(torch.equal(p, q) for p, q in zip(a, b))
+
+
+def test_layer_step_with_bf16_parameters(gpu):
+    """Parameters that are bf16 themselves keep the operators on bf16 tiles and get bf16 gradients."""
+    from looped_blockell.layers import MLPBlock
+    torch.manual_seed(0)
+    m = MLPBlock(128, 256, use_swiglu=True, tile_size=32, density=0.5, device="cuda")
+    ref = MLPBlock(128, 256, use_swiglu=True, tile_size=32, density=0.5, device="cuda")
+    m.load_state_dict(ref.state_dict())
+    for n in ("w_gate", "w_up", "w_down"):
+        getattr(m, n).values.data = getattr(ref, n).values.data.to(torch.bfloat16)
+    x = torch.randn(50, 128, device="cuda").to(torch.bfloat16)
+    y, yr = m(x), ref(x)
+    assert torch.equal(y, yr)
+    y.float().square().sum().backward()
+    yr.float().square().sum().backward()
+    for n in ("w_gate", "w_up", "w_down"):
+        a, b = getattr(m, n).values.grad, getattr(ref, n).values.grad
+        assert a.dtype == torch.bfloat16 and b.dtype == torch.float32 and torch.equal(a, b.to(torch.bfloat16))
