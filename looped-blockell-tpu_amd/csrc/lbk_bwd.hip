@@ -485,9 +485,8 @@ template <int B, int MT, int NW>
 static int launch_dh_panel_t(const TProdArgs& a0, hipStream_t st) {
   constexpr size_t lds = (size_t)16 * MT * (8192 / MT);
   auto kern = dh_panel_kernel<B, MT, NW>;
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)lds) != hipSuccess)
-    return -1;
+  static std::atomic<uint64_t> done{0};
+  if (set_lds_limit_once(reinterpret_cast<const void*>(kern), (int)lds, done)) return -1;
   TProdArgs a = a0;
   set_kdiv(a);
   const int64_t ntb = (a.N + 16 * MT - 1) / (16 * MT);
@@ -714,9 +713,8 @@ template <int B, int OPW, int NW>
 static int launch_dx_stage_t(const TProdArgs& a, hipStream_t st) {
   constexpr size_t lds = 2 * (size_t)64 * DxStage<B>::COLS * 2;
   auto kern = dx_stage_kernel<B, OPW, NW>;
-  if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-    return -1;
+  static std::atomic<uint64_t> done{0};
+  if (lds > 65536 && set_lds_limit_once(reinterpret_cast<const void*>(kern), (int)lds, done)) return -1;
   hipLaunchKernelGGL(kern, dim3((unsigned)((a.N + 63) / 64 * a.nsl)), dim3(64 * NW), lds, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -914,9 +912,8 @@ static int launch_dxf(const TProdArgs& a0, hipStream_t st) {
   a.nsl = (a.C + DXF_WAVES - 1) / DXF_WAVES;
   const int64_t grid = a.nsl == 1 ? ntb : 8 * a.nsl * ((ntb + 7) / 8);
   auto kern = dxf_kernel<B, DXF_RING>;
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)lds) != hipSuccess)
-    return -1;
+  static std::atomic<uint64_t> done{0};
+  if (set_lds_limit_once(reinterpret_cast<const void*>(kern), (int)lds, done)) return -1;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * DXF_WAVES), lds, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

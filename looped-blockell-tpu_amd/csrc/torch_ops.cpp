@@ -13,6 +13,7 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
 
 #include <vector>
@@ -92,6 +93,7 @@ at::Tensor opt_bias(const c10::optional<at::Tensor>& b, int64_t n, const at::Ten
   if (!b.has_value() || !b->defined()) return at::Tensor();
   check_gpu(*b, op, name);
   TORCH_CHECK(b->numel() == n, "titan::", op, ": ", name, " must have ", n, " elements, got ", b->numel());
+  if (b->scalar_type() == at::kFloat && b->device() == x.device() && b->is_contiguous()) return *b;
   return b->to(x.device(), at::kFloat).contiguous();
 }
 const float* fptr(const at::Tensor& t) { return t.defined() ? t.data_ptr<float>() : nullptr; }
@@ -890,6 +892,84 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tenso
   return {dx, dvg, dvu, dvd, dbg, dbu, dbd};
 }
 
+// The differentiable SwiGLU on fp32 tiles as one native autograd node: forward and backward each
+// one operator call, with no Python in the backward thread (a 128 x 256 step took 212 us of host
+// time as a torch.autograd.Function in Python).  The calls go through the dispatcher, so a
+// backward under create_graph records the operators' nodes, which raise when differentiated again.
+using at::Tensor;
+using OptTensor = c10::optional<at::Tensor>;
+using Seven = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor>;
+
+Seven call_fwd_train(const Tensor& x, const Tensor& vg, const Tensor& cg, const OptTensor& bg, const Tensor& vu,
+                     const Tensor& cu, const OptTensor& bu, const Tensor& vd, const Tensor& cd, const OptTensor& bd,
+                     bool add_residual) {
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("titan::block_ell_swiglu_fwd_train", "")
+                             .typed<decltype(swiglu_fwd_train)>();
+  return op.call(x, vg, cg, bg, vu, cu, bu, vd, cd, bd, add_residual);
+}
+
+Seven call_bwd_train(const Tensor& dy, const Tensor& x, const Tensor& gp, const Tensor& uo, const Tensor& h,
+                     const Tensor& wg, const Tensor& cg, const Tensor& wu, const Tensor& cu, const Tensor& wd,
+                     const Tensor& cd, bool add_residual, bool biases) {
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("titan::block_ell_swiglu_bwd_train", "")
+                             .typed<decltype(swiglu_bwd_train)>();
+  return op.call(dy, x, gp, uo, h, wg, cg, wu, cu, wd, cd, add_residual, biases);
+}
+
+struct SwigluTrain : public torch::autograd::Function<SwigluTrain> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& vg, const Tensor& cg,
+                        const OptTensor& bg, const Tensor& vu, const Tensor& cu, const OptTensor& bu,
+                        const Tensor& vd, const Tensor& cd, const OptTensor& bd, bool add_residual) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    auto [out, h, gp, uo, wg, wu, wd] = call_fwd_train(x, vg, cg, bg, vu, cu, bu, vd, cd, bd, add_residual);
+    ctx->save_for_backward({x, h, gp, uo, wg, cg, wu, cu, wd, cd});
+    // per bias: its dtype, or -1
+    auto dt = [](const OptTensor& b) {
+      return b.has_value() && b->defined() ? (int64_t)b->scalar_type() : (int64_t)-1;
+    };
+    ctx->saved_data["bias"] = std::vector<int64_t>{dt(bg), dt(bu), dt(bd)};
+    ctx->saved_data["res"] = add_residual;
+    return out;
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    torch::autograd::variable_list r(11);
+    if (!grads[0].defined()) return r;
+    const auto s = ctx->get_saved_variables();
+    const auto dt = ctx->saved_data["bias"].toIntVector();
+    const bool biases = dt[0] >= 0 || dt[1] >= 0 || dt[2] >= 0;
+    auto [dx, dvg, dvu, dvd, dbg, dbu, dbd] =
+        call_bwd_train(grads[0].to(at::kBFloat16).contiguous(), s[0], s[2], s[3], s[1], s[4], s[5], s[6], s[7], s[8],
+                       s[9], ctx->saved_data["res"].toBool(), biases);
+    auto bias = [&](const Tensor& d, int t) {
+      return dt[t] >= 0 ? d.to(static_cast<at::ScalarType>(dt[t])) : Tensor();
+    };
+    r[0] = dx;
+    r[1] = dvg;
+    r[3] = bias(dbg, 0);
+    r[4] = dvu;
+    r[6] = bias(dbu, 1);
+    r[7] = dvd;
+    r[9] = bias(dbd, 2);
+    return r;
+  }
+};
+
+Tensor swiglu_train(const Tensor& x, const Tensor& vg, const Tensor& cg, const OptTensor& bg, const Tensor& vu,
+                    const Tensor& cu, const OptTensor& bu, const Tensor& vd, const Tensor& cd, const OptTensor& bd,
+                    bool add_residual) {
+  return std::get<0>(call_fwd_train(x, vg, cg, bg, vu, cu, bu, vd, cd, bd, add_residual));
+}
+
+Tensor swiglu_train_autograd(const Tensor& x, const Tensor& vg, const Tensor& cg, const OptTensor& bg,
+                             const Tensor& vu, const Tensor& cu, const OptTensor& bu, const Tensor& vd,
+                             const Tensor& cd, const OptTensor& bd, bool add_residual) {
+  return SwigluTrain::apply(x, vg, cg, bg, vu, cu, bu, vd, cd, bd, add_residual);
+}
+
 // the reference operator: dx always includes grad_out (the forward's residual)
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> swiglu_bwd(
     const at::Tensor& dy, const at::Tensor& x, const at::Tensor& gp, const at::Tensor& uo, const at::Tensor& h,
@@ -953,6 +1033,9 @@ TORCH_LIBRARY(titan, m) {
   m.def("block_ell_swiglu_fwd_train(Tensor x, Tensor values_gate, Tensor col_indices_gate, Tensor? b_gate, "
         "Tensor values_up, Tensor col_indices_up, Tensor? b_up, Tensor values_down, Tensor col_indices_down, "
         "Tensor? b_down, bool add_residual) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
+  m.def("block_ell_swiglu_train(Tensor x, Tensor values_gate, Tensor col_indices_gate, Tensor? b_gate, "
+        "Tensor values_up, Tensor col_indices_up, Tensor? b_up, Tensor values_down, Tensor col_indices_down, "
+        "Tensor? b_down, bool add_residual) -> Tensor");
   m.def("block_ell_swiglu_bwd_train(Tensor grad_out, Tensor x, Tensor gate_pre_act, Tensor up_out, Tensor h, "
         "Tensor values_gate, Tensor col_indices_gate, Tensor values_up, Tensor col_indices_up, Tensor values_down, "
         "Tensor col_indices_down, bool add_residual, bool biases) "
@@ -1013,6 +1096,7 @@ TORCH_LIBRARY_IMPL(titan, CUDA, m) {
   m.impl("block_ell_matmul_bwd", &block_ell_matmul_bwd);
   m.impl("block_ell_matmul_bwd_bias", &block_ell_matmul_bwd_bias);
   m.impl("block_ell_swiglu_fwd_train", &swiglu_fwd_train);
+  m.impl("block_ell_swiglu_train", &swiglu_train);
   m.impl("block_ell_swiglu_bwd_train", &swiglu_bwd_train);
   m.impl("block_ell_matmul_prepack", &block_ell_matmul_prepack);
   m.impl("block_ell_matmul_prepacked", &block_ell_matmul_prepacked);
@@ -1038,11 +1122,12 @@ TORCH_LIBRARY_IMPL(titan, CUDA, m) {
 
 TORCH_LIBRARY_IMPL(titan, CompositeExplicitAutograd, m) { m.impl("unpin_weights_l2", &unpin_weights_l2); }
 
-// No operator here has an autograd formula of its own (the differentiable ones are wrapped by
-// torch.autograd.Function in looped_blockell.kernels, which call them with grad mode off).
+// block_ell_swiglu_train is differentiable; no other operator has an autograd formula of its own
+// (torch.autograd.Function in looped_blockell.kernels wraps them and calls them with grad mode off).
 // Outputs of an op called on inputs that require grad get a node that raises on backward,
 // instead of silently carrying no gradient.
 TORCH_LIBRARY_IMPL(titan, Autograd, m) {
+  m.impl("block_ell_swiglu_train", &swiglu_train_autograd);
   for (const char* name :
        {"block_ell_swiglu_fwd", "block_ell_swiglu_fwd_with_intermediate", "block_ell_swiglu_bwd",
         "persistent_mlp_step", "block_ell_matmul", "block_ell_matmul_bwd", "block_ell_matmul_bwd_bias",
@@ -1127,6 +1212,10 @@ TORCH_LIBRARY_IMPL(titan, Meta, m) {
   m.impl("block_ell_matmul_bwd", [](const at::Tensor&, const at::Tensor& x, const at::Tensor& v, const at::Tensor&) {
     return std::make_tuple(at::empty_like(x), at::empty_like(v));
   });
+  m.impl("block_ell_swiglu_train",
+         [](const at::Tensor& x, const at::Tensor&, const at::Tensor&, const c10::optional<at::Tensor>&,
+            const at::Tensor&, const at::Tensor&, const c10::optional<at::Tensor>&, const at::Tensor&,
+            const at::Tensor&, const c10::optional<at::Tensor>&, bool) { return at::empty_like(x); });
   m.impl("block_ell_swiglu_fwd_train",
          [](const at::Tensor& x, const at::Tensor& vg, const at::Tensor&, const c10::optional<at::Tensor>&,
             const at::Tensor& vu, const at::Tensor&, const c10::optional<at::Tensor>&, const at::Tensor& vd,

@@ -165,37 +165,16 @@ class _SwiGLUBiasFunction(torch.autograd.Function):
         return dx, dvg, None, db[0], dvu, None, db[1], dvd, None, db[2], None
 
 
-class _SwiGLUTrainFunction(torch.autograd.Function):
-    """Differentiable SwiGLU FFN on fp32 master tiles: ``titan::block_ell_swiglu_fwd_train`` rounds
-    and packs the three weights in one launch, ``..._bwd_train`` returns their gradients in fp32 as
-    summed; the column indices get no gradient."""
-
-    @staticmethod
-    def forward(ctx, x, v_gate, ci_gate, b_gate, v_up, ci_up, b_up, v_down, ci_down, b_down, add_residual):
-        out, h, gp, uo, wg, wu, wd = ops().block_ell_swiglu_fwd_train(x, v_gate, ci_gate, b_gate, v_up, ci_up, b_up,
-                                                                      v_down, ci_down, b_down, add_residual)
-        ctx.save_for_backward(x, h, gp, uo, wg, ci_gate, wu, ci_up, wd, ci_down)
-        ctx.add_residual = add_residual
-        ctx.bias_dtypes = tuple(b.dtype if b is not None else None for b in (b_gate, b_up, b_down))
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        x, h, gp, uo, wg, cg, wu, cu, wd, cd = ctx.saved_tensors
-        biased = any(t is not None for t in ctx.bias_dtypes)
-        dx, dvg, dvu, dvd, *db = ops().block_ell_swiglu_bwd_train(
-            grad_out.to(torch.bfloat16).contiguous(), x, gp, uo, h, wg, cg, wu, cu, wd, cd, ctx.add_residual, biased)
-        db = [d.to(t) if t is not None else None for d, t in zip(db, ctx.bias_dtypes)]
-        return dx, dvg, None, db[0], dvu, None, db[1], dvd, None, db[2], None
-
-
 def swiglu_train(x, v_gate, ci_gate, v_up, ci_up, v_down, ci_down, add_residual: bool = False,
                  b_gate=None, b_up=None, b_down=None):
-    """``swiglu`` for fp32 values when gradients are needed: their rounding to bf16 is part of the
-    operator, and their gradients come back in fp32."""
+    """``swiglu`` for fp32 values when gradients are needed: ``titan::block_ell_swiglu_train``, one
+    native autograd node.  The values' rounding to bf16 is part of the operator, and their
+    gradients come back in fp32."""
     _gpu(x, v_gate, v_down)
-    return _SwiGLUTrainFunction.apply(x, v_gate, ci_gate, b_gate, v_up, ci_up, b_up, v_down, ci_down, b_down,
-                                      add_residual)
+    if torch._C._are_functorch_transforms_active():
+        raise RuntimeError("the differentiable SwiGLU has no rules for functorch transforms")
+    return ops().block_ell_swiglu_train(x, v_gate, ci_gate, b_gate, v_up, ci_up, b_up, v_down, ci_down, b_down,
+                                        add_residual)
 
 
 def swiglu(x, v_gate, ci_gate, v_up, ci_up, v_down, ci_down, add_residual: bool = False,

@@ -37,6 +37,25 @@ from .. import kernels
 from .block_ell import BlockELLConfig, BlockELLTensor, create_random_topology
 
 
+def _tensors(lin):
+    """(values, col_indices, alive_mask) of a projection, without ``nn.Module``'s attribute lookup
+    (about 0.4 us a name, and a small forward reads nine)."""
+    try:
+        b = lin._buffers
+        return lin._parameters["values"], b["col_indices"], b["alive_mask"]
+    except KeyError:                                     # parametrized or replaced by plain attributes
+        return lin.values, lin.col_indices, lin.alive_mask
+
+
+def _versions(lins):
+    """Pointer and version of every value tensor, column-index buffer and alive mask of ``lins``."""
+    key = []
+    for lin in lins:
+        v, c, a = _tensors(lin)
+        key += (v.data_ptr(), v._version, c.data_ptr(), c._version, a.data_ptr(), a._version)
+    return key
+
+
 class BlockELLLinear(nn.Module):
     """Single Block-ELL linear layer (reference ``mlp.py:28-95``).
 
@@ -75,13 +94,13 @@ class BlockELLLinear(nn.Module):
 
     def effective_col_indices(self) -> torch.Tensor:
         """col_indices with dead tiles (alive_mask False) set to the -1 sentinel (cached per version)."""
-        key = (self.col_indices.data_ptr(), self.col_indices._version, self.alive_mask.data_ptr(),
-               self.alive_mask._version)
+        _, cols, alive = _tensors(self)
+        key = (cols.data_ptr(), cols._version, alive.data_ptr(), alive._version)
         if self._eff_cache is None or self._eff_cache[0] != key:
             # an ordinary tensor even when built under inference mode: a later forward with
             # gradients saves it for the backward
             with torch.inference_mode(False):
-                eff = torch.where(self.alive_mask, self.col_indices, torch.full_like(self.col_indices, -1))
+                eff = torch.where(alive, cols, torch.full_like(cols, -1))
                 self._eff_cache = (key, eff.to(torch.int32).contiguous())
         return self._eff_cache[1]
 
@@ -169,10 +188,7 @@ class MLPBlock(nn.Module):
 
     def _frozen_swiglu(self):
         """(kernel-form weights, packed copy), rebuilt when any weight's version changes."""
-        lins = (self.w_gate, self.w_up, self.w_down)
-        for lin in lins:
-            lin.effective_col_indices()                  # refreshes each topology key
-        key = tuple((lin.values.data_ptr(), lin.values._version, lin._eff_cache[0]) for lin in lins)
+        key = _versions((self.w_gate, self.w_up, self.w_down))
         if self._frozen is None or self._frozen[0] != key:
             w = self.swiglu_weights()
             self._frozen = (key, w, kernels.swiglu_prepack(*w))
@@ -187,7 +203,6 @@ class MLPBlock(nn.Module):
         return self.w_gate.bias, self.w_up.bias, self.w_down.bias
 
     def forward(self, x: torch.Tensor, deterministic: bool = True) -> torch.Tensor:
-        lead = x.shape[:-1]
         if self.use_swiglu:
             x2 = x.reshape(-1, self.d_model).to(torch.bfloat16).contiguous()
             bg, bu, bd = self.swiglu_biases()
@@ -197,7 +212,8 @@ class MLPBlock(nn.Module):
             else:
                 w, packed = self._frozen_swiglu()
                 out = kernels.swiglu_fwd_prepacked(x2, packed, *w, add_residual=False, b_gate=bg, b_up=bu, b_down=bd)
-            out = out.reshape(*lead, self.d_model)
+            if x.dim() != 2 or x.shape[1] != self.d_model:
+                out = out.reshape(*x.shape[:-1], self.d_model)
         else:
             out = self.fc2(F.gelu(self.fc1(x).float(), approximate="tanh").to(torch.bfloat16))
         if self.dropout > 0.0 and not deterministic:

@@ -75,3 +75,58 @@ def test_layer_step_with_bf16_parameters(gpu):
     for n in ("w_gate", "w_up", "w_down"):
         a, b = getattr(m, n).values.grad, getattr(ref, n).values.grad
         assert a.dtype == torch.bfloat16 and b.dtype == torch.float32 and torch.equal(a, b.to(torch.bfloat16))
+
+
+def test_train_node_hooks_double_backward_and_transforms(gpu):
+    """The native node keeps what a Python autograd function did: saved-tensor hooks see its saved
+    tensors, a second derivative and functorch transforms are refused, frozen tiles get no gradient."""
+    from looped_blockell.layers import MLPBlock
+    torch.manual_seed(1)
+    m = MLPBlock(64, 128, use_swiglu=True, tile_size=32, density=0.5, device="cuda")
+    x = torch.randn(3, 5, 64, device="cuda").to(torch.bfloat16).requires_grad_(True)
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (seen.append(t.shape), t)[1], lambda t: t):
+        y = m(x)
+    assert y.shape == x.shape and torch.Size([15, 128]) in seen and m.w_gate.values.shape in seen
+    y.float().sum().backward()
+    gx = x.grad.clone()
+    x.grad = None
+    m.w_up.values.requires_grad_(False)
+    m.w_up.values.grad = None
+    m(x).float().sum().backward()
+    assert torch.equal(x.grad, gx) and m.w_up.values.grad is None and m.w_gate.values.grad is not None
+    g, = torch.autograd.grad(m(x).float().sum(), x, create_graph=True)
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(g.float().sum(), m.w_down.values)
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda t: m(t).float().sum())(x.detach())
+    with torch.autograd.forward_ad.dual_level():
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            m(torch.autograd.forward_ad.make_dual(x.detach(), torch.ones_like(x)))
+
+
+def test_frozen_weights_follow_replacement(gpu):
+    """Gradient-free forwards notice in-place writes, replaced parameters and replaced topologies."""
+    from looped_blockell.layers import MLPBlock
+    torch.manual_seed(2)
+    m = MLPBlock(64, 128, use_swiglu=True, tile_size=32, density=0.5, device="cuda")
+    x = torch.randn(70, 64, device="cuda").to(torch.bfloat16)
+
+    def fresh():
+        n = MLPBlock(64, 128, use_swiglu=True, tile_size=32, density=0.5, device="cuda")
+        n.load_state_dict(m.state_dict())
+        with torch.no_grad():
+            return n(x)
+
+    with torch.no_grad():
+        first = m(x)
+        m.w_gate.values.mul_(2)
+        assert torch.equal(m(x), fresh()) and not torch.equal(m(x), first)
+        m.w_down.values = torch.nn.Parameter(torch.randn_like(m.w_down.values) * 0.02)
+        assert torch.equal(m(x), fresh())
+        m.w_up.alive_mask[0, 0] = False
+        assert torch.equal(m(x), fresh())
+        m.w_up.col_indices = m.w_up.col_indices.flip(0).contiguous()
+        assert torch.equal(m(x), fresh())
+    with pytest.raises(RuntimeError):
+        m(torch.zeros(4, 128, device="cuda", dtype=torch.bfloat16))
