@@ -598,6 +598,33 @@ int lbk_block_ell_matmul_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t*
                                        uint16_t* d_values, float* d_bias, void* workspace,
                                        size_t workspace_bytes, void* stream);
 
+/*
+ * The GELU FFN out = W2 gelu(W1 x + b1) + b2 (tanh form; reference looped_blockell/layers/mlp.py:156),
+ * w1 [d_ff, d_model], w2 [d_model, d_ff], biases fp32 and optional.
+ *   prepacked   the two weights' lbk_block_ell_matmul_prepack_bf16 copies (NULL where a weight has none)
+ *   train       rounds the fp32 tiles v1, v2 to the copies vb1, vb2 (16-byte aligned), as
+ *               lbk_swiglu_fwd_train does, and exports h and the pre-activation
+ *   bwd_train   dx, fp32 tile gradients and (each optional) fp32 bias gradients
+ * Workspaces: lbk_gelu_workspace_bytes(..., prepacked, want_h) with (1, 0) and (0, 1) for the two
+ * forwards, lbk_gelu_bwd_workspace_bytes for the backward.
+ */
+size_t lbk_gelu_workspace_bytes(int64_t N, int32_t d_model, const lbk_bell* w1, const lbk_bell* w2,
+                                int prepacked, int want_h);
+int lbk_gelu_fwd_prepacked_bf16(const uint16_t* x, int64_t N, int32_t d_model, const lbk_bell* w1,
+                                const lbk_bell* w2, const void* packed1, size_t packed1_bytes,
+                                const void* packed2, size_t packed2_bytes, const float* b1,
+                                const float* b2, uint16_t* out, void* workspace, size_t workspace_bytes,
+                                void* stream);
+int lbk_gelu_fwd_train(const uint16_t* x, int64_t N, int32_t d_model, const lbk_bell* w1,
+                       const lbk_bell* w2, const float* v1, const float* v2, uint16_t* vb1, uint16_t* vb2,
+                       const float* b1, const float* b2, uint16_t* out, uint16_t* h_out,
+                       uint16_t* pre_out, void* workspace, size_t workspace_bytes, void* stream);
+size_t lbk_gelu_bwd_workspace_bytes(int64_t N, int32_t d_model, const lbk_bell* w1, const lbk_bell* w2);
+int lbk_gelu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint16_t* pre,
+                       const uint16_t* h, int64_t N, int32_t d_model, const lbk_bell* w1,
+                       const lbk_bell* w2, uint16_t* dx, float* d_v1, float* d_v2, float* d_b1,
+                       float* d_b2, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---- prune-time topology transforms (integer and copy work; alive masks are one byte per slot,
  * nonzero = alive).  Replaces the JAX functions of looped_blockell/opt/compaction.py and
  * looped_blockell/opt/column_reorder.py on device. */

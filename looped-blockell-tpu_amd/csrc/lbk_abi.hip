@@ -1305,6 +1305,215 @@ int lbk_swiglu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint
                          workspace, workspace_bytes, stream);
 }
 
+// ---- the GELU FFN out = W2 gelu(W1 x + b1) + b2
+static int check_gelu(int64_t N, int32_t d_model, const lbk_bell* w1, const lbk_bell* w2) {
+  int st;
+  if ((st = check_bell(w1)) || (st = check_bell(w2))) return st;
+  if (w1->B != w2->B) return LBK_ERR_TILE;
+  if (N < 0) return LBK_ERR_ARG;
+  if (d_model <= 0 || d_model % w1->B || (int64_t)w2->R * w2->B != d_model) return LBK_ERR_SHAPE;
+  return LBK_OK;
+}
+
+static size_t gelu_packed_bytes(int32_t in_features, const lbk_bell* w) {
+  return lbk_block_ell_matmul_workspace_bytes(1, in_features, w);
+}
+
+size_t lbk_gelu_workspace_bytes(int64_t N, int32_t d_model, const lbk_bell* w1, const lbk_bell* w2, int prepacked,
+                                int want_h) {
+  if (!w1 || !w2 || check_gelu(N, d_model, w1, w2)) return 0;
+  const size_t h = want_h ? 0 : align256((size_t)N * w1->R * w1->B * 2);
+  return h + (prepacked ? 0 : gelu_packed_bytes(d_model, w1) + gelu_packed_bytes(w1->R * w1->B, w2));
+}
+
+// h = gelu(x W1 + b1), the pre-activation to `pre` (optional): in the epilogue where the product's
+// kernel has one, else a pass over it
+static int gelu_product(const uint16_t* x, int64_t N, int32_t d_model, const lbk_bell* w, const void* pk,
+                        const float* bias, uint16_t* h, uint16_t* pre, hipStream_t s) {
+  const int64_t out_f = (int64_t)w->R * w->B;
+  if (matmul_path(d_model, w) == MM_LIN) {
+    GUArgs g{};
+    g.x = x; g.N = N; g.d_model = d_model;
+    g.pg = pk; g.cg = w->col_idx; g.Kg = w->K;
+    g.R_ff = w->R; g.h = h; g.gpre = pre; g.bg = bias;
+    return launch_lin_gelu(w->B, g, s) == 0 ? LBK_OK : LBK_ERR_LAUNCH;
+  }
+  if (w->B == 64 && w->R > 0) {
+    RowblockLaunch a{};
+    a.x = x; a.N = N; a.ldx = d_model; a.C = d_model / w->B; a.R = w->R;
+    a.v0 = w->values; a.c0 = w->col_idx; a.K0 = w->K;
+    a.bias = bias; a.y = h; a.ldy = out_f;
+    a.gelu = 1; a.aux0 = pre; a.ldaux = out_f;
+    const int rc = launch_t64(0, a, s);
+    if (rc != -2) return rc == 0 ? LBK_OK : LBK_ERR_LAUNCH;
+  }
+  uint16_t* y = pre ? pre : h;
+  const int st = matmul_impl(x, N, d_model, w, pk, pk ? gelu_packed_bytes(d_model, w) : 0, bias, y, nullptr, 0, s);
+  if (st) return st;
+  return launch_gelu(y, N * out_f, h, s) == 0 ? LBK_OK : LBK_ERR_LAUNCH;
+}
+
+static int gelu_fwd_impl(const uint16_t* x, int64_t N, int32_t d_model, const lbk_bell* w1, const lbk_bell* w2,
+                         const void* packed1, size_t packed1_bytes, const void* packed2, size_t packed2_bytes,
+                         const float* const master[2], uint16_t* const raw[2], const float* b1, const float* b2,
+                         uint16_t* out, uint16_t* h_out, uint16_t* pre_out, void* workspace, size_t workspace_bytes,
+                         hipStream_t s) {
+  int st = check_gelu(N, d_model, w1, w2);
+  if (st) return st;
+  const int32_t d_ff = w1->R * w1->B;
+  const lbk_bell* w[2] = {w1, w2};
+  const int32_t in[2] = {d_model, d_ff};
+  const size_t pb[2] = {gelu_packed_bytes(d_model, w1), gelu_packed_bytes(d_ff, w2)};
+  if (N > 0) {
+    if (!x || !out) return LBK_ERR_NULL;
+    for (const void* p : {(const void*)x, (const void*)out, (const void*)h_out, (const void*)pre_out})
+      if (p && !a16(p)) return LBK_ERR_ALIGN;
+    if (d_model % 8) return LBK_ERR_ALIGN;
+  }
+  const size_t need = lbk_gelu_workspace_bytes(N, d_model, w1, w2, master ? 0 : 1, h_out != nullptr);
+  if (need > 0 && (!workspace || workspace_bytes < need)) return LBK_ERR_WORKSPACE;
+  if (need > 0 && !a16(workspace)) return LBK_ERR_ALIGN;
+  char* p = static_cast<char*>(workspace);
+  const void* pk[2] = {packed1, packed2};
+  if (master) {
+    PackJob jobs[2];
+    int nj = 0;
+    for (int t = 0; t < 2; ++t) {
+      const int64_t nt = (int64_t)w[t]->R * w[t]->K;
+      pk[t] = pb[t] ? p : nullptr;
+      if (nt > 0 || pb[t])
+        jobs[nj++] = PackJob{w[t]->values, w[t]->col_idx, nt, in[t] / w[t]->B, reinterpret_cast<uint32_t*>(pb[t] ? p : nullptr),
+                             0, matmul_path(in[t], w[t]) == MM_LIN, master[t], raw[t]};
+      p += pb[t];
+    }
+    if (nj && launch_pack_bf16_multi(jobs, nj, w1->B, s)) return LBK_ERR_LAUNCH;
+  } else if (N > 0) {
+    const size_t got[2] = {packed1_bytes, packed2_bytes};
+    for (int t = 0; t < 2; ++t) {
+      if (pb[t] == 0) continue;
+      if (!pk[t]) return LBK_ERR_NULL;
+      if (got[t] < pb[t]) return LBK_ERR_WORKSPACE;
+      if (!a16(pk[t])) return LBK_ERR_ALIGN;
+    }
+  }
+  if (N == 0) return LBK_OK;
+  uint16_t* h = h_out ? h_out : reinterpret_cast<uint16_t*>(p);
+  if ((st = gelu_product(x, N, d_model, w1, pb[0] ? pk[0] : nullptr, b1, h, pre_out, s))) return st;
+  return matmul_impl(h, N, d_ff, w2, pb[1] ? pk[1] : nullptr, pb[1], b2, out, nullptr, 0, s);
+}
+
+int lbk_gelu_fwd_prepacked_bf16(const uint16_t* x, int64_t N, int32_t d_model, const lbk_bell* w1,
+                                const lbk_bell* w2, const void* packed1, size_t packed1_bytes, const void* packed2,
+                                size_t packed2_bytes, const float* b1, const float* b2, uint16_t* out,
+                                void* workspace, size_t workspace_bytes, void* stream) {
+  return gelu_fwd_impl(x, N, d_model, w1, w2, packed1, packed1_bytes, packed2, packed2_bytes, nullptr, nullptr, b1, b2,
+                       out, nullptr, nullptr, workspace, workspace_bytes, S(stream));
+}
+
+int lbk_gelu_fwd_train(const uint16_t* x, int64_t N, int32_t d_model, const lbk_bell* w1, const lbk_bell* w2,
+                       const float* v1, const float* v2, uint16_t* vb1, uint16_t* vb2, const float* b1,
+                       const float* b2, uint16_t* out, uint16_t* h_out, uint16_t* pre_out, void* workspace,
+                       size_t workspace_bytes, void* stream) {
+  if (!w1 || !w2) return LBK_ERR_NULL;
+  lbk_bell w[2] = {*w1, *w2};
+  const float* m[2] = {v1, v2};
+  uint16_t* raw[2] = {vb1, vb2};
+  for (int t = 0; t < 2; ++t) {
+    w[t].values = raw[t];
+    const int st = check_bell(&w[t]);
+    if (st) return st;
+    if ((int64_t)w[t].R * w[t].K > 0) {
+      if (!m[t]) return LBK_ERR_NULL;
+      if (!a16(m[t]) || !a16(raw[t])) return LBK_ERR_ALIGN;
+    }
+  }
+  if (N > 0 && (!h_out || !pre_out)) return LBK_ERR_NULL;
+  return gelu_fwd_impl(x, N, d_model, &w[0], &w[1], nullptr, 0, nullptr, 0, m, raw, b1, b2, out, h_out, pre_out,
+                       workspace, workspace_bytes, S(stream));
+}
+
+size_t lbk_gelu_bwd_workspace_bytes(int64_t N, int32_t d_model, const lbk_bell* w1, const lbk_bell* w2) {
+  if (!w1 || !w2 || check_gelu(N, d_model, w1, w2)) return 0;
+  const int64_t d_ff = (int64_t)w1->R * w1->B;
+  const int C_in = d_model / w1->B, C_d = w1->R;
+  return tlist_bytes(w2, C_d) + tlist_bytes(w1, C_in) + align256((size_t)N * d_ff * 2) +
+         align256((dw_part_floats(N, w1, C_in, d_ff) + dw_part_floats(N, w2, C_d, d_model)) * 4) +
+         align256(colsum_bytes(N, d_ff + d_model));
+}
+
+int lbk_gelu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint16_t* pre, const uint16_t* h,
+                       int64_t N, int32_t d_model, const lbk_bell* w1, const lbk_bell* w2, uint16_t* dx,
+                       float* d_v1, float* d_v2, float* d_b1, float* d_b2, void* workspace, size_t workspace_bytes,
+                       void* stream) {
+  int st = check_gelu(N, d_model, w1, w2);
+  if (st) return st;
+  const int B = w1->B;
+  const int64_t d_ff = (int64_t)w1->R * B, t1 = (int64_t)w1->R * w1->K, t2 = (int64_t)w2->R * w2->K;
+  const int C_in = d_model / B, C_d = w1->R;
+  if ((t1 && !d_v1) || (t2 && !d_v2)) return LBK_ERR_NULL;
+  for (const void* q : {(const void*)d_v1, (const void*)d_v2, (const void*)w1->values, (const void*)w2->values})
+    if (q && !a16(q)) return LBK_ERR_ALIGN;
+  if (N > 0) {
+    if (!grad_out || !x || !pre || !h || !dx) return LBK_ERR_NULL;
+    for (const void* q : {(const void*)grad_out, (const void*)x, (const void*)pre, (const void*)h, (const void*)dx})
+      if (!a16(q)) return LBK_ERR_ALIGN;
+    if (d_model % 8) return LBK_ERR_ALIGN;
+  }
+  const size_t need = lbk_gelu_bwd_workspace_bytes(N, d_model, w1, w2);
+  if (!workspace || workspace_bytes < need) return LBK_ERR_WORKSPACE;
+  if (!a16(workspace)) return LBK_ERR_ALIGN;
+  hipStream_t s = S(stream);
+  char* p = static_cast<char*>(workspace);
+  auto take = [&](size_t bytes) {
+    char* q = p;
+    p += align256(bytes);
+    return q;
+  };
+  const lbk_bell* w[2] = {w2, w1};
+  const int c[2] = {C_d, C_in};
+  TListJob lj[2], ljn[2];
+  int nl = 0;
+  for (int t = 0; t < 2; ++t) {
+    lj[t] = TListJob{w[t]->col_idx, w[t]->R, w[t]->K, c[t], nullptr, nullptr};
+    lj[t].cnt = reinterpret_cast<int32_t*>(take((size_t)c[t] * 4));
+    lj[t].list = reinterpret_cast<int32_t*>(take((size_t)c[t] * w[t]->R * w[t]->K * 4));
+    if ((int64_t)w[t]->R * w[t]->K > 0) ljn[nl++] = lj[t];
+  }
+  uint16_t* da = reinterpret_cast<uint16_t*>(take((size_t)N * d_ff * 2));
+  const size_t f1 = dw_part_floats(N, w1, C_in, d_ff), f2 = dw_part_floats(N, w2, C_d, d_model);
+  float* part = reinterpret_cast<float*>(take((f1 + f2) * 4));
+  float* cpart = reinterpret_cast<float*>(p);
+  if (N > 0) {
+    if (nl && launch_tlist(ljn, nl, s)) return LBK_ERR_LAUNCH;
+    // da = (dy W2) gelu'(pre)
+    TProdArgs a{};
+    if (t2 > 0) a.src[a.nsrc++] = TProdSrc{grad_out, d_model, w2->values, w2->K, lj[0].cnt, lj[0].list, t2};
+    a.N = N; a.C = C_d; a.ldo = d_ff;
+    a.g = pre; a.dg = da;
+    if (launch_tprod(B, 2, a, s)) return LBK_ERR_LAUNCH;
+    // dx = da W1
+    TProdArgs b{};
+    if (t1 > 0) b.src[b.nsrc++] = TProdSrc{da, d_ff, w1->values, w1->K, lj[1].cnt, lj[1].list, t1};
+    b.N = N; b.C = C_in; b.ldo = d_model;
+    b.out = dx;
+    if (launch_tprod(B, 1, b, s)) return LBK_ERR_LAUNCH;
+  }
+  DWJob dj[2];
+  int nj = 0;
+  if (t1 > 0)
+    dj[nj++] = DWJob{x, d_model, da, d_ff, w1->col_idx, w1->R, w1->K, C_in, part, nullptr, d_v1, nullptr, nullptr, 0, 0};
+  if (t2 > 0)
+    dj[nj++] = DWJob{h, d_ff, grad_out, d_model, w2->col_idx, w2->R, w2->K, C_d, part + f1, nullptr, d_v2,
+                     N > 0 ? lj[0].cnt : nullptr, N > 0 ? lj[0].list : nullptr, 0, 0};
+  if (nj && launch_dw(B, dj, nj, N, s)) return LBK_ERR_LAUNCH;
+  ColsumJob cj[2];
+  int nc = 0;
+  if (d_b1 && d_ff > 0) cj[nc++] = ColsumJob{da, d_ff, (int)d_ff, d_b1, nullptr, 0};
+  if (d_b2) cj[nc++] = ColsumJob{grad_out, d_model, d_model, d_b2, nullptr, 0};
+  if (nc && launch_colsum(cj, nc, N, cpart, s)) return LBK_ERR_LAUNCH;
+  return LBK_OK;
+}
+
 size_t lbk_block_ell_matmul_bwd_workspace_bytes(int64_t N, int32_t in_features, const lbk_bell* w) {
   if (!w || N < 0 || in_features <= 0 || !tile_ok(w->B) || in_features % w->B) return 0;
   const int C = in_features / w->B;

@@ -637,6 +637,24 @@ int launch_injection(const uint16_t* h, const uint16_t* e, const float* log_A, c
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+// y = gelu(x) in place or not, 8 values a thread: the products whose kernel has no GELU epilogue
+__global__ __launch_bounds__(256) void gelu_kernel(const uint16_t* x, int64_t n8, uint16_t* y) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= n8) return;
+  float v[8];
+  unpack8_bf16(reinterpret_cast<const u32x4*>(x)[e], v);
+#pragma unroll
+  for (int q = 0; q < 8; ++q) v[q] = gelu_f(v[q]);
+  store_bf16x<8>(y + 8 * e, v);
+}
+
+int launch_gelu(const uint16_t* x, int64_t n, uint16_t* y, hipStream_t st) {
+  if (n == 0) return 0;
+  if (n % 8) return -2;
+  hipLaunchKernelGGL(gelu_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, st, x, n / 8, y);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 // ---------------------------------------------------------------------------
 // bf16 tiles [R*K, B, B] ([B_in, B_out] each) -> fragment-major packed tiles
 // (layout described with PackedTile in lbk_device.h), one thread per dword.

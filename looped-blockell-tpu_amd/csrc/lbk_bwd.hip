@@ -19,7 +19,8 @@
 //                  needs), the activation rows the B operand, so each lane ends
 //                  with 4 consecutive output columns of one token; two list
 //                  entries are in flight at a time.  Epilogue:
-//                  the SiLU*mul backward (dh -> dg, du) or the optional + dy (-> dx).
+//                  the SiLU*mul backward (dh -> dg, du), the optional + dy (-> dx) or
+//                  the GELU backward (dh -> dg, for a layer without an up weight).
 //   dh_panel_kernel  dh -> dg, du when d_model <= 2048: the dy rows of 64 (32)
 //                  tokens sit in LDS as the forward's XOR-swizzled panel and each
 //                  of NW waves (8; 16 at B = 16) streams the list entries of its
@@ -119,7 +120,7 @@ __device__ __forceinline__ int op_row(int i, int m) {
 }
 
 // epilogue of one token row: the lane's accumulator values v8 (8 consecutive columns starting at
-// col, or 4 for B = 16): SiLU*mul backward (MODE 0) or + residual (MODE 1)
+// col, or 4 for B = 16): SiLU*mul backward (MODE 0), + residual (MODE 1) or GELU backward (MODE 2)
 template <int MODE, int NV>
 __device__ __forceinline__ void tprod_epilogue(const TProdArgs& a, int64_t off, const float (&v)[NV]) {
   if constexpr (MODE == 0) {
@@ -134,6 +135,12 @@ __device__ __forceinline__ void tprod_epilogue(const TProdArgs& a, int64_t off, 
     }
     store_bf16x<NV>(a.dg + off, dgv);
     store_bf16x<NV>(a.du + off, duv);
+  } else if constexpr (MODE == 2) {
+    float gv[NV], dgv[NV];
+    load_bf16x<NV>(a.g + off, gv);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) dgv[j] = v[j] * gelu_grad_f(gv[j]);
+    store_bf16x<NV>(a.dg + off, dgv);
   } else {
     float rv[NV], o[NV];
 #pragma unroll
@@ -273,7 +280,8 @@ __device__ __forceinline__ int kdiv(const TProdSrc& S, int e) {
   return (int)((__umulhi((uint32_t)e, S.kmul) + (uint32_t)e) >> S.ksh);
 }
 
-template <int B, int MT, int NW>
+// GELU: the epilogue is dg = dh gelu'(g), with no up stream
+template <int B, int MT, int NW, bool GELU>
 __global__ __launch_bounds__(64 * NW, 1) void dh_panel_kernel(TProdArgs a) {
   constexpr int NT = 64 * NW;
   constexpr int CW = B / 16;
@@ -390,7 +398,7 @@ __global__ __launch_bounds__(64 * NW, 1) void dh_panel_kernel(TProdArgs a) {
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
         graw[q][p] = *reinterpret_cast<const raw_t*>(a.g + row + col_of(c, p));
-        uraw[q][p] = *reinterpret_cast<const raw_t*>(a.u + row + col_of(c, p));
+        if constexpr (!GELU) uraw[q][p] = *reinterpret_cast<const raw_t*>(a.u + row + col_of(c, p));
       }
     }
 #pragma unroll
@@ -465,14 +473,20 @@ __global__ __launch_bounds__(64 * NW, 1) void dh_panel_kernel(TProdArgs a) {
         for (int j = 0; j < NV; ++j) dh[j] = acc[q][CW == 1 ? 0 : 2 * p + j / 4][j % 4];
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-          const uint32_t gw = graw[q][p][j / 2], uw = uraw[q][p][j / 2];
-          const float gv = (j & 1) ? bf_hi(gw) : bf_lo(gw), uv = (j & 1) ? bf_hi(uw) : bf_lo(uw);
+          const uint32_t gw = graw[q][p][j / 2];
+          const float gv = (j & 1) ? bf_hi(gw) : bf_lo(gw);
+          if constexpr (GELU) {
+            dgv[j] = dh[j] * gelu_grad_f(gv);
+            continue;
+          }
+          const uint32_t uw = uraw[q][p][j / 2];
+          const float uv = (j & 1) ? bf_hi(uw) : bf_lo(uw);
           const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-gv));   // sigmoid(g)
           dgv[j] = dh[j] * uv * (sg + gv * sg * (1.0f - sg));
           duv[j] = dh[j] * gv * sg;
         }
         store_bf16x<NV>(a.dg + tn * a.ldo + col_of(c, p), dgv);
-        store_bf16x<NV>(a.du + tn * a.ldo + col_of(c, p), duv);
+        if constexpr (!GELU) store_bf16x<NV>(a.du + tn * a.ldo + col_of(c, p), duv);
       }
     }
   }
@@ -481,10 +495,10 @@ __global__ __launch_bounds__(64 * NW, 1) void dh_panel_kernel(TProdArgs a) {
 // dh through the LDS panel when the dy rows of 16*MT tokens fit (d_model <= 2048, one source)
 // With fewer token blocks than CUs, the column blocks are split over nsl workgroups per token
 // block (about 256 workgroups, at least one column block per wave), each loading the dy panel.
-template <int B, int MT, int NW>
+template <int B, int MT, int NW, bool GELU>
 static int launch_dh_panel_t(const TProdArgs& a0, hipStream_t st) {
   constexpr size_t lds = (size_t)16 * MT * (8192 / MT);
-  auto kern = dh_panel_kernel<B, MT, NW>;
+  auto kern = dh_panel_kernel<B, MT, NW, GELU>;
   static std::atomic<uint64_t> done{0};
   if (set_lds_limit_once(reinterpret_cast<const void*>(kern), (int)lds, done)) return -1;
   TProdArgs a = a0;
@@ -496,14 +510,15 @@ static int launch_dh_panel_t(const TProdArgs& a0, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+template <bool GELU>
 static int launch_dh_panel(int B, const TProdArgs& a, hipStream_t st) {
   const int64_t d_model = a.src[0].lda;
   const int mt = d_model <= 1024 ? 4 : (d_model <= 2048 ? 2 : 0);
   if (mt == 0 || d_model % 8) return -2;
   // 16 waves at B = 16 (their registers fit 128 VGPRs): B = 16 backward at d_model 1024, d_ff 4096
   // 1.93 -> 1.87 ms; at B = 32 16 waves spill (0.739 against 0.715 ms)
-  if (B == 16 && mt == 4) return launch_dh_panel_t<16, 4, 16>(a, st);
-#define LBK_DH(BB, MM) if (B == BB && mt == MM) return launch_dh_panel_t<BB, MM, 8>(a, st);
+  if (B == 16 && mt == 4) return launch_dh_panel_t<16, 4, 16, GELU>(a, st);
+#define LBK_DH(BB, MM) if (B == BB && mt == MM) return launch_dh_panel_t<BB, MM, 8, GELU>(a, st);
   LBK_DH(16, 4) LBK_DH(16, 2) LBK_DH(32, 4) LBK_DH(32, 2) LBK_DH(64, 4) LBK_DH(64, 2)
 #undef LBK_DH
   return -2;
@@ -961,7 +976,11 @@ static int launch_dx_stage(int B, const TProdArgs& a0, hipStream_t st) {
 int launch_tprod(int B, int mode, const TProdArgs& a, hipStream_t st) {
   if (a.N == 0 || a.C == 0) return 0;
   if (mode == 0 && a.nsrc == 1) {
-    const int rc = launch_dh_panel(B, a, st);
+    const int rc = launch_dh_panel<false>(B, a, st);
+    if (rc != -2) return rc;
+  }
+  if (mode == 2 && a.nsrc == 1) {
+    const int rc = launch_dh_panel<true>(B, a, st);
     if (rc != -2) return rc;
   }
   if (mode == 1) {
@@ -972,6 +991,7 @@ int launch_tprod(int B, int mode, const TProdArgs& a, hipStream_t st) {
 #define LBK_TP(BB)                                                                      \
   if (B == BB) {                                                                        \
     if (mode == 0) hipLaunchKernelGGL((tprod_kernel<BB, 0>), grid, dim3(256), 0, st, a); \
+    else if (mode == 2) hipLaunchKernelGGL((tprod_kernel<BB, 2>), grid, dim3(256), 0, st, a); \
     else hipLaunchKernelGGL((tprod_kernel<BB, 1>), grid, dim3(256), 0, st, a);           \
     return hipGetLastError() == hipSuccess ? 0 : -1;                                    \
   }

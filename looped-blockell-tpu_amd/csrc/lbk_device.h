@@ -73,6 +73,17 @@ __device__ __forceinline__ float silu_f(float z) {
   return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z));
 }
 
+// GELU in its tanh form, z (1 + tanh u) / 2 with u = sqrt(2 / pi) (z + 0.044715 z^3), as
+// z sigmoid(2 u), and its derivative s + z s (1 - s) 2 u', s = sigmoid(2 u).
+__device__ __forceinline__ float gelu_gate(float z) {
+  return __builtin_amdgcn_rcpf(1.0f + __expf(-1.5957691216f * (z + 0.044715f * z * z * z)));
+}
+__device__ __forceinline__ float gelu_f(float z) { return z * gelu_gate(z); }
+__device__ __forceinline__ float gelu_grad_f(float z) {
+  const float s = gelu_gate(z);
+  return s + z * s * (1.0f - s) * (1.5957691216f * (1.0f + 0.134145f * z * z));
+}
+
 // Wave-uniform value (forces scalar registers / scalar branches).
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 

@@ -21,6 +21,8 @@ struct RowblockLaunch {
   const uint16_t* resid; int64_t ldr;              // MODE 2, optional
   uint16_t* y; int64_t ldy;
   uint16_t* aux0; uint16_t* aux1; int64_t ldaux;    // MODE 1 optional pre-activations
+  int gelu;                                         // MODE 0 of launch_t64: y = gelu(product), the
+                                                    // pre-activation to aux0 (optional)
 };
 
 // B = 64 products of more tokens than the decode kernels take (lbk_tile64.hip); -2: an operand's
@@ -111,6 +113,10 @@ bool split_supported(int B, int d_model, int R_ff, int R_m, int Kg, int Ku, int 
 // a.d_model = in, output in a.h with row stride R*B): the gate/up kernel's gate stream alone
 bool lin_supported(int B, int in_features, int R, int K);
 int launch_lin(int B, const GUArgs& a, hipStream_t st);
+// the same with h = gelu(product) and the pre-activation to a.gpre (optional)
+int launch_lin_gelu(int B, const GUArgs& a, hipStream_t st);
+// y = gelu(x) over n bf16 values (n % 8 == 0, 16-byte aligned; y may be x)
+int launch_gelu(const uint16_t* x, int64_t n, uint16_t* y, hipStream_t st);
 // looped block in one launch: gate/up (RMSNorm of the fp32 state) and down per token block
 // for all L iterations; gu.xf == dn.state == the fp32 state, gu.h == dn.h
 // one core block of the persistent looped kernel (packed tiles, columns, norm scale, biases)
@@ -301,11 +307,11 @@ struct TProdSrc {
 struct TProdArgs {
   TProdSrc src[2]; int nsrc;
   int64_t N; int C; int64_t ldo;    // output [N, C*B], row stride ldo (also of g, u, resid)
-  const uint16_t* g; const uint16_t* u; uint16_t* dg; uint16_t* du;   // mode 0
+  const uint16_t* g; const uint16_t* u; uint16_t* dg; uint16_t* du;   // mode 0 (mode 2: g and dg)
   const uint16_t* resid; uint16_t* out;                               // mode 1 (resid optional)
   int nsl;                          // output column slices per token block (set by the launcher)
 };
-// mode 0: dh -> dg, du (SiLU*mul backward); mode 1: out = product + resid
+// mode 0: dh -> dg, du (SiLU*mul backward); mode 1: out = product + resid; mode 2: dh -> dg = dh gelu'(g)
 int launch_tprod(int B, int mode, const TProdArgs& a, hipStream_t st);
 // tile gradients dW[e] = X[:, col(e)]^T G[:, row(e)] through fp32 per-chunk partials
 struct DWJob {

@@ -120,8 +120,9 @@ struct GUPanel { static constexpr int ROWB = 8192 / MT; };
 // the gate's weights and columns for up too, with SHARED), no SiLU.
 // NW, RING: waves of the workgroup and ring depth (12 waves with a 2-deep ring for the plain
 // x-panel path, where three waves per SIMD fit the register budget).
+// GELU (with LIN): a.h gets gelu of the product, a.gpre (optional) the product
 template <int B, int MT, bool NORM, bool INTER, bool SHARED, bool READY = false, bool BIAS = false, bool LIN = false,
-          int NW = 8, int RING = GU_RING>
+          int NW = 8, int RING = GU_RING, bool GELU = false>
 __device__ __forceinline__ void gu_tile(const GUArgs& a, int64_t tb, int r_lo, int nrs, unsigned char* smem,
                                         int tid) {
   constexpr int CW = TileShape<B>::CW;
@@ -528,13 +529,15 @@ __device__ __forceinline__ void gu_tile(const GUArgs& a, int64_t tb, int r_lo, i
             gv[4 * m + v] += bgv[4 * m + v];
             uv[4 * m + v] += buv[4 * m + v];
           }
-          o[4 * m + v] = LIN ? gv[4 * m + v] : silu_f(gv[4 * m + v]) * uv[4 * m + v];
+          o[4 * m + v] = GELU  ? gelu_f(gv[4 * m + v])
+                         : LIN ? gv[4 * m + v]
+                               : silu_f(gv[4 * m + v]) * uv[4 * m + v];
         }
       if (t < a.N) {
         store_bf16x<4 * CW>(a.h + t * d_ff + col0, o);
         if constexpr (INTER) {
           if (a.gpre) store_bf16x<4 * CW>(a.gpre + t * d_ff + col0, gv);
-          if (a.uout) store_bf16x<4 * CW>(a.uout + t * d_ff + col0, uv);
+          if (!LIN && a.uout) store_bf16x<4 * CW>(a.uout + t * d_ff + col0, uv);
         }
       }
     }
@@ -597,14 +600,16 @@ __global__ __launch_bounds__((64 * gu_w12_waves<B, SHARED>()), 1) void gu_kernel
 // (at most 92 VGPRs); at the headline gate shape (16384 x 1024 -> 4096, B = 32) a call with
 // per-call packing took 0.0535 ms against 0.0615 with 8 waves and a 4-deep ring (12 waves:
 // 0.0551 with a 2-deep ring, 0.0535 with a 4-deep one)
+// With GELU the activation runs in the epilogue (as passes of their own over 8192 x 4096 values the
+// two casts and the activation took 103 us of a 245 us forward).
 constexpr int LIN_WAVES = 16;
-template <int B, int MT, bool BIAS>
+template <int B, int MT, bool BIAS, bool GELU>
 __global__ __launch_bounds__(64 * LIN_WAVES, 1) void lin_kernel(GUArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   int64_t tb;
   int r_lo, nrs;
   gu_slice(a, tb, r_lo, nrs);
-  gu_tile<B, MT, false, false, true, false, BIAS, true, LIN_WAVES, 2>(a, tb, r_lo, nrs, smem, (int)threadIdx.x);
+  gu_tile<B, MT, false, GELU, true, false, BIAS, true, LIN_WAVES, 2, GELU>(a, tb, r_lo, nrs, smem, (int)threadIdx.x);
 }
 
 // ===========================================================================
@@ -1517,9 +1522,9 @@ int launch_gu(int B, bool norm, const GUArgs& a0, hipStream_t st) {
   return -2;
 }
 
-template <int B, int MT, bool BIAS>
+template <int B, int MT, bool BIAS, bool GELU>
 static int launch_lin_t(const GUArgs& a, hipStream_t st) {
-  auto kern = lin_kernel<B, MT, BIAS>;
+  auto kern = lin_kernel<B, MT, BIAS, GELU>;
   static std::atomic<uint64_t> configured{0};
   if (set_lds_limit_once((const void*)kern, 163840, configured)) return -1;
   const int TM = 16 * MT;
@@ -1536,7 +1541,8 @@ bool lin_supported(int B, int in_features, int R, int K) {
   return (R * B) % 8 == 0;
 }
 
-int launch_lin(int B, const GUArgs& a0, hipStream_t st) {
+template <bool GELU>
+static int launch_lin_g(int B, const GUArgs& a0, hipStream_t st) {
   if (a0.N == 0) return 0;
   GUArgs a = a0;   // the up operands are the gate's (never read as weights)
   a.pu = a.pg;
@@ -1546,11 +1552,15 @@ int launch_lin(int B, const GUArgs& a0, hipStream_t st) {
   if (mt == 0) return -2;
   a.H = gu_slices((a.N + 16 * mt - 1) / (16 * mt), a.R_ff);
 #define LBK_LIN(BB, MM)                                                                     \
-  if (B == BB && mt == MM) return a.bg ? launch_lin_t<BB, MM, true>(a, st) : launch_lin_t<BB, MM, false>(a, st);
+  if (B == BB && mt == MM)                                                                  \
+    return a.bg ? launch_lin_t<BB, MM, true, GELU>(a, st) : launch_lin_t<BB, MM, false, GELU>(a, st);
   LBK_LIN(16, 4) LBK_LIN(16, 2) LBK_LIN(32, 4) LBK_LIN(32, 2)
 #undef LBK_LIN
   return -2;
 }
+
+int launch_lin(int B, const GUArgs& a, hipStream_t st) { return launch_lin_g<false>(B, a, st); }
+int launch_lin_gelu(int B, const GUArgs& a, hipStream_t st) { return launch_lin_g<true>(B, a, st); }
 
 template <int B, int MT, int RPW, int NW, int SC, int KC>
 static int launch_dn_k(const DNArgs& a0, hipStream_t st) {

@@ -217,6 +217,11 @@ __global__ __launch_bounds__(256, 2) void t64_kernel(T64Args a) {
         if (MODE == 2 && a.resid) load_bf16x<4>(a.resid + t * a.ldr + oc, rv);
 #pragma unroll
         for (int v = 0; v < 4; ++v) o[v] = acc[0][q][m][v] + b0[v] + rv[v];
+        if (MODE == 0 && a.gelu) {
+          if (a.aux0) store_bf16x<4>(a.aux0 + t * a.ldaux + oc, o);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) o[v] = gelu_f(o[v]);
+        }
       }
       store_bf16x<4>(a.y + t * a.ldy + oc, o);
     }
@@ -268,7 +273,7 @@ int launch_t64(int mode, const RowblockLaunch& a, hipStream_t st) {
   auto bad = [](const void* p, uintptr_t m) { return (reinterpret_cast<uintptr_t>(p) & m) != 0; };
   // 16-byte loads of activations and tiles, 8-byte stores; 32-bit offsets within a token block
   if (bad(a.x, 15) || a.ldx % 8 || bad(a.v0, 15) || (mode == 1 && bad(a.v1, 15)) || bad(a.y, 7) || a.ldy % 4 ||
-      (mode == 1 && ((a.aux0 && bad(a.aux0, 7)) || (a.aux1 && bad(a.aux1, 7)) || a.ldaux % 4)) ||
+      ((mode == 1 || a.gelu) && ((a.aux0 && bad(a.aux0, 7)) || (a.aux1 && bad(a.aux1, 7)) || a.ldaux % 4)) ||
       (mode == 2 && a.resid && (bad(a.resid, 7) || a.ldr % 4)) || a.ldx > (1 << 22))
     return -2;
   // the largest token block that leaves two workgroups per CU (2048 tokens, 2048 -> 8192 at 0.5: 159

@@ -970,6 +970,154 @@ Tensor swiglu_train_autograd(const Tensor& x, const Tensor& vg, const Tensor& cg
   return SwigluTrain::apply(x, vg, cg, bg, vu, cu, bu, vd, cd, bd, add_residual);
 }
 
+// ------------------------------------------------------------------ GELU FFN
+using Five = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor>;
+
+void check_gelu_shapes(const lbk_bell& w1, const lbk_bell& w2, int64_t d_model, const char* op) {
+  TORCH_CHECK(w1.B == w2.B, "titan::", op, ": the two weights must have one tile size");
+  TORCH_CHECK(d_model % w1.B == 0, "titan::", op, ": in_features ", d_model, " not a multiple of B=", w1.B);
+  TORCH_CHECK((int64_t)w2.R * w2.B == d_model, "titan::", op, ": the second weight's ", (int64_t)w2.R * w2.B,
+              " output features are not d_model=", d_model);
+}
+
+// gradient-free forward from the two weights' block_ell_matmul_prepack copies
+Tensor gelu_fwd_prepacked(const Tensor& x_, const Tensor& p1, const Tensor& v1_, const Tensor& c1_,
+                          const OptTensor& b1_, const Tensor& p2, const Tensor& v2_, const Tensor& c2_,
+                          const OptTensor& b2_) {
+  const char* op = "block_ell_gelu_fwd_prepacked";
+  Tensor v1 = v1_, c1 = c1_, v2 = v2_, c2 = c2_;
+  Tensor x = check_x2d(x_, op);
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
+  lbk_bell w1 = make_bell(v1, c1, op, "w1"), w2 = make_bell(v2, c2, op, "w2");
+  const int64_t N = x.size(0), d_model = x.size(1);
+  check_gelu_shapes(w1, w2, d_model, op);
+  for (const Tensor* p : {&p1, &p2}) {
+    check_gpu(*p, op, "packed");
+    TORCH_CHECK(p->scalar_type() == at::kByte && p->dim() == 1 && p->is_contiguous(), "titan::", op,
+                ": packed must be the uint8 tensor of block_ell_matmul_prepack");
+  }
+  const int32_t d_ff = w1.R * w1.B;
+  const size_t n1 = lbk_block_ell_matmul_prepacked_bytes((int32_t)d_model, &w1),
+               n2 = lbk_block_ell_matmul_prepacked_bytes(d_ff, &w2);
+  TORCH_CHECK((size_t)p1.numel() >= n1 && (size_t)p2.numel() >= n2, "titan::", op, ": the packed copies hold ",
+              p1.numel(), " and ", p2.numel(), " bytes, these weights need ", n1, " and ", n2);
+  const Tensor b1 = opt_bias(b1_, d_ff, x, op, "b1"), b2 = opt_bias(b2_, d_model, x, op, "b2");
+  Tensor out = at::empty({N, d_model}, x.options());
+  const size_t wsb = lbk_gelu_workspace_bytes(N, (int32_t)d_model, &w1, &w2, 1, 0);
+  Tensor ws = wsb ? workspace(wsb, x) : Tensor();
+  LBK_CALL("block_ell_gelu_fwd_prepacked",
+           lbk_gelu_fwd_prepacked_bf16(bf(x), N, (int32_t)d_model, &w1, &w2, n1 ? p1.data_ptr() : nullptr,
+                                       (size_t)p1.numel(), n2 ? p2.data_ptr() : nullptr, (size_t)p2.numel(), fptr(b1),
+                                       fptr(b2), bfm(out), wsb ? ws.data_ptr() : nullptr, wsb, cur_stream(x)));
+  return out;
+}
+
+// (out, h, pre-activation, and the bf16 copies of the two weights that the backward reads)
+Five gelu_fwd_train(const Tensor& x_, const Tensor& v1_, const Tensor& c1_, const OptTensor& b1_, const Tensor& v2_,
+                    const Tensor& c2_, const OptTensor& b2_) {
+  const char* op = "block_ell_gelu_fwd_train";
+  Tensor v1 = v1_, c1 = c1_, v2 = v2_, c2 = c2_;
+  Tensor x = check_x2d(x_, op);
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
+  lbk_bell w1 = make_master(v1, c1, op, "w1"), w2 = make_master(v2, c2, op, "w2");
+  const int64_t N = x.size(0), d_model = x.size(1);
+  check_gelu_shapes(w1, w2, d_model, op);
+  const int64_t d_ff = (int64_t)w1.R * w1.B;
+  const Tensor b1 = opt_bias(b1_, d_ff, x, op, "b1"), b2 = opt_bias(b2_, d_model, x, op, "b2");
+  Tensor out = at::empty({N, d_model}, x.options()), h = at::empty({N, d_ff}, x.options()),
+         pre = at::empty({N, d_ff}, x.options());
+  Tensor r1 = at::empty(v1.sizes(), x.options()), r2 = at::empty(v2.sizes(), x.options());
+  w1.values = bf(r1);
+  w2.values = bf(r2);
+  const size_t wsb = lbk_gelu_workspace_bytes(N, (int32_t)d_model, &w1, &w2, 0, 1);
+  Tensor ws = wsb ? workspace(wsb, x) : Tensor();
+  LBK_CALL("block_ell_gelu_fwd_train",
+           lbk_gelu_fwd_train(bf(x), N, (int32_t)d_model, &w1, &w2, v1.data_ptr<float>(), v2.data_ptr<float>(),
+                              bfm(r1), bfm(r2), fptr(b1), fptr(b2), bfm(out), bfm(h), bfm(pre),
+                              wsb ? ws.data_ptr() : nullptr, wsb, cur_stream(x)));
+  return {out, h, pre, r1, r2};
+}
+
+// (dx, fp32 gradients of the two weights' tiles and of the biases; the last two empty without biases)
+Five gelu_bwd_train(const Tensor& dy_, const Tensor& x_, const Tensor& pre_, const Tensor& h_, const Tensor& r1_,
+                    const Tensor& c1_, const Tensor& r2_, const Tensor& c2_, bool biases) {
+  const char* op = "block_ell_gelu_bwd_train";
+  Tensor v1 = r1_, c1 = c1_, v2 = r2_, c2 = c2_;
+  Tensor x = check_x2d(x_, op), dy = check_x2d(dy_, op), pre = check_x2d(pre_, op), h = check_x2d(h_, op);
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
+  lbk_bell w1 = make_bell(v1, c1, op, "w1"), w2 = make_bell(v2, c2, op, "w2");
+  const int64_t N = x.size(0), d_model = x.size(1), d_ff = (int64_t)w1.R * w1.B;
+  check_gelu_shapes(w1, w2, d_model, op);
+  TORCH_CHECK(dy.sizes() == x.sizes() && pre.size(0) == N && pre.size(1) == d_ff && h.sizes() == pre.sizes(),
+              "titan::", op, ": grad_out must match x, and the pre-activation and h be [", N, ", ", d_ff, "]");
+  const auto f32 = x.options().dtype(at::kFloat);
+  Tensor dx = at::empty({N, d_model}, x.options()), d1 = at::empty(v1.sizes(), f32), d2 = at::empty(v2.sizes(), f32);
+  Tensor db1 = at::empty({biases ? d_ff : 0}, f32), db2 = at::empty({biases ? d_model : 0}, f32);
+  const size_t wsb = lbk_gelu_bwd_workspace_bytes(N, (int32_t)d_model, &w1, &w2);
+  Tensor ws = workspace(wsb, x);
+  LBK_CALL("block_ell_gelu_bwd_train",
+           lbk_gelu_bwd_train(bf(dy), bf(x), bf(pre), bf(h), N, (int32_t)d_model, &w1, &w2, bfm(dx),
+                              d1.data_ptr<float>(), d2.data_ptr<float>(), biases ? db1.data_ptr<float>() : nullptr,
+                              biases ? db2.data_ptr<float>() : nullptr, ws.data_ptr(), wsb, cur_stream(x)));
+  return {dx, d1, d2, db1, db2};
+}
+
+Five call_gelu_fwd_train(const Tensor& x, const Tensor& v1, const Tensor& c1, const OptTensor& b1, const Tensor& v2,
+                         const Tensor& c2, const OptTensor& b2) {
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("titan::block_ell_gelu_fwd_train", "")
+                             .typed<decltype(gelu_fwd_train)>();
+  return op.call(x, v1, c1, b1, v2, c2, b2);
+}
+
+Five call_gelu_bwd_train(const Tensor& dy, const Tensor& x, const Tensor& pre, const Tensor& h, const Tensor& r1,
+                         const Tensor& c1, const Tensor& r2, const Tensor& c2, bool biases) {
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("titan::block_ell_gelu_bwd_train", "")
+                             .typed<decltype(gelu_bwd_train)>();
+  return op.call(dy, x, pre, h, r1, c1, r2, c2, biases);
+}
+
+struct GeluTrain : public torch::autograd::Function<GeluTrain> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& v1, const Tensor& c1,
+                        const OptTensor& b1, const Tensor& v2, const Tensor& c2, const OptTensor& b2) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    auto [out, h, pre, r1, r2] = call_gelu_fwd_train(x, v1, c1, b1, v2, c2, b2);
+    ctx->save_for_backward({x, pre, h, r1, c1, r2, c2});
+    auto dt = [](const OptTensor& b) {
+      return b.has_value() && b->defined() ? (int64_t)b->scalar_type() : (int64_t)-1;
+    };
+    ctx->saved_data["bias"] = std::vector<int64_t>{dt(b1), dt(b2)};
+    return out;
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    torch::autograd::variable_list r(7);
+    if (!grads[0].defined()) return r;
+    const auto s = ctx->get_saved_variables();
+    const auto dt = ctx->saved_data["bias"].toIntVector();
+    auto [dx, d1, d2, db1, db2] = call_gelu_bwd_train(grads[0].to(at::kBFloat16).contiguous(), s[0], s[1], s[2], s[3],
+                                                      s[4], s[5], s[6], dt[0] >= 0 || dt[1] >= 0);
+    r[0] = dx;
+    r[1] = d1;
+    if (dt[0] >= 0) r[3] = db1.to(static_cast<at::ScalarType>(dt[0]));
+    r[4] = d2;
+    if (dt[1] >= 0) r[6] = db2.to(static_cast<at::ScalarType>(dt[1]));
+    return r;
+  }
+};
+
+Tensor gelu_train(const Tensor& x, const Tensor& v1, const Tensor& c1, const OptTensor& b1, const Tensor& v2,
+                  const Tensor& c2, const OptTensor& b2) {
+  return std::get<0>(call_gelu_fwd_train(x, v1, c1, b1, v2, c2, b2));
+}
+
+Tensor gelu_train_autograd(const Tensor& x, const Tensor& v1, const Tensor& c1, const OptTensor& b1, const Tensor& v2,
+                           const Tensor& c2, const OptTensor& b2) {
+  return GeluTrain::apply(x, v1, c1, b1, v2, c2, b2);
+}
+
 // the reference operator: dx always includes grad_out (the forward's residual)
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> swiglu_bwd(
     const at::Tensor& dy, const at::Tensor& x, const at::Tensor& gp, const at::Tensor& uo, const at::Tensor& h,
@@ -1033,6 +1181,15 @@ TORCH_LIBRARY(titan, m) {
   m.def("block_ell_swiglu_fwd_train(Tensor x, Tensor values_gate, Tensor col_indices_gate, Tensor? b_gate, "
         "Tensor values_up, Tensor col_indices_up, Tensor? b_up, Tensor values_down, Tensor col_indices_down, "
         "Tensor? b_down, bool add_residual) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
+  m.def("block_ell_gelu_fwd_prepacked(Tensor x, Tensor packed1, Tensor values1, Tensor col_indices1, Tensor? b1, "
+        "Tensor packed2, Tensor values2, Tensor col_indices2, Tensor? b2) -> Tensor");
+  m.def("block_ell_gelu_fwd_train(Tensor x, Tensor values1, Tensor col_indices1, Tensor? b1, Tensor values2, "
+        "Tensor col_indices2, Tensor? b2) -> (Tensor, Tensor, Tensor, Tensor, Tensor)");
+  m.def("block_ell_gelu_train(Tensor x, Tensor values1, Tensor col_indices1, Tensor? b1, Tensor values2, "
+        "Tensor col_indices2, Tensor? b2) -> Tensor");
+  m.def("block_ell_gelu_bwd_train(Tensor grad_out, Tensor x, Tensor pre_act, Tensor h, Tensor values1, "
+        "Tensor col_indices1, Tensor values2, Tensor col_indices2, bool biases) "
+        "-> (Tensor, Tensor, Tensor, Tensor, Tensor)");
   m.def("block_ell_swiglu_train(Tensor x, Tensor values_gate, Tensor col_indices_gate, Tensor? b_gate, "
         "Tensor values_up, Tensor col_indices_up, Tensor? b_up, Tensor values_down, Tensor col_indices_down, "
         "Tensor? b_down, bool add_residual) -> Tensor");
@@ -1097,6 +1254,10 @@ TORCH_LIBRARY_IMPL(titan, CUDA, m) {
   m.impl("block_ell_matmul_bwd_bias", &block_ell_matmul_bwd_bias);
   m.impl("block_ell_swiglu_fwd_train", &swiglu_fwd_train);
   m.impl("block_ell_swiglu_train", &swiglu_train);
+  m.impl("block_ell_gelu_fwd_prepacked", &gelu_fwd_prepacked);
+  m.impl("block_ell_gelu_fwd_train", &gelu_fwd_train);
+  m.impl("block_ell_gelu_train", &gelu_train);
+  m.impl("block_ell_gelu_bwd_train", &gelu_bwd_train);
   m.impl("block_ell_swiglu_bwd_train", &swiglu_bwd_train);
   m.impl("block_ell_matmul_prepack", &block_ell_matmul_prepack);
   m.impl("block_ell_matmul_prepacked", &block_ell_matmul_prepacked);
@@ -1122,16 +1283,18 @@ TORCH_LIBRARY_IMPL(titan, CUDA, m) {
 
 TORCH_LIBRARY_IMPL(titan, CompositeExplicitAutograd, m) { m.impl("unpin_weights_l2", &unpin_weights_l2); }
 
-// block_ell_swiglu_train is differentiable; no other operator has an autograd formula of its own
+// The _train operators are differentiable; no other operator has an autograd formula of its own
 // (torch.autograd.Function in looped_blockell.kernels wraps them and calls them with grad mode off).
 // Outputs of an op called on inputs that require grad get a node that raises on backward,
 // instead of silently carrying no gradient.
 TORCH_LIBRARY_IMPL(titan, Autograd, m) {
   m.impl("block_ell_swiglu_train", &swiglu_train_autograd);
+  m.impl("block_ell_gelu_train", &gelu_train_autograd);
   for (const char* name :
        {"block_ell_swiglu_fwd", "block_ell_swiglu_fwd_with_intermediate", "block_ell_swiglu_bwd",
         "persistent_mlp_step", "block_ell_matmul", "block_ell_matmul_bwd", "block_ell_matmul_bwd_bias",
         "block_ell_swiglu_fwd_train", "block_ell_swiglu_bwd_train",
+        "block_ell_gelu_fwd_prepacked", "block_ell_gelu_fwd_train", "block_ell_gelu_bwd_train",
         "block_ell_swiglu_bwd_ex",
         "block_ell_matmul_prepack", "block_ell_matmul_prepacked",
         "looped_swiglu", "looped_swiglu_persistent", "looped_swiglu_launches", "looped_core", "rmsnorm",
@@ -1212,6 +1375,28 @@ TORCH_LIBRARY_IMPL(titan, Meta, m) {
   m.impl("block_ell_matmul_bwd", [](const at::Tensor&, const at::Tensor& x, const at::Tensor& v, const at::Tensor&) {
     return std::make_tuple(at::empty_like(x), at::empty_like(v));
   });
+  m.impl("block_ell_gelu_fwd_prepacked",
+         [](const at::Tensor& x, const at::Tensor&, const at::Tensor&, const at::Tensor&,
+            const c10::optional<at::Tensor>&, const at::Tensor&, const at::Tensor&, const at::Tensor&,
+            const c10::optional<at::Tensor>&) { return at::empty_like(x); });
+  m.impl("block_ell_gelu_train",
+         [](const at::Tensor& x, const at::Tensor&, const at::Tensor&, const c10::optional<at::Tensor>&,
+            const at::Tensor&, const at::Tensor&, const c10::optional<at::Tensor>&) { return at::empty_like(x); });
+  m.impl("block_ell_gelu_fwd_train",
+         [](const at::Tensor& x, const at::Tensor& v1, const at::Tensor&, const c10::optional<at::Tensor>&,
+            const at::Tensor& v2, const at::Tensor&, const c10::optional<at::Tensor>&) {
+           auto act = [&]() { return at::empty({x.size(0), v1.size(0) * v1.size(2)}, x.options()); };
+           return std::make_tuple(at::empty_like(x), act(), act(), at::empty(v1.sizes(), x.options()),
+                                  at::empty(v2.sizes(), x.options()));
+         });
+  m.impl("block_ell_gelu_bwd_train",
+         [](const at::Tensor&, const at::Tensor& x, const at::Tensor&, const at::Tensor&, const at::Tensor& r1,
+            const at::Tensor&, const at::Tensor& r2, const at::Tensor&, bool biases) {
+           const auto f = x.options().dtype(at::kFloat);
+           return std::make_tuple(at::empty_like(x), at::empty(r1.sizes(), f), at::empty(r2.sizes(), f),
+                                  at::empty({biases ? r1.size(0) * r1.size(2) : 0}, f),
+                                  at::empty({biases ? x.size(1) : 0}, f));
+         });
   m.impl("block_ell_swiglu_train",
          [](const at::Tensor& x, const at::Tensor&, const at::Tensor&, const c10::optional<at::Tensor>&,
             const at::Tensor&, const at::Tensor&, const c10::optional<at::Tensor>&, const at::Tensor&,

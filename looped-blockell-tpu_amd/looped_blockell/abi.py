@@ -108,6 +108,12 @@ SIGNATURES = {
                                                 _P, _P, _P, _P, _SZ, _P]),
     "lbk_swiglu_bwd_workspace_bytes": (_SZ, [_I64, _I32, _PB, _PB, _PB]),
     "lbk_swiglu_bwd_bias_workspace_bytes": (_SZ, [_I64, _I32, _PB, _PB, _PB]),
+    "lbk_gelu_workspace_bytes": (C.c_size_t, [_I64, _I32, _PB, _PB, C.c_int, C.c_int]),
+    "lbk_gelu_fwd_prepacked_bf16": (C.c_int, [_P, _I64, _I32, _PB, _PB, _P, C.c_size_t, _P, C.c_size_t, _P, _P, _P, _P,
+                                              C.c_size_t, _P]),
+    "lbk_gelu_fwd_train": (C.c_int, [_P, _I64, _I32, _PB, _PB, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_size_t, _P]),
+    "lbk_gelu_bwd_workspace_bytes": (C.c_size_t, [_I64, _I32, _PB, _PB]),
+    "lbk_gelu_bwd_train": (C.c_int, [_P, _P, _P, _P, _I64, _I32, _PB, _PB, _P, _P, _P, _P, _P, _P, C.c_size_t, _P]),
     "lbk_swiglu_fwd_train": (C.c_int, [_P, _I64, _I32, _PB, _PB, _PB, _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_int, _P,
                                        _P, _P, _P, _P, C.c_size_t, _P]),
     "lbk_swiglu_bwd_train": (C.c_int, [_P, _P, _P, _P, _P, _I64, _I32, _PB, _PB, _PB, C.c_int, _P, _P, _P, _P, _P, _P,

@@ -165,14 +165,18 @@ class _SwiGLUBiasFunction(torch.autograd.Function):
         return dx, dvg, None, db[0], dvu, None, db[1], dvd, None, db[2], None
 
 
+def _no_transforms():
+    if torch._C._are_functorch_transforms_active():
+        raise RuntimeError("the differentiable FFN operators have no rules for functorch transforms")
+
+
 def swiglu_train(x, v_gate, ci_gate, v_up, ci_up, v_down, ci_down, add_residual: bool = False,
                  b_gate=None, b_up=None, b_down=None):
     """``swiglu`` for fp32 values when gradients are needed: ``titan::block_ell_swiglu_train``, one
     native autograd node.  The values' rounding to bf16 is part of the operator, and their
     gradients come back in fp32."""
     _gpu(x, v_gate, v_down)
-    if torch._C._are_functorch_transforms_active():
-        raise RuntimeError("the differentiable SwiGLU has no rules for functorch transforms")
+    _no_transforms()
     return ops().block_ell_swiglu_train(x, v_gate, ci_gate, b_gate, v_up, ci_up, b_up, v_down, ci_down, b_down,
                                         add_residual)
 
@@ -196,6 +200,21 @@ def swiglu(x, v_gate, ci_gate, v_up, ci_up, v_down, ci_down, add_residual: bool 
     if grad:
         return _SwiGLUFunction.apply(x, v_gate, ci_gate, v_up, ci_up, v_down, ci_down, add_residual)
     return swiglu_fwd(x, v_gate, ci_gate, v_up, ci_up, v_down, ci_down, add_residual)
+
+
+def gelu_train(x, v1, ci1, v2, ci2, b1=None, b2=None):
+    """``gelu(x W1 + b1) W2 + b2`` (tanh form) on fp32 values, differentiable as one native
+    autograd node (``titan::block_ell_gelu_train``); gradients of the values in fp32."""
+    _gpu(x, v1, v2)
+    _no_transforms()
+    return ops().block_ell_gelu_train(x, v1, ci1, b1, v2, ci2, b2)
+
+
+def gelu_fwd_prepacked(x, packed1, v1, ci1, packed2, v2, ci2, b1=None, b2=None):
+    """The same without gradients, from the two weights' ``block_ell_matmul_prepack`` copies: the
+    activation runs in the first product's epilogue."""
+    _gpu(x, v1, v2)
+    return ops().block_ell_gelu_fwd_prepacked(x, packed1, v1, ci1, b1, packed2, v2, ci2, b2)
 
 
 def block_ell_matmul_prepack(values, col_indices, in_features: int):

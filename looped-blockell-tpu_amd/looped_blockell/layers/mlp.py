@@ -25,6 +25,9 @@ a column-index buffer or an alive mask changes (tensor version counters), so suc
 the gate/up and down launches only.  Writes through ``.data`` bypass the version counter: call
 ``release_inference_cache()`` after them.  The cache holds about two bytes per weight element
 twice (bf16 tiles, packed tiles); ``release_inference_cache()`` drops it.
+
+The GELU form is one operator too (``titan::block_ell_gelu_fwd_prepacked``, ``..._gelu_train``)
+unless a hook, a subclass or a replaced method of ``fc1`` / ``fc2`` has to see the two calls.
 """
 
 from __future__ import annotations
@@ -54,6 +57,18 @@ def _versions(lins):
         v, c, a = _tensors(lin)
         key += (v.data_ptr(), v._version, c.data_ptr(), c._version, a.data_ptr(), a._version)
     return key
+
+
+_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+
+
+def _plain(lin):
+    """Whether calling ``lin`` does no more than ``BlockELLLinear.forward``: no subclass, no replaced
+    forward, no hooks on it or on every module."""
+    d = lin.__dict__
+    g = nn.modules.module
+    return (type(lin) is BlockELLLinear and "forward" not in d and "kernel_values" not in d
+            and not any(d[h] for h in _HOOKS) and not any(getattr(g, "_global" + h) for h in _HOOKS))
 
 
 class BlockELLLinear(nn.Module):
@@ -112,9 +127,9 @@ class BlockELLLinear(nn.Module):
 
     def _frozen_weight(self):
         """(bf16 tiles, effective columns, packed copy), rebuilt when the values or the topology change."""
-        cols = self.effective_col_indices()
-        key = (self.values.data_ptr(), self.values._version, self._eff_cache[0])
+        key = _versions((self,))
         if self._frozen is None or self._frozen[0] != key:
+            cols = self.effective_col_indices()
             with torch.inference_mode(False):
                 v = self.kernel_values()
                 self._frozen = (key, v, cols, kernels.block_ell_matmul_prepack(v, cols, self.in_features))
@@ -202,6 +217,20 @@ class MLPBlock(nn.Module):
         """(b_gate, b_up, b_down): the projections' biases (None where a projection has none)."""
         return self.w_gate.bias, self.w_up.bias, self.w_down.bias
 
+    def _gelu(self, x):
+        """The GELU form as one operator, the activation in the first product's epilogue."""
+        fc1, fc2 = self.fc1, self.fc2
+        x2 = x.reshape(-1, x.shape[-1]).to(torch.bfloat16).contiguous()
+        if torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters())):
+            if fc1.values.dtype != torch.float32 or fc2.values.dtype != torch.float32:
+                return fc2(F.gelu(fc1(x).float(), approximate="tanh").to(torch.bfloat16))
+            out = kernels.gelu_train(x2, fc1.values, fc1.effective_col_indices(), fc2.values,
+                                     fc2.effective_col_indices(), fc1.bias, fc2.bias)
+        else:
+            (v1, c1, p1), (v2, c2, p2) = fc1._frozen_weight(), fc2._frozen_weight()
+            out = kernels.gelu_fwd_prepacked(x2, p1, v1, c1, p2, v2, c2, fc1.bias, fc2.bias)
+        return out if x.dim() == 2 else out.reshape(*x.shape[:-1], out.shape[-1])
+
     def forward(self, x: torch.Tensor, deterministic: bool = True) -> torch.Tensor:
         if self.use_swiglu:
             x2 = x.reshape(-1, self.d_model).to(torch.bfloat16).contiguous()
@@ -214,7 +243,9 @@ class MLPBlock(nn.Module):
                 out = kernels.swiglu_fwd_prepacked(x2, packed, *w, add_residual=False, b_gate=bg, b_up=bu, b_down=bd)
             if x.dim() != 2 or x.shape[1] != self.d_model:
                 out = out.reshape(*x.shape[:-1], self.d_model)
-        else:
+        elif x.shape[-1] == self.d_model and _plain(self.fc1) and _plain(self.fc2):
+            out = self._gelu(x)
+        else:                       # the two layers one by one: their hooks and overrides see each
             out = self.fc2(F.gelu(self.fc1(x).float(), approximate="tanh").to(torch.bfloat16))
         if self.dropout > 0.0 and not deterministic:
             out = F.dropout(out, p=self.dropout, training=True)

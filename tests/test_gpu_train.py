@@ -130,3 +130,82 @@ def test_frozen_weights_follow_replacement(gpu):
         assert torch.equal(m(x), fresh())
     with pytest.raises(RuntimeError):
         m(torch.zeros(4, 128, device="cuda", dtype=torch.bfloat16))
+
+
+def _dense(v, c, C):
+    R, K, B, _ = v.shape
+    w = torch.zeros(R, C, B, B, dtype=torch.float64, device=v.device)
+    for k in range(K):
+        col = c[:, k].long()
+        ok = (col >= 0) & (col < C)
+        w[torch.arange(R, device=v.device)[ok], col[ok]] += v[ok, k].double().transpose(-1, -2)
+    return w.permute(0, 2, 1, 3).reshape(R * B, C * B)
+
+
+def _gelu_grad(z):
+    z = z.detach().requires_grad_(True)
+    y = torch.nn.functional.gelu(z, approximate="tanh")
+    return torch.autograd.grad(y.sum(), z)[0]
+
+
+# epilogues of the panel product (B = 16, 32, up to 2048 wide) and of the B = 64 product, and the pass
+# over the product's result (wider inputs, more than 128 slots a row); the backward's panel kernel and
+# the general one (d_model above 2048); one and several token chunks
+@pytest.mark.parametrize("case", [(256, 512, 16, 0.5, 70), (256, 1024, 32, 0.25, 2100), (2048, 256, 32, 0.1, 33),
+                                  (2176, 256, 32, 0.1, 65), (128, 2304, 16, 1.0, 20), (512, 1024, 64, 0.25, 130),
+                                  (256, 512, 64, 0.5, 2), (128, 256, 32, 1.0, 0)])
+def test_gelu_operators(gpu, case):
+    from looped_blockell import kernels
+    d, ff, B, dens, N = case
+    rng = np.random.default_rng(N + d + ff)
+    v1, c1, _, _, v2, c2 = _weights(rng, d, ff, B, dens, 0.1)
+    v1 *= 20.0                                   # pre-activations of order 1
+    b1, b2 = (T.to_gpu((0.3 * rng.standard_normal(n)).astype(np.float32)) for n in (ff, d))
+    x, dy = T.to_gpu_bf16(T.act(rng, N, d)), T.to_gpu_bf16(T.act(rng, N, d))
+    ops = kernels.ops()
+    out, h, pre, r1, r2 = ops.block_ell_gelu_fwd_train(x, v1, c1, b1, v2, c2, b2)
+    assert torch.equal(r1, v1.to(torch.bfloat16)) and torch.equal(r2, v2.to(torch.bfloat16))
+    assert torch.equal(pre, ops.block_ell_matmul(x, r1, c1, b1))
+    assert torch.equal(out, ops.block_ell_matmul(h, r2, c2, b2))
+    # the epilogue applies GELU to the fp32 sum: the exported pre-activation differs by its bf16
+    # rounding (2^-9 of it, slope at most 1.13), h by its own
+    hr = torch.nn.functional.gelu(pre.double(), approximate="tanh")
+    assert ((h.double() - hr).abs() <= 2.0 ** -8 * (hr.abs() + pre.double().abs()) + 1e-6).all()
+    p1, p2 = ops.block_ell_matmul_prepack(r1, c1, d), ops.block_ell_matmul_prepack(r2, c2, ff)
+    assert torch.equal(out, kernels.gelu_fwd_prepacked(x, p1, r1, c1, p2, r2, c2, b1, b2))
+    dx, d1, d2, db1, db2 = ops.block_ell_gelu_bwd_train(dy, x, pre, h, r1, c1, r2, c2, True)
+    w1, w2 = _dense(r1, c1, d // B), _dense(r2, c2, ff // B)
+    da = (dy.double() @ w2) * _gelu_grad(pre.double())
+    D1, D2 = da.T @ x.double(), dy.double().T @ h.double()
+    # bf16 da and dx: 2^-9 each of values that add up over a row; sums in fp32
+    rel = 6e-3
+    for got, want in ((dx, da @ w1), (db1, da.sum(0)), (db2, dy.double().sum(0))):
+        assert (got.double() - want).norm() <= rel * want.norm() + 1e-12
+    for got, c, D, C in ((d1, c1, D1, d // B), (d2, c2, D2, ff // B)):
+        R, K = c.shape
+        tiles = D.reshape(R, B, C, B)[torch.arange(R, device=c.device)[:, None], :, c.clamp(min=0).long()]
+        tiles = tiles.transpose(-1, -2) * (c >= 0)[:, :, None, None]
+        assert got.dtype == torch.float32 and (got[c < 0] == 0).all()
+        assert (got.double() - tiles).norm() <= rel * tiles.norm() + 1e-12
+    none = ops.block_ell_gelu_bwd_train(dy, x, pre, h, r1, c1, r2, c2, False)
+    assert torch.equal(none[0], dx) and none[3].numel() == 0
+
+
+def test_gelu_layer_hooks_and_extremes(gpu):
+    """A hook on fc1 or fc2 still sees its call; the fused forward agrees with the two layers, also at
+    pre-activations where the exponential overflows."""
+    from looped_blockell.layers import MLPBlock
+    torch.manual_seed(4)
+    m = MLPBlock(128, 256, tile_size=32, density=0.5, device="cuda")
+    x = torch.randn(2, 70, 128, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        m.fc1.bias[:4] = torch.tensor([-1e15, 1e15, -60.0, 60.0])
+        fused = m(x)
+        seen = []
+        hook = m.fc1.register_forward_hook(lambda mod, args, y: seen.append(y.shape))
+        split = m(x)
+        hook.remove()
+    assert seen == [torch.Size([2, 70, 256])] and fused.shape == x.shape and torch.isfinite(fused).all()
+    assert (fused.double() - split.double()).norm() <= 8e-3 * split.double().norm()
+    m(x).float().sum().backward()
+    assert all(torch.isfinite(p.grad).all() for p in m.parameters())
