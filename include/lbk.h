@@ -625,6 +625,34 @@ int lbk_gelu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint16
                        const lbk_bell* w2, uint16_t* dx, float* d_v1, float* d_v2, float* d_b1,
                        float* d_b2, void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * Training of the looped block h <- h + SwiGLU(RMSNorm(h)), L >= 1 applications with shared weights,
+ * N >= 1 rows.  The state and its gradient stay in fp32 between the applications.  The forward
+ * rounds the fp32 tiles as lbk_swiglu_fwd_train does and exports per application l, each
+ * [L, N, .] bf16: states (the norm's input), normed (its result), h, gate_pre, up_out.  The backward
+ * returns dh, the norm scale's gradient, fp32 tile gradients and (each optional) bias gradients,
+ * summed over the applications in a fixed order.  The reference differentiates its scan
+ * (looped_blockell/looping/looped_model.py:342-350).
+ */
+size_t lbk_looped_fwd_train_workspace_bytes(int64_t N, int32_t d_model, const lbk_bell* gate,
+                                            const lbk_bell* up, const lbk_bell* down);
+int lbk_looped_fwd_train(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale,
+                         float eps, int32_t L, const lbk_bell* gate, const lbk_bell* up,
+                         const lbk_bell* down, const float* v_gate, const float* v_up, const float* v_down,
+                         uint16_t* vb_gate, uint16_t* vb_up, uint16_t* vb_down, const float* b_gate,
+                         const float* b_up, const float* b_down, uint16_t* out, uint16_t* states,
+                         uint16_t* normed, uint16_t* h, uint16_t* gate_pre, uint16_t* up_out,
+                         void* workspace, size_t workspace_bytes, void* stream);
+size_t lbk_looped_bwd_train_workspace_bytes(int64_t N, int32_t d_model, int32_t L, const lbk_bell* gate,
+                                            const lbk_bell* up, const lbk_bell* down);
+int lbk_looped_bwd_train(const uint16_t* grad_out, const uint16_t* states, const uint16_t* normed,
+                         const uint16_t* h, const uint16_t* gate_pre, const uint16_t* up_out, int64_t N,
+                         int32_t d_model, const float* norm_scale, float eps, int32_t L,
+                         const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down, uint16_t* dh,
+                         float* d_scale, float* d_gate_values, float* d_up_values, float* d_down_values,
+                         float* d_b_gate, float* d_b_up, float* d_b_down, void* workspace,
+                         size_t workspace_bytes, void* stream);
+
 /* ---- prune-time topology transforms (integer and copy work; alive masks are one byte per slot,
  * nonzero = alive).  Replaces the JAX functions of looped_blockell/opt/compaction.py and
  * looped_blockell/opt/column_reorder.py on device. */

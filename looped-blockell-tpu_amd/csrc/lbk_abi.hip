@@ -1261,7 +1261,7 @@ static int swiglu_bwd_impl(const uint16_t* grad_out, const uint16_t* x, const ui
                  int t, const TListJob* tl) {
     const int64_t nt = (int64_t)w->R * w->K;
     if (nt == 0) return;
-    dj[nj++] = DWJob{xx, ldx, gy, ldg, w->col_idx, w->R, w->K, C, part + poff, dw.dv[t], dw.dv32[t],
+    dj[nj++] = DWJob{xx, ldx, gy, ldg, w->col_idx, w->R, w->K, C, part + poff, dw.dv[t], dw.dv32[t], 0,
                      tl ? tl->cnt : nullptr, tl ? tl->list : nullptr, 0, 0};
     poff += dw_part_floats(N, w, C, ldg);
   };
@@ -1275,9 +1275,9 @@ static int swiglu_bwd_impl(const uint16_t* grad_out, const uint16_t* x, const ui
     float* cpart = reinterpret_cast<float*>(reinterpret_cast<char*>(part) + align256(poff * 4));
     ColsumJob cj[3];
     int nc = 0;
-    if (d_b_gate) cj[nc++] = ColsumJob{dg, d_ff, (int)d_ff, d_b_gate, nullptr, 0};
-    if (d_b_up) cj[nc++] = ColsumJob{du, d_ff, (int)d_ff, d_b_up, nullptr, 0};
-    if (d_b_down) cj[nc++] = ColsumJob{grad_out, d_model, d_model, d_b_down, nullptr, 0};
+    if (d_b_gate) cj[nc++] = ColsumJob{dg, d_ff, (int)d_ff, d_b_gate, nullptr, 0, 0};
+    if (d_b_up) cj[nc++] = ColsumJob{du, d_ff, (int)d_ff, d_b_up, nullptr, 0, 0};
+    if (d_b_down) cj[nc++] = ColsumJob{grad_out, d_model, d_model, d_b_down, nullptr, 0, 0};
     if (launch_colsum(cj, nc, N, cpart, s)) return LBK_ERR_LAUNCH;
   }
   return LBK_OK;
@@ -1303,6 +1303,230 @@ int lbk_swiglu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint
   return swiglu_bwd_impl(grad_out, x, gate_pre_act, up_output, h, N, d_model, gate, up, down, add_residual, dx,
                          BwdGrads{{}, {d_gate_values, d_up_values, d_down_values}}, d_b_gate, d_b_up, d_b_down,
                          workspace, workspace_bytes, stream);
+}
+
+// ---- training of the looped block h <- h + SwiGLU(RMSNorm(h)), L times with shared weights
+size_t lbk_looped_fwd_train_workspace_bytes(int64_t N, int32_t d_model, const lbk_bell* gate, const lbk_bell* up,
+                                            const lbk_bell* down) {
+  if (!gate || !up || !down || N <= 0 || d_model <= 0) return 0;
+  // [fp32 state] [y, the products' result where the down kernel does not add to the state] [packed tiles]
+  return align256((size_t)N * d_model * 4) + align256((size_t)N * d_model * 2) +
+         (use_split(gate, up, down, d_model) ? packed_ffn_bytes(gate, up, down) : 0);
+}
+
+int lbk_looped_fwd_train(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale, float eps,
+                         int32_t L, const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down,
+                         const float* v_gate, const float* v_up, const float* v_down, uint16_t* vb_gate,
+                         uint16_t* vb_up, uint16_t* vb_down, const float* b_gate, const float* b_up,
+                         const float* b_down, uint16_t* out, uint16_t* states, uint16_t* normed, uint16_t* h,
+                         uint16_t* gate_pre, uint16_t* up_out, void* workspace, size_t workspace_bytes,
+                         void* stream) {
+  if (!gate || !up || !down) return LBK_ERR_NULL;
+  const MasterFFN m{{v_gate, v_up, v_down}, {vb_gate, vb_up, vb_down}};
+  lbk_bell w3[3] = {*gate, *up, *down};
+  int st;
+  for (int t = 0; t < 3; ++t) {
+    w3[t].values = m.raw[t];
+    if ((st = check_bell(&w3[t]))) return st;
+    if ((int64_t)w3[t].R * w3[t].K > 0) {
+      if (!m.v[t]) return LBK_ERR_NULL;
+      if (!a16(m.v[t]) || !a16(m.raw[t])) return LBK_ERR_ALIGN;
+    }
+  }
+  int64_t d_ff = 0;
+  if ((st = check_ffn(&w3[0], &w3[1], &w3[2], d_model, &d_ff))) return st;
+  if (N <= 0 || L < 1 || !(eps >= 0.f)) return LBK_ERR_ARG;
+  for (const void* q : {(const void*)h_in, (const void*)out, (const void*)states, (const void*)normed, (const void*)h,
+                        (const void*)gate_pre, (const void*)up_out}) {
+    if (!q) return LBK_ERR_NULL;
+    if (!a16(q)) return LBK_ERR_ALIGN;
+  }
+  if (!norm_scale) return LBK_ERR_NULL;
+  if (d_model % 8) return LBK_ERR_ALIGN;
+  if (!workspace || workspace_bytes < lbk_looped_fwd_train_workspace_bytes(N, d_model, gate, up, down))
+    return LBK_ERR_WORKSPACE;
+  if (!a16(workspace)) return LBK_ERR_ALIGN;
+  hipStream_t s = S(stream);
+  char* p = static_cast<char*>(workspace);
+  float* state = reinterpret_cast<float*>(p);
+  p += align256((size_t)N * d_model * 4);
+  uint16_t* y = reinterpret_cast<uint16_t*>(p);
+  p += align256((size_t)N * d_model * 2);
+  const bool split = use_split(&w3[0], &w3[1], &w3[2], d_model);
+  PackedFFN pk{};
+  if ((st = split ? pack_ffn(&w3[0], &w3[1], &w3[2], p, &pk, s, &m) : cast_ffn(&w3[0], &w3[1], &w3[2], m, s)))
+    return st;
+  const Biases bs{b_gate, b_up, b_down};
+  const int64_t nd = N * d_model, nf = N * d_ff;
+  if (launch_state_init(h_in, nd, state, states, s)) return LBK_ERR_LAUNCH;
+  for (int l = 0; l < L; ++l) {
+    const uint16_t* xn = normed + l * nd;
+    uint16_t* next = l + 1 < L ? states + (l + 1) * nd : out;     // bf16 of the state after this application
+    if (launch_rmsnorm(states + l * nd, N, d_model, norm_scale, eps, normed + l * nd, s)) return LBK_ERR_LAUNCH;
+    if (split) {
+      if ((st = swiglu_split(xn, nullptr, nullptr, 0.f, N, d_model, &w3[0], &w3[1], &w3[2], pk, nullptr, state, next,
+                             h + l * nf, gate_pre + l * nf, up_out + l * nf, s, bs)))
+        return st;
+    } else {
+      if ((st = swiglu_general(xn, N, d_model, &w3[0], &w3[1], &w3[2], nullptr, y, h + l * nf, gate_pre + l * nf,
+                               up_out + l * nf, s, bs)))
+        return st;
+      if (launch_core_update(state, y, nullptr, 0, nullptr, nullptr, N, d_model, next, s)) return LBK_ERR_LAUNCH;
+    }
+  }
+  return LBK_OK;
+}
+
+// Applications whose dg, du and dy the backward keeps before one pass over all of their tokens sums
+// the weight gradients: as many as fit 2 GiB of dg and du
+static int64_t loop_group(int64_t N, int64_t d_ff, int32_t L) {
+  const int64_t g = ((int64_t)1 << 31) / (N * d_ff * 4 > 0 ? N * d_ff * 4 : 1);
+  return g < 1 ? 1 : g < L ? g : L;
+}
+
+struct LoopBwdLayout {
+  size_t lists, dg, dy, dy_next, dxn, tmp, g, dw, cs, rms, total;
+};
+static LoopBwdLayout loop_bwd_layout(int64_t N, int32_t d_model, int32_t L, const lbk_bell* gate, const lbk_bell* up,
+                                     const lbk_bell* down) {
+  const int C_in = d_model / gate->B, C_d = gate->R;
+  const int64_t d_ff = (int64_t)gate->R * gate->B, G = loop_group(N, d_ff, L);
+  LoopBwdLayout l{};
+  l.lists = tlist_bytes(down, C_d) + tlist_bytes(gate, C_in) + tlist_bytes(up, C_in);
+  l.dg = align256((size_t)G * N * d_ff * 2);
+  l.dy = align256((size_t)G * N * d_model * 2);
+  l.dy_next = l.dxn = l.tmp = align256((size_t)N * d_model * 2);
+  l.g = align256((size_t)N * d_model * 4);
+  // token counts of the passes: whole groups, and the last one
+  for (const int64_t n : {G * N, (L % G) * N}) {
+    if (n == 0) continue;
+    const size_t dw = align256((dw_part_floats(n, gate, C_in, d_ff) + dw_part_floats(n, up, C_in, d_ff) +
+                                dw_part_floats(n, down, C_d, d_model)) * 4);
+    const size_t cs = align256(colsum_bytes(n, 2 * d_ff + d_model));
+    l.dw = dw > l.dw ? dw : l.dw;
+    l.cs = cs > l.cs ? cs : l.cs;
+  }
+  l.rms = align256((size_t)G * rmsnorm_bwd_bytes(N, d_model));
+  l.total = l.lists + 2 * l.dg + l.dy + l.dy_next + l.dxn + l.tmp + l.g + l.dw + l.cs + l.rms;
+  return l;
+}
+
+size_t lbk_looped_bwd_train_workspace_bytes(int64_t N, int32_t d_model, int32_t L, const lbk_bell* gate,
+                                            const lbk_bell* up, const lbk_bell* down) {
+  int64_t d_ff = 0;
+  if (check_bell(gate) || check_bell(up) || check_bell(down) || check_ffn(gate, up, down, d_model, &d_ff)) return 0;
+  if (N <= 0 || L < 1) return 0;
+  return loop_bwd_layout(N, d_model, L, gate, up, down).total;
+}
+
+int lbk_looped_bwd_train(const uint16_t* grad_out, const uint16_t* states, const uint16_t* normed, const uint16_t* h,
+                         const uint16_t* gate_pre, const uint16_t* up_out, int64_t N, int32_t d_model,
+                         const float* norm_scale, float eps, int32_t L, const lbk_bell* gate, const lbk_bell* up,
+                         const lbk_bell* down, uint16_t* dh, float* d_scale, float* d_gate_values, float* d_up_values,
+                         float* d_down_values, float* d_b_gate, float* d_b_up, float* d_b_down, void* workspace,
+                         size_t workspace_bytes, void* stream) {
+  int st;
+  if ((st = check_bell(gate)) || (st = check_bell(up)) || (st = check_bell(down))) return st;
+  int64_t d_ff = 0;
+  if ((st = check_ffn(gate, up, down, d_model, &d_ff))) return st;
+  if (N <= 0 || L < 1 || !(eps >= 0.f)) return LBK_ERR_ARG;
+  const int B = gate->B;
+  const int64_t tg = (int64_t)gate->R * gate->K, tu = (int64_t)up->R * up->K, td = (int64_t)down->R * down->K;
+  if (!norm_scale || !d_scale || (tg && !d_gate_values) || (tu && !d_up_values) || (td && !d_down_values))
+    return LBK_ERR_NULL;
+  for (const void* q : {(const void*)grad_out, (const void*)states, (const void*)normed, (const void*)h,
+                        (const void*)gate_pre, (const void*)up_out, (const void*)dh}) {
+    if (!q) return LBK_ERR_NULL;
+    if (!a16(q)) return LBK_ERR_ALIGN;
+  }
+  for (const void* q : {(const void*)d_gate_values, (const void*)d_up_values, (const void*)d_down_values,
+                        (const void*)gate->values, (const void*)up->values, (const void*)down->values})
+    if (q && !a16(q)) return LBK_ERR_ALIGN;
+  if (d_model % 8) return LBK_ERR_ALIGN;
+  const LoopBwdLayout lay = loop_bwd_layout(N, d_model, L, gate, up, down);
+  if (!workspace || workspace_bytes < lay.total) return LBK_ERR_WORKSPACE;
+  if (!a16(workspace)) return LBK_ERR_ALIGN;
+  hipStream_t s = S(stream);
+  const int C_in = d_model / B, C_d = gate->R;
+  char* p = static_cast<char*>(workspace);
+  auto take = [&](size_t bytes) {
+    char* q = p;
+    p += align256(bytes);
+    return q;
+  };
+  const lbk_bell* w3[3] = {down, gate, up};
+  const int c3[3] = {C_d, C_in, C_in};
+  TListJob lj[3], ljn[3];
+  int nl = 0;
+  for (int t = 0; t < 3; ++t) {
+    lj[t] = TListJob{w3[t]->col_idx, w3[t]->R, w3[t]->K, c3[t], nullptr, nullptr};
+    lj[t].cnt = reinterpret_cast<int32_t*>(take((size_t)c3[t] * 4));
+    lj[t].list = reinterpret_cast<int32_t*>(take((size_t)c3[t] * w3[t]->R * w3[t]->K * 4));
+    if ((int64_t)w3[t]->R * w3[t]->K > 0) ljn[nl++] = lj[t];
+  }
+  uint16_t* dg = reinterpret_cast<uint16_t*>(take(lay.dg));
+  uint16_t* du = reinterpret_cast<uint16_t*>(take(lay.dg));
+  uint16_t* dy = reinterpret_cast<uint16_t*>(take(lay.dy));
+  uint16_t* dy_next = reinterpret_cast<uint16_t*>(take(lay.dy_next));
+  uint16_t* dxn = reinterpret_cast<uint16_t*>(take(lay.dxn));
+  uint16_t* tmp = reinterpret_cast<uint16_t*>(take(lay.tmp));
+  float* g = reinterpret_cast<float*>(take(lay.g));
+  float* part = reinterpret_cast<float*>(take(lay.dw));
+  float* cpart = reinterpret_cast<float*>(take(lay.cs));
+  float* rpart = reinterpret_cast<float*>(p);
+  if (nl && launch_tlist(ljn, nl, s)) return LBK_ERR_LAUNCH;
+  const int64_t nd = N * d_model, nf = N * d_ff, G = loop_group(N, d_ff, L);
+  for (int64_t hi = L; hi > 0;) {
+    const int64_t lo = hi > G ? hi - G : 0, n = hi - lo;
+    const int acc = hi < L;
+    // the gradient of the state after application hi - 1, into its slot (and, at the end of the
+    // block, into the fp32 state gradient)
+    if (launch_state_init(acc ? dy_next : grad_out, nd, acc ? nullptr : g, dy + (n - 1) * nd, s)) return LBK_ERR_LAUNCH;
+    int64_t nblk = 0;
+    for (int64_t t = hi - 1; t >= lo; --t) {
+      const int64_t q = t - lo;
+      TProdArgs a{};
+      if (td > 0) a.src[a.nsrc++] = TProdSrc{dy + q * nd, d_model, down->values, down->K, lj[0].cnt, lj[0].list, td};
+      a.N = N; a.C = C_d; a.ldo = d_ff;
+      a.g = gate_pre + t * nf; a.u = up_out + t * nf; a.dg = dg + q * nf; a.du = du + q * nf;
+      if (launch_tprod(B, 0, a, s)) return LBK_ERR_LAUNCH;
+      TProdArgs b{};
+      if (tg > 0) b.src[b.nsrc++] = TProdSrc{dg + q * nf, d_ff, gate->values, gate->K, lj[1].cnt, lj[1].list, tg};
+      if (tu > 0) b.src[b.nsrc++] = TProdSrc{du + q * nf, d_ff, up->values, up->K, lj[2].cnt, lj[2].list, tu};
+      b.N = N; b.C = C_in; b.ldo = d_model;
+      b.out = dxn;
+      if (launch_tprod(B, 1, b, s)) return LBK_ERR_LAUNCH;
+      uint16_t* prev = t == 0 ? dh : q > 0 ? dy + (q - 1) * nd : dy_next;
+      nblk = rmsnorm_bwd_blocks(states + t * nd, dxn, N, d_model, norm_scale, prev);
+      if (launch_rmsnorm_bwd_part(states + t * nd, dxn, N, d_model, norm_scale, eps, g, prev, tmp,
+                                  rpart + q * nblk * d_model, s))
+        return LBK_ERR_LAUNCH;
+    }
+    // the group's weight, bias and scale gradients over its n N tokens
+    DWJob dj[3];
+    int nj = 0;
+    size_t poff = 0;
+    auto add = [&](const uint16_t* xx, int64_t ldx, const uint16_t* gy, int64_t ldg, const lbk_bell* w, int C,
+                   float* dst, const TListJob* tl) {
+      if ((int64_t)w->R * w->K == 0) return;
+      dj[nj++] = DWJob{xx, ldx, gy, ldg, w->col_idx, w->R, w->K, C, part + poff, nullptr, dst, acc,
+                       tl ? tl->cnt : nullptr, tl ? tl->list : nullptr, 0, 0};
+      poff += dw_part_floats(n * N, w, C, ldg);
+    };
+    add(normed + lo * nd, d_model, dg, d_ff, gate, C_in, d_gate_values, nullptr);
+    add(normed + lo * nd, d_model, du, d_ff, up, C_in, d_up_values, nullptr);
+    add(h + lo * nf, d_ff, dy, d_model, down, C_d, d_down_values, &lj[0]);
+    if (nj && launch_dw(B, dj, nj, n * N, s)) return LBK_ERR_LAUNCH;
+    ColsumJob cj[3];
+    int nc = 0;
+    if (d_b_gate) cj[nc++] = ColsumJob{dg, d_ff, (int)d_ff, d_b_gate, nullptr, 0, acc};
+    if (d_b_up) cj[nc++] = ColsumJob{du, d_ff, (int)d_ff, d_b_up, nullptr, 0, acc};
+    if (d_b_down) cj[nc++] = ColsumJob{dy, d_model, d_model, d_b_down, nullptr, 0, acc};
+    if (nc && launch_colsum(cj, nc, n * N, cpart, s)) return LBK_ERR_LAUNCH;
+    if (launch_rmsnorm_dscale(rpart, n * nblk, d_model, d_scale, acc, s)) return LBK_ERR_LAUNCH;
+    hi = lo;
+  }
+  return LBK_OK;
 }
 
 // ---- the GELU FFN out = W2 gelu(W1 x + b1) + b2
@@ -1501,15 +1725,15 @@ int lbk_gelu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint16
   DWJob dj[2];
   int nj = 0;
   if (t1 > 0)
-    dj[nj++] = DWJob{x, d_model, da, d_ff, w1->col_idx, w1->R, w1->K, C_in, part, nullptr, d_v1, nullptr, nullptr, 0, 0};
+    dj[nj++] = DWJob{x, d_model, da, d_ff, w1->col_idx, w1->R, w1->K, C_in, part, nullptr, d_v1, 0, nullptr, nullptr, 0, 0};
   if (t2 > 0)
-    dj[nj++] = DWJob{h, d_ff, grad_out, d_model, w2->col_idx, w2->R, w2->K, C_d, part + f1, nullptr, d_v2,
+    dj[nj++] = DWJob{h, d_ff, grad_out, d_model, w2->col_idx, w2->R, w2->K, C_d, part + f1, nullptr, d_v2, 0,
                      N > 0 ? lj[0].cnt : nullptr, N > 0 ? lj[0].list : nullptr, 0, 0};
   if (nj && launch_dw(B, dj, nj, N, s)) return LBK_ERR_LAUNCH;
   ColsumJob cj[2];
   int nc = 0;
-  if (d_b1 && d_ff > 0) cj[nc++] = ColsumJob{da, d_ff, (int)d_ff, d_b1, nullptr, 0};
-  if (d_b2) cj[nc++] = ColsumJob{grad_out, d_model, d_model, d_b2, nullptr, 0};
+  if (d_b1 && d_ff > 0) cj[nc++] = ColsumJob{da, d_ff, (int)d_ff, d_b1, nullptr, 0, 0};
+  if (d_b2) cj[nc++] = ColsumJob{grad_out, d_model, d_model, d_b2, nullptr, 0, 0};
   if (nc && launch_colsum(cj, nc, N, cpart, s)) return LBK_ERR_LAUNCH;
   return LBK_OK;
 }
@@ -1578,7 +1802,7 @@ int lbk_block_ell_matmul_bwd_bias_bf16(const uint16_t* grad_out, const uint16_t*
   if (d_values && nt > 0) {
     // the transposed lists exist when dx was computed above
     const bool lists = dx && N > 0;
-    DWJob dj{x, in_features, grad_out, out_f, w->col_idx, w->R, w->K, C, part, d_values, nullptr,
+    DWJob dj{x, in_features, grad_out, out_f, w->col_idx, w->R, w->K, C, part, d_values, nullptr, 0,
              lists ? lj.cnt : nullptr, lists ? lj.list : nullptr, 0, 0};
     if (launch_dw(B, &dj, 1, N, s)) return LBK_ERR_LAUNCH;
   }

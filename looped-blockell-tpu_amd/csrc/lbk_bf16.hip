@@ -257,11 +257,13 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const uint16_t* __rest
 // `rows` rows go to its four waves in turn, the next row's loads in flight; the waves' dscale
 // partials meet in LDS.  2048 x 512: 56.2 -> 4.6 us (and the reduction of 256
 // partials 5.0 us, 8.4 for 32 partials one thread a column).
-template <int NC>
+// STATE: dx is added to the fp32 state gradient gs, whose bf16 rounding is stored as dx.
+template <int NC, bool STATE>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_vec_kernel(const uint16_t* __restrict__ x,
                                                               const uint16_t* __restrict__ dy, int64_t N, int d,
                                                               const float* __restrict__ scale, float eps, int rows,
-                                                              uint16_t* __restrict__ dx, float* __restrict__ part) {
+                                                              float* __restrict__ gs, uint16_t* __restrict__ dx,
+                                                              float* __restrict__ part) {
   __shared__ float sums[4][512 * NC];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t r0 = (int64_t)blockIdx.x * rows;
@@ -321,7 +323,19 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_vec_kernel(const uint16_t* __
         o[q] = rs * sc[j][q] * gv[j][q] - xv[j][q] * coef;
         ds[j][q] += gv[j][q] * xv[j][q] * rs;
       }
-      if (col < d) store_bf16x<8>(dx + (r0 + rr) * d + col, o);
+      if (col >= d) continue;
+      const int64_t off = (r0 + rr) * d + col;
+      if constexpr (STATE) {
+        f32x4 g0 = *reinterpret_cast<const f32x4*>(gs + off), g1 = *reinterpret_cast<const f32x4*>(gs + off + 4);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          o[q] = g0[q] += o[q];
+          o[4 + q] = g1[q] += o[4 + q];
+        }
+        *reinterpret_cast<f32x4*>(gs + off) = g0;
+        *reinterpret_cast<f32x4*>(gs + off + 4) = g1;
+      }
+      store_bf16x<8>(dx + off, o);
     }
   }
 #pragma unroll
@@ -410,7 +424,10 @@ __global__ __launch_bounds__(256) void colsum_reduce_kernel(ColsumJobs jobs) {
   }
   sums[tq][tc] = s;
   __syncthreads();
-  if (tq == 0 && c < J.C) J.out[c] = (sums[0][tc] + sums[1][tc]) + (sums[2][tc] + sums[3][tc]);
+  if (tq == 0 && c < J.C) {
+    const float t = (sums[0][tc] + sums[1][tc]) + (sums[2][tc] + sums[3][tc]);
+    J.out[c] = J.acc ? J.out[c] + t : t;
+  }
 }
 
 // rows per chunk: 64 keeps thousands of workgroups on short inputs, 256 keeps the partials a 128th
@@ -465,28 +482,73 @@ static bool aligned16(std::initializer_list<const void*> ps) {
   return true;
 }
 
-int launch_rmsnorm_bwd(const uint16_t* x, const uint16_t* dy, int64_t N, int d, const float* scale, float eps,
-                       uint16_t* dx, float* dscale, float* part, hipStream_t st) {
-  const bool vec = d % 8 == 0 && d <= 2048 && aligned16({x, dy, scale, dx});
-  const int rows = vec ? rmsnorm_bwd_rows(N) : RMS_BWD_ROWS;
-  const int64_t nblk = (N + rows - 1) / rows;
+static bool rmsnorm_bwd_vec(const uint16_t* x, const uint16_t* dy, int d, const float* scale, const uint16_t* dx) {
+  return d % 8 == 0 && d <= 2048 && aligned16({x, dy, scale, dx});
+}
+
+int64_t rmsnorm_bwd_blocks(const uint16_t* x, const uint16_t* dy, int64_t N, int d, const float* scale,
+                           const uint16_t* dx) {
+  const int rows = rmsnorm_bwd_vec(x, dy, d, scale, dx) ? rmsnorm_bwd_rows(N) : RMS_BWD_ROWS;
+  return (N + rows - 1) / rows;
+}
+
+int launch_rmsnorm_bwd_part(const uint16_t* x, const uint16_t* dy, int64_t N, int d, const float* scale, float eps,
+                            float* gs, uint16_t* dx, uint16_t* dx_tmp, float* part, hipStream_t st) {
+  const int64_t nblk = rmsnorm_bwd_blocks(x, dy, N, d, scale, dx);
   if (nblk > 0x7fffffff) return -2;
-  if (nblk > 0) {
-    const dim3 grid((unsigned)nblk), block(256);
-    if (!vec)
-      hipLaunchKernelGGL(rmsnorm_bwd_kernel, grid, block, 0, st, x, dy, N, d, scale, eps, dx, part);
-    else if (d <= 512)
-      hipLaunchKernelGGL(rmsnorm_bwd_vec_kernel<1>, grid, block, 0, st, x, dy, N, d, scale, eps, rows, dx, part);
-    else if (d <= 1024)
-      hipLaunchKernelGGL(rmsnorm_bwd_vec_kernel<2>, grid, block, 0, st, x, dy, N, d, scale, eps, rows, dx, part);
-    else
-      hipLaunchKernelGGL(rmsnorm_bwd_vec_kernel<4>, grid, block, 0, st, x, dy, N, d, scale, eps, rows, dx, part);
+  if (nblk == 0) return 0;
+  const dim3 grid((unsigned)nblk), block(256);
+  if (!rmsnorm_bwd_vec(x, dy, d, scale, dx)) {
+    hipLaunchKernelGGL(rmsnorm_bwd_kernel, grid, block, 0, st, x, dy, N, d, scale, eps, gs ? dx_tmp : dx, part);
     if (hipGetLastError() != hipSuccess) return -1;
+    return gs ? launch_core_update(gs, dx_tmp, nullptr, 0, nullptr, nullptr, N, d, dx, st) : 0;
   }
+  const int rows = rmsnorm_bwd_rows(N);
+#define LBK_RMSB(NC)                                                                                              \
+  {                                                                                                               \
+    if (gs) hipLaunchKernelGGL((rmsnorm_bwd_vec_kernel<NC, true>), grid, block, 0, st, x, dy, N, d, scale, eps, rows, \
+                               gs, dx, part);                                                                     \
+    else hipLaunchKernelGGL((rmsnorm_bwd_vec_kernel<NC, false>), grid, block, 0, st, x, dy, N, d, scale, eps, rows,  \
+                            gs, dx, part);                                                                        \
+  }
+  if (d <= 512) LBK_RMSB(1) else if (d <= 1024) LBK_RMSB(2) else LBK_RMSB(4)
+#undef LBK_RMSB
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int launch_rmsnorm_dscale(float* part, int64_t nblk, int d, float* dscale, int acc, hipStream_t st) {
+  if (nblk > 0x7fffffff) return -2;
   ColsumJobs J{};
   J.n = 1;
-  J.job[0] = ColsumJob{nullptr, 0, d, dscale, part, (int)nblk};
+  J.job[0] = ColsumJob{nullptr, 0, d, dscale, part, (int)nblk, acc};
   hipLaunchKernelGGL(colsum_reduce_kernel, dim3((unsigned)((d + 63) / 64)), dim3(256), 0, st, J);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int launch_rmsnorm_bwd(const uint16_t* x, const uint16_t* dy, int64_t N, int d, const float* scale, float eps,
+                       uint16_t* dx, float* dscale, float* part, hipStream_t st) {
+  const int rc = launch_rmsnorm_bwd_part(x, dy, N, d, scale, eps, nullptr, dx, nullptr, part, st);
+  return rc ? rc : launch_rmsnorm_dscale(part, rmsnorm_bwd_blocks(x, dy, N, d, scale, dx), d, dscale, 0, st);
+}
+
+__global__ __launch_bounds__(256) void state_init_kernel(const uint16_t* __restrict__ x, int64_t n8,
+                                                         float* __restrict__ y32, uint16_t* __restrict__ y16) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= n8) return;
+  const u32x4 v = reinterpret_cast<const u32x4*>(x)[e];
+  if (y16) reinterpret_cast<u32x4*>(y16)[e] = v;
+  if (y32) {
+    float f[8];
+    unpack8_bf16(v, f);
+    reinterpret_cast<f32x4*>(y32)[2 * e] = f32x4{f[0], f[1], f[2], f[3]};
+    reinterpret_cast<f32x4*>(y32)[2 * e + 1] = f32x4{f[4], f[5], f[6], f[7]};
+  }
+}
+
+int launch_state_init(const uint16_t* x, int64_t n, float* y32, uint16_t* y16, hipStream_t st) {
+  if (n == 0) return 0;
+  if (n % 8) return -2;
+  hipLaunchKernelGGL(state_init_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, st, x, n / 8, y32, y16);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

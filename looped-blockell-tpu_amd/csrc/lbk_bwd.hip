@@ -1871,6 +1871,7 @@ __global__ __launch_bounds__(256) void dw_reduce_kernel(DWJobs jobs, int B) {
     }
   }
   if (J.dw32) {
+    if (J.acc) s += *reinterpret_cast<const f32x4*>(J.dw32 + idx);
     *reinterpret_cast<f32x4*>(J.dw32 + idx) = s;
   } else {
     const float o[4] = {s[0], s[1], s[2], s[3]};

@@ -191,6 +191,7 @@ struct ColsumJob {
   float* out;
   float* part;               // set by launch_colsum
   int nchunk;
+  int acc;                   // add to out instead of writing it
 };
 struct ColsumJobs {
   static constexpr int kMax = 3;
@@ -203,6 +204,17 @@ size_t colsum_bytes(int64_t N, int64_t C);
 int launch_colsum(const ColsumJob* jobs, int n, int64_t N, float* part, hipStream_t st);
 int launch_rmsnorm_bwd(const uint16_t* x, const uint16_t* dy, int64_t N, int d, const float* scale, float eps,
                        uint16_t* dx, float* dscale, float* part, hipStream_t st);
+// the backward's first launch alone, for the looped block's training: dscale's partials of
+// rmsnorm_bwd_blocks workgroups to part, and with the fp32 state gradient gs [N, d]
+// gs += dx, dx = bf16(gs) (dx_tmp [N, d] holds the product where the kernel has no such epilogue)
+int64_t rmsnorm_bwd_blocks(const uint16_t* x, const uint16_t* dy, int64_t N, int d, const float* scale,
+                           const uint16_t* dx);
+int launch_rmsnorm_bwd_part(const uint16_t* x, const uint16_t* dy, int64_t N, int d, const float* scale, float eps,
+                            float* gs, uint16_t* dx, uint16_t* dx_tmp, float* part, hipStream_t st);
+// dscale (+)= the sum of nblk partials
+int launch_rmsnorm_dscale(float* part, int64_t nblk, int d, float* dscale, int acc, hipStream_t st);
+// y32 (optional) = x in fp32, y16 (optional) = x; n % 8 == 0, 16-byte aligned
+int launch_state_init(const uint16_t* x, int64_t n, float* y32, uint16_t* y16, hipStream_t st);
 int launch_injection(const uint16_t* h, const uint16_t* e, const float* log_A, const float* log_dt, int64_t N,
                      int d, uint16_t* out, hipStream_t st);
 size_t injection_bwd_bytes(int64_t N, int d);   // fp32 column partials (two per row block)
@@ -321,6 +333,7 @@ struct DWJob {
   float* part;                       // [nchunk, R*K, B, B]
   uint16_t* dw;                      // [R, K, B, B] bf16
   float* dw32;                       // the same in fp32, unrounded (one of the two)
+  int acc;                           // with dw32: add to it instead of writing it
   // optional transposed topology of launch_tlist (per column block c: tcnt[c] slots e at
   // tlist[c * R * K ..]); lets a weight with wide input rows and narrow output rows (the down
   // projection) stage its G rows whole and walk the slots of each input column block

@@ -970,6 +970,157 @@ Tensor swiglu_train_autograd(const Tensor& x, const Tensor& vg, const Tensor& cg
   return SwigluTrain::apply(x, vg, cg, bg, vu, cu, bu, vd, cd, bd, add_residual);
 }
 
+// ------------------------------------------------------------------ looped block
+// [out, states, normed, h, gate_pre, up_out, and the bf16 copies of the three weights]
+std::vector<Tensor> looped_fwd_train(const Tensor& h_, const Tensor& scale_, const Tensor& vg_, const Tensor& cg_,
+                                     const OptTensor& bg_, const Tensor& vu_, const Tensor& cu_, const OptTensor& bu_,
+                                     const Tensor& vd_, const Tensor& cd_, const OptTensor& bd_, int64_t L,
+                                     double eps) {
+  const char* op = "looped_swiglu_fwd_train";
+  Tensor vg = vg_, cg = cg_, vu = vu_, cu = cu_, vd = vd_, cd = cd_;
+  Tensor x = check_x2d(h_, op);
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
+  lbk_bell g = make_master(vg, cg, op, "gate"), u = make_master(vu, cu, op, "up"),
+           d = make_master(vd, cd, op, "down");
+  const int64_t N = x.size(0), d_model = x.size(1);
+  TORCH_CHECK(N >= 1 && L >= 1, "titan::", op, ": needs at least one row and one application");
+  TORCH_CHECK((int64_t)d.R * d.B == d_model, "titan::", op, ": values_down R_model=", d.R,
+              " inconsistent with d_model=", d_model);
+  TORCH_CHECK(g.R == u.R, "titan::", op, ": gate and up must have same R_ff");
+  Tensor sc = scale_.to(x.device(), at::kFloat).contiguous();
+  TORCH_CHECK(sc.numel() == d_model, "titan::", op, ": norm scale must have d_model elements");
+  const int64_t d_ff = (int64_t)g.R * g.B;
+  const Tensor bg = opt_bias(bg_, d_ff, x, op, "b_gate"), bu = opt_bias(bu_, d_ff, x, op, "b_up"),
+               bd = opt_bias(bd_, d_model, x, op, "b_down");
+  Tensor out = at::empty({N, d_model}, x.options()), states = at::empty({L, N, d_model}, x.options()),
+         normed = at::empty({L, N, d_model}, x.options()), h = at::empty({L, N, d_ff}, x.options()),
+         gp = at::empty({L, N, d_ff}, x.options()), uo = at::empty({L, N, d_ff}, x.options());
+  Tensor wg = at::empty(vg.sizes(), x.options()), wu = at::empty(vu.sizes(), x.options()),
+         wd = at::empty(vd.sizes(), x.options());
+  g.values = bf(wg);
+  u.values = bf(wu);
+  d.values = bf(wd);
+  const size_t wsb = lbk_looped_fwd_train_workspace_bytes(N, (int32_t)d_model, &g, &u, &d);
+  Tensor ws = workspace(wsb, x);
+  LBK_CALL("looped_swiglu_fwd_train",
+           lbk_looped_fwd_train(bf(x), N, (int32_t)d_model, sc.data_ptr<float>(), (float)eps, (int32_t)L, &g, &u, &d,
+                                vg.data_ptr<float>(), vu.data_ptr<float>(), vd.data_ptr<float>(), bfm(wg), bfm(wu),
+                                bfm(wd), fptr(bg), fptr(bu), fptr(bd), bfm(out), bfm(states), bfm(normed), bfm(h),
+                                bfm(gp), bfm(uo), ws.data_ptr(), wsb, cur_stream(x)));
+  return {out, states, normed, h, gp, uo, wg, wu, wd};
+}
+
+// [dh, d_scale, fp32 tile gradients of gate, up, down, fp32 bias gradients (empty without biases)]
+std::vector<Tensor> looped_bwd_train(const Tensor& dy_, const Tensor& states_, const Tensor& normed_,
+                                     const Tensor& h_, const Tensor& gp_, const Tensor& uo_, const Tensor& scale_,
+                                     const Tensor& wg_, const Tensor& cg_, const Tensor& wu_, const Tensor& cu_,
+                                     const Tensor& wd_, const Tensor& cd_, double eps, bool biases) {
+  const char* op = "looped_swiglu_bwd_train";
+  Tensor vg = wg_, cg = cg_, vu = wu_, cu = cu_, vd = wd_, cd = cd_;
+  Tensor dy = check_x2d(dy_, op);
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(dy.device());
+  lbk_bell g = make_bell(vg, cg, op, "gate"), u = make_bell(vu, cu, op, "up"), d = make_bell(vd, cd, op, "down");
+  const int64_t N = dy.size(0), d_model = dy.size(1), d_ff = (int64_t)g.R * g.B, L = states_.size(0);
+  auto act = [&](const Tensor& t, int64_t cols, const char* name) {
+    check_gpu(t, op, name);
+    TORCH_CHECK(t.scalar_type() == at::kBFloat16 && t.dim() == 3 && t.size(0) == L && t.size(1) == N &&
+                    t.size(2) == cols, "titan::", op, ": ", name, " must be bf16 [", L, ", ", N, ", ", cols, "], got ",
+                t.sizes());
+    return t.contiguous();
+  };
+  Tensor states = act(states_, d_model, "states"), normed = act(normed_, d_model, "normed"),
+         h = act(h_, d_ff, "h"), gp = act(gp_, d_ff, "gate_pre_act"), uo = act(uo_, d_ff, "up_output");
+  Tensor sc = scale_.to(dy.device(), at::kFloat).contiguous();
+  TORCH_CHECK(sc.numel() == d_model, "titan::", op, ": norm scale must have d_model elements");
+  const auto f32 = dy.options().dtype(at::kFloat);
+  Tensor dh = at::empty({N, d_model}, dy.options()), ds = at::empty({d_model}, f32);
+  Tensor dvg = at::empty(vg.sizes(), f32), dvu = at::empty(vu.sizes(), f32), dvd = at::empty(vd.sizes(), f32);
+  Tensor dbg = at::empty({biases ? d_ff : 0}, f32), dbu = at::empty({biases ? d_ff : 0}, f32),
+         dbd = at::empty({biases ? d_model : 0}, f32);
+  auto fp = [&](Tensor& t) { return biases ? t.data_ptr<float>() : nullptr; };
+  const size_t wsb = lbk_looped_bwd_train_workspace_bytes(N, (int32_t)d_model, (int32_t)L, &g, &u, &d);
+  Tensor ws = workspace(wsb, dy);
+  LBK_CALL("looped_swiglu_bwd_train",
+           lbk_looped_bwd_train(bf(dy), bf(states), bf(normed), bf(h), bf(gp), bf(uo), N, (int32_t)d_model,
+                                sc.data_ptr<float>(), (float)eps, (int32_t)L, &g, &u, &d, bfm(dh),
+                                ds.data_ptr<float>(), dvg.data_ptr<float>(), dvu.data_ptr<float>(),
+                                dvd.data_ptr<float>(), fp(dbg), fp(dbu), fp(dbd), ws.data_ptr(), wsb, cur_stream(dy)));
+  return {dh, ds, dvg, dvu, dvd, dbg, dbu, dbd};
+}
+
+std::vector<Tensor> call_looped_fwd_train(const Tensor& h, const Tensor& sc, const Tensor& vg, const Tensor& cg,
+                                          const OptTensor& bg, const Tensor& vu, const Tensor& cu, const OptTensor& bu,
+                                          const Tensor& vd, const Tensor& cd, const OptTensor& bd, int64_t L,
+                                          double eps) {
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("titan::looped_swiglu_fwd_train", "")
+                             .typed<decltype(looped_fwd_train)>();
+  return op.call(h, sc, vg, cg, bg, vu, cu, bu, vd, cd, bd, L, eps);
+}
+
+std::vector<Tensor> call_looped_bwd_train(const Tensor& dy, const Tensor& st, const Tensor& xn, const Tensor& h,
+                                          const Tensor& gp, const Tensor& uo, const Tensor& sc, const Tensor& wg,
+                                          const Tensor& cg, const Tensor& wu, const Tensor& cu, const Tensor& wd,
+                                          const Tensor& cd, double eps, bool biases) {
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("titan::looped_swiglu_bwd_train", "")
+                             .typed<decltype(looped_bwd_train)>();
+  return op.call(dy, st, xn, h, gp, uo, sc, wg, cg, wu, cu, wd, cd, eps, biases);
+}
+
+// All L applications as one native autograd node
+struct LoopedTrain : public torch::autograd::Function<LoopedTrain> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& sc, const Tensor& vg,
+                        const Tensor& cg, const OptTensor& bg, const Tensor& vu, const Tensor& cu,
+                        const OptTensor& bu, const Tensor& vd, const Tensor& cd, const OptTensor& bd, int64_t L,
+                        double eps) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const auto r = call_looped_fwd_train(x, sc, vg, cg, bg, vu, cu, bu, vd, cd, bd, L, eps);
+    ctx->save_for_backward({r[1], r[2], r[3], r[4], r[5], sc, r[6], cg, r[7], cu, r[8], cd});
+    auto dt = [](const OptTensor& b) {
+      return b.has_value() && b->defined() ? (int64_t)b->scalar_type() : (int64_t)-1;
+    };
+    ctx->saved_data["bias"] = std::vector<int64_t>{dt(bg), dt(bu), dt(bd)};
+    ctx->saved_data["eps"] = eps;
+    return r[0];
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    torch::autograd::variable_list r(13);
+    if (!grads[0].defined()) return r;
+    const auto s = ctx->get_saved_variables();
+    const auto dt = ctx->saved_data["bias"].toIntVector();
+    const auto d = call_looped_bwd_train(grads[0].to(at::kBFloat16).contiguous(), s[0], s[1], s[2], s[3], s[4], s[5],
+                                         s[6], s[7], s[8], s[9], s[10], s[11], ctx->saved_data["eps"].toDouble(),
+                                         dt[0] >= 0 || dt[1] >= 0 || dt[2] >= 0);
+    auto bias = [&](const Tensor& b, int t) {
+      return dt[t] >= 0 ? b.to(static_cast<at::ScalarType>(dt[t])) : Tensor();
+    };
+    r[0] = d[0];
+    r[1] = d[1].to(s[5].scalar_type()).reshape(s[5].sizes());
+    r[2] = d[2];
+    r[4] = bias(d[5], 0);
+    r[5] = d[3];
+    r[7] = bias(d[6], 1);
+    r[8] = d[4];
+    r[10] = bias(d[7], 2);
+    return r;
+  }
+};
+
+Tensor looped_train(const Tensor& x, const Tensor& sc, const Tensor& vg, const Tensor& cg, const OptTensor& bg,
+                    const Tensor& vu, const Tensor& cu, const OptTensor& bu, const Tensor& vd, const Tensor& cd,
+                    const OptTensor& bd, int64_t L, double eps) {
+  return call_looped_fwd_train(x, sc, vg, cg, bg, vu, cu, bu, vd, cd, bd, L, eps)[0];
+}
+
+Tensor looped_train_autograd(const Tensor& x, const Tensor& sc, const Tensor& vg, const Tensor& cg,
+                             const OptTensor& bg, const Tensor& vu, const Tensor& cu, const OptTensor& bu,
+                             const Tensor& vd, const Tensor& cd, const OptTensor& bd, int64_t L, double eps) {
+  return LoopedTrain::apply(x, sc, vg, cg, bg, vu, cu, bu, vd, cd, bd, L, eps);
+}
+
 // ------------------------------------------------------------------ GELU FFN
 using Five = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor>;
 
@@ -1181,6 +1332,15 @@ TORCH_LIBRARY(titan, m) {
   m.def("block_ell_swiglu_fwd_train(Tensor x, Tensor values_gate, Tensor col_indices_gate, Tensor? b_gate, "
         "Tensor values_up, Tensor col_indices_up, Tensor? b_up, Tensor values_down, Tensor col_indices_down, "
         "Tensor? b_down, bool add_residual) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
+  m.def("looped_swiglu_fwd_train(Tensor h, Tensor norm_scale, Tensor values_gate, Tensor col_indices_gate, "
+        "Tensor? b_gate, Tensor values_up, Tensor col_indices_up, Tensor? b_up, Tensor values_down, "
+        "Tensor col_indices_down, Tensor? b_down, int L, float eps) -> Tensor[]");
+  m.def("looped_swiglu_train(Tensor h, Tensor norm_scale, Tensor values_gate, Tensor col_indices_gate, "
+        "Tensor? b_gate, Tensor values_up, Tensor col_indices_up, Tensor? b_up, Tensor values_down, "
+        "Tensor col_indices_down, Tensor? b_down, int L, float eps) -> Tensor");
+  m.def("looped_swiglu_bwd_train(Tensor grad_out, Tensor states, Tensor normed, Tensor h, Tensor gate_pre_act, "
+        "Tensor up_out, Tensor norm_scale, Tensor values_gate, Tensor col_indices_gate, Tensor values_up, "
+        "Tensor col_indices_up, Tensor values_down, Tensor col_indices_down, float eps, bool biases) -> Tensor[]");
   m.def("block_ell_gelu_fwd_prepacked(Tensor x, Tensor packed1, Tensor values1, Tensor col_indices1, Tensor? b1, "
         "Tensor packed2, Tensor values2, Tensor col_indices2, Tensor? b2) -> Tensor");
   m.def("block_ell_gelu_fwd_train(Tensor x, Tensor values1, Tensor col_indices1, Tensor? b1, Tensor values2, "
@@ -1256,6 +1416,9 @@ TORCH_LIBRARY_IMPL(titan, CUDA, m) {
   m.impl("block_ell_swiglu_train", &swiglu_train);
   m.impl("block_ell_gelu_fwd_prepacked", &gelu_fwd_prepacked);
   m.impl("block_ell_gelu_fwd_train", &gelu_fwd_train);
+  m.impl("looped_swiglu_fwd_train", &looped_fwd_train);
+  m.impl("looped_swiglu_train", &looped_train);
+  m.impl("looped_swiglu_bwd_train", &looped_bwd_train);
   m.impl("block_ell_gelu_train", &gelu_train);
   m.impl("block_ell_gelu_bwd_train", &gelu_bwd_train);
   m.impl("block_ell_swiglu_bwd_train", &swiglu_bwd_train);
@@ -1290,11 +1453,13 @@ TORCH_LIBRARY_IMPL(titan, CompositeExplicitAutograd, m) { m.impl("unpin_weights_
 TORCH_LIBRARY_IMPL(titan, Autograd, m) {
   m.impl("block_ell_swiglu_train", &swiglu_train_autograd);
   m.impl("block_ell_gelu_train", &gelu_train_autograd);
+  m.impl("looped_swiglu_train", &looped_train_autograd);
   for (const char* name :
        {"block_ell_swiglu_fwd", "block_ell_swiglu_fwd_with_intermediate", "block_ell_swiglu_bwd",
         "persistent_mlp_step", "block_ell_matmul", "block_ell_matmul_bwd", "block_ell_matmul_bwd_bias",
         "block_ell_swiglu_fwd_train", "block_ell_swiglu_bwd_train",
         "block_ell_gelu_fwd_prepacked", "block_ell_gelu_fwd_train", "block_ell_gelu_bwd_train",
+        "looped_swiglu_fwd_train", "looped_swiglu_bwd_train",
         "block_ell_swiglu_bwd_ex",
         "block_ell_matmul_prepack", "block_ell_matmul_prepacked",
         "looped_swiglu", "looped_swiglu_persistent", "looped_swiglu_launches", "looped_core", "rmsnorm",
@@ -1375,6 +1540,33 @@ TORCH_LIBRARY_IMPL(titan, Meta, m) {
   m.impl("block_ell_matmul_bwd", [](const at::Tensor&, const at::Tensor& x, const at::Tensor& v, const at::Tensor&) {
     return std::make_tuple(at::empty_like(x), at::empty_like(v));
   });
+  m.impl("looped_swiglu_train",
+         [](const at::Tensor& h, const at::Tensor&, const at::Tensor&, const at::Tensor&,
+            const c10::optional<at::Tensor>&, const at::Tensor&, const at::Tensor&, const c10::optional<at::Tensor>&,
+            const at::Tensor&, const at::Tensor&, const c10::optional<at::Tensor>&, int64_t, double) {
+           return at::empty_like(h);
+         });
+  m.impl("looped_swiglu_fwd_train",
+         [](const at::Tensor& h, const at::Tensor&, const at::Tensor& vg, const at::Tensor&,
+            const c10::optional<at::Tensor>&, const at::Tensor& vu, const at::Tensor&,
+            const c10::optional<at::Tensor>&, const at::Tensor& vd, const at::Tensor&,
+            const c10::optional<at::Tensor>&, int64_t L, double) {
+           auto act = [&](int64_t c) { return at::empty({L, h.size(0), c}, h.options()); };
+           const int64_t d = h.size(1), d_ff = vg.size(0) * vg.size(2);
+           return std::vector<at::Tensor>{at::empty_like(h), act(d), act(d), act(d_ff), act(d_ff), act(d_ff),
+                                          at::empty(vg.sizes(), h.options()), at::empty(vu.sizes(), h.options()),
+                                          at::empty(vd.sizes(), h.options())};
+         });
+  m.impl("looped_swiglu_bwd_train",
+         [](const at::Tensor& dy, const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&,
+            const at::Tensor&, const at::Tensor&, const at::Tensor& wg, const at::Tensor&, const at::Tensor& wu,
+            const at::Tensor&, const at::Tensor& wd, const at::Tensor&, double, bool biases) {
+           const auto f = dy.options().dtype(at::kFloat);
+           const int64_t d_ff = biases ? wg.size(0) * wg.size(2) : 0, d = biases ? dy.size(1) : 0;
+           return std::vector<at::Tensor>{at::empty_like(dy), at::empty({dy.size(1)}, f), at::empty(wg.sizes(), f),
+                                          at::empty(wu.sizes(), f), at::empty(wd.sizes(), f), at::empty({d_ff}, f),
+                                          at::empty({d_ff}, f), at::empty({d}, f)};
+         });
   m.impl("block_ell_gelu_fwd_prepacked",
          [](const at::Tensor& x, const at::Tensor&, const at::Tensor&, const at::Tensor&,
             const c10::optional<at::Tensor>&, const at::Tensor&, const at::Tensor&, const at::Tensor&,

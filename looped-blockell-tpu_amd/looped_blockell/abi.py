@@ -114,6 +114,12 @@ SIGNATURES = {
     "lbk_gelu_fwd_train": (C.c_int, [_P, _I64, _I32, _PB, _PB, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_size_t, _P]),
     "lbk_gelu_bwd_workspace_bytes": (C.c_size_t, [_I64, _I32, _PB, _PB]),
     "lbk_gelu_bwd_train": (C.c_int, [_P, _P, _P, _P, _I64, _I32, _PB, _PB, _P, _P, _P, _P, _P, _P, C.c_size_t, _P]),
+    "lbk_looped_fwd_train_workspace_bytes": (C.c_size_t, [_I64, _I32, _PB, _PB, _PB]),
+    "lbk_looped_fwd_train": (C.c_int, [_P, _I64, _I32, _P, C.c_float, _I32, _PB, _PB, _PB, _P, _P, _P, _P, _P, _P, _P, _P,
+                                       _P, _P, _P, _P, _P, _P, _P, _P, C.c_size_t, _P]),
+    "lbk_looped_bwd_train_workspace_bytes": (C.c_size_t, [_I64, _I32, _I32, _PB, _PB, _PB]),
+    "lbk_looped_bwd_train": (C.c_int, [_P, _P, _P, _P, _P, _P, _I64, _I32, _P, C.c_float, _I32, _PB, _PB, _PB, _P, _P, _P,
+                                       _P, _P, _P, _P, _P, _P, C.c_size_t, _P]),
     "lbk_swiglu_fwd_train": (C.c_int, [_P, _I64, _I32, _PB, _PB, _PB, _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_int, _P,
                                        _P, _P, _P, _P, C.c_size_t, _P]),
     "lbk_swiglu_bwd_train": (C.c_int, [_P, _P, _P, _P, _P, _I64, _I32, _PB, _PB, _PB, C.c_int, _P, _P, _P, _P, _P, _P,

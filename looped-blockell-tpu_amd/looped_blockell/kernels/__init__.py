@@ -263,6 +263,17 @@ def looped_swiglu_bias(h, norm_scale, v_gate, ci_gate, b_gate, v_up, ci_up, b_up
                                     b_down, L, eps)
 
 
+def looped_swiglu_train(h, norm_scale, v_gate, ci_gate, b_gate, v_up, ci_up, b_up, v_down, ci_down, b_down,
+                        L: int, eps: float = 1e-5):
+    """``looped_swiglu_bias`` on fp32 values, differentiable as one native autograd node
+    (``titan::looped_swiglu_train``): the state and its gradient stay in fp32 between the
+    applications, and one pass over all applications' tokens sums the weight gradients."""
+    _gpu(h, v_gate, v_down)
+    _no_transforms()
+    return ops().looped_swiglu_train(h, norm_scale, v_gate, ci_gate, b_gate, v_up, ci_up, b_up, v_down, ci_down,
+                                     b_down, L, eps)
+
+
 def looped_swiglu_persistent(h, norm_scale, v_gate, ci_gate, v_up, ci_up, v_down, ci_down, L: int,
                              eps: float = 1e-5):
     """``looped_swiglu`` in one persistent launch: each workgroup owns a 64-token block for all L

@@ -6,8 +6,9 @@ the core loop ``looped_blockell/looping/looped_model.py:293-350`` and the MLP pa
 ``csrc/loop/persistent_core.cu:315-335``), one operator call
 (``titan::looped_swiglu``): the weights are packed once, then a gate/up and a down launch per
 application with the carried state in fp32 (``titan::looped_swiglu_persistent`` runs all L in
-one launch).  With gradients required the applications
-run one by one through the differentiable RMSNorm and SwiGLU instead.
+one launch).  With gradients required it is one
+operator too (``titan::looped_swiglu_train``), or the applications one by one through the
+differentiable RMSNorm and SwiGLU where those modules' own calls have to be made.
 """
 
 from __future__ import annotations
@@ -16,7 +17,7 @@ import torch
 from torch import nn
 
 from .. import kernels
-from .mlp import MLPBlock
+from .mlp import MLPBlock, _plain
 from .norms import RMSNorm
 
 
@@ -34,7 +35,16 @@ class LoopedSwiGLU(nn.Module):
         d = h.shape[-1]
         h2 = h.reshape(-1, d).to(torch.bfloat16).contiguous()
         if torch.is_grad_enabled() and (h.requires_grad or any(p.requires_grad for p in self.parameters())):
-            # training: the L applications one by one through the differentiable RMSNorm and
+            if (self.L >= 1 and h2.shape[0] > 0 and d == self.mlp.d_model and _plain(self.norm, RMSNorm)
+                    and _plain(self.mlp, MLPBlock) and self.mlp._fp32_values()):
+                cg, cu, cd = self.mlp.swiglu_columns()
+                bg, bu, bd = self.mlp.swiglu_biases()
+                m = self.mlp
+                out = kernels.looped_swiglu_train(h2, self.norm.scale, m.w_gate.values, cg, bg, m.w_up.values, cu, bu,
+                                                  m.w_down.values, cd, bd, self.L, self.norm.eps)
+                return out.reshape(*lead, d)
+            # where a hook, a subclass or other parameter types have to see the modules' calls:
+            # the L applications one by one through the differentiable RMSNorm and
             # SwiGLU (titan::rmsnorm_bwd, titan::block_ell_swiglu_bwd_bias), as the reference's
             # scan is differentiated (looped_blockell/looping/looped_model.py:342-350); the
             # carried state stays in fp32 as in the operator path

@@ -62,12 +62,12 @@ def _versions(lins):
 _HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
 
 
-def _plain(lin):
-    """Whether calling ``lin`` does no more than ``BlockELLLinear.forward``: no subclass, no replaced
-    forward, no hooks on it or on every module."""
-    d = lin.__dict__
+def _plain(mod, cls):
+    """Whether calling ``mod`` does no more than ``cls.forward``: no subclass, no replaced method, no
+    hooks on it or on every module."""
+    d = mod.__dict__
     g = nn.modules.module
-    return (type(lin) is BlockELLLinear and "forward" not in d and "kernel_values" not in d
+    return (type(mod) is cls and "forward" not in d and "kernel_values" not in d
             and not any(d[h] for h in _HOOKS) and not any(getattr(g, "_global" + h) for h in _HOOKS))
 
 
@@ -191,11 +191,14 @@ class MLPBlock(nn.Module):
         cg, cu, cd = self.swiglu_columns()
         return (self.w_gate.kernel_values(), cg, self.w_up.kernel_values(), cu, self.w_down.kernel_values(), cd)
 
+    def _fp32_values(self):
+        """Whether the projections' values are fp32 and rounded to bf16 without more ado."""
+        return all(lin.values.dtype == torch.float32 and type(lin).kernel_values is BlockELLLinear.kernel_values
+                   and "kernel_values" not in lin.__dict__ for lin in (self.w_gate, self.w_up, self.w_down))
+
     def _swiglu_grad(self, x2, bg, bu, bd):
         """The differentiable forward: fp32 values go to the kernels as they are, rounded there."""
-        lins = (self.w_gate, self.w_up, self.w_down)
-        if all(lin.values.dtype == torch.float32 and type(lin).kernel_values is BlockELLLinear.kernel_values
-               for lin in lins):
+        if self._fp32_values():
             cg, cu, cd = self.swiglu_columns()
             return kernels.swiglu_train(x2, self.w_gate.values, cg, self.w_up.values, cu, self.w_down.values, cd,
                                         add_residual=False, b_gate=bg, b_up=bu, b_down=bd)
@@ -243,7 +246,7 @@ class MLPBlock(nn.Module):
                 out = kernels.swiglu_fwd_prepacked(x2, packed, *w, add_residual=False, b_gate=bg, b_up=bu, b_down=bd)
             if x.dim() != 2 or x.shape[1] != self.d_model:
                 out = out.reshape(*x.shape[:-1], self.d_model)
-        elif x.shape[-1] == self.d_model and _plain(self.fc1) and _plain(self.fc2):
+        elif x.shape[-1] == self.d_model and _plain(self.fc1, BlockELLLinear) and _plain(self.fc2, BlockELLLinear):
             out = self._gelu(x)
         else:                       # the two layers one by one: their hooks and overrides see each
             out = self.fc2(F.gelu(self.fc1(x).float(), approximate="tanh").to(torch.bfloat16))

@@ -209,3 +209,74 @@ def test_gelu_layer_hooks_and_extremes(gpu):
     assert (fused.double() - split.double()).norm() <= 8e-3 * split.double().norm()
     m(x).float().sum().backward()
     assert all(torch.isfinite(p.grad).all() for p in m.parameters())
+
+
+def _loop_pair(d, ff, B, dens, L, shared, bias):
+    """A looped block, and the same one whose modules' calls are made one by one (a hook asks for it)."""
+    from looped_blockell.layers import LoopedSwiGLU
+    ms = []
+    for _ in range(2):
+        torch.manual_seed(11)
+        m = LoopedSwiGLU(d, ff, L, tile_size=B, density=dens, device="cuda", bias=bias)
+        with torch.no_grad():
+            m.norm.scale.uniform_(0.8, 1.2)
+            for lin in (m.mlp.w_gate, m.mlp.w_up, m.mlp.w_down):
+                lin.values.normal_(0, 0.05)
+                lin.alive_mask.copy_(torch.rand(lin.R, lin.K) >= 0.1)
+                if lin.bias is not None:
+                    lin.bias.normal_(0, 0.1)
+            if not shared:
+                m.mlp.w_up.alive_mask.copy_(torch.rand(m.mlp.w_up.R, m.mlp.w_up.K) >= 0.1)
+        ms.append(m)
+    ms[1].mlp.register_forward_hook(lambda *a: None)
+    return ms
+
+
+# state kept by the down kernel (B = 16, 32) and by a pass of its own (B = 64, wide rows); odd widths of
+# the norm's kernels; one row
+@pytest.mark.parametrize("case", [(256, 512, 16, 0.5, 70, 3), (256, 1024, 32, 0.25, 700, 4), (128, 256, 64, 0.5, 200, 2),
+                                  (2112, 128, 64, 0.2, 20, 2), (128, 256, 32, 1.0, 1, 5), (256, 512, 32, 0.5, 33, 1)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_looped_training_matches_the_modules(gpu, case, bias):
+    d, ff, B, dens, N, L = case
+    one, many = _loop_pair(d, ff, B, dens, L, shared=bias, bias=bias)
+    x = torch.randn(N, d, device="cuda").to(torch.bfloat16)
+    dy = torch.randn(N, d, device="cuda").to(torch.bfloat16)
+    got, want = [], []
+    for m, res in ((one, got), (many, want)):
+        xi = x.clone().requires_grad_(True)
+        y = m(xi)
+        res += [y.detach(), *torch.autograd.grad(y, [xi] + list(m.parameters()), dy)]
+    # the module path rounds y and the norm's gradient to bf16 at every application (2^-9 each)
+    for a, b in zip(got, want):
+        assert a.dtype == b.dtype and a.shape == b.shape
+        assert (a.double() - b.double()).norm() <= 4e-3 * (1 + L) * b.double().norm() + 1e-12
+    again = one(x.clone().requires_grad_(True))
+    assert torch.equal(again, got[0])
+
+
+def test_looped_training_groups_of_applications(gpu):
+    """The backward's weight-gradient passes over several groups of applications (the last one shorter)
+    add up: the operator on 5 applications of a size where a group holds two."""
+    from looped_blockell import kernels
+    rng = np.random.default_rng(6)
+    d, ff, B, N, L = 64, 8192, 32, 32768, 5          # 2 GiB of dg and du: two applications
+    ws = _weights(rng, d, ff, B, 0.5, 0.0)
+    x = T.to_gpu_bf16(T.act(rng, N, d))
+    dy = T.to_gpu_bf16(T.act(rng, N, d))
+    sc = torch.ones(d, device="cuda")
+    ops = kernels.ops()
+    out, st, xn, h, gp, uo, wg, wu, wd = ops.looped_swiglu_fwd_train(x, sc, ws[0], ws[1], None, ws[2], ws[3], None, ws[4],
+                                                                     ws[5], None, L, 1e-5)
+    got = ops.looped_swiglu_bwd_train(dy, st, xn, h, gp, uo, sc, wg, ws[1], wu, ws[3], wd, ws[5], 1e-5, True)
+    # the same applications one at a time, the state gradient carried in fp32
+    g, tot = dy.float(), None
+    for t in range(L - 1, -1, -1):
+        r = ops.block_ell_swiglu_bwd_train(g.to(torch.bfloat16), xn[t], gp[t], uo[t], h[t], wg, ws[1], wu, ws[3], wd,
+                                           ws[5], False, True)
+        dx, ds = ops.rmsnorm_bwd(r[0], st[t], sc, 1e-5)
+        g = g + dx.float()
+        parts = [ds, *r[1:]]
+        tot = parts if tot is None else [a + b for a, b in zip(tot, parts)]
+    for a, b in zip(got, [g.to(torch.bfloat16), *tot]):
+        assert (a.double() - b.double()).norm() <= 4e-3 * b.double().norm()
