@@ -1141,7 +1141,7 @@ static size_t tlist_bytes(const lbk_bell* w, int C) {
 }
 // fp32 partial tiles of one weight's tile gradients (the token chunking of launch_dw)
 static size_t dw_part_floats(int64_t N, const lbk_bell* w, int C, int64_t ldg) {
-  const int64_t ch = dw_job_chunk(w->B, w->R, C, ldg, N);
+  const int64_t ch = dw_job_chunk(w->B, w->R, w->K, C, ldg, N);
   return (size_t)((N + ch - 1) / ch) * w->R * w->K * w->B * w->B;
 }
 

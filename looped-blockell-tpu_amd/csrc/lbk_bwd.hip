@@ -26,11 +26,12 @@
 //                  of NW waves (8; 16 at B = 16) streams the list entries of its
 //                  column blocks (c = w, w + NW, ...): tile rows from global memory,
 //                  dy fragments from the panel.
-//   dx_stage_kernel  dx when the output blocks fit the waves' accumulators (16
-//                  waves where they fit 128 VGPRs, else 8): the dg and du columns
-//                  of 64 tokens pass through LDS 512 at a time, and a cursor per
-//                  output block walks its sorted list, whose first 64 entries
-//                  stay in a register.
+//   dx_stage_kernel  dx at B = 64 when the output blocks fit the waves' accumulators:
+//                  the dg and du columns of 64 tokens pass through LDS 256 at a
+//                  time, and a cursor per output block walks its sorted list, whose
+//                  first 64 entries stay in a register.
+//   dx16_kernel    dx at B = 16: the same walk with wider stages, list entries in
+//                  pairs through a ring.
 //   dxf_kernel     dx at B = 32: the same stages, one output block per wave and a
 //                  4-slot ring of tiles over the wave's whole list (both sources,
 //                  all stages), the list entries read one pass ahead.
@@ -556,8 +557,6 @@ __global__ __launch_bounds__(64 * NW, 1) void dx_stage_kernel(TProdArgs a) {
   // workgroup -> (64-token block, slice sl of nsl: output blocks sl + nsl (w + NW o))
   const int sl = (int)(blockIdx.x % (unsigned)a.nsl);
   const int64_t t0 = (int64_t)(blockIdx.x / (unsigned)a.nsl) * 64;
-  const int gk = (B == 16) ? (g & 1) : g;
-  const bool kz = (B == 16) && g >= 2;
 
   // stages: source s covers ceil(R_s / G) stages; global stage -> (source, first block)
   const int R0 = (int)(a.src[0].lda / B);
@@ -598,7 +597,6 @@ __global__ __launch_bounds__(64 * NW, 1) void dx_stage_kernel(TProdArgs a) {
 
   struct Ent {
     u32x4 av[NKS][CW];
-    u32x2 a16;                                       // B = 16: the 16x16x16 fragment
     int r;                                           // source column block
   };
   const uint32_t lbase = (uint32_t)(i * MT * SROWB);
@@ -627,15 +625,11 @@ __global__ __launch_bounds__(64 * NW, 1) void dx_stage_kernel(TProdArgs a) {
     const unsigned char* sb = stg + (s & 1) * SBYTES;
     const int rlo = st * G, rhi = rlo + G;           // source column blocks of this stage
     auto load = [&](int e, Ent& E) {
-      if constexpr (B == 16) {
-        E.a16 = *reinterpret_cast<const u32x2*>(S.w + (int64_t)e * B * B + i * B + 4 * g);
-      } else {
-        const uint16_t* tile = S.w + (int64_t)e * B * B + 8 * gk;
+      const uint16_t* tile = S.w + (int64_t)e * B * B + 8 * g;
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks)
+      for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
-          for (int m = 0; m < CW; ++m) E.av[ks][m] = ld16(tile + op_row<CW>(i, m) * B + 32 * ks);
-      }
+        for (int m = 0; m < CW; ++m) E.av[ks][m] = ld16(tile + op_row<CW>(i, m) * B + 32 * ks);
       E.r = e / S.K;
     };
 #pragma unroll
@@ -644,20 +638,12 @@ __global__ __launch_bounds__(64 * NW, 1) void dx_stage_kernel(TProdArgs a) {
       if (c >= a.C) continue;
       auto compute = [&](const Ent& E) {
         const int rb = uniform(E.r) - rlo;           // column block within the stage
-        if constexpr (B == 16) {
-          const uint32_t pa = lbase + ((uint32_t)(((rb * 2 + (g >> 1)) ^ i) << 4) | (uint32_t)((g & 1) << 3));
-#pragma unroll
-          for (int q = 0; q < MT; ++q)
-            acc[o][q][0] = mfma_bf16_k16(E.a16, *reinterpret_cast<const u32x2*>(sb + pa + q * SROWB), acc[o][q][0]);
-          return;
-        }
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
-          const uint32_t pa = lbase + (((rb * (B / 8) + 4 * ks + gk) ^ i) << 4);
+          const uint32_t pa = lbase + (((rb * (B / 8) + 4 * ks + g) ^ i) << 4);
 #pragma unroll
           for (int q = 0; q < MT; ++q) {
-            const u32x4 bv0 = *reinterpret_cast<const u32x4*>(sb + pa + q * SROWB);
-            const u32x4 bv = kz ? u32x4{0, 0, 0, 0} : bv0;
+            const u32x4 bv = *reinterpret_cast<const u32x4*>(sb + pa + q * SROWB);
 #pragma unroll
             for (int m = 0; m < CW; ++m) acc[o][q][m] = mfma_bf16(E.av[ks][m], bv, acc[o][q][m]);
           }
@@ -678,29 +664,13 @@ __global__ __launch_bounds__(64 * NW, 1) void dx_stage_kernel(TProdArgs a) {
         const int n = __builtin_popcountll(m);       // a contiguous run of lanes (sorted list)
         if (n == 0) break;
         auto ent = [&](int jj) { return __builtin_amdgcn_readlane(lv, base + (jj < n ? jj : n - 1)); };
-        if constexpr (B == 16) {
-          // 8-byte tile fragments: a 3-entry ring keeps two loads in flight ahead of the MFMAs
-          // (positions past the run reload its last entry and are not computed)
-          constexpr int DXR = 3;
-          Ent E[DXR];
-#pragma unroll
-          for (int k = 0; k < DXR - 1; ++k) load(ent(k), E[k]);
-          for (int jj = 0; jj < n; jj += DXR) {
-#pragma unroll
-            for (int k = 0; k < DXR; ++k) {
-              load(ent(jj + k + DXR - 1), E[(k + DXR - 1) % DXR]);
-              if (jj + k < n) compute(E[k]);
-            }
-          }
-        } else {
-          Ent E0, E1;
-          load(ent(0), E0);
-          for (int jj = 0; jj < n; jj += 2) {
-            load(ent(jj + 1), E1);
-            compute(E0);
-            load(ent(jj + 2), E0);
-            if (jj + 1 < n) compute(E1);
-          }
+        Ent E0, E1;
+        load(ent(0), E0);
+        for (int jj = 0; jj < n; jj += 2) {
+          load(ent(jj + 1), E1);
+          compute(E0);
+          load(ent(jj + 2), E0);
+          if (jj + 1 < n) compute(E1);
         }
         jc += n;
         if (base + n < 64) break;                    // the run ended inside this chunk
@@ -731,6 +701,168 @@ static int launch_dx_stage_t(const TProdArgs& a, hipStream_t st) {
   static std::atomic<uint64_t> done{0};
   if (lds > 65536 && set_lds_limit_once(reinterpret_cast<const void*>(kern), (int)lds, done)) return -1;
   hipLaunchKernelGGL(kern, dim3((unsigned)((a.N + 63) / 64 * a.nsl)), dim3(64 * NW), lds, st, a);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// dx16_kernel<OPW, MT, NW>: dx at B = 16 (wave w of NW owns output blocks sl + nsl (w + NW o) of
+// 16 MT tokens).  A step of a wave is one list entry and little work, so the kernel is bound by the latency of its tile
+// loads: entries go in pairs (one 16x16x32 MFMA per token tile, lanes g < 2 with entry 2p, the
+// others with 2p + 1, 16 bytes a lane) through a four-pair ring, as in the dh panel kernel, and a
+// stage holds 512 to 2048 activation columns (64 or 128 KB of LDS, the next stage in registers
+// meanwhile), so that a block's run within a stage is long enough to fill the ring.
+constexpr int dx16_cols(int OPW, int MT) { return MT == 2 ? 2048 : OPW == 1 ? 1024 : 512; }
+template <int OPW, int MT, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void dx16_kernel(TProdArgs a) {
+  constexpr int NT = 64 * NW, TM = 16 * MT, B = 16;
+  constexpr int COLS = dx16_cols(OPW, MT);
+  constexpr int G = COLS / B;                        // source column blocks per stage
+  constexpr int SROWB = COLS * 2;                    // bytes per token row of a stage
+  constexpr int PER_T = TM * SROWB / 16 / NT;        // 16-byte chunks per thread per stage
+  extern __shared__ __attribute__((aligned(16))) unsigned char stg[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = uniform(tid >> 6);
+  const int i = lane & 15, g = lane >> 4;
+  const int sl = (int)(blockIdx.x % (unsigned)a.nsl);
+  const int64_t t0 = (int64_t)(blockIdx.x / (unsigned)a.nsl) * TM;
+  const int ns0 = (int)((a.src[0].lda + COLS - 1) / COLS);
+  const int ns1 = a.nsrc > 1 ? (int)((a.src[1].lda + COLS - 1) / COLS) : 0;
+  const int nstages = ns0 + ns1;
+
+  u32x4 sreg[PER_T];
+  auto stage_fetch = [&](int s) {
+    const TProdSrc& S = a.src[s < ns0 ? 0 : 1];
+    const int64_t col0 = (int64_t)(s < ns0 ? s : s - ns0) * COLS;
+#pragma unroll
+    for (int u = 0; u < PER_T; ++u) {
+      const int e = tid + NT * u;
+      const int row = e / (SROWB / 16), cc = e - row * (SROWB / 16);
+      const int64_t t = t0 + row, col = col0 + 8 * cc;
+      const bool ok = t < a.N && col < S.lda;
+      const u32x4 v = ld16(S.a + (ok ? t : t0) * S.lda + (ok ? col : 0));
+      sreg[u] = ok ? v : u32x4{0, 0, 0, 0};
+    }
+  };
+  auto stage_store = [&]() {
+#pragma unroll
+    for (int u = 0; u < PER_T; ++u) {
+      const int e = tid + NT * u;
+      const int row = e / (SROWB / 16), cc = e - row * (SROWB / 16);
+      *reinterpret_cast<u32x4*>(stg + bpanel_addr<MT>(row, cc, SROWB)) = sreg[u];
+    }
+  };
+
+  f32x4 acc[OPW][MT];
+#pragma unroll
+  for (int o = 0; o < OPW; ++o)
+#pragma unroll
+    for (int q = 0; q < MT; ++q) acc[o][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t lbase = (uint32_t)(i * MT * SROWB);
+  int cur[OPW];                                      // list cursors of the current source
+  int lvr[OPW];                                      // first 64 list entries of each output block
+  int cnts[OPW];
+
+  stage_fetch(0);
+  for (int s = 0; s < nstages; ++s) {
+    const int src = s < ns0 ? 0 : 1;
+    const int st = s < ns0 ? s : s - ns0;
+    const TProdSrc& S = a.src[src];
+    if (st == 0) {
+      // a new source: each output block's first 64 list entries into a register (lane j holds
+      // entry j), so that a stage finds its run with a ballot instead of a global load
+#pragma unroll
+      for (int o = 0; o < OPW; ++o) {
+        cur[o] = 0;
+        const int c = sl + a.nsl * (w + NW * o);
+        cnts[o] = c < a.C ? S.cnt[c] : 0;
+        lvr[o] = lane < cnts[o] ? S.list[(int64_t)c * S.cap + lane] : 0x7fffffff;
+      }
+    }
+    if (s > 0) __syncthreads();                      // the previous stage has been read
+    stage_store();
+    __syncthreads();
+    if (s + 1 < nstages) stage_fetch(s + 1);
+    const int rlo = st * G, rhi = rlo + G;           // source column blocks of this stage
+    struct Ent {
+      u32x4 av;
+      int r;
+    };
+#pragma unroll
+    for (int o = 0; o < OPW; ++o) {
+      const int c = sl + a.nsl * (w + NW * o);
+      const int cnt = cnts[o];
+      int jc = cur[o];
+      while (jc < cnt) {
+        // entries of this stage: the run from jc whose source block is below rhi.  Within the
+        // first 64 entries they come from the register (lanes jc .. jc + n - 1), beyond them
+        // from the next 64 entries loaded here (lanes 0 .. n - 1)
+        const bool inreg = jc < 64;
+        const int lv = inreg ? lvr[o] : ((jc + lane < cnt) ? S.list[(int64_t)c * S.cap + jc + lane] : 0x7fffffff);
+        const int base = inreg ? jc : 0;
+        const int lim = inreg ? (cnt < 64 ? cnt : 64) : cnt - jc;
+        const int rv = kdiv(S, lv);                  // source block (lanes at or past lim: not used)
+        const uint64_t m = __ballot(lane >= base && lane < lim && rv < rhi);
+        const int n = __builtin_popcountll(m);       // a contiguous run of lanes (sorted list)
+        if (n == 0) break;
+        const int np = (n + 1) >> 1;
+        constexpr int D = 4;
+        Ent E[D];
+        auto loadp = [&](int p, Ent& E) {
+          const int j1 = 2 * p < n ? 2 * p : n - 1, j2 = 2 * p + 1 < n ? 2 * p + 1 : n - 1;
+          const int e1 = __builtin_amdgcn_readlane(lv, base + j1), e2 = __builtin_amdgcn_readlane(lv, base + j2);
+          const int e = g < 2 ? e1 : e2;
+          E.av = *reinterpret_cast<const u32x4*>(S.w + (int64_t)e * (B * B) + i * B + 8 * (g & 1));
+          E.r = (__builtin_amdgcn_readlane(rv, base + j1) - rlo) | ((__builtin_amdgcn_readlane(rv, base + j2) - rlo) << 10) |
+                (2 * p + 1 < n ? 1 << 20 : 0);
+        };
+        auto computep = [&](const Ent& E) {
+          const int rr = uniform(E.r);
+          const int rl = g < 2 ? (rr & 1023) : ((rr >> 10) & 1023);
+          const u32x4 av = (g < 2 || ((rr >> 20) & 1)) ? E.av : u32x4{0, 0, 0, 0};
+          const uint32_t pa = lbase + ((uint32_t)((rl * 2 + (g & 1)) ^ i) << 4);
+#pragma unroll
+          for (int q = 0; q < MT; ++q)
+            acc[o][q] = mfma_bf16(av, *reinterpret_cast<const u32x4*>(stg + pa + q * SROWB), acc[o][q]);
+        };
+#pragma unroll
+        for (int k = 0; k < D - 1; ++k) loadp(k, E[k]);
+        for (int pp = 0; pp < np; pp += D) {
+#pragma unroll
+          for (int k = 0; k < D; ++k) {
+            loadp(pp + k + D - 1, E[(k + D - 1) % D]);
+            if (k == 0 || pp + k < np) computep(E[k]);
+          }
+        }
+        jc += n;
+        if (base + n < 64) break;                    // the run ended inside this chunk
+      }
+      cur[o] = jc;
+    }
+  }
+
+  // epilogue: dx = acc (+ dy)
+#pragma unroll
+  for (int o = 0; o < OPW; ++o) {
+    const int c = sl + a.nsl * (w + NW * o);
+    if (c >= a.C) continue;
+#pragma unroll
+    for (int q = 0; q < MT; ++q) {
+      const int64_t tn = t0 + 16 * q + i;
+      f32x4 v[1] = {acc[o][q]};
+      if (tn < a.N) tprod_store<1, 1>(a, tn, c, g, v);
+    }
+  }
+}
+
+template <int OPW, int MT, int NW>
+static int launch_dx16_t(const TProdArgs& a0, hipStream_t st) {
+  constexpr int lds = 16 * MT * 2 * dx16_cols(OPW, MT);
+  auto kern = dx16_kernel<OPW, MT, NW>;
+  static std::atomic<uint64_t> done{0};
+  if (set_lds_limit_once(reinterpret_cast<const void*>(kern), lds, done)) return -1;
+  TProdArgs a = a0;
+  set_kdiv(a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((a.N + 16 * MT - 1) / (16 * MT) * a.nsl)), dim3(64 * NW), lds, st,
+                     a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -949,21 +1081,24 @@ static int launch_dx_stage(int B, const TProdArgs& a0, hipStream_t st) {
   // B = 32: the deep-ring kernel (headline backward 0.710 -> 0.688 ms; 64 / 1024 / 4096 tokens
   // 0.109 / 0.131 / 0.213 -> 0.105 / 0.127 / 0.199 ms)
   if (B == 32) return launch_dxf<32>(a0, st);
-  // 16 waves (four per SIMD to hide the tile loads) when their accumulators fit 128 VGPRs:
-  // headline backward 0.785 -> 0.740 ms, B = 16 at d_model 512 / 1024 0.497 -> 0.447 and
-  // 2.10 -> 1.95 ms against 8 waves; B = 64 keeps 8 waves (16 would spill)
-  const int o16 = (cs + 15) / 16;
-  if (B == 16 && o16 <= 1) return launch_dx_stage_t<16, 1, 16>(a, st);
-  if (B == 16 && o16 <= 2) return launch_dx_stage_t<16, 2, 16>(a, st);
-  if (B == 16 && o16 <= 4) return launch_dx_stage_t<16, 4, 16>(a, st);
-  if (B == 32 && o16 <= 1) return launch_dx_stage_t<32, 1, 16>(a, st);
-  if (B == 32 && o16 <= 2) return launch_dx_stage_t<32, 2, 16>(a, st);
+  if (B == 16) {
+    // 64-token blocks with 16 waves where those fill the CUs; else 32-token blocks and 8 waves, one
+    // output block each, whose panel reads and staging spread over four times the CUs (us a step,
+    // 2000 x 512, d_ff 2048 / looped x4 of 2048 x 512 / 1000 x 1024, d_ff 4096: 164 / 603 / 206 with
+    // 64 tokens and 16 waves, 156 / 563 / 191 so, 161 / 590 / 203 with 64 tokens and 8 waves, 176 /
+    // 653 / 216 with 32 and 4; the eight-byte single-entry kernel before it 189 / 786 / 238)
+    if (ntb * ((a.C + 15) / 16) < 256) {
+      a.nsl = (a.C + 7) / 8;
+      return launch_dx16_t<1, 2, 8>(a, st);
+    }
+    const int opw = (cs + 15) / 16;
+    if (opw <= 1) return launch_dx16_t<1, 4, 16>(a, st);
+    if (opw <= 2) return launch_dx16_t<2, 4, 16>(a, st);
+    if (opw <= 4) return launch_dx16_t<4, 4, 16>(a, st);
+  }
   const int opw = (cs + 7) / 8;
-#define LBK_DX(BB, OO) if (B == BB && opw <= OO) return launch_dx_stage_t<BB, OO, 8>(a, st);
-  if (B == 16) { LBK_DX(16, 1) LBK_DX(16, 2) LBK_DX(16, 4) LBK_DX(16, 8) }
-  if (B == 32) { LBK_DX(32, 1) LBK_DX(32, 2) LBK_DX(32, 4) }
-  if (B == 64) { LBK_DX(64, 1) LBK_DX(64, 2) }
-#undef LBK_DX
+  if (B == 64 && opw <= 1) return launch_dx_stage_t<64, 1, 8>(a, st);
+  if (B == 64 && opw <= 2) return launch_dx_stage_t<64, 2, 8>(a, st);
   // B = 16 with more output blocks than the staged kernel's accumulators hold (N >= 16321 tokens
   // and more than 64 output blocks): the deep-ring kernel, one output block per wave, in place of
   // the per-entry kernel (1024 x 8192 product backward at 16384 tokens 1.275 -> 0.658 ms).  Where
@@ -1887,21 +2022,47 @@ static bool dwt_shape(int B, int R, int C, int64_t ldg) {
   return false;
 }
 
-int dw_job_chunk(int B, int R, int C, int64_t ldg, int64_t N) {
+// The kernel that a weight's tile gradients take and the tokens of a partial tile.  The kernels that
+// stage whole rows (dwg, dwt) read each operand once per 8 or 16 block rows instead of once per slot
+// group, but a workgroup fills a CU (up to 160 KB of LDS), so they are taken where they fill the
+// chip.  B = 16: the tokens are cut into chunks down to 256 for that (each chunk costs a write and a
+// read of the partial tiles): looped x4 of 2048 x 512 0.709 -> 0.605 ms, 4096 x 1024 at d_ff 4096
+// 0.552 -> 0.416; below 64 workgroups a weight the slot-per-wave kernel is as fast.  B = 32: chunks
+// of 2048 (dwg) or 1024 (dwt) and 256 workgroups, smaller chunks measured slower (2821 x 1024
+// 0.291 ms against 0.306 to 0.346).
+struct DWPlan {
+  enum { SLOTS, ROWS, OUT } kind;
+  int chunk;
+};
+static DWPlan dw_plan(int B, int R, int K, int C, int64_t ldg, int64_t N) {
+  auto chunks = [&](int64_t c) { return (N + c - 1) / c; };
   const bool wide_in = (int64_t)C * B > 1024;
-  // one workgroup per CU (160 KB of LDS): with fewer than 256 the slot-per-wave kernel is faster
-  // (at 128 workgroups: 151 against 117 us for the config-2 down weight)
-  const int64_t half = DW_CHUNK / 2;
-  const bool fills = (int64_t)(C / dwt_blocks(B)) * ((N + half - 1) / half) >= 256;
-  return wide_in && dwt_shape(B, R, C, ldg) && fills ? (int)half : DW_CHUNK;
+  if (B == 16) {
+    const bool rows = K <= 16 && R % 16 == 0 && (C == 16 || C == 32 || C == 64);
+    const bool out = wide_in && dwt_shape(B, R, C, ldg);
+    if (rows || out) {
+      const int64_t groups = rows ? R / 16 : C / 16;
+      int c = DW_CHUNK;
+      while (c > 256 && groups * chunks(c) < 128) c /= 2;
+      if (groups * chunks(c) >= (rows ? 64 : 128)) return {rows ? DWPlan::ROWS : DWPlan::OUT, c};
+    }
+    return {DWPlan::SLOTS, DW_CHUNK};
+  }
+  if (wide_in && dwt_shape(B, R, C, ldg) && (C / dwt_blocks(B)) * chunks(DW_CHUNK / 2) >= 256)
+    return {DWPlan::OUT, DW_CHUNK / 2};
+  return {DWPlan::SLOTS, DW_CHUNK};
 }
+
+int dw_job_chunk(int B, int R, int K, int C, int64_t ldg, int64_t N) { return dw_plan(B, R, K, C, ldg, N).chunk; }
 
 int launch_dw(int B, const DWJob* jobs_in, int n, int64_t N, hipStream_t st) {
   if (n < 1 || n > DWJobs::kMax) return -2;
   DWJob jobs[DWJobs::kMax];
+  DWPlan plan[DWJobs::kMax];
   for (int t = 0; t < n; ++t) {
     jobs[t] = jobs_in[t];
-    jobs[t].chunk = dw_job_chunk(B, jobs[t].R, jobs[t].C, jobs[t].ldg, N);   // whole slices of 32 and 64 tokens
+    plan[t] = dw_plan(B, jobs[t].R, jobs[t].K, jobs[t].C, jobs[t].ldg, N);
+    jobs[t].chunk = plan[t].chunk;                   // whole slices of 32, 64 and 128 tokens
     jobs[t].nchunk = N > 0 ? (int)((N + jobs[t].chunk - 1) / jobs[t].chunk) : 0;
   }
   DWJobs J{};
@@ -1953,27 +2114,19 @@ int launch_dw(int B, const DWJob* jobs_in, int n, int64_t N, hipStream_t st) {
   // B = 16 weights with at most 16 slots per row, rows in whole groups of 16 and input rows of
   // 256 to 1024 elements (the gate and up weights of such models) take dwg16_kernel
   // (XI = C / 16 in {1, 2, 4}: C in {16, 32, 64})
-  auto narrow16 = [&](const DWJob& j) {
-    return B == 16 && j.K <= 16 && j.R % 16 == 0 && (j.C == 16 || j.C == 32 || j.C == 64) &&
-           j.ldx >= (int64_t)j.C * 16;
-  };
+  auto narrow16 = [&](int t) { return plan[t].kind == DWPlan::ROWS && jobs[t].ldx >= (int64_t)jobs[t].C * 16; };
   for (int t = 0; t < n; ++t) {
-    if (taken[t] || !narrow16(jobs[t])) continue;
+    if (taken[t] || !narrow16(t)) continue;
     DWJobs G = J;
     G.n = 0;
     int64_t gb = 0;
     for (int u = t; u < n; ++u)
-      if (!taken[u] && narrow16(jobs[u]) && jobs[u].C == jobs[t].C) {
+      if (!taken[u] && narrow16(u) && jobs[u].C == jobs[t].C) {
         taken[u] = true;
         G.job[G.n] = jobs[u];
         G.first[G.n++] = gb;
         gb += (int64_t)(jobs[u].R / 16) * jobs[u].nchunk;
       }
-    if (gb < 256) {
-      for (int u = t; u < n; ++u)
-        if (narrow16(jobs[u]) && jobs[u].C == jobs[t].C) taken[u] = false;
-      continue;
-    }
     const int xi = jobs[t].C / 16;                   // 1 KB load instructions of x per wave and slice
     const size_t lds = (size_t)2 * 32 * 2 * (jobs[t].C * 16 + DWG::GW);
     auto kern = xi == 4 ? dwg16_kernel<4> : xi == 2 ? dwg16_kernel<2> : dwg16_kernel<1>;
@@ -1983,17 +2136,16 @@ int launch_dw(int B, const DWJob* jobs_in, int n, int64_t N, hipStream_t st) {
     hipLaunchKernelGGL(kern, dim3((unsigned)gb), dim3(1024), lds, st, G);
     if (hipGetLastError() != hipSuccess) return -1;
   }
-  // weights given the half chunk (narrow output rows, R B <= 1024: the down weight of d_model <=
-  // 1024, with enough workgroups) and their transposed lists take dwt_kernel (dwt16_kernel at
-  // B = 16), one launch per output width
-  auto narrow_out = [&](const DWJob& j) { return j.chunk == DW_CHUNK / 2 && j.tcnt && j.tlist; };
+  // weights with narrow output rows (R B <= 1024: the down weight of d_model <= 1024) and their
+  // transposed lists take dwt_kernel (dwt16_kernel at B = 16), one launch per output width
+  auto narrow_out = [&](int t) { return plan[t].kind == DWPlan::OUT && jobs[t].tcnt && jobs[t].tlist; };
   for (int t = 0; t < n; ++t) {
-    if (taken[t] || !narrow_out(jobs[t])) continue;
+    if (taken[t] || !narrow_out(t)) continue;
     DWJobs G = J;
     G.n = 0;
     int64_t gb = 0;
     for (int u = t; u < n; ++u)
-      if (!taken[u] && narrow_out(jobs[u]) && jobs[u].R == jobs[t].R) {
+      if (!taken[u] && narrow_out(u) && jobs[u].R == jobs[t].R) {
         taken[u] = true;
         G.job[G.n] = jobs[u];
         G.first[G.n++] = gb;

@@ -348,10 +348,8 @@ struct DWJobs {
 };
 constexpr int DW_CHUNK = 2048;   // tokens per partial tile
 // tokens per partial tile of a weight [R, K, B, B] with C input column blocks, G rows of ldg
-// elements and N tokens: DW_CHUNK / 2 where the tile gradients take the transposed-list kernel
-// (input rows too wide to stage whole, output rows at most 1024 wide, and at least 256 of its
-// workgroups at that chunk), else DW_CHUNK
-int dw_job_chunk(int B, int R, int C, int64_t ldg, int64_t N);
+// elements and N tokens (at most DW_CHUNK; the kernel that the weight takes decides)
+int dw_job_chunk(int B, int R, int K, int C, int64_t ldg, int64_t N);
 // per job: chunk = dw_job_chunk(...) (a multiple of 64), partials [ceil(N / chunk), R*K, B, B]
 int launch_dw(int B, const DWJob* jobs, int n, int64_t N, hipStream_t st);
 
