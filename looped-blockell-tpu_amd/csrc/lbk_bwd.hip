@@ -722,8 +722,16 @@ __global__ __launch_bounds__(64 * NW, 1) void dx16_kernel(TProdArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = uniform(tid >> 6);
   const int i = lane & 15, g = lane >> 4;
-  const int sl = (int)(blockIdx.x % (unsigned)a.nsl);
-  const int64_t t0 = (int64_t)(blockIdx.x / (unsigned)a.nsl) * TM;
+  // workgroup -> (token block tb, slice sl); the slices of a token block share an XCD
+  int64_t tb = blockIdx.x;
+  int sl = 0;
+  if (a.nsl > 1) {
+    const int64_t b = blockIdx.x, rest = b >> 3;
+    sl = (int)(rest % a.nsl);
+    tb = 8 * (rest / a.nsl) + (b & 7);
+  }
+  const int64_t t0 = tb * TM;
+  if (t0 >= a.N) return;                             // the whole workgroup, before any barrier
   const int ns0 = (int)((a.src[0].lda + COLS - 1) / COLS);
   const int ns1 = a.nsrc > 1 ? (int)((a.src[1].lda + COLS - 1) / COLS) : 0;
   const int nstages = ns0 + ns1;
@@ -861,8 +869,9 @@ static int launch_dx16_t(const TProdArgs& a0, hipStream_t st) {
   if (set_lds_limit_once(reinterpret_cast<const void*>(kern), lds, done)) return -1;
   TProdArgs a = a0;
   set_kdiv(a);
-  hipLaunchKernelGGL(kern, dim3((unsigned)((a.N + 16 * MT - 1) / (16 * MT) * a.nsl)), dim3(64 * NW), lds, st,
-                     a);
+  const int64_t ntb = (a.N + 16 * MT - 1) / (16 * MT);
+  const int64_t grid = a.nsl == 1 ? ntb : 8 * a.nsl * ((ntb + 7) / 8);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), lds, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -577,22 +577,19 @@ __global__ __launch_bounds__(512, 1) void gu_kernel(GUArgs a) {
 }
 
 // gate/up with distinct gate/up topologies, without exported pre-activations or biases, one row
-// slice, with 12 waves and a 2-deep
-// ring: at most 168 VGPRs fit three waves per SIMD, and the extra waves hide more of the
-// panel-read and weight-load latency than the shallower ring gives up.  B = 16 with a shared
-// topology (slot pairs, so a 2-deep ring keeps four slots in flight) takes the same shape; B = 16
-// with distinct topologies, with a quarter of the accumulators and 8-byte fragments (113 VGPRs),
-// runs 16 waves with a 4-deep ring (forward at d_model 1024, d_ff 4096, 25 %, 16384 tokens:
-// 0.2490 ms with 12 waves, 0.2467 with 16).
-template <int B, bool SHARED> constexpr int gu_w12_waves() { return B == 16 && !SHARED ? 16 : 12; }
-template <int B, bool SHARED> constexpr int gu_w12_ring() { return B == 16 && !SHARED ? 4 : 2; }
-// (B = 16 also takes shared topologies and biases here)
-template <int B, int MT, bool NORM, bool SHARED = false, bool BIAS = false>
-__global__ __launch_bounds__((64 * gu_w12_waves<B, SHARED>()), 1) void gu_kernel_w12(GUArgs a) {
+// slice, with 12 waves and a 2-deep ring (B = 32): at most 168 VGPRs fit three waves per SIMD, and
+// the extra waves hide more of the panel-read and weight-load latency than the shallower ring gives
+// up.  B = 16, with a quarter of the accumulators and 8-byte fragments, runs 16 waves (forward at
+// d_model 1024, d_ff 4096, 25 %, 16384 tokens: 0.2490 ms with 12 waves, 0.2467 with 16).
+// (B = 16 also takes shared topologies, biases, exports and row slices here)
+template <int B, int MT, bool NORM, bool SHARED = false, bool BIAS = false, bool INTER = false, int NW = 12, int RING = 2>
+__global__ __launch_bounds__(64 * NW, 1) void gu_kernel_w12(GUArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  if (a.tdepth && !block_runs(a.tdepth, a.it, (int64_t)blockIdx.x * 16 * MT, 16 * MT, a.N, (int)threadIdx.x)) return;
-  gu_tile<B, MT, NORM, false, SHARED, false, BIAS, false, gu_w12_waves<B, SHARED>(), gu_w12_ring<B, SHARED>()>(
-      a, (int64_t)blockIdx.x, 0, a.R_ff, smem, (int)threadIdx.x);
+  int64_t tb;
+  int r_lo, nrs;
+  gu_slice(a, tb, r_lo, nrs);
+  if (a.tdepth && !block_runs(a.tdepth, a.it, tb * 16 * MT, 16 * MT, a.N, (int)threadIdx.x)) return;
+  gu_tile<B, MT, NORM, INTER, SHARED, false, BIAS, false, NW, RING>(a, tb, r_lo, nrs, smem, (int)threadIdx.x);
 }
 
 // plain Block-ELL product y = x W (+ bias) over an LDS panel of x (the gate/up kernel's gate
@@ -1413,16 +1410,23 @@ static size_t gu_lds(int R_ff, int K, int mt) {
   return (size_t)16 * mt * (8192 / mt) + (((size_t)R_ff * K * 2 + 15) & ~(size_t)15);
 }
 
-// Row slices per token block for the gate/up kernels: with fewer token blocks than CUs, each
-// block's h rows are split so that about 256 workgroups run (a workgroup streams the weights of
-// its rows only), keeping at least 8 rows (one per wave) per slice; above 4 slices the count is
-// a multiple of 8, so that one slice's workgroups share an XCD.
-static int gu_slices(int64_t ntb, int R_ff) {
-  if (ntb >= 256) return 1;
-  const int hmax = R_ff / 8 > 1 ? R_ff / 8 : 1;
-  int H = (int)((256 + ntb - 1) / ntb);
-  if (H > 4) H = (H + 7) / 8 * 8;
-  return H < hmax ? H : hmax;
+// Row slices per token block for the gate/up kernels (one workgroup of NW waves fills a CU): the split
+// with the least rounds of 256 workgroups times the rows a wave walks in each (two more for the panel
+// fill).  About 256 workgroups whatever the token count leaves a last round of a few: 4099 x 512, d_ff
+// 2048 at density 1, B = 16 (65 token blocks), 65 us in four slices of two rounds, 40 in three of one.
+// Above 4 slices the count is a multiple of 8, so that one slice's workgroups share an XCD.
+static int gu_slices(int64_t ntb, int R_ff, int NW) {
+  int best = 1;
+  int64_t cost = 0;
+  for (int H = 1; H <= R_ff; H = H < 4 ? H + 1 : (H / 8 + 1) * 8) {
+    const int rows = (R_ff + H - 1) / H;
+    const int64_t c = (ntb * H + 255) / 256 * ((rows + NW - 1) / NW + 2);
+    if (H == 1 || c < cost) {
+      cost = c;
+      best = H;
+    }
+  }
+  return best;
 }
 
 bool split_supported(int B, int d_model, int R_ff, int R_m, int Kg, int Ku, int Kd) {
@@ -1448,14 +1452,20 @@ static int launch_gu_b(const GUArgs& a, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-template <int B, int MT, bool NORM, bool SHARED = false, bool BIAS = false>
+template <int B, int MT, bool NORM, bool SHARED = false, bool BIAS = false, bool INTER = false, int NW = 12, int RING = 2>
 static int launch_gu_w12(const GUArgs& a, hipStream_t st) {
-  auto kern = gu_kernel_w12<B, MT, NORM, SHARED, BIAS>;
+  auto kern = gu_kernel_w12<B, MT, NORM, SHARED, BIAS, INTER, NW, RING>;
   static std::atomic<uint64_t> configured{0};
   if (set_lds_limit_once((const void*)kern, 163840, configured)) return -1;
-  hipLaunchKernelGGL(kern, dim3((unsigned)((a.N + 16 * MT - 1) / (16 * MT))), dim3(64 * gu_w12_waves<B, SHARED>()),
+  hipLaunchKernelGGL(kern, dim3((unsigned)((a.N + 16 * MT - 1) / (16 * MT) * a.H)), dim3(64 * NW),
                      gu_lds(a.R_ff, a.Kg, MT), st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+// B = 16 runs 16 waves: a shared topology's slot pairs two deep (four slots in flight), distinct
+// topologies' single slots four deep, or two where the exported pre-activations would spill
+template <int MT, bool NORM, bool SHARED, bool BIAS, bool INTER>
+static int launch_gu16(const GUArgs& a, hipStream_t st) {
+  return launch_gu_w12<16, MT, NORM, SHARED, BIAS, INTER, 16, SHARED || INTER ? 2 : 4>(a, st);
 }
 
 // the bias-free kernels carry no bias code (a bias is an epilogue add and two loads per column)
@@ -1470,7 +1480,8 @@ int launch_gu(int B, bool norm, const GUArgs& a0, hipStream_t st) {
   const int mt = gu_mt(a0.d_model);
   if (mt == 0) return -2;
   GUArgs a = a0;
-  a.H = gu_slices((a.N + 16 * mt - 1) / (16 * mt), a.R_ff);
+  const int64_t ntb = (a.N + 16 * mt - 1) / (16 * mt);
+  a.H = gu_slices(ntb, a.R_ff, 8);
   const bool inter = a.gpre || a.uout;
   // gate and up passing the same column-index buffer share their topology (the reference
   // layer initialises both from the same seed)
@@ -1481,33 +1492,28 @@ int launch_gu(int B, bool norm, const GUArgs& a0, hipStream_t st) {
   // fast or faster, 0.1378 against 0.1381-0.1429 ms)
   if (B == 32 && mt == 4 && a.H == 1 && !inter && !shared && !a.bg && !a.bu)
     return norm ? launch_gu_w12<32, 4, true>(a, st) : launch_gu_w12<32, 4, false>(a, st);
-  // B = 16 with one row slice and no exports: 16 waves for every topology and bias combination
-  // (at most 113 VGPRs; reference-default layer forward 0.2615 -> 0.2408 ms against 8 waves)
-  // the same at 32-token panels (d_model 2048), bias-free or not, shared or not; the normalising
-  // fill of 2048-wide rows would spill at 16 waves (the reference's large tile-16 layer, d_ff 8192,
-  // 25 %, biases, shared topology, 16384 tokens: 1.276 -> 1.198 ms per forward)
-  if (B == 16 && mt == 2 && a.H == 1 && !inter && !norm) {
+  // B = 16: 16 waves for every topology, bias and export combination (at most 128 VGPRs; against 8
+  // waves: reference-default layer forward 0.2615 -> 0.2408 ms, 3000 x 1024 with biases 103 -> 90 us,
+  // 3000 x 2048 190 -> 143).  The normalising fill of 2048-wide rows would spill: 8 waves there.
+  if (B == 16 && !(mt == 2 && norm)) {
+    a.H = gu_slices(ntb, a.R_ff, 16);
     const int sel = (shared ? 2 : 0) | ((a.bg || a.bu) ? 1 : 0);
-    switch (sel) {
-      case 0: return launch_gu_w12<16, 2, false, false, false>(a, st);
-      case 1: return launch_gu_w12<16, 2, false, false, true>(a, st);
-      case 2: return launch_gu_w12<16, 2, false, true, false>(a, st);
-      default: return launch_gu_w12<16, 2, false, true, true>(a, st);
-    }
+#define LBK_GU16(MM, NO, IN)                                                     \
+  switch (sel) {                                                                 \
+    case 0: return launch_gu16<MM, NO, false, false, IN>(a, st);                 \
+    case 1: return launch_gu16<MM, NO, false, true, IN>(a, st);                  \
+    case 2: return launch_gu16<MM, NO, true, false, IN>(a, st);                  \
+    default: return launch_gu16<MM, NO, true, true, IN>(a, st);                  \
   }
-  if (B == 16 && mt == 4 && a.H == 1 && !inter) {
-    const int sel = (norm ? 4 : 0) | (shared ? 2 : 0) | ((a.bg || a.bu) ? 1 : 0);
-    switch (sel) {
-      case 0: return launch_gu_w12<16, 4, false, false, false>(a, st);
-      case 1: return launch_gu_w12<16, 4, false, false, true>(a, st);
-      case 2: return launch_gu_w12<16, 4, false, true, false>(a, st);
-      case 3: return launch_gu_w12<16, 4, false, true, true>(a, st);
-      case 4: return launch_gu_w12<16, 4, true, false, false>(a, st);
-      case 5: return launch_gu_w12<16, 4, true, false, true>(a, st);
-      case 6: return launch_gu_w12<16, 4, true, true, false>(a, st);
-      default: return launch_gu_w12<16, 4, true, true, true>(a, st);
-    }
+    if (mt == 2 && inter) { LBK_GU16(2, false, true) }
+    if (mt == 2) { LBK_GU16(2, false, false) }
+    if (norm) { LBK_GU16(4, true, false) }
+    if (inter) { LBK_GU16(4, false, true) }
+    LBK_GU16(4, false, false)
+#undef LBK_GU16
   }
+  if (B == 16)
+    return shared ? launch_gu_t<16, 2, true, false, true>(a, st) : launch_gu_t<16, 2, true, false, false>(a, st);
 #define LBK_GU2(BB, MM, SH)                                                                          \
   if (norm) return launch_gu_t<BB, MM, true, false, SH>(a, st);                                     \
   return inter ? launch_gu_t<BB, MM, false, true, SH>(a, st) : launch_gu_t<BB, MM, false, false, SH>(a, st);
@@ -1516,7 +1522,7 @@ int launch_gu(int B, bool norm, const GUArgs& a0, hipStream_t st) {
     if (shared) { LBK_GU2(BB, MM, true) }                                                       \
     LBK_GU2(BB, MM, false)                                                                      \
   }
-  LBK_GU(16, 4) LBK_GU(16, 2) LBK_GU(32, 4) LBK_GU(32, 2)
+  LBK_GU(32, 4) LBK_GU(32, 2)
 #undef LBK_GU
 #undef LBK_GU2
   return -2;
@@ -1550,7 +1556,7 @@ static int launch_lin_g(int B, const GUArgs& a0, hipStream_t st) {
   a.Ku = a.Kg;
   const int mt = gu_mt(a.d_model);
   if (mt == 0) return -2;
-  a.H = gu_slices((a.N + 16 * mt - 1) / (16 * mt), a.R_ff);
+  a.H = gu_slices((a.N + 16 * mt - 1) / (16 * mt), a.R_ff, LIN_WAVES);
 #define LBK_LIN(BB, MM)                                                                     \
   if (B == BB && mt == MM)                                                                  \
     return a.bg ? launch_lin_t<BB, MM, true, GELU>(a, st) : launch_lin_t<BB, MM, false, GELU>(a, st);
