@@ -28,6 +28,9 @@
 // two-slot ring that also prefetches the next stage's first tiles.  The
 // epilogue adds the residual, or carries an fp32 state for the looped block.
 //
+// dnr_kernel: the down kernel where those leave CUs idle, and at B = 16: smaller workgroups, wider
+// stages and a ring (its own comment).
+//
 // dnf_kernel<B, D>: the plain forward's down kernel at B = 32 on 64-token blocks: the same
 // workgroup and stages, but each wave streams its row through a D-slot ring across the stages
 // (no pair padding, stage changes taken inline); see its comment.
@@ -1072,6 +1075,192 @@ __global__ __launch_bounds__(64 * NW, 1) void dn_kernel(DNArgs a) {
 }
 
 // ===========================================================================
+// down projection, ring over wide stages
+// ===========================================================================
+// dnr_kernel<B, MT, NW, OPW, COLS, KC, BIAS>: 16 MT tokens, NW waves of OPW down rows each (wave w owns
+// rows w, w + NW, ... of its group).  With one row a wave a step is one tile and little work, so the
+// kernel is bound by the latency of its tile loads: they run through a D-deep ring (pairs of slots at
+// B = 16: one 16x16x32 MFMA per token tile, lanes g < 2 with slot 2p, the others with 2p + 1), and a
+// stage holds COLS columns of h (one LDS buffer, the next stage in registers meanwhile) so that a
+// row's run within a stage fills the ring.  The tile is the MFMA's A operand, so a lane ends with
+// 4 (B = 16) or 8 (B = 32) consecutive columns of one token.
+template <int B, int MT, int NW, int OPW, int COLS, int KC, bool BIAS>
+__global__ __launch_bounds__(64 * NW, 1) void dnr_kernel(DNArgs a) {
+  constexpr int NT = 64 * NW, TM = 16 * MT, CW = B / 16, D = 4;
+  constexpr int G = COLS / B, SROWB = COLS * 2;
+  constexpr int PER_T = TM * SROWB / 16 / NT;        // 16-byte chunks per thread per stage
+  static_assert(TM * SROWB / 16 % NT == 0, "whole chunks per thread");
+  extern __shared__ __attribute__((aligned(16))) unsigned char dn_smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = uniform(tid >> 6);
+  const int i = lane & 15, g = lane >> 4;
+  // workgroup -> (token block, row group), as in dn_kernel
+  int tb = (int)blockIdx.x, rg = 0;
+  if (a.nrg > 1) {
+    const int b = (int)blockIdx.x, rest = b >> 3;
+    rg = rest % a.nrg;
+    tb = 8 * (rest / a.nrg) + (b & 7);
+  }
+  const int64_t t0 = (int64_t)tb * TM;
+  if (t0 >= a.N) return;                             // the whole workgroup, before any barrier
+  const int row0 = rg * NW * OPW + w;
+  const int nstages = (a.C_d + G - 1) / G;
+
+  u32x4 sreg[PER_T];
+  auto stage_fetch = [&](int s) {
+#pragma unroll
+    for (int u = 0; u < PER_T; ++u) {
+      const int e = tid + NT * u;
+      const int row = e / (SROWB / 16), cc = e - row * (SROWB / 16);
+      const int64_t t = t0 + row, col = (int64_t)s * COLS + 8 * cc;
+      const bool ok = t < a.N && col < a.d_ff;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(a.h + (ok ? t : t0) * a.d_ff + (ok ? col : 0));
+      sreg[u] = ok ? v : u32x4{0, 0, 0, 0};
+    }
+  };
+  auto stage_store = [&]() {
+#pragma unroll
+    for (int u = 0; u < PER_T; ++u) {
+      const int e = tid + NT * u;
+      const int row = e / (SROWB / 16), cc = e - row * (SROWB / 16);
+      *reinterpret_cast<u32x4*>(dn_smem + panel_addr<MT>(row, cc, SROWB)) = sreg[u];
+    }
+  };
+
+  int colreg[OPW][KC];                               // lane l: the column of slot 64 kc + l (-1 beyond)
+#pragma unroll
+  for (int o = 0; o < OPW; ++o)
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc) {
+      const int rm = row0 + NW * o, k = 64 * kc + lane;
+      colreg[o][kc] = (rm < a.R_m && k < a.Kd) ? a.cd[(int64_t)rm * a.Kd + k] : -1;
+    }
+  f32x4 acc[OPW][MT][CW];
+#pragma unroll
+  for (int o = 0; o < OPW; ++o)
+#pragma unroll
+    for (int q = 0; q < MT; ++q)
+#pragma unroll
+      for (int m = 0; m < CW; ++m) acc[o][q][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const uint32_t lbase = (uint32_t)(i * MT * SROWB);
+  const u32x4* pd = static_cast<const u32x4*>(a.pd);
+  struct Slot {
+    u32x4 f[CW];
+    int cb;   // column block within the stage (B = 16: of both slots, and whether the second counts)
+  };
+  stage_fetch(0);
+  for (int s = 0; s < nstages; ++s) {
+    if (s > 0) __syncthreads();                      // the previous stage has been read
+    stage_store();
+    __syncthreads();
+    if (s + 1 < nstages) stage_fetch(s + 1);
+    const int c0 = s * G;
+#pragma unroll
+    for (int o = 0; o < OPW; ++o)
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) {
+        const int cl = colreg[o][kc] - c0;
+        uint64_t m = __ballot(cl >= 0 && cl < G && colreg[o][kc] < a.C_d);
+        const int n = __builtin_popcountll(m);
+        if (n == 0) continue;
+        const int64_t e0 = (int64_t)(row0 + NW * o) * a.Kd + 64 * kc;
+        int last = 0;
+        // the next hit (past the end: the last one again)
+        auto next = [&]() {
+          if (m) {
+            last = __builtin_ctzll(m);
+            m &= m - 1;
+          }
+          return last;
+        };
+        auto fetch = [&](Slot& S) {
+          if constexpr (B == 16) {
+            const int b1 = next();
+            const int two = m ? 1 << 20 : 0;
+            const int b2 = next();
+            const int b = g < 2 ? b1 : b2;
+            S.f[0] = pd[(e0 + b) * PackedTile<B>::U32X4 + i + 16 * (g & 1)];
+            S.cb = __builtin_amdgcn_readlane(cl, b1) | (__builtin_amdgcn_readlane(cl, b2) << 10) | two;
+          } else {
+            const int b1 = next();
+            const u32x4* tp = pd + (e0 + b1) * PackedTile<B>::U32X4 + lane;
+#pragma unroll
+            for (int mm = 0; mm < CW; ++mm) S.f[mm] = tp[64 * mm];
+            S.cb = __builtin_amdgcn_readlane(cl, b1);
+          }
+        };
+        auto compute = [&](const Slot& S) {
+          const int cb = uniform(S.cb);
+          if constexpr (B == 16) {
+            const int rl = g < 2 ? (cb & 1023) : ((cb >> 10) & 1023);
+            const u32x4 f = (g < 2 || ((cb >> 20) & 1)) ? S.f[0] : u32x4{0, 0, 0, 0};
+            const uint32_t pa = lbase + ((uint32_t)((rl * 2 + (g & 1)) ^ i) << 4);
+#pragma unroll
+            for (int q = 0; q < MT; ++q) acc[o][q][0] = mfma_bf16(f, lds16(dn_smem, pa + q * SROWB), acc[o][q][0]);
+          } else {
+            const uint32_t pa = lbase + ((uint32_t)((cb * (B / 8) + g) ^ i) << 4);
+#pragma unroll
+            for (int q = 0; q < MT; ++q) {
+              const u32x4 hv = lds16(dn_smem, pa + q * SROWB);
+#pragma unroll
+              for (int mm = 0; mm < CW; ++mm) acc[o][q][mm] = mfma_bf16(S.f[mm], hv, acc[o][q][mm]);
+            }
+          }
+        };
+        const int np = B == 16 ? (n + 1) >> 1 : n;
+        Slot S[D];
+#pragma unroll
+        for (int k = 0; k < D - 1; ++k) fetch(S[k]);
+        for (int p = 0; p < np; p += D) {
+#pragma unroll
+          for (int k = 0; k < D; ++k) {
+            fetch(S[(k + D - 1) % D]);
+            if (k == 0 || p + k < np) compute(S[k]);
+          }
+        }
+      }
+  }
+
+  // lane (i, g): token 16 q + i, columns NV g .. + NV - 1 of its row (B = 32: accumulator m, v is
+  // column 8 g + 2 v + m, as the tiles are packed)
+  constexpr int NV = 4 * CW;
+#pragma unroll
+  for (int o = 0; o < OPW; ++o) {
+    const int rm = row0 + NW * o;
+    if (rm >= a.R_m) continue;
+    const int col = rm * B + NV * g;
+    float bv[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) bv[j] = BIAS && a.bd ? a.bd[col + j] : 0.f;
+#pragma unroll
+    for (int q = 0; q < MT; ++q) {
+      const int64_t t = t0 + 16 * q + i;
+      if (t >= a.N) continue;
+      const int64_t off = t * a.d_model + col;
+      float v[NV];
+#pragma unroll
+      for (int j = 0; j < NV; ++j) v[j] = acc[o][q][j % CW][j / CW] + bv[j];
+      if (a.state) {
+#pragma unroll
+        for (int j = 0; j < NV; j += 4) {
+          f32x4 sv = *reinterpret_cast<const f32x4*>(a.state + off + j);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[j + u] = sv[u] += v[j + u];
+          *reinterpret_cast<f32x4*>(a.state + off + j) = sv;
+        }
+      } else if (a.resid) {
+        float rv[NV];
+        load_bf16x<NV>(a.resid + off, rv);
+#pragma unroll
+        for (int j = 0; j < NV; ++j) v[j] += rv[j];
+      }
+      if (a.out) store_bf16x<NV>(a.out + off, v);
+    }
+  }
+}
+
+// ===========================================================================
 // down projection with a deep ring (the plain forward)
 // ===========================================================================
 // dnf_kernel<B, D>: the dn_kernel workgroup (16 waves, 64 tokens, one down row per wave, h staged
@@ -1618,18 +1807,60 @@ static int launch_dnf(const DNArgs& a0, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+template <int B, int MT, int NW, int OPW, int COLS, int KC>
+static int launch_dnr_k(const DNArgs& a0, hipStream_t st) {
+  constexpr int TM = 16 * MT, lds = TM * COLS * 2;
+  DNArgs a = a0;
+  const int64_t ntb = (a.N + TM - 1) / TM;
+  a.nrg = (a.R_m + NW * OPW - 1) / (NW * OPW);
+  const int64_t grid = a.nrg == 1 ? ntb : 8 * a.nrg * ((ntb + 7) / 8);
+  auto kern = a.bd ? dnr_kernel<B, MT, NW, OPW, COLS, KC, true> : dnr_kernel<B, MT, NW, OPW, COLS, KC, false>;
+  static std::atomic<uint64_t> done[2] = {{0}, {0}};
+  if (lds > 65536 && set_lds_limit_once(reinterpret_cast<const void*>(kern), lds, done[a.bd ? 1 : 0])) return -1;
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), lds, st, a);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+template <int B, int MT, int NW, int OPW, int COLS>
+static int launch_dnr(const DNArgs& a, hipStream_t st) {
+  return a.Kd > 64 ? launch_dnr_k<B, MT, NW, OPW, COLS, 2>(a, st) : launch_dnr_k<B, MT, NW, OPW, COLS, 1>(a, st);
+}
+
+// The ring kernel's form for a token count and row count (-2: the kernels with 512-column stages are
+// faster).  Workgroups of 64 tokens while they fill about half the CUs or more, then 32 tokens and 8
+// rows (1024-column stages, two workgroups a CU, above 256 of them), then 16 tokens and 4 rows.  us a
+// forward or looped forward, in the order 64 x 16 (B = 16) or 64 x 8 rows (B = 32) / 32 x 8 with 2048
+// columns / with 1024 / 16 x 4 / the two-slot kernel before it:
+//   B = 16  4099 x 512 K 128: 61 / 79 / 70 / 94 / 105     2048 x 512 x4 training: 529 / 491 / 499 / 521 / 531
+//           5000 x 256 x8: 330 / 356 / 308 / 394 / 433    300 x 512 x8: 239 / 181 / 194 / 167 / 210
+//   B = 32  3000 x 1024: 50 / 55 / 58 / 58 / 61           2338 x 512 x7: 247 / 213 / 220 / 222 / 245
+//           700 x 1024: 35 / 26 / 29 / 24 / 31            1313 x 512 x8: 269 / 221 / 231 / 213 / 253
+// At B = 32 whole rounds of 64 tokens and 16 rows stay with dnf_kernel and dn_kernel (16384 x 1024:
+// 166 us, 181 here), and at B = 16 those whose rows have few slots in a stage (3000 x 2048 at 0.1:
+// 144, 147 here).
+template <int B>
+static int launch_dn_ring(const DNArgs& a, int64_t w16, hipStream_t st) {
+  const int64_t w8 = (a.N + 63) / 64 * ((a.R_m + 7) / 8), w2 = (a.N + 31) / 32 * ((a.R_m + 7) / 8);
+  if (B == 16 && w16 >= 256 && (int64_t)a.Kd * 1024 < 8 * a.d_ff) return -2;
+  if (B == 16 && w16 >= 128) return launch_dnr<16, 4, 16, 1, 1024>(a, st);
+  if (B == 32 && w16 >= 200) return -2;
+  if (B == 32 && w8 >= 160) return launch_dnr<32, 4, 8, 1, 1024>(a, st);
+  if (w2 > 256) return launch_dnr<B, 2, 8, 1, 1024>(a, st);
+  if (w2 >= 128) return launch_dnr<B, 2, 8, 1, 2048>(a, st);
+  return launch_dnr<B, 1, 4, 1, 2048>(a, st);
+}
+
 int launch_dn(int B, const DNArgs& a, hipStream_t st) {
   if (a.N == 0) return 0;
   // the deep-ring kernel takes the plain forward (with an fp32 state, as the looped block's
   // iterations run it, it measured slower: L = 8 at the headline geometry 1.270 -> 1.281 ms)
   const bool plain = !a.state && !a.tdepth && !a.inj_e && a.out && a.Kd <= 64;
-  // Fewer 64-token blocks than the 16-row groups need to fill the CUs: smaller workgroups with
-  // longer stages, so that more of them run and each walks fewer stages -- 16 tokens and 4 rows
-  // per workgroup with 2048-column stages (1024 for B = 16) while they number at most 128, else
-  // 32 tokens and 8 rows with 1024-column stages.  Measured at d_model 1024, d_ff 4096, B = 32
-  // (forward per N = 64 / 256 / 1024 / 2048 / 4096): 20.0 / 21.0 / 28.6 / 37.3 / 62.3 us, against
-  // 38.4 / 40.3 / 44.4 / 50.9 / 61.9 with 64 tokens and 4 rows at 256-column stages.
-  if ((a.N + 63) / 64 * ((a.R_m + 15) / 16) < 256) {
+  const int64_t w16 = (a.N + 63) / 64 * ((a.R_m + 15) / 16);   // 64-token workgroups of 16 rows
+  if (!a.tdepth && !a.inj_e) {
+    const int rc = B == 16 ? launch_dn_ring<16>(a, w16, st) : B == 32 ? launch_dn_ring<32>(a, w16, st) : -2;
+    if (rc != -2) return rc;
+  } else if (w16 < 256) {
+    // the looped core's state update, with too few workgroups of 64 tokens and 16 rows: smaller ones
+    // with longer stages (1024 columns, 2048 at 16 tokens and B = 32)
     if ((a.N + 15) / 16 * ((a.R_m + 3) / 4) <= 128) {
       if (B == 16) return launch_dn_t<16, 1, 1, 4, 1024>(a, st);
       if (B == 32) return launch_dn_t<32, 1, 1, 4, 2048>(a, st);
