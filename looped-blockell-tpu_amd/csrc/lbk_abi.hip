@@ -255,6 +255,16 @@ static size_t packed_ffn_bytes(const lbk_bell* gate, const lbk_bell* up, const l
          align256(packed_bf16_bytes((int64_t)down->R * down->K, B));
 }
 
+// the three parts of a copy made by lbk_swiglu_prepack_bf16
+static PackedFFN packed_ffn_at(const char* p, const lbk_bell* gate, const lbk_bell* up) {
+  PackedFFN pk{};
+  pk.g = p;
+  p += align256(packed_bf16_bytes((int64_t)gate->R * gate->K, gate->B));
+  pk.u = p;
+  pk.d = p + align256(packed_bf16_bytes((int64_t)up->R * up->K, gate->B));
+  return pk;
+}
+
 // fp32 master tiles of gate, up and down and the buffers of their bf16 copies
 struct MasterFFN {
   const float* v[3];
@@ -393,11 +403,7 @@ static int swiglu_fwd_impl(const uint16_t* x, int64_t N, int32_t d_model, const 
   if (split) {
     PackedFFN pk{};
     if (prepacked) {
-      const int B = gate->B;
-      pk.g = prepacked;
-      pk.u = prepacked + align256(packed_bf16_bytes((int64_t)gate->R * gate->K, B));
-      pk.d = static_cast<const char*>(pk.u) + align256(packed_bf16_bytes((int64_t)up->R * up->K, B));
-      pk.bytes = pbytes;
+      pk = packed_ffn_at(prepacked, gate, up);
     } else if ((st = pack_ffn(gate, up, down, ws, &pk, s, master))) {
       return st;
     }
@@ -568,7 +574,8 @@ static int looped_persistent(const uint16_t* h_in, int64_t N, int32_t d_model, c
                              uint16_t* h_out, void* workspace, size_t workspace_bytes, void* stream, Biases bs);
 static int looped_launches(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale, float eps,
                            int32_t L, const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down,
-                           uint16_t* h_out, void* workspace, size_t workspace_bytes, void* stream, Biases bs);
+                           uint16_t* h_out, void* workspace, size_t workspace_bytes, void* stream, Biases bs,
+                           const char* prepacked = nullptr);
 
 int lbk_looped_swiglu_bf16(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale, float eps,
                            int32_t L, const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down,
@@ -589,6 +596,22 @@ int lbk_looped_swiglu_bias_bf16(const uint16_t* h_in, int64_t N, int32_t d_model
                          stream, bs);
 }
 
+int lbk_looped_swiglu_prepacked_bf16(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale,
+                                     float eps, int32_t L, const lbk_bell* gate, const lbk_bell* up,
+                                     const lbk_bell* down, const void* packed, size_t packed_bytes,
+                                     const float* b_gate, const float* b_up, const float* b_down, uint16_t* h_out,
+                                     void* workspace, size_t workspace_bytes, void* stream) {
+  if (!gate || !up || !down) return LBK_ERR_NULL;
+  const size_t need = lbk_swiglu_prepacked_bytes(d_model, gate, up, down);
+  if (need && N > 0) {
+    if (!packed) return LBK_ERR_NULL;
+    if (packed_bytes < need) return LBK_ERR_WORKSPACE;
+    if (!a16(packed)) return LBK_ERR_ALIGN;
+  }
+  return looped_launches(h_in, N, d_model, norm_scale, eps, L, gate, up, down, h_out, workspace, workspace_bytes,
+                         stream, Biases{b_gate, b_up, b_down}, need ? static_cast<const char*>(packed) : nullptr);
+}
+
 int lbk_looped_swiglu_launches_bf16(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale,
                                     float eps, int32_t L, const lbk_bell* gate, const lbk_bell* up,
                                     const lbk_bell* down, uint16_t* h_out, void* workspace, size_t workspace_bytes,
@@ -599,7 +622,8 @@ int lbk_looped_swiglu_launches_bf16(const uint16_t* h_in, int64_t N, int32_t d_m
 
 static int looped_launches(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale, float eps,
                            int32_t L, const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down,
-                           uint16_t* h_out, void* workspace, size_t workspace_bytes, void* stream, Biases bs) {
+                           uint16_t* h_out, void* workspace, size_t workspace_bytes, void* stream, Biases bs,
+                           const char* prepacked) {
   int st;
   if ((st = check_bell(gate)) || (st = check_bell(up)) || (st = check_bell(down))) return st;
   int64_t d_ff = 0;
@@ -650,7 +674,8 @@ static int looped_launches(const uint16_t* h_in, int64_t N, int32_t d_model, con
     // fp32 state carried across the L applications; bf16 written once, after the last
     float* state = reinterpret_cast<float*>(ws);
     PackedFFN pk{};
-    if ((st = pack_ffn(gate, up, down, ws + sbytes + hbytes, &pk, s))) return st;
+    if (prepacked) pk = packed_ffn_at(prepacked, gate, up);
+    else if ((st = pack_ffn(gate, up, down, ws + sbytes + hbytes, &pk, s))) return st;
     if (launch_bf16_to_f32(h_in, N * d_model, state, s) != 0) return LBK_ERR_LAUNCH;
     for (int l = 0; l < L; ++l)
       if ((st = swiglu_split(nullptr, state, norm_scale, eps, N, d_model, gate, up, down, pk, nullptr, state,
@@ -1139,6 +1164,8 @@ int lbk_swiglu_fwd_ternary_prepared(const int8_t* xq, const float* sx, int64_t N
 static size_t tlist_bytes(const lbk_bell* w, int C) {
   return align256((size_t)C * 4) + align256((size_t)C * w->R * w->K * 4);
 }
+// floats of the column sums that dh's kernel forms per token block (blocks of 32 tokens at most 2 N / 64 + 1)
+static size_t dh_sum_floats(int64_t N, int64_t d_ff) { return (size_t)((N + 31) / 32) * (size_t)d_ff; }
 // fp32 partial tiles of one weight's tile gradients (the token chunking of launch_dw)
 static size_t dw_part_floats(int64_t N, const lbk_bell* w, int C, int64_t ldg) {
   const int64_t ch = dw_job_chunk(w->B, w->R, w->K, C, ldg, N);
@@ -1162,7 +1189,7 @@ size_t lbk_swiglu_bwd_bias_workspace_bytes(int64_t N, int32_t d_model, const lbk
   const size_t base = lbk_swiglu_bwd_workspace_bytes(N, d_model, gate, up, down);
   if (!base) return 0;
   const int64_t d_ff = (int64_t)gate->R * gate->B;
-  return base + align256(colsum_bytes(N, 2 * d_ff + d_model));
+  return base + align256(colsum_bytes(N, 2 * d_ff + d_model)) + 2 * align256(dh_sum_floats(N, d_ff) * 4);
 }
 
 int lbk_swiglu_bwd_bf16(const uint16_t* grad_out, const uint16_t* x, const uint16_t* gate_pre_act,
@@ -1230,6 +1257,15 @@ static int swiglu_bwd_impl(const uint16_t* grad_out, const uint16_t* x, const ui
   uint16_t* dg = reinterpret_cast<uint16_t*>(take((size_t)N * d_ff * 2));
   uint16_t* du = reinterpret_cast<uint16_t*>(take((size_t)N * d_ff * 2));
   float* part = reinterpret_cast<float*>(p);
+  // after the tile partials: the column sums of dg and du that dh's kernel forms, and the partials of
+  // those (and of grad_out) read as matrices
+  const size_t parts = dw_part_floats(N, gate, C_in, d_ff) + dw_part_floats(N, up, C_in, d_ff) +
+                       dw_part_floats(N, down, C_d, d_model);
+  char* tail = reinterpret_cast<char*>(part) + align256(parts * 4);
+  float* gsum = reinterpret_cast<float*>(tail);
+  float* usum = reinterpret_cast<float*>(tail + align256(dh_sum_floats(N, d_ff) * 4));
+  float* cpart = reinterpret_cast<float*>(tail + 2 * align256(dh_sum_floats(N, d_ff) * 4));
+  int64_t sum_rows = 0;
   // slots of a weight with no tiles (R * K == 0) take no part in the lists
   int nl = 0;
   TListJob ljn[3];
@@ -1243,6 +1279,8 @@ static int swiglu_bwd_impl(const uint16_t* grad_out, const uint16_t* x, const ui
     if (td > 0) a.src[a.nsrc++] = TProdSrc{grad_out, d_model, down->values, down->K, lj[0].cnt, lj[0].list, td};
     a.N = N; a.C = C_d; a.ldo = d_ff;
     a.g = gate_pre_act; a.u = up_output; a.dg = dg; a.du = du;
+    if (d_b_gate || d_b_up) sum_rows = dh_sum_blocks(B, a);
+    if (sum_rows) { a.dgsum = gsum; a.dusum = usum; }
     if (launch_tprod(B, 0, a, s)) return LBK_ERR_LAUNCH;
     // dx = dg W_gate + du W_up (+ dy)
     TProdArgs b{};
@@ -1272,11 +1310,11 @@ static int swiglu_bwd_impl(const uint16_t* grad_out, const uint16_t* x, const ui
   if (nj && launch_dw(B, dj, nj, N, s)) return LBK_ERR_LAUNCH;
   // bias gradients: column sums of dg, du and grad_out (the partials after the tile partials)
   if (want_db) {
-    float* cpart = reinterpret_cast<float*>(reinterpret_cast<char*>(part) + align256(poff * 4));
     ColsumJob cj[3];
     int nc = 0;
-    if (d_b_gate) cj[nc++] = ColsumJob{dg, d_ff, (int)d_ff, d_b_gate, nullptr, 0, 0};
-    if (d_b_up) cj[nc++] = ColsumJob{du, d_ff, (int)d_ff, d_b_up, nullptr, 0, 0};
+    const bool have = sum_rows > 0;
+    if (d_b_gate) cj[nc++] = ColsumJob{have ? nullptr : dg, d_ff, (int)d_ff, d_b_gate, gsum, (int)sum_rows, 0};
+    if (d_b_up) cj[nc++] = ColsumJob{have ? nullptr : du, d_ff, (int)d_ff, d_b_up, usum, (int)sum_rows, 0};
     if (d_b_down) cj[nc++] = ColsumJob{grad_out, d_model, d_model, d_b_down, nullptr, 0, 0};
     if (launch_colsum(cj, nc, N, cpart, s)) return LBK_ERR_LAUNCH;
   }
@@ -1385,7 +1423,7 @@ static int64_t loop_group(int64_t N, int64_t d_ff, int32_t L) {
 }
 
 struct LoopBwdLayout {
-  size_t lists, dg, dy, dy_next, dxn, tmp, g, dw, cs, rms, total;
+  size_t lists, dg, dy, dy_next, dxn, tmp, g, dw, cs, sums, rms, total;
 };
 static LoopBwdLayout loop_bwd_layout(int64_t N, int32_t d_model, int32_t L, const lbk_bell* gate, const lbk_bell* up,
                                      const lbk_bell* down) {
@@ -1407,7 +1445,8 @@ static LoopBwdLayout loop_bwd_layout(int64_t N, int32_t d_model, int32_t L, cons
     l.cs = cs > l.cs ? cs : l.cs;
   }
   l.rms = align256((size_t)G * rmsnorm_bwd_bytes(N, d_model));
-  l.total = l.lists + 2 * l.dg + l.dy + l.dy_next + l.dxn + l.tmp + l.g + l.dw + l.cs + l.rms;
+  l.sums = align256((size_t)G * dh_sum_floats(N, d_ff) * 4);
+  l.total = l.lists + 2 * l.dg + l.dy + l.dy_next + l.dxn + l.tmp + l.g + l.dw + l.cs + 2 * l.sums + l.rms;
   return l;
 }
 
@@ -1473,6 +1512,8 @@ int lbk_looped_bwd_train(const uint16_t* grad_out, const uint16_t* states, const
   float* g = reinterpret_cast<float*>(take(lay.g));
   float* part = reinterpret_cast<float*>(take(lay.dw));
   float* cpart = reinterpret_cast<float*>(take(lay.cs));
+  float* gsum = reinterpret_cast<float*>(take(lay.sums));
+  float* usum = reinterpret_cast<float*>(take(lay.sums));
   float* rpart = reinterpret_cast<float*>(p);
   if (nl && launch_tlist(ljn, nl, s)) return LBK_ERR_LAUNCH;
   const int64_t nd = N * d_model, nf = N * d_ff, G = loop_group(N, d_ff, L);
@@ -1482,13 +1523,18 @@ int lbk_looped_bwd_train(const uint16_t* grad_out, const uint16_t* states, const
     // the gradient of the state after application hi - 1, into its slot (and, at the end of the
     // block, into the fp32 state gradient)
     if (launch_state_init(acc ? dy_next : grad_out, nd, acc ? nullptr : g, dy + (n - 1) * nd, s)) return LBK_ERR_LAUNCH;
-    int64_t nblk = 0;
+    int64_t nblk = 0, sum_rows = 0;
     for (int64_t t = hi - 1; t >= lo; --t) {
       const int64_t q = t - lo;
       TProdArgs a{};
       if (td > 0) a.src[a.nsrc++] = TProdSrc{dy + q * nd, d_model, down->values, down->K, lj[0].cnt, lj[0].list, td};
       a.N = N; a.C = C_d; a.ldo = d_ff;
       a.g = gate_pre + t * nf; a.u = up_out + t * nf; a.dg = dg + q * nf; a.du = du + q * nf;
+      if (d_b_gate || d_b_up) sum_rows = dh_sum_blocks(B, a);
+      if (sum_rows) {
+        a.dgsum = gsum + q * sum_rows * d_ff;
+        a.dusum = usum + q * sum_rows * d_ff;
+      }
       if (launch_tprod(B, 0, a, s)) return LBK_ERR_LAUNCH;
       TProdArgs b{};
       if (tg > 0) b.src[b.nsrc++] = TProdSrc{dg + q * nf, d_ff, gate->values, gate->K, lj[1].cnt, lj[1].list, tg};
@@ -1519,8 +1565,10 @@ int lbk_looped_bwd_train(const uint16_t* grad_out, const uint16_t* states, const
     if (nj && launch_dw(B, dj, nj, n * N, s)) return LBK_ERR_LAUNCH;
     ColsumJob cj[3];
     int nc = 0;
-    if (d_b_gate) cj[nc++] = ColsumJob{dg, d_ff, (int)d_ff, d_b_gate, nullptr, 0, acc};
-    if (d_b_up) cj[nc++] = ColsumJob{du, d_ff, (int)d_ff, d_b_up, nullptr, 0, acc};
+    const bool have = sum_rows > 0;
+    const int rows = (int)(n * sum_rows);
+    if (d_b_gate) cj[nc++] = ColsumJob{have ? nullptr : dg, d_ff, (int)d_ff, d_b_gate, gsum, rows, acc};
+    if (d_b_up) cj[nc++] = ColsumJob{have ? nullptr : du, d_ff, (int)d_ff, d_b_up, usum, rows, acc};
     if (d_b_down) cj[nc++] = ColsumJob{dy, d_model, d_model, d_b_down, nullptr, 0, acc};
     if (nc && launch_colsum(cj, nc, n * N, cpart, s)) return LBK_ERR_LAUNCH;
     if (launch_rmsnorm_dscale(rpart, n * nblk, d_model, d_scale, acc, s)) return LBK_ERR_LAUNCH;
@@ -1662,7 +1710,7 @@ size_t lbk_gelu_bwd_workspace_bytes(int64_t N, int32_t d_model, const lbk_bell* 
   const int C_in = d_model / w1->B, C_d = w1->R;
   return tlist_bytes(w2, C_d) + tlist_bytes(w1, C_in) + align256((size_t)N * d_ff * 2) +
          align256((dw_part_floats(N, w1, C_in, d_ff) + dw_part_floats(N, w2, C_d, d_model)) * 4) +
-         align256(colsum_bytes(N, d_ff + d_model));
+         align256(dh_sum_floats(N, d_ff) * 4) + align256(colsum_bytes(N, d_ff + d_model));
 }
 
 int lbk_gelu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint16_t* pre, const uint16_t* h,
@@ -1706,7 +1754,9 @@ int lbk_gelu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint16
   uint16_t* da = reinterpret_cast<uint16_t*>(take((size_t)N * d_ff * 2));
   const size_t f1 = dw_part_floats(N, w1, C_in, d_ff), f2 = dw_part_floats(N, w2, C_d, d_model);
   float* part = reinterpret_cast<float*>(take((f1 + f2) * 4));
+  float* asum = reinterpret_cast<float*>(take(dh_sum_floats(N, d_ff) * 4));
   float* cpart = reinterpret_cast<float*>(p);
+  int64_t sum_rows = 0;
   if (N > 0) {
     if (nl && launch_tlist(ljn, nl, s)) return LBK_ERR_LAUNCH;
     // da = (dy W2) gelu'(pre)
@@ -1714,6 +1764,8 @@ int lbk_gelu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint16
     if (t2 > 0) a.src[a.nsrc++] = TProdSrc{grad_out, d_model, w2->values, w2->K, lj[0].cnt, lj[0].list, t2};
     a.N = N; a.C = C_d; a.ldo = d_ff;
     a.g = pre; a.dg = da;
+    if (d_b1) sum_rows = dh_sum_blocks(B, a);
+    if (sum_rows) a.dgsum = asum;
     if (launch_tprod(B, 2, a, s)) return LBK_ERR_LAUNCH;
     // dx = da W1
     TProdArgs b{};
@@ -1732,7 +1784,8 @@ int lbk_gelu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint16
   if (nj && launch_dw(B, dj, nj, N, s)) return LBK_ERR_LAUNCH;
   ColsumJob cj[2];
   int nc = 0;
-  if (d_b1 && d_ff > 0) cj[nc++] = ColsumJob{da, d_ff, (int)d_ff, d_b1, nullptr, 0, 0};
+  if (d_b1 && d_ff > 0)
+    cj[nc++] = ColsumJob{sum_rows ? nullptr : da, d_ff, (int)d_ff, d_b1, asum, (int)sum_rows, 0};
   if (d_b2) cj[nc++] = ColsumJob{grad_out, d_model, d_model, d_b2, nullptr, 0, 0};
   if (nc && launch_colsum(cj, nc, N, cpart, s)) return LBK_ERR_LAUNCH;
   return LBK_OK;

@@ -351,7 +351,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_vec_kernel(const uint16_t* __
 // (bias gradients), all of a call's matrices in two launches.  Bound by reading the matrices once.
 // A workgroup sums `rows` rows of 256 columns: 32 lanes of 16 bytes cover the columns (512
 // contiguous bytes a row), the 8 half-waves take every eighth row, four row loads in flight each,
-// and LDS adds the eight.  colsum_reduce_kernel adds the row chunks, four strands a column.  Every
+// and LDS adds the eight.  colsum_reduce_kernel adds the row chunks, 16 strands a column.  Every
 // sum has a fixed order.  dg, du [16384, 4096] and dy [16384, 1024]: 1322 us with one row loop a
 // thread over 2-byte loads and 64-row workgroups, 66 us so (302 MB at 4.6 TB/s; a copy reaches 4.9).
 __global__ __launch_bounds__(256) void colsum_part_kernel(ColsumJobs jobs) {
@@ -398,34 +398,36 @@ __global__ __launch_bounds__(256) void colsum_part_kernel(ColsumJobs jobs) {
   }
 }
 
-// out[c] = sum over the chunks of part[chunk, c]: 64 columns a workgroup, chunks q, q + 4, ... by
-// strand q, eight loads in flight
+// out[c] = sum over the chunks of part[chunk, c]: 16 columns a workgroup, chunks q, q + 16, ... by
+// strand q, eight loads in flight (1024 chunks of 512 columns: 12.9 us in 64 columns and 4 strands)
 __global__ __launch_bounds__(256) void colsum_reduce_kernel(ColsumJobs jobs) {
-  __shared__ float sums[4][64];
+  __shared__ float sums[16][17];
   int jt = 0;
 #pragma unroll
   for (int u = 1; u < ColsumJobs::kMax; ++u)
     if (u < jobs.n && (int)blockIdx.x >= jobs.rfirst[u]) jt = u;
   const ColsumJob& J = jobs.job[jt];
-  const int tc = threadIdx.x & 63, tq = threadIdx.x >> 6;
-  const int c = ((int)blockIdx.x - jobs.rfirst[jt]) * 64 + tc;
+  const int tc = threadIdx.x & 15, tq = threadIdx.x >> 4;
+  const int c = ((int)blockIdx.x - jobs.rfirst[jt]) * 16 + tc;
   float s = 0.f;
   if (c < J.C) {
     const float* p = J.part + c;
     int ch = tq;
-    for (; ch + 28 < J.nchunk; ch += 32) {
+    for (; ch + 112 < J.nchunk; ch += 128) {
       float v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)(ch + 4 * u) * J.C];
+      for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)(ch + 16 * u) * J.C];
 #pragma unroll
       for (int u = 0; u < 8; ++u) s += v[u];
     }
-    for (; ch < J.nchunk; ch += 4) s += p[(int64_t)ch * J.C];
+    for (; ch < J.nchunk; ch += 16) s += p[(int64_t)ch * J.C];
   }
   sums[tq][tc] = s;
   __syncthreads();
   if (tq == 0 && c < J.C) {
-    const float t = (sums[0][tc] + sums[1][tc]) + (sums[2][tc] + sums[3][tc]);
+    float t = sums[0][tc];
+#pragma unroll
+    for (int q = 1; q < 16; ++q) t += sums[q][tc];
     J.out[c] = J.acc ? J.out[c] + t : t;
   }
 }
@@ -448,13 +450,14 @@ int launch_colsum(const ColsumJob* in, int n, int64_t N, float* part, hipStream_
     const int64_t nchunk = colsum_chunks(N);
     if (in[t].C <= 0 || nchunk > 0x7fffffff) return -2;
     J.job[t] = in[t];
+    J.first[t] = (int)blocks;
+    J.rfirst[t] = (int)rblocks;
+    rblocks += (in[t].C + 15) / 16;
+    if (!in[t].a) continue;                          // its partial sums are there already
     J.job[t].nchunk = (int)nchunk;
     J.job[t].part = part;
     part += nchunk * in[t].C;
-    J.first[t] = (int)blocks;
-    J.rfirst[t] = (int)rblocks;
     blocks += nchunk * ((in[t].C + 255) / 256);
-    rblocks += (in[t].C + 63) / 64;
   }
   if (blocks > 0x7fffffff) return -2;
   if (blocks > 0) {
@@ -521,7 +524,7 @@ int launch_rmsnorm_dscale(float* part, int64_t nblk, int d, float* dscale, int a
   ColsumJobs J{};
   J.n = 1;
   J.job[0] = ColsumJob{nullptr, 0, d, dscale, part, (int)nblk, acc};
-  hipLaunchKernelGGL(colsum_reduce_kernel, dim3((unsigned)((d + 63) / 64)), dim3(256), 0, st, J);
+  hipLaunchKernelGGL(colsum_reduce_kernel, dim3((unsigned)((d + 15) / 16)), dim3(256), 0, st, J);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

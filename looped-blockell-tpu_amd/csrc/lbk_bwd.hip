@@ -282,6 +282,15 @@ __device__ __forceinline__ int kdiv(const TProdSrc& S, int e) {
 }
 
 // GELU: the epilogue is dg = dh gelu'(g), with no up stream
+// sum over the 16 lanes of a DPP row (every lane gets it): rotations by 8, 4, 2 and 1
+__device__ __forceinline__ float row_sum16(float v) {
+#define LBK_ROR(n) \
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + n, 0xf, 0xf, true));
+  LBK_ROR(8) LBK_ROR(4) LBK_ROR(2) LBK_ROR(1)
+#undef LBK_ROR
+  return v;
+}
+
 template <int B, int MT, int NW, bool GELU>
 __global__ __launch_bounds__(64 * NW, 1) void dh_panel_kernel(TProdArgs a) {
   constexpr int NT = 64 * NW;
@@ -463,6 +472,11 @@ __global__ __launch_bounds__(64 * NW, 1) void dh_panel_kernel(TProdArgs a) {
     }
     // epilogue: lane (i, g) of acc[q] holds dh of token t0 + 16q + i (columns as op_row
     // arranges them): dg = dh * u * silu'(g), du = dh * silu(g)
+    float sg_[NP][NV], su_[NP][NV];                  // the lane's column sums (the bias gradients)
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int j = 0; j < NV; ++j) sg_[p][j] = su_[p][j] = 0.f;
 #pragma unroll
     for (int q = 0; q < MT; ++q) {
       const int64_t tn = t0 + 16 * q + i;
@@ -486,9 +500,32 @@ __global__ __launch_bounds__(64 * NW, 1) void dh_panel_kernel(TProdArgs a) {
           dgv[j] = dh[j] * uv * (sg + gv * sg * (1.0f - sg));
           duv[j] = dh[j] * gv * sg;
         }
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+          sg_[p][j] += dgv[j];
+          if constexpr (!GELU) su_[p][j] += duv[j];
+        }
         store_bf16x<NV>(a.dg + tn * a.ldo + col_of(c, p), dgv);
         if constexpr (!GELU) store_bf16x<NV>(a.du + tn * a.ldo + col_of(c, p), duv);
       }
+    }
+    if (a.dgsum) {
+      const int64_t srow = t0 / TM * a.ldo;
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int j0 = 0; j0 < NV; j0 += 4) {
+          f32x4 vg, vu;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            vg[j] = row_sum16(sg_[p][j0 + j]);
+            vu[j] = GELU ? 0.f : row_sum16(su_[p][j0 + j]);
+          }
+          if (i == 0) {
+            *reinterpret_cast<f32x4*>(a.dgsum + srow + col_of(c, p) + j0) = vg;
+            if constexpr (!GELU) *reinterpret_cast<f32x4*>(a.dusum + srow + col_of(c, p) + j0) = vu;
+          }
+        }
     }
   }
 }
@@ -511,11 +548,20 @@ static int launch_dh_panel_t(const TProdArgs& a0, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+static int dh_mt(const TProdArgs& a) {
+  const int64_t d_model = a.nsrc == 1 ? a.src[0].lda : 0;
+  return d_model <= 0 || d_model % 8 ? 0 : d_model <= 1024 ? 4 : d_model <= 2048 ? 2 : 0;
+}
+
+int64_t dh_sum_blocks(int B, const TProdArgs& a) {
+  const int mt = B == 16 || B == 32 || B == 64 ? dh_mt(a) : 0;
+  return mt ? (a.N + 16 * mt - 1) / (16 * mt) : 0;
+}
+
 template <bool GELU>
 static int launch_dh_panel(int B, const TProdArgs& a, hipStream_t st) {
-  const int64_t d_model = a.src[0].lda;
-  const int mt = d_model <= 1024 ? 4 : (d_model <= 2048 ? 2 : 0);
-  if (mt == 0 || d_model % 8) return -2;
+  const int mt = dh_mt(a);
+  if (mt == 0) return -2;
   // 16 waves at B = 16 (their registers fit 128 VGPRs): B = 16 backward at d_model 1024, d_ff 4096
   // 1.93 -> 1.87 ms; at B = 32 16 waves spill (0.739 against 0.715 ms)
   if (B == 16 && mt == 4) return launch_dh_panel_t<16, 4, 16, GELU>(a, st);

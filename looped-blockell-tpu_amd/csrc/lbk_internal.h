@@ -183,14 +183,15 @@ int launch_rmsnorm_f32(const float* x, int64_t N, int d, const float* scale, flo
                        hipStream_t st);
 size_t rmsnorm_bwd_bytes(int64_t N, int d);   // fp32 dscale partials of the workgroups
 // fp32 column sums out[C] of up to three bf16 [N, C] matrices (C % 8 == 0, 16-byte aligned rows);
-// part: colsum_bytes(N, the sum of their C), 4-byte aligned
+// part: colsum_bytes(N, the sum of their C), 4-byte aligned.  A job without a matrix (a null) gives its
+// own nchunk rows of partial sums.
 struct ColsumJob {
   const uint16_t* a;
   int64_t lda;
   int C;
   float* out;
-  float* part;               // set by launch_colsum
-  int nchunk;
+  float* part;               // set by launch_colsum (given when a is null)
+  int nchunk;                // the same
   int acc;                   // add to out instead of writing it
 };
 struct ColsumJobs {
@@ -322,7 +323,12 @@ struct TProdArgs {
   const uint16_t* g; const uint16_t* u; uint16_t* dg; uint16_t* du;   // mode 0 (mode 2: g and dg)
   const uint16_t* resid; uint16_t* out;                               // mode 1 (resid optional)
   int nsl;                          // output column slices per token block (set by the launcher)
+  // modes 0, 2: optional fp32 column sums of dg and du over each token block, [dh_sum_blocks, C*B]
+  // (given only where that is not 0)
+  float* dgsum; float* dusum;
 };
+// rows of those sums: the token blocks of the kernel that forms them, 0 where the product takes another
+int64_t dh_sum_blocks(int B, const TProdArgs& a);
 // mode 0: dh -> dg, du (SiLU*mul backward); mode 1: out = product + resid; mode 2: dh -> dg = dh gelu'(g)
 int launch_tprod(int B, int mode, const TProdArgs& a, hipStream_t st);
 // tile gradients dW[e] = X[:, col(e)]^T G[:, row(e)] through fp32 per-chunk partials

@@ -563,6 +563,12 @@ __device__ __forceinline__ bool block_runs(const int32_t* tdepth, int it, int64_
 // to the 8 XCDs round robin), so each XCD's L2 holds the weights of its slices only
 __device__ __forceinline__ void gu_slice(const GUArgs& a, int64_t& tb, int& r_lo, int& nrs) {
   const int64_t b = blockIdx.x;
+  if (a.H == 1) {
+    tb = b;
+    r_lo = 0;
+    nrs = a.R_ff;
+    return;
+  }
   const int H = a.H, hs = (int)(b % H);
   tb = b / H;
   r_lo = (int)((int64_t)hs * a.R_ff / H);

@@ -52,10 +52,11 @@ class LoopedSwiGLU(nn.Module):
             for _ in range(self.L):
                 hf = hf + self.mlp(self.norm(hf.to(torch.bfloat16))).float()
             return hf.to(torch.bfloat16).reshape(*lead, d)
-        vg, cg, vu, cu, vd, cd = self.mlp.swiglu_weights()
+        # the weights as MLPBlock keeps them for gradient-free forwards (rounded and packed once a version)
+        (vg, cg, vu, cu, vd, cd), packed = self.mlp._frozen_swiglu()
         bg, bu, bd = self.mlp.swiglu_biases()
-        out = kernels.looped_swiglu_bias(h2, self.norm.scale, vg, cg, bg, vu, cu, bu, vd, cd, bd, L=self.L,
-                                         eps=self.norm.eps)
+        out = kernels.looped_swiglu_prepacked(h2, self.norm.scale, packed, vg, cg, bg, vu, cu, bu, vd, cd, bd, L=self.L,
+                                              eps=self.norm.eps)
         return out.reshape(*lead, d)
 
 
