@@ -280,3 +280,29 @@ def test_looped_training_groups_of_applications(gpu):
         tot = parts if tot is None else [a + b for a, b in zip(tot, parts)]
     for a, b in zip(got, [g.to(torch.bfloat16), *tot]):
         assert (a.double() - b.double()).norm() <= 4e-3 * b.double().norm()
+
+
+@pytest.mark.parametrize("kind", ["tile64", "gelu16", "gelu64", "loop16", "down16"])
+def test_gradient_free_forwards_replay_from_a_graph(gpu, kind):
+    """The forwards captured once replay on new inputs, with eager work between the replays."""
+    from looped_blockell.layers import LoopedSwiGLU, MLPBlock
+    torch.manual_seed(8)
+    kw = dict(device="cuda")
+    m = {"tile64": lambda: MLPBlock(256, 512, use_swiglu=True, tile_size=64, density=0.5, **kw),
+         "gelu16": lambda: MLPBlock(256, 512, tile_size=16, density=0.5, **kw),
+         "gelu64": lambda: MLPBlock(256, 512, tile_size=64, density=0.5, **kw),
+         "loop16": lambda: LoopedSwiGLU(256, 512, 3, tile_size=16, density=0.5, **kw),
+         "down16": lambda: MLPBlock(256, 2048, use_swiglu=True, tile_size=16, density=1.0, **kw)}[kind]()
+    x = torch.randn(130, 256, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        m(x)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            y = m(x)
+        for k in range(3):
+            x.copy_(torch.randn(130, 256, device="cuda"))
+            g.replay()
+            torch.cuda.synchronize()
+            got = y.clone()
+            assert torch.equal(got, m(x)), k
