@@ -1174,6 +1174,10 @@ int launch_tprod(int B, int mode, const TProdArgs& a, hipStream_t st) {
     if (rc != -2) return rc;
   }
   if (mode == 1) {
+    if (B == 64) {
+      const int rc = launch_t64_dx(a, st);
+      if (rc != -2) return rc;
+    }
     const int rc = launch_dx_stage(B, a, st);
     if (rc != -2) return rc;
   }

@@ -331,6 +331,8 @@ struct TProdArgs {
 int64_t dh_sum_blocks(int B, const TProdArgs& a);
 // mode 0: dh -> dg, du (SiLU*mul backward); mode 1: out = product + resid; mode 2: dh -> dg = dh gelu'(g)
 int launch_tprod(int B, int mode, const TProdArgs& a, hipStream_t st);
+// mode 1 at B = 64 (lbk_tile64.hip); -2: an operand's alignment or stride does not fit
+int launch_t64_dx(const TProdArgs& a, hipStream_t st);
 // tile gradients dW[e] = X[:, col(e)]^T G[:, row(e)] through fp32 per-chunk partials
 struct DWJob {
   const uint16_t* x; int64_t ldx;    // [N, C*B]

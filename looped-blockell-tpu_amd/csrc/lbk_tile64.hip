@@ -1,4 +1,4 @@
-// lbk_tile64.hip — Block-ELL products at B = 64 for more tokens than the decode kernels take
+// lbk_tile64.hip — Block-ELL products at B = 64 (forward: more tokens than the decode kernels take)
 // (gfx950, bf16 MFMA): y = x W (+ bias), h = silu(x Wg) * (x Wu), out = h Wd (+ residual).
 //
 // t64_kernel<MODE, MT, ST>: a workgroup of four waves owns 64 MT tokens and one block row, wave w
@@ -290,6 +290,170 @@ int launch_t64(int mode, const RowblockLaunch& a, hipStream_t st) {
   LBK_T64(0) LBK_T64(1) LBK_T64(2)
 #undef LBK_T64
   return -2;
+}
+
+// ---------------------------------------------------------------------------
+// the transposed product: dx[:, c] = sum over the list entries of column block c of A[:, r] W[e]^T
+// ---------------------------------------------------------------------------
+// t64_dx_kernel<MT, ST>: the kernel above for the backward's dx at B = 64.  The steps are the entries
+// of the transposed topology of an output column block, dg's and then du's, into one accumulator; the
+// tile's rows are the output columns, so it is read as it lies (rows of 16-byte chunks, chunk c at
+// c ^ (row & 7), as the tokens' pieces).  3000 x 1024, d_ff 4096 at 0.5: 232 us with the activations
+// staged 256 columns at a time by 94 workgroups, 51 us so.
+template <int MT, int ST>
+__global__ __launch_bounds__(256, 2) void t64_dx_kernel(TProdArgs a, int tg) {
+  constexpr int TM = 64 * MT;
+  constexpr int STEP = TM * 128 + T64_TILE;
+  constexpr int NLD = 2 * MT + 2;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = uniform(tid >> 6);
+  const int i = lane & 15, g = lane >> 4;
+  // workgroup -> (token block, output column block), as in t64_kernel
+  const int xcd = (int)(blockIdx.x & 7), rgs = 8 / tg;
+  const int64_t j8 = blockIdx.x >> 3;
+  const int rl = (a.C + rgs - 1) / rgs;
+  const int64_t tl = j8 / rl;
+  const int c = (int)(j8 - tl * rl) * rgs + xcd / tg;
+  const int64_t tb = tl * tg + xcd % tg;
+  if (c >= a.C || tb * TM >= a.N) return;            // the whole workgroup, before any barrier
+  const int64_t t0 = tb * TM;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_byte*)smem;
+  const TProdSrc& S0 = a.src[0];
+  const TProdSrc& S1 = a.src[a.nsrc > 1 ? 1 : 0];
+  const int64_t lda = S0.lda;                        // both sources' (the launcher checks it)
+
+  uint32_t xoff[2 * MT], woff[2];
+#pragma unroll
+  for (int j = 0; j < 2 * MT; ++j) {
+    const int row = 16 * MT * w + 8 * j + (lane >> 3);
+    const int64_t left = a.N - 1 - t0;
+    const int rc = row < left ? row : (int)left;
+    xoff[j] = (uint32_t)rc * (uint32_t)(lda * 2) + (uint32_t)(((lane & 7) ^ (row & 7)) << 4);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int row = 16 * w + 8 * j + (lane >> 3);
+    woff[j] = (uint32_t)(row * 128 + (((lane & 7) ^ (row & 7)) << 4));
+  }
+
+  // the list, 64 entries at a time: lane l holds entry base + l and its source block
+  const int n0 = S0.cnt[c], T = n0 + (a.nsrc > 1 ? S1.cnt[c] : 0);
+  int base = 0, ev = 0, rv = 0, pos = 0;
+  auto window = [&]() {
+    const int j = base + lane;
+    const bool s1 = j >= n0;
+    const int32_t* p = s1 ? S1.list + (int64_t)c * S1.cap + (j - n0) : S0.list + (int64_t)c * S0.cap + j;
+    ev = j < T ? *p : 0;
+    rv = ev / (s1 ? S1.K : S0.K);
+    pos = 0;
+  };
+  if (T > 0) window();
+  int issued = 0;
+  auto issue = [&](int slot) {
+    if (base + pos >= T) return false;
+    if (pos == 64) {
+      base += 64;
+      window();
+    }
+    const int e = __builtin_amdgcn_readlane(ev, pos), r = __builtin_amdgcn_readlane(rv, pos);
+    const bool s1 = base + pos >= n0;
+    ++pos;
+    const char* wp = reinterpret_cast<const char*>(s1 ? S1.w : S0.w) + (int64_t)e * T64_TILE;
+    const char* xp = reinterpret_cast<const char*>((s1 ? S1.a : S0.a) + t0 * lda) + (int64_t)r * 128;
+    const uint32_t l0 = lds0 + (uint32_t)(slot * STEP);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) t64_load(wp, woff[j], l0 + (uint32_t)(TM * 128 + (2 * w + j) * 1024));
+#pragma unroll
+    for (int j = 0; j < 2 * MT; ++j) t64_load(xp, xoff[j], l0 + (uint32_t)((2 * MT * w + j) * 1024));
+    ++issued;
+    return true;
+  };
+
+  f32x4 acc[MT][4];
+#pragma unroll
+  for (int q = 0; q < MT; ++q)
+#pragma unroll
+    for (int m = 0; m < 4; ++m) acc[q][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t xl = (uint32_t)((16 * MT * w + i) * 128), wl = (uint32_t)(TM * 128 + i * 128);
+  const uint32_t ch0 = (uint32_t)((g ^ (i & 7)) << 4), ch1 = (uint32_t)(((4 + g) ^ (i & 7)) << 4);
+#pragma unroll
+  for (int s = 0; s < ST - 1; ++s)
+    if (!issue(s)) break;
+  int slot = 0, islot = ST - 1;
+  for (int s = 0; s < issued; ++s) {
+    // this wave's loads of step s have landed once only the later steps' are in flight
+    const int later = issued - s - 1;
+    if (ST > 3 && later >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NLD) : "memory");
+    else if (ST > 2 && later >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NLD) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    t64_barrier();           // every wave's have, and step s - 1 is read: its ring slot is free
+    if (issue(islot)) islot = islot + 1 == ST ? 0 : islot + 1;
+    const uint32_t s0 = (uint32_t)(slot * STEP);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const uint32_t ch = ks ? ch1 : ch0;
+      u32x4 wf[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) wf[m] = *reinterpret_cast<const u32x4*>(smem + s0 + wl + (uint32_t)(m * 2048) + ch);
+#pragma unroll
+      for (int q = 0; q < MT; ++q) {
+        const u32x4 xf = *reinterpret_cast<const u32x4*>(smem + s0 + xl + (uint32_t)(q * 2048) + ch);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) acc[q][m] = mfma_bf16(wf[m], xf, acc[q][m]);
+      }
+    }
+    slot = slot + 1 == ST ? 0 : slot + 1;
+  }
+
+  // lane (i, g) of acc[q][m]: token 16 q + i of the wave, columns 16 m + 4 g .. + 3
+#pragma unroll
+  for (int q = 0; q < MT; ++q) {
+    const int64_t t = t0 + 16 * MT * w + 16 * q + i;
+    if (t >= a.N) continue;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int64_t off = t * a.ldo + (int64_t)c * 64 + 16 * m + 4 * g;
+      float o[4], rr[4] = {0.f, 0.f, 0.f, 0.f};
+      if (a.resid) load_bf16x<4>(a.resid + off, rr);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) o[v] = acc[q][m][v] + rr[v];
+      store_bf16x<4>(a.out + off, o);
+    }
+  }
+}
+
+template <int MT, int ST>
+static int launch_t64_dx_t(const TProdArgs& a, hipStream_t st) {
+  constexpr int lds = ST * (64 * MT * 128 + T64_TILE);
+  auto kern = t64_dx_kernel<MT, ST>;
+  static std::atomic<uint64_t> done{0};
+  if (lds > 65536 && set_lds_limit_once(reinterpret_cast<const void*>(kern), lds, done)) return -1;
+  const int64_t ntb = (a.N + 64 * MT - 1) / (64 * MT);
+  RowblockLaunch b{};                                // the traffic that decides the token groups
+  b.N = a.N;
+  b.C = (int)(a.src[0].lda / 64);
+  b.R = a.C;
+  b.K0 = (int)(a.src[0].cap / a.C);
+  b.K1 = a.nsrc > 1 ? (int)(a.src[1].cap / a.C) : 0;
+  const int tg = t64_groups(b, ntb), rgs = 8 / tg;
+  const int64_t grid = 8 * ((a.C + rgs - 1) / rgs) * ((ntb + tg - 1) / tg);
+  if (grid > 0x7fffffff) return -2;
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, st, a, tg);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int launch_t64_dx(const TProdArgs& a, hipStream_t st) {
+  auto bad = [](const void* p, uintptr_t m) { return (reinterpret_cast<uintptr_t>(p) & m) != 0; };
+  if (a.nsrc < 1 || a.nsrc > 2 || a.C < 1 || bad(a.out, 7) || (a.resid && bad(a.resid, 7)) || a.ldo % 4) return -2;
+  for (int s = 0; s < a.nsrc; ++s)
+    if (bad(a.src[s].a, 15) || bad(a.src[s].w, 15) || a.src[s].lda != a.src[0].lda || a.src[s].lda % 64 ||
+        a.src[s].lda > (1 << 22) || a.src[s].K < 1)
+      return -2;
+  auto wgs = [&](int tm) { return (int64_t)a.C * ((a.N + tm - 1) / tm); };
+  if (wgs(256) >= 256) return launch_t64_dx_t<4, 2>(a, st);
+  if (wgs(128) >= 256) return launch_t64_dx_t<2, 3>(a, st);
+  return launch_t64_dx_t<1, 4>(a, st);
 }
 
 }  // namespace lbk

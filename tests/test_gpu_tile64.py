@@ -87,3 +87,40 @@ def test_unaligned_tiles_take_the_rowblock_kernel(gpu):
     off.copy_(v)
     x = T.to_gpu_bf16(T.act(rng, 200, 6 * 64))
     assert _close(kernels.block_ell_matmul(x, off, c), x.double() @ _dense(v, c, 6).T)
+
+
+# the transposed product of the backward: token blocks of 64, 128 and 256, one and two sources, lists past
+# one 64-entry window, an input block that no slot reads, output blocks that are no multiple of 8
+@pytest.mark.parametrize("case", [(1, 3, 2, 1), (65, 8, 5, 3), (700, 80, 16, 16), (3000, 40, 17, 9), (8200, 20, 12, 5),
+                                  (127, 130, 3, 3)])
+def test_product_backward(gpu, case):
+    from looped_blockell import kernels
+    N, R, C, K = case
+    rng = np.random.default_rng(N)
+    vals, col = T.bell_weight(rng, R, C, K, 64)
+    col[rng.random(col.shape) < 0.15] = -1
+    if C > 2 * K:
+        col[col == 1] = -1
+    v, c = T.gpu_weight((vals, col))
+    x, dy = T.to_gpu_bf16(T.act(rng, N, C * 64)), T.to_gpu_bf16(T.act(rng, N, R * 64))
+    dx, _ = kernels.ops().block_ell_matmul_bwd(dy, x, v, c)
+    ref = dy.double() @ _dense(v, c, C)
+    assert ((dx.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4 * ref.abs().amax()).all()
+
+
+@pytest.mark.parametrize("N", [130, 2100])
+def test_swiglu_backward_two_sources(gpu, N):
+    from looped_blockell import kernels
+    d, ff = 512, 1024
+    rng = np.random.default_rng(N)
+    g, u, dn = (_weight(rng, *s, dead=0.1) for s in ((ff // 64, d // 64, 5), (ff // 64, d // 64, 5), (d // 64, ff // 64, 7)))
+    x, dy = T.to_gpu_bf16(T.act(rng, N, d)), T.to_gpu_bf16(T.act(rng, N, d))
+    ops = kernels.ops()
+    _, h, gp, uo = ops.block_ell_swiglu_fwd_with_intermediate(x, *g, *u, *dn, True)
+    wg, wu, wd = (_dense(*w, C) for w, C in ((g, d // 64), (u, d // 64), (dn, ff // 64)))
+    G, U, dh = gp.double(), uo.double(), dy.double() @ wd
+    s = torch.sigmoid(G)
+    ref = (dh * U * (s + G * s * (1 - s))) @ wg + (dh * G * s) @ wu
+    for res in (False, True):
+        dx = ops.block_ell_swiglu_bwd_ex(dy, x, gp, uo, h, *g, *u, *dn, res)[0]
+        assert _close(dx, ref + (dy.double() if res else 0))
