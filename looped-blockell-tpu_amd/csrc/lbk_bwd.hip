@@ -26,12 +26,9 @@
 //                  of NW waves (8; 16 at B = 16) streams the list entries of its
 //                  column blocks (c = w, w + NW, ...): tile rows from global memory,
 //                  dy fragments from the panel.
-//   dx_stage_kernel  dx at B = 64 when the output blocks fit the waves' accumulators:
-//                  the dg and du columns of 64 tokens pass through LDS 256 at a
-//                  time, and a cursor per output block walks its sorted list, whose
-//                  first 64 entries stay in a register.
-//   dx16_kernel    dx at B = 16: the same walk with wider stages, list entries in
-//                  pairs through a ring.
+//   dx16_kernel    dx at B = 16: the dg and du columns of 32 or 64 tokens pass through
+//                  LDS, and a cursor per output block walks its sorted list, whose first
+//                  64 entries stay in a register, in pairs through a ring.
 //   dxf_kernel     dx at B = 32: the same stages, one output block per wave and a
 //                  4-slot ring of tiles over the wave's whole list (both sources,
 //                  all stages), the list entries read one pass ahead.
@@ -574,181 +571,11 @@ static int launch_dh_panel(int B, const TProdArgs& a, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // dx = dg W_gate + du W_up (+ dy) with the activations staged through LDS
 // ---------------------------------------------------------------------------
-// A workgroup owns 64 tokens and every output column block: wave w owns blocks c = w + 8 o
-// (o < OPW).  The columns of dg, then du, pass through LDS 512 at a time (double buffered, the
-// next stage's loads in flight during the current one, as in the forward's down kernel).  A
-// block's list is sorted by slot, hence by the source column block r = e / K, so the entries of
-// a stage are the next run of the list: a cursor per block walks it, 64 entries at a time held
-// one per lane.
-// activation columns per stage: 512 (longer runs of a block's list per stage), 256 for B = 64
-// (its larger accumulators leave no registers for the bigger stage)
-template <int B>
-struct DxStage { static constexpr int COLS = B == 64 ? 256 : 512; };
-
-template <int B, int OPW, int NW>
-__global__ __launch_bounds__(64 * NW, 1) void dx_stage_kernel(TProdArgs a) {
-  constexpr int NT = 64 * NW;
-  constexpr int CW = B / 16;
-  constexpr int NKS = B >= 32 ? B / 32 : 1;
-  constexpr int MT = 4;
-  constexpr int COLS = DxStage<B>::COLS;
-  constexpr int G = COLS / B;                        // source column blocks per stage
-  constexpr int SROWB = COLS * 2;                    // bytes per token row of a stage
-  constexpr int SBYTES = 64 * SROWB;                 // 64 KB (32 KB for B = 64)
-  constexpr int PER_T = SBYTES / 16 / NT;            // 16-byte chunks per thread per stage
-  extern __shared__ __attribute__((aligned(16))) unsigned char stg[];   // two stages
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = uniform(tid >> 6);
-  const int i = lane & 15, g = lane >> 4;
-  // workgroup -> (64-token block, slice sl of nsl: output blocks sl + nsl (w + NW o))
-  const int sl = (int)(blockIdx.x % (unsigned)a.nsl);
-  const int64_t t0 = (int64_t)(blockIdx.x / (unsigned)a.nsl) * 64;
-
-  // stages: source s covers ceil(R_s / G) stages; global stage -> (source, first block)
-  const int R0 = (int)(a.src[0].lda / B);
-  const int ns0 = (R0 + G - 1) / G;
-  const int ns1 = a.nsrc > 1 ? ((int)(a.src[1].lda / B) + G - 1) / G : 0;
-  const int nstages = ns0 + ns1;
-
-  u32x4 sreg[PER_T];
-  auto stage_fetch = [&](int s) {
-    const TProdSrc& S = a.src[s < ns0 ? 0 : 1];
-    const int64_t col0 = (int64_t)(s < ns0 ? s : s - ns0) * COLS;
-#pragma unroll
-    for (int u = 0; u < PER_T; ++u) {
-      const int e = tid + NT * u;
-      const int row = e / (SROWB / 16), cc = e - row * (SROWB / 16);
-      const int64_t t = t0 + row, col = col0 + 8 * cc;
-      const bool ok = t < a.N && col < S.lda;
-      const u32x4 v = ld16(S.a + (ok ? t : t0) * S.lda + (ok ? col : 0));
-      sreg[u] = ok ? v : u32x4{0, 0, 0, 0};
-    }
-  };
-  auto stage_store = [&](int buf) {
-#pragma unroll
-    for (int u = 0; u < PER_T; ++u) {
-      const int e = tid + NT * u;
-      const int row = e / (SROWB / 16), cc = e - row * (SROWB / 16);
-      *reinterpret_cast<u32x4*>(stg + buf * SBYTES + bpanel_addr<MT>(row, cc, SROWB)) = sreg[u];
-    }
-  };
-
-  f32x4 acc[OPW][MT][CW];
-#pragma unroll
-  for (int o = 0; o < OPW; ++o)
-#pragma unroll
-    for (int q = 0; q < MT; ++q)
-#pragma unroll
-      for (int m = 0; m < CW; ++m) acc[o][q][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  struct Ent {
-    u32x4 av[NKS][CW];
-    int r;                                           // source column block
-  };
-  const uint32_t lbase = (uint32_t)(i * MT * SROWB);
-  int cur[OPW];                                      // list cursors of the current source
-  int lvr[OPW];                                      // first 64 list entries of each output block
-
-  stage_fetch(0);
-  stage_store(0);
-  __syncthreads();
-  for (int s = 0; s < nstages; ++s) {
-    const int src = s < ns0 ? 0 : 1;
-    const int st = s < ns0 ? s : s - ns0;
-    const TProdSrc& S = a.src[src];
-    if (st == 0) {
-      // a new source: each output block's first 64 list entries into a register (lane j holds
-      // entry j), so that a stage finds its run with a ballot instead of a global load
-#pragma unroll
-      for (int o = 0; o < OPW; ++o) {
-        cur[o] = 0;
-        const int c = sl + a.nsl * (w + NW * o);
-        const int cnt = c < a.C ? S.cnt[c] : 0;
-        lvr[o] = lane < cnt ? S.list[(int64_t)c * S.cap + lane] : 0x7fffffff;
-      }
-    }
-    if (s + 1 < nstages) stage_fetch(s + 1);
-    const unsigned char* sb = stg + (s & 1) * SBYTES;
-    const int rlo = st * G, rhi = rlo + G;           // source column blocks of this stage
-    auto load = [&](int e, Ent& E) {
-      const uint16_t* tile = S.w + (int64_t)e * B * B + 8 * g;
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks)
-#pragma unroll
-        for (int m = 0; m < CW; ++m) E.av[ks][m] = ld16(tile + op_row<CW>(i, m) * B + 32 * ks);
-      E.r = e / S.K;
-    };
-#pragma unroll
-    for (int o = 0; o < OPW; ++o) {
-      const int c = sl + a.nsl * (w + NW * o);
-      if (c >= a.C) continue;
-      auto compute = [&](const Ent& E) {
-        const int rb = uniform(E.r) - rlo;           // column block within the stage
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-          const uint32_t pa = lbase + (((rb * (B / 8) + 4 * ks + g) ^ i) << 4);
-#pragma unroll
-          for (int q = 0; q < MT; ++q) {
-            const u32x4 bv = *reinterpret_cast<const u32x4*>(sb + pa + q * SROWB);
-#pragma unroll
-            for (int m = 0; m < CW; ++m) acc[o][q][m] = mfma_bf16(E.av[ks][m], bv, acc[o][q][m]);
-          }
-        }
-      };
-      const int cnt = S.cnt[c];
-      const int32_t* L = S.list + (int64_t)c * S.cap;
-      int jc = cur[o];
-      while (jc < cnt) {
-        // entries of this stage: the run from jc whose source block is below rhi.  Within the
-        // first 64 entries they come from the register (lanes jc .. jc + n - 1), beyond them
-        // from the next 64 entries loaded here (lanes 0 .. n - 1)
-        const bool inreg = jc < 64;
-        const int lv = inreg ? lvr[o] : ((jc + lane < cnt) ? L[jc + lane] : 0x7fffffff);
-        const int base = inreg ? jc : 0;
-        const int lim = inreg ? (cnt < 64 ? cnt : 64) : cnt - jc;
-        const uint64_t m = __ballot(lane >= base && lane < lim && lv / S.K < rhi);
-        const int n = __builtin_popcountll(m);       // a contiguous run of lanes (sorted list)
-        if (n == 0) break;
-        auto ent = [&](int jj) { return __builtin_amdgcn_readlane(lv, base + (jj < n ? jj : n - 1)); };
-        Ent E0, E1;
-        load(ent(0), E0);
-        for (int jj = 0; jj < n; jj += 2) {
-          load(ent(jj + 1), E1);
-          compute(E0);
-          load(ent(jj + 2), E0);
-          if (jj + 1 < n) compute(E1);
-        }
-        jc += n;
-        if (base + n < 64) break;                    // the run ended inside this chunk
-      }
-      cur[o] = jc;
-    }
-    if (s + 1 < nstages) stage_store((s + 1) & 1);
-    __syncthreads();
-  }
-
-  // epilogue: dx = acc (+ dy)
-#pragma unroll
-  for (int o = 0; o < OPW; ++o) {
-    const int c = sl + a.nsl * (w + NW * o);
-    if (c >= a.C) continue;
-#pragma unroll
-    for (int q = 0; q < MT; ++q) {
-      const int64_t tn = t0 + 16 * q + i;
-      if (tn < a.N) tprod_store<1, CW>(a, tn, c, g, acc[o][q]);
-    }
-  }
-}
-
-template <int B, int OPW, int NW>
-static int launch_dx_stage_t(const TProdArgs& a, hipStream_t st) {
-  constexpr size_t lds = 2 * (size_t)64 * DxStage<B>::COLS * 2;
-  auto kern = dx_stage_kernel<B, OPW, NW>;
-  static std::atomic<uint64_t> done{0};
-  if (lds > 65536 && set_lds_limit_once(reinterpret_cast<const void*>(kern), (int)lds, done)) return -1;
-  hipLaunchKernelGGL(kern, dim3((unsigned)((a.N + 63) / 64 * a.nsl)), dim3(64 * NW), lds, st, a);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
+// The columns of dg, then du, pass through LDS in stages, the next stage's loads in flight during the
+// current one, as in the forward's down kernels.  A block's list is sorted by slot, hence by the
+// source column block r = e / K, so the entries of a stage are the next run of the list.  (B = 64:
+// t64_dx_kernel of lbk_tile64.hip.)
+constexpr int DX_COLS = 512;                         // activation columns per stage (dxf_kernel)
 
 // dx16_kernel<OPW, MT, NW>: dx at B = 16 (wave w of NW owns output blocks sl + nsl (w + NW o) of
 // 16 MT tokens).  A step of a wave is one list entry and little work, so the kernel is bound by the latency of its tile
@@ -925,8 +752,7 @@ static int launch_dx16_t(const TProdArgs& a0, hipStream_t st) {
 // block per wave (16 waves; the output blocks are dealt to nsl workgroups per 64-token block,
 // which share an XCD) and a D-slot ring of tiles that
 // runs over the wave's whole list -- the sorted entries of source 0, then of source 1 -- across
-// the 512-column stages of both sources, so D tile loads stay in flight where dx_stage_kernel
-// had one.  A stage change is a workgroup barrier taken inline when the next entry lies in a
+// the 512-column stages of both sources, so D tile loads stay in flight.  A stage change is a workgroup barrier taken inline when the next entry lies in a
 // later stage; every wave passes all of them.  The list entries a pass fetches are read one pass
 // ahead (lane j of a window holds entry j of the pass), so no load waits on a list read.
 constexpr int DXF_WAVES = 16;
@@ -935,7 +761,7 @@ template <int B, int D>
 __global__ __launch_bounds__(64 * DXF_WAVES, 1) void dxf_kernel(TProdArgs a) {
   constexpr int NW = DXF_WAVES, NT = 64 * NW;
   constexpr int CW = B / 16, MT = 4;
-  constexpr int COLS = DxStage<B>::COLS;
+  constexpr int COLS = DX_COLS;
   constexpr int G = COLS / B;                        // source column blocks per stage
   constexpr int SROWB = COLS * 2;
   constexpr int SBYTES = 64 * SROWB;
@@ -1107,7 +933,7 @@ __global__ __launch_bounds__(64 * DXF_WAVES, 1) void dxf_kernel(TProdArgs a) {
 
 template <int B>
 static int launch_dxf(const TProdArgs& a0, hipStream_t st) {
-  constexpr size_t lds = 2 * (size_t)64 * DxStage<B>::COLS * 2;
+  constexpr size_t lds = 2 * (size_t)64 * DX_COLS * 2;
   TProdArgs a = a0;
   set_kdiv(a);
   const int64_t ntb = (a.N + 63) / 64;
@@ -1122,7 +948,7 @@ static int launch_dxf(const TProdArgs& a0, hipStream_t st) {
 
 // staged dx when every output block fits the waves' accumulators (OPW * B / 16 <= 8) and the
 // sources' widths are whole stages of 16-byte chunks
-static int launch_dx_stage(int B, const TProdArgs& a0, hipStream_t st) {
+static int launch_dx(int B, const TProdArgs& a0, hipStream_t st) {
   if (a0.nsrc < 1 || a0.nsrc > 2) return -2;
   for (int s = 0; s < a0.nsrc; ++s)
     if (a0.src[s].lda % B) return -2;
@@ -1130,8 +956,7 @@ static int launch_dx_stage(int B, const TProdArgs& a0, hipStream_t st) {
   // token block so that each wave owns one (each workgroup stages all the activation columns).
   TProdArgs a = a0;
   const int64_t ntb = (a.N + 63) / 64;
-  const int per_wg = B == 64 ? 8 : 16;
-  a.nsl = ntb >= 256 ? 1 : (a.C + per_wg - 1) / per_wg;
+  a.nsl = ntb >= 256 ? 1 : (a.C + 15) / 16;
   const int cs = (a.C + a.nsl - 1) / a.nsl;        // output blocks per slice
   // B = 32: the deep-ring kernel (headline backward 0.710 -> 0.688 ms; 64 / 1024 / 4096 tokens
   // 0.109 / 0.131 / 0.213 -> 0.105 / 0.127 / 0.199 ms)
@@ -1151,9 +976,6 @@ static int launch_dx_stage(int B, const TProdArgs& a0, hipStream_t st) {
     if (opw <= 2) return launch_dx16_t<2, 4, 16>(a, st);
     if (opw <= 4) return launch_dx16_t<4, 4, 16>(a, st);
   }
-  const int opw = (cs + 7) / 8;
-  if (B == 64 && opw <= 1) return launch_dx_stage_t<64, 1, 8>(a, st);
-  if (B == 64 && opw <= 2) return launch_dx_stage_t<64, 2, 8>(a, st);
   // B = 16 with more output blocks than the staged kernel's accumulators hold (N >= 16321 tokens
   // and more than 64 output blocks): the deep-ring kernel, one output block per wave, in place of
   // the per-entry kernel (1024 x 8192 product backward at 16384 tokens 1.275 -> 0.658 ms).  Where
@@ -1178,7 +1000,7 @@ int launch_tprod(int B, int mode, const TProdArgs& a, hipStream_t st) {
       const int rc = launch_t64_dx(a, st);
       if (rc != -2) return rc;
     }
-    const int rc = launch_dx_stage(B, a, st);
+    const int rc = launch_dx(B, a, st);
     if (rc != -2) return rc;
   }
   const dim3 grid((unsigned)((a.N + 63) / 64), (unsigned)((a.C + 3) / 4));
