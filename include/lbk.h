@@ -374,14 +374,6 @@ int lbk_looped_swiglu_bias_bf16(const uint16_t* h_in, int64_t N, int32_t d_model
                                 const float* b_gate, const float* b_up, const float* b_down,
                                 uint16_t* h_out, void* workspace, size_t workspace_bytes,
                                 void* stream);
-/* The same from weights packed once (lbk_swiglu_prepack_bf16; packed may be NULL where the geometry has
- * no packed form).  The workspace is lbk_looped_workspace_bytes. */
-int lbk_looped_swiglu_prepacked_bf16(const uint16_t* h_in, int64_t N, int32_t d_model,
-                                     const float* norm_scale, float eps, int32_t L, const lbk_bell* gate,
-                                     const lbk_bell* up, const lbk_bell* down, const void* packed,
-                                     size_t packed_bytes, const float* b_gate, const float* b_up,
-                                     const float* b_down, uint16_t* h_out, void* workspace,
-                                     size_t workspace_bytes, void* stream);
 
 /*
  * lbk_looped_swiglu_bf16 as separate launches per iteration: the weight packing and an fp32

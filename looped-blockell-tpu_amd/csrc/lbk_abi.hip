@@ -574,8 +574,7 @@ static int looped_persistent(const uint16_t* h_in, int64_t N, int32_t d_model, c
                              uint16_t* h_out, void* workspace, size_t workspace_bytes, void* stream, Biases bs);
 static int looped_launches(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale, float eps,
                            int32_t L, const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down,
-                           uint16_t* h_out, void* workspace, size_t workspace_bytes, void* stream, Biases bs,
-                           const char* prepacked = nullptr);
+                           uint16_t* h_out, void* workspace, size_t workspace_bytes, void* stream, Biases bs);
 
 int lbk_looped_swiglu_bf16(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale, float eps,
                            int32_t L, const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down,
@@ -596,22 +595,6 @@ int lbk_looped_swiglu_bias_bf16(const uint16_t* h_in, int64_t N, int32_t d_model
                          stream, bs);
 }
 
-int lbk_looped_swiglu_prepacked_bf16(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale,
-                                     float eps, int32_t L, const lbk_bell* gate, const lbk_bell* up,
-                                     const lbk_bell* down, const void* packed, size_t packed_bytes,
-                                     const float* b_gate, const float* b_up, const float* b_down, uint16_t* h_out,
-                                     void* workspace, size_t workspace_bytes, void* stream) {
-  if (!gate || !up || !down) return LBK_ERR_NULL;
-  const size_t need = lbk_swiglu_prepacked_bytes(d_model, gate, up, down);
-  if (need && N > 0) {
-    if (!packed) return LBK_ERR_NULL;
-    if (packed_bytes < need) return LBK_ERR_WORKSPACE;
-    if (!a16(packed)) return LBK_ERR_ALIGN;
-  }
-  return looped_launches(h_in, N, d_model, norm_scale, eps, L, gate, up, down, h_out, workspace, workspace_bytes,
-                         stream, Biases{b_gate, b_up, b_down}, need ? static_cast<const char*>(packed) : nullptr);
-}
-
 int lbk_looped_swiglu_launches_bf16(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale,
                                     float eps, int32_t L, const lbk_bell* gate, const lbk_bell* up,
                                     const lbk_bell* down, uint16_t* h_out, void* workspace, size_t workspace_bytes,
@@ -622,8 +605,7 @@ int lbk_looped_swiglu_launches_bf16(const uint16_t* h_in, int64_t N, int32_t d_m
 
 static int looped_launches(const uint16_t* h_in, int64_t N, int32_t d_model, const float* norm_scale, float eps,
                            int32_t L, const lbk_bell* gate, const lbk_bell* up, const lbk_bell* down,
-                           uint16_t* h_out, void* workspace, size_t workspace_bytes, void* stream, Biases bs,
-                           const char* prepacked) {
+                           uint16_t* h_out, void* workspace, size_t workspace_bytes, void* stream, Biases bs) {
   int st;
   if ((st = check_bell(gate)) || (st = check_bell(up)) || (st = check_bell(down))) return st;
   int64_t d_ff = 0;
@@ -674,8 +656,7 @@ static int looped_launches(const uint16_t* h_in, int64_t N, int32_t d_model, con
     // fp32 state carried across the L applications; bf16 written once, after the last
     float* state = reinterpret_cast<float*>(ws);
     PackedFFN pk{};
-    if (prepacked) pk = packed_ffn_at(prepacked, gate, up);
-    else if ((st = pack_ffn(gate, up, down, ws + sbytes + hbytes, &pk, s))) return st;
+    if ((st = pack_ffn(gate, up, down, ws + sbytes + hbytes, &pk, s))) return st;
     if (launch_bf16_to_f32(h_in, N * d_model, state, s) != 0) return LBK_ERR_LAUNCH;
     for (int l = 0; l < L; ++l)
       if ((st = swiglu_split(nullptr, state, norm_scale, eps, N, d_model, gate, up, down, pk, nullptr, state,

@@ -391,11 +391,11 @@ at::Tensor looped_impl(const at::Tensor& h, const at::Tensor& scale_, at::Tensor
   return out;
 }
 
-at::Tensor looped_bias_impl(const at::Tensor& h_, const at::Tensor& scale_, const at::Tensor* packed,
-                            const at::Tensor& vg_, const at::Tensor& cg_, const c10::optional<at::Tensor>& bg_, const at::Tensor& vu_,
+at::Tensor looped_swiglu_bias(const at::Tensor& h_, const at::Tensor& scale_, const at::Tensor& vg_,
+                              const at::Tensor& cg_, const c10::optional<at::Tensor>& bg_, const at::Tensor& vu_,
                               const at::Tensor& cu_, const c10::optional<at::Tensor>& bu_, const at::Tensor& vd_,
-                              const at::Tensor& cd_, const c10::optional<at::Tensor>& bd_, int64_t L, double eps,
-                            const char* op) {
+                              const at::Tensor& cd_, const c10::optional<at::Tensor>& bd_, int64_t L, double eps) {
+  const char* op = "looped_swiglu_bias";
   at::Tensor x = check_x2d(h_, op);
   const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
   at::Tensor vg = vg_, cg = cg_, vu = vu_, cu = cu_, vd = vd_, cd = cd_;
@@ -409,40 +409,11 @@ at::Tensor looped_bias_impl(const at::Tensor& h_, const at::Tensor& scale_, cons
   at::Tensor out = at::empty_like(x);
   const size_t wsb = lbk_looped_workspace_bytes(x.size(0), (int32_t)x.size(1), &g, &u, &d);
   at::Tensor ws = wsb ? workspace(wsb, x) : at::Tensor();
-  if (packed) {
-    check_gpu(*packed, op, "packed");
-    TORCH_CHECK(packed->scalar_type() == at::kByte && packed->dim() == 1 && packed->is_contiguous(), "titan::", op,
-                ": packed must be the contiguous uint8 tensor of block_ell_swiglu_prepack");
-    const size_t need = lbk_swiglu_prepacked_bytes((int32_t)x.size(1), &g, &u, &d);
-    TORCH_CHECK((size_t)packed->numel() >= need, "titan::", op, ": packed holds ", packed->numel(),
-                " bytes, this geometry needs ", need);
-    LBK_CALL("looped_swiglu_prepacked",
-             lbk_looped_swiglu_prepacked_bf16(bf(x), x.size(0), (int32_t)x.size(1), s.data_ptr<float>(), (float)eps,
-                                              (int32_t)L, &g, &u, &d, need ? packed->data_ptr() : nullptr,
-                                              (size_t)packed->numel(), fptr(bg), fptr(bu), fptr(bd), bfm(out),
-                                              wsb ? ws.data_ptr() : nullptr, wsb, cur_stream(x)));
-    return out;
-  }
   LBK_CALL("looped_swiglu_bias",
            lbk_looped_swiglu_bias_bf16(bf(x), x.size(0), (int32_t)x.size(1), s.data_ptr<float>(), (float)eps,
                                        (int32_t)L, &g, &u, &d, fptr(bg), fptr(bu), fptr(bd), bfm(out),
                                        wsb ? ws.data_ptr() : nullptr, wsb, cur_stream(x)));
   return out;
-}
-
-at::Tensor looped_swiglu_bias(const at::Tensor& h, const at::Tensor& scale, const at::Tensor& vg, const at::Tensor& cg,
-                              const c10::optional<at::Tensor>& bg, const at::Tensor& vu, const at::Tensor& cu,
-                              const c10::optional<at::Tensor>& bu, const at::Tensor& vd, const at::Tensor& cd,
-                              const c10::optional<at::Tensor>& bd, int64_t L, double eps) {
-  return looped_bias_impl(h, scale, nullptr, vg, cg, bg, vu, cu, bu, vd, cd, bd, L, eps, "looped_swiglu_bias");
-}
-
-at::Tensor looped_swiglu_prepacked(const at::Tensor& h, const at::Tensor& scale, const at::Tensor& packed,
-                                   const at::Tensor& vg, const at::Tensor& cg, const c10::optional<at::Tensor>& bg,
-                                   const at::Tensor& vu, const at::Tensor& cu, const c10::optional<at::Tensor>& bu,
-                                   const at::Tensor& vd, const at::Tensor& cd, const c10::optional<at::Tensor>& bd,
-                                   int64_t L, double eps) {
-  return looped_bias_impl(h, scale, &packed, vg, cg, bg, vu, cu, bu, vd, cd, bd, L, eps, "looped_swiglu_prepacked");
 }
 
 at::Tensor looped_swiglu_persistent(const at::Tensor& h, const at::Tensor& scale, const at::Tensor& vg,
@@ -1355,9 +1326,6 @@ TORCH_LIBRARY(titan, m) {
   m.def("block_ell_swiglu_bwd_bias(Tensor grad_out, Tensor x, Tensor gate_pre_act, Tensor up_out, Tensor h, "
         "Tensor v_gate, Tensor ci_gate, Tensor v_up, Tensor ci_up, Tensor v_down, Tensor ci_down, "
         "bool add_residual) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
-  m.def("looped_swiglu_prepacked(Tensor h, Tensor norm_scale, Tensor packed, Tensor v_gate, Tensor ci_gate, "
-        "Tensor? b_gate, Tensor v_up, Tensor ci_up, Tensor? b_up, Tensor v_down, Tensor ci_down, Tensor? b_down, "
-        "int L, float eps=1e-05) -> Tensor");
   m.def("looped_swiglu_bias(Tensor h, Tensor norm_scale, Tensor v_gate, Tensor ci_gate, Tensor? b_gate, "
         "Tensor v_up, Tensor ci_up, Tensor? b_up, Tensor v_down, Tensor ci_down, Tensor? b_down, int L, "
         "float eps=1e-05) -> Tensor");
@@ -1439,7 +1407,6 @@ TORCH_LIBRARY_IMPL(titan, CUDA, m) {
   m.impl("block_ell_swiglu_prepack", &swiglu_prepack);
   m.impl("block_ell_swiglu_fwd_prepacked", &swiglu_fwd_prepacked);
   m.impl("looped_swiglu_bias", &looped_swiglu_bias);
-  m.impl("looped_swiglu_prepacked", &looped_swiglu_prepacked);
   m.impl("pin_weights_l2", &pin_weights_l2);
   m.impl("persistent_mlp_step", &persistent_mlp_step);
   m.impl("block_ell_matmul", &block_ell_matmul);
@@ -1492,7 +1459,7 @@ TORCH_LIBRARY_IMPL(titan, Autograd, m) {
         "persistent_mlp_step", "block_ell_matmul", "block_ell_matmul_bwd", "block_ell_matmul_bwd_bias",
         "block_ell_swiglu_fwd_train", "block_ell_swiglu_bwd_train",
         "block_ell_gelu_fwd_prepacked", "block_ell_gelu_fwd_train", "block_ell_gelu_bwd_train",
-        "looped_swiglu_fwd_train", "looped_swiglu_bwd_train", "looped_swiglu_prepacked",
+        "looped_swiglu_fwd_train", "looped_swiglu_bwd_train",
         "block_ell_swiglu_bwd_ex",
         "block_ell_matmul_prepack", "block_ell_matmul_prepacked",
         "looped_swiglu", "looped_swiglu_persistent", "looped_swiglu_launches", "looped_core", "rmsnorm",
@@ -1573,12 +1540,6 @@ TORCH_LIBRARY_IMPL(titan, Meta, m) {
   m.impl("block_ell_matmul_bwd", [](const at::Tensor&, const at::Tensor& x, const at::Tensor& v, const at::Tensor&) {
     return std::make_tuple(at::empty_like(x), at::empty_like(v));
   });
-  m.impl("looped_swiglu_prepacked",
-         [](const at::Tensor& h, const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&,
-            const c10::optional<at::Tensor>&, const at::Tensor&, const at::Tensor&, const c10::optional<at::Tensor>&,
-            const at::Tensor&, const at::Tensor&, const c10::optional<at::Tensor>&, int64_t, double) {
-           return at::empty_like(h);
-         });
   m.impl("looped_swiglu_train",
          [](const at::Tensor& h, const at::Tensor&, const at::Tensor&, const at::Tensor&,
             const c10::optional<at::Tensor>&, const at::Tensor&, const at::Tensor&, const c10::optional<at::Tensor>&,

@@ -120,8 +120,6 @@ SIGNATURES = {
     "lbk_looped_bwd_train_workspace_bytes": (C.c_size_t, [_I64, _I32, _I32, _PB, _PB, _PB]),
     "lbk_looped_bwd_train": (C.c_int, [_P, _P, _P, _P, _P, _P, _I64, _I32, _P, C.c_float, _I32, _PB, _PB, _PB, _P, _P, _P,
                                        _P, _P, _P, _P, _P, _P, C.c_size_t, _P]),
-    "lbk_looped_swiglu_prepacked_bf16": (C.c_int, [_P, _I64, _I32, _P, C.c_float, _I32, _PB, _PB, _PB, _P, C.c_size_t,
-                                                   _P, _P, _P, _P, _P, C.c_size_t, _P]),
     "lbk_swiglu_fwd_train": (C.c_int, [_P, _I64, _I32, _PB, _PB, _PB, _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_int, _P,
                                        _P, _P, _P, _P, C.c_size_t, _P]),
     "lbk_swiglu_bwd_train": (C.c_int, [_P, _P, _P, _P, _P, _I64, _I32, _PB, _PB, _PB, C.c_int, _P, _P, _P, _P, _P, _P,

@@ -263,14 +263,6 @@ def looped_swiglu_bias(h, norm_scale, v_gate, ci_gate, b_gate, v_up, ci_up, b_up
                                     b_down, L, eps)
 
 
-def looped_swiglu_prepacked(h, norm_scale, packed, v_gate, ci_gate, b_gate, v_up, ci_up, b_up, v_down, ci_down, b_down,
-                            L: int, eps: float = 1e-5):
-    """``looped_swiglu_bias`` from a ``swiglu_prepack`` copy of the weights."""
-    _gpu(h, v_gate, v_down)
-    return ops().looped_swiglu_prepacked(h, norm_scale, packed, v_gate, ci_gate, b_gate, v_up, ci_up, b_up, v_down,
-                                         ci_down, b_down, L, eps)
-
-
 def looped_swiglu_train(h, norm_scale, v_gate, ci_gate, b_gate, v_up, ci_up, b_up, v_down, ci_down, b_down,
                         L: int, eps: float = 1e-5):
     """``looped_swiglu_bias`` on fp32 values, differentiable as one native autograd node

@@ -21,13 +21,6 @@ from .mlp import MLPBlock, _plain
 from .norms import RMSNorm
 
 
-# Rows from which a gradient-free looped forward packs its weights in the call.  The pack is 6 us, but
-# a long run of nothing but matrix kernels is clocked lower on this card than one with a memory kernel
-# between the passes (the gate/up kernel 80 us at first, 95 to 101 once they follow each other): 16384 x
-# 1024, 8 applications, 1251 us packing per call, 1287 with the kept copy; 96 x 256, 4: 60 and 38.
-_PACK_PER_CALL = 8192
-
-
 class LoopedSwiGLU(nn.Module):
     def __init__(self, d_model: int, d_ff: int, L: int, tile_size: int = 16, density: float = 1.0,
                  eps: float = 1e-5, device=None, bias: bool = True):
@@ -59,15 +52,11 @@ class LoopedSwiGLU(nn.Module):
             for _ in range(self.L):
                 hf = hf + self.mlp(self.norm(hf.to(torch.bfloat16))).float()
             return hf.to(torch.bfloat16).reshape(*lead, d)
-        # the weights as MLPBlock keeps them for gradient-free forwards (rounded and packed once a version)
-        (vg, cg, vu, cu, vd, cd), packed = self.mlp._frozen_swiglu()
+        # rounded and packed in the call: it follows any write to the weights, also replayed from a graph
+        vg, cg, vu, cu, vd, cd = self.mlp.swiglu_weights()
         bg, bu, bd = self.mlp.swiglu_biases()
-        if h2.shape[0] >= _PACK_PER_CALL:
-            out = kernels.looped_swiglu_bias(h2, self.norm.scale, vg, cg, bg, vu, cu, bu, vd, cd, bd, L=self.L,
-                                             eps=self.norm.eps)
-        else:
-            out = kernels.looped_swiglu_prepacked(h2, self.norm.scale, packed, vg, cg, bg, vu, cu, bu, vd, cd, bd,
-                                                  L=self.L, eps=self.norm.eps)
+        out = kernels.looped_swiglu_bias(h2, self.norm.scale, vg, cg, bg, vu, cu, bu, vd, cd, bd, L=self.L,
+                                         eps=self.norm.eps)
         return out.reshape(*lead, d)
 
 

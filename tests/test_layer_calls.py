@@ -1,0 +1,112 @@
+"""Which weights the layers hand to the kernels (host logic only: the kernel calls are recorded)."""
+
+import pytest
+import torch
+
+from looped_blockell import kernels
+
+
+@pytest.fixture
+def looped(monkeypatch):
+    """A CPU LoopedSwiGLU and the (gate, up, down) values that each of its calls passed to a kernel."""
+    from looped_blockell.layers import LoopedSwiGLU
+    seen = []
+
+    def looped_bias(h, scale, vg, cg, bg, vu, cu, bu, vd, cd, bd, L, eps=1e-5):
+        seen.append((vg, vu, vd))
+        return h * vg.flatten()[0]
+
+    monkeypatch.setattr(kernels, "looped_swiglu_bias", looped_bias)
+    monkeypatch.setattr(kernels, "looped_swiglu_prepacked",
+                        lambda h, scale, packed, *w, **kw: looped_bias(h, scale, *w, **kw), raising=False)
+    monkeypatch.setattr(kernels, "swiglu_prepack", lambda *w: torch.zeros(1, dtype=torch.uint8))
+    return LoopedSwiGLU(64, 128, 2, tile_size=16, density=0.5), seen
+
+
+def test_looped_forward_reads_the_weights_of_the_call(looped):
+    """A gradient-free looped forward rounds the weights as they are at the call, whether or not the write
+    before it raised a version (a captured call then holds the rounding, and replays follow the weights)."""
+    m, seen = looped
+    h = torch.zeros(3, 64, dtype=torch.bfloat16)
+    with torch.no_grad():
+        m(h)
+        for write in (lambda p: p.data.mul_(2), lambda p: p.data.copy_(torch.randn(p.shape)), lambda p: p.mul_(3)):
+            for lin in (m.mlp.w_gate, m.mlp.w_up, m.mlp.w_down):
+                write(lin.values)
+            m(h)
+            for got, lin in zip(seen[-1], (m.mlp.w_gate, m.mlp.w_up, m.mlp.w_down)):
+                assert torch.equal(got, lin.values.detach().to(torch.bfloat16))
+    assert m.mlp._frozen is None          # no copy outlives the call
+
+
+def test_looped_forward_under_vmap_over_weights(looped):
+    m, _ = looped
+    gates = torch.randn(2, *m.mlp.w_gate.values.shape)
+    h = torch.ones(3, 64, dtype=torch.bfloat16)
+    with torch.no_grad():
+        out = torch.func.vmap(lambda v: torch.func.functional_call(m, {"mlp.w_gate.values": v}, (h,)))(gates)
+    assert torch.equal(out[:, 0, 0], gates.flatten(1)[:, 0].to(torch.bfloat16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [5, 130])
+@pytest.mark.parametrize("tile", [16, 64])
+def test_captured_looped_forward_follows_its_weights(gpu, N, tile):
+    """Replays of a captured gradient-free looped forward use the weights of the moment, with eager
+    forwards (which must not disturb what the graph reads) and weight writes between them."""
+    from looped_blockell.layers import LoopedSwiGLU
+    torch.manual_seed(4)
+
+    def make():
+        return LoopedSwiGLU(256, 512, 3, tile_size=tile, density=0.5, device="cuda")
+
+    m, x = make(), torch.randn(N, 256, device="cuda").to(torch.bfloat16)
+
+    def fresh():
+        n = make()
+        n.load_state_dict(m.state_dict())
+        return n(x)
+
+    with torch.no_grad():
+        m(x)
+        for p in m.parameters():
+            p.mul_(1.5)                       # the first forward after this write is the captured one
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            y = m(x)
+        assert torch.equal(m(x), fresh())
+        last = None
+        for k in range(4):
+            for lin in (m.mlp.w_gate, m.mlp.w_up, m.mlp.w_down):
+                w = torch.randn_like(lin.values) * 0.05
+                if k % 2:
+                    lin.values.data.copy_(w)
+                else:
+                    lin.values.copy_(w)
+            if k >= 2:
+                assert torch.equal(m(x), fresh())
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, fresh()), k
+            assert last is None or not torch.equal(y, last)
+            last = y.clone()
+
+
+@pytest.mark.gpu
+def test_looped_forward_on_two_streams(gpu):
+    """A forward on another stream right after a weight write on that stream sees the written weights."""
+    from looped_blockell.layers import LoopedSwiGLU
+    torch.manual_seed(5)
+    m = LoopedSwiGLU(256, 512, 2, tile_size=16, density=0.5, device="cuda")
+    x = torch.randn(70, 256, device="cuda").to(torch.bfloat16)
+    s = torch.cuda.Stream()
+    with torch.no_grad():
+        m(x)
+        for _ in range(3):
+            s.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(s):
+                m.mlp.w_gate.values.mul_(1.25)
+                a = m(x)
+            torch.cuda.current_stream().wait_stream(s)
+            assert torch.equal(a, m(x))
