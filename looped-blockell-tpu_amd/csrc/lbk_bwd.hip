@@ -1162,12 +1162,9 @@ __device__ __forceinline__ void dwd_load(const uint16_t* src, int64_t ld, int64_
   int row, c;
   DWD<B>::pos(64 * j + lane, row, c);
   const int64_t t = t0 + row < N ? t0 + row : N - 1;
-  // issued from inline assembly, so the compiler counts no load of its own here and inserts no
-  // wait for these LDS writes before the reads of the other buffer; the kernel waits explicitly
   const uint32_t lds = static_cast<uint32_t>(
       reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)(slice + 512 * j)));
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src + t * ld + col0 + 8 * c),
-               "s"(lds) : "memory", "m0");
+  lds_load16(src + t * ld + col0 + 8 * c, lds);
 }
 
 // barrier without a fence: this wave's LDS reads have returned, its loads in flight stay so
@@ -1323,15 +1320,14 @@ __device__ __forceinline__ void dwg_load(const uint16_t* src, int64_t ld, int64_
   const int64_t tt = t0 + t < N ? t0 + t : N - 1;
   const uint32_t lds = static_cast<uint32_t>(
       reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)(slice + 512 * j)));
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src + tt * ld + col0 + 8 * c),
-               "s"(lds) : "memory", "m0");
+  lds_load16(src + tt * ld + col0 + 8 * c, lds);
 }
 // 1 KB of a slice into LDS at slice_j from this lane's source address (dwg_load's transfer with
 // the address formed by the caller)
 __device__ __forceinline__ void dwt_load(const uint16_t* src, uint16_t* slice_j) {
   const uint32_t lds = static_cast<uint32_t>(
       reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)slice_j));
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory", "m0");
+  lds_load16(src, lds);
 }
 }  // namespace
 

@@ -84,6 +84,19 @@ __device__ __forceinline__ float gelu_grad_f(float z) {
   return s + z * s * (1.0f - s) * (1.5957691216f * (1.0f + 0.134145f * z * z));
 }
 
+// 1 KB from global memory to LDS: lane l's 16 bytes at p (or at base + off) land at lds + 16 l.  Inline
+// assembly, so that the compiler counts no load of its own and puts no wait for these LDS writes before
+// reads of other buffers; the kernels wait explicitly.  The compiler's hazard pass does not look into it
+// either: the s_nop is the wait state that gfx9 needs between a scalar write of M0 (the LDS address) and
+// a load to LDS, without which the piece could land at the previous load's address.
+__device__ __forceinline__ void lds_load16(const void* p, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ void lds_load16(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+               : "memory", "m0");
+}
+
 // Wave-uniform value (forces scalar registers / scalar branches).
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 

@@ -26,11 +26,6 @@ namespace {
 
 constexpr int T64_TILE = 64 * 64 * 2;    // bytes of a tile, and of 64 tokens' column block
 
-// 1 KB to LDS: lane l's 16 bytes at base + off(l) land at lds + 16 l.  Inline assembly, so that
-// the compiler counts no load of its own and puts no wait for it before reads of other steps.
-__device__ __forceinline__ void t64_load(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
-}
 // barrier without a fence: this wave's LDS reads have returned, its loads in flight stay so
 __device__ __forceinline__ void t64_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -123,9 +118,9 @@ __global__ __launch_bounds__(256, 2) void t64_kernel(T64Args a) {
     const char* xp = xb + (int64_t)col * 128;
     const uint32_t l0 = lds0 + (uint32_t)(slot * STEP);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) t64_load(wp, woff[j], l0 + (uint32_t)(TM * 128 + (2 * w + j) * 1024));
+    for (int j = 0; j < 2; ++j) lds_load16(wp, woff[j], l0 + (uint32_t)(TM * 128 + (2 * w + j) * 1024));
 #pragma unroll
-    for (int j = 0; j < 2 * MT; ++j) t64_load(xp, xoff[j], l0 + (uint32_t)((2 * MT * w + j) * 1024));
+    for (int j = 0; j < 2 * MT; ++j) lds_load16(xp, xoff[j], l0 + (uint32_t)((2 * MT * w + j) * 1024));
     if (MODE == 1) upmask = (upmask & ~(1u << slot)) | ((up ? 1u : 0u) << slot);
     ++issued;
     return true;
@@ -363,9 +358,9 @@ __global__ __launch_bounds__(256, 2) void t64_dx_kernel(TProdArgs a, int tg) {
     const char* xp = reinterpret_cast<const char*>((s1 ? S1.a : S0.a) + t0 * lda) + (int64_t)r * 128;
     const uint32_t l0 = lds0 + (uint32_t)(slot * STEP);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) t64_load(wp, woff[j], l0 + (uint32_t)(TM * 128 + (2 * w + j) * 1024));
+    for (int j = 0; j < 2; ++j) lds_load16(wp, woff[j], l0 + (uint32_t)(TM * 128 + (2 * w + j) * 1024));
 #pragma unroll
-    for (int j = 0; j < 2 * MT; ++j) t64_load(xp, xoff[j], l0 + (uint32_t)((2 * MT * w + j) * 1024));
+    for (int j = 0; j < 2 * MT; ++j) lds_load16(xp, xoff[j], l0 + (uint32_t)((2 * MT * w + j) * 1024));
     ++issued;
     return true;
   };
