@@ -580,7 +580,8 @@ constexpr int DX_COLS = 512;                         // activation columns per s
 // dx16_kernel<OPW, MT, NW>: dx at B = 16 (wave w of NW owns output blocks sl + nsl (w + NW o) of
 // 16 MT tokens).  A step of a wave is one list entry and little work, so the kernel is bound by the latency of its tile
 // loads: entries go in pairs (one 16x16x32 MFMA per token tile, lanes g < 2 with entry 2p, the
-// others with 2p + 1, 16 bytes a lane) through a four-pair ring, as in the dh panel kernel, and a
+// others with 2p + 1, 16 bytes a lane; an odd run's last entry is a 16x16x16 MFMA, as a zero tile in
+// the missing half would turn an infinite gradient into NaN) through a four-pair ring, as in the dh panel kernel, and a
 // stage holds 512 to 2048 activation columns (64 or 128 KB of LDS, the next stage in registers
 // meanwhile), so that a block's run within a stage is long enough to fill the ring.
 constexpr int dx16_cols(int OPW, int MT) { return MT == 2 ? 2048 : OPW == 1 ? 1024 : 512; }
@@ -684,34 +685,49 @@ __global__ __launch_bounds__(64 * NW, 1) void dx16_kernel(TProdArgs a) {
         const uint64_t m = __ballot(lane >= base && lane < lim && rv < rhi);
         const int n = __builtin_popcountll(m);       // a contiguous run of lanes (sorted list)
         if (n == 0) break;
-        const int np = (n + 1) >> 1;
+        // an odd run's last entry by itself, as a 16x16x16 MFMA: its load goes out ahead of the pairs'
+        u32x2 odd;
+        int orl = 0;
+        if (n & 1) {
+          const int e = __builtin_amdgcn_readlane(lv, base + n - 1);
+          odd = *reinterpret_cast<const u32x2*>(S.w + (int64_t)e * (B * B) + i * B + 4 * g);
+          orl = __builtin_amdgcn_readlane(rv, base + n - 1) - rlo;
+        }
+        const int np = n >> 1;
         constexpr int D = 4;
         Ent E[D];
         auto loadp = [&](int p, Ent& E) {
-          const int j1 = 2 * p < n ? 2 * p : n - 1, j2 = 2 * p + 1 < n ? 2 * p + 1 : n - 1;
-          const int e1 = __builtin_amdgcn_readlane(lv, base + j1), e2 = __builtin_amdgcn_readlane(lv, base + j2);
+          const int j1 = p < np ? 2 * p : 2 * np - 2;
+          const int e1 = __builtin_amdgcn_readlane(lv, base + j1), e2 = __builtin_amdgcn_readlane(lv, base + j1 + 1);
           const int e = g < 2 ? e1 : e2;
           E.av = *reinterpret_cast<const u32x4*>(S.w + (int64_t)e * (B * B) + i * B + 8 * (g & 1));
-          E.r = (__builtin_amdgcn_readlane(rv, base + j1) - rlo) | ((__builtin_amdgcn_readlane(rv, base + j2) - rlo) << 10) |
-                (2 * p + 1 < n ? 1 << 20 : 0);
+          E.r = (__builtin_amdgcn_readlane(rv, base + j1) - rlo) |
+                ((__builtin_amdgcn_readlane(rv, base + j1 + 1) - rlo) << 10);
         };
         auto computep = [&](const Ent& E) {
           const int rr = uniform(E.r);
-          const int rl = g < 2 ? (rr & 1023) : ((rr >> 10) & 1023);
-          const u32x4 av = (g < 2 || ((rr >> 20) & 1)) ? E.av : u32x4{0, 0, 0, 0};
+          const int rl = g < 2 ? (rr & 1023) : (rr >> 10);
           const uint32_t pa = lbase + ((uint32_t)((rl * 2 + (g & 1)) ^ i) << 4);
 #pragma unroll
           for (int q = 0; q < MT; ++q)
-            acc[o][q] = mfma_bf16(av, *reinterpret_cast<const u32x4*>(stg + pa + q * SROWB), acc[o][q]);
+            acc[o][q] = mfma_bf16(E.av, *reinterpret_cast<const u32x4*>(stg + pa + q * SROWB), acc[o][q]);
         };
+        if (np > 0) {
 #pragma unroll
-        for (int k = 0; k < D - 1; ++k) loadp(k, E[k]);
+          for (int k = 0; k < D - 1; ++k) loadp(k, E[k]);
+        }
         for (int pp = 0; pp < np; pp += D) {
 #pragma unroll
           for (int k = 0; k < D; ++k) {
             loadp(pp + k + D - 1, E[(k + D - 1) % D]);
             if (k == 0 || pp + k < np) computep(E[k]);
           }
+        }
+        if (n & 1) {
+          const uint32_t pa = lbase + ((uint32_t)((orl * 2 + (g >> 1)) ^ i) << 4) + (uint32_t)((g & 1) << 3);
+#pragma unroll
+          for (int q = 0; q < MT; ++q)
+            acc[o][q] = mfma_bf16_k16(odd, *reinterpret_cast<const u32x2*>(stg + pa + q * SROWB), acc[o][q]);
         }
         jc += n;
         if (base + n < 64) break;                    // the run ended inside this chunk

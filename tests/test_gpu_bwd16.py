@@ -84,3 +84,28 @@ def test_swiglu_backward(gpu, case):
     assert _close(dbg, dG.sum(0)) and _close(dbu, dU.sum(0)) and _close(dbd, dy.double().sum(0))
     again = ops.block_ell_swiglu_bwd_train(dy, x, gp, uo, h, vg, cg, vu, cu, vd, cd, False, True)
     assert all(torch.equal(a, b) for a, b in zip(again, (dx, dvg, dvu, dvd, dbg, dbu, dbd)))
+
+
+# 32-token blocks, and 64-token blocks with 1, 2 and 4 output blocks a wave
+@pytest.mark.parametrize("case", [(70, 40, 9, 3), (16400, 20, 9, 4), (16400, 66, 24, 7), (16400, 16, 64, 33)])
+def test_infinite_gradients_stay_infinite(gpu, case):
+    """An infinite gradient reaches the inputs of its block row's live tiles as an infinity of the
+    weight's sign, in runs of odd and even length, and no other value."""
+    from looped_blockell import kernels
+    N, R, C, K = case
+    B = 16
+    rng = np.random.default_rng(R)
+    vals, col = T.bell_weight(rng, R, C, K, B)
+    col[rng.random(col.shape) < 0.15] = -1
+    v, c = T.gpu_weight((vals, col))
+    x, dy = T.to_gpu_bf16(T.act(rng, N, C * B)), T.to_gpu_bf16(T.act(rng, N, R * B))
+    w = _dense(v, c, C)
+    ref = dy.double() @ w
+    for r in range(R):                                      # token r: infinite in block row r
+        f = r * B + (r * 5) % B
+        ref[r] = torch.where(w[f] != 0, torch.sign(w[f]) * float("inf"), ref[r] - dy[r, f].double() * w[f])
+        dy[r, f] = float("inf")
+    dx = kernels.ops().block_ell_matmul_bwd(dy, x, v, c)[0].double()
+    assert torch.equal(torch.isinf(dx), torch.isinf(ref)) and torch.equal(dx[torch.isinf(ref)], ref[torch.isinf(ref)])
+    ok = torch.isfinite(ref)
+    assert not torch.isnan(dx).any() and _close(dx[ok], ref[ok])
