@@ -1086,9 +1086,10 @@ __global__ __launch_bounds__(64 * NW, 1) void dn_kernel(DNArgs a) {
 // dnr_kernel<B, MT, NW, OPW, COLS, KC, BIAS>: 16 MT tokens, NW waves of OPW down rows each (wave w owns
 // rows w, w + NW, ... of its group).  With one row a wave a step is one tile and little work, so the
 // kernel is bound by the latency of its tile loads: they run through a D-deep ring (pairs of slots at
-// B = 16: one 16x16x32 MFMA per token tile, lanes g < 2 with slot 2p, the others with 2p + 1), and a
-// stage holds COLS columns of h (one LDS buffer, the next stage in registers meanwhile) so that a
-// row's run within a stage fills the ring.  The tile is the MFMA's A operand, so a lane ends with
+// B = 16: one 16x16x32 MFMA per token tile, lanes g < 2 with slot 2p, the others with 2p + 1; an odd
+// run's last slot is a 16x16x16 MFMA, as a zero tile in the missing half would turn an infinite h into
+// NaN), and a stage holds COLS columns of h (one LDS buffer, the next stage in registers meanwhile) so
+// that a row's run within a stage fills the ring.  The tile is the MFMA's A operand, so a lane ends with
 // 4 (B = 16) or 8 (B = 32) consecutive columns of one token.
 template <int B, int MT, int NW, int OPW, int COLS, int KC, bool BIAS>
 __global__ __launch_bounds__(64 * NW, 1) void dnr_kernel(DNArgs a) {
@@ -1153,7 +1154,7 @@ __global__ __launch_bounds__(64 * NW, 1) void dnr_kernel(DNArgs a) {
   const u32x4* pd = static_cast<const u32x4*>(a.pd);
   struct Slot {
     u32x4 f[CW];
-    int cb;   // column block within the stage (B = 16: of both slots, and whether the second counts)
+    int cb;   // column block within the stage (B = 16: of both slots)
   };
   stage_fetch(0);
   for (int s = 0; s < nstages; ++s) {
@@ -1171,6 +1172,15 @@ __global__ __launch_bounds__(64 * NW, 1) void dnr_kernel(DNArgs a) {
         const int n = __builtin_popcountll(m);
         if (n == 0) continue;
         const int64_t e0 = (int64_t)(row0 + NW * o) * a.Kd + 64 * kc;
+        // B = 16: the last hit of an odd run by itself, its load ahead of the pairs'
+        u32x2 odd;
+        int ocb = 0;
+        if (B == 16 && (n & 1)) {
+          const int b = 63 - __builtin_clzll(m);
+          m &= ~(1ull << b);
+          odd = load_pfrag16(pd + (e0 + b) * PackedTile<B>::U32X4, pfrag16_off(lane));
+          ocb = __builtin_amdgcn_readlane(cl, b);
+        }
         int last = 0;
         // the next hit (past the end: the last one again)
         auto next = [&]() {
@@ -1182,12 +1192,10 @@ __global__ __launch_bounds__(64 * NW, 1) void dnr_kernel(DNArgs a) {
         };
         auto fetch = [&](Slot& S) {
           if constexpr (B == 16) {
-            const int b1 = next();
-            const int two = m ? 1 << 20 : 0;
-            const int b2 = next();
+            const int b1 = next(), b2 = next();
             const int b = g < 2 ? b1 : b2;
             S.f[0] = pd[(e0 + b) * PackedTile<B>::U32X4 + i + 16 * (g & 1)];
-            S.cb = __builtin_amdgcn_readlane(cl, b1) | (__builtin_amdgcn_readlane(cl, b2) << 10) | two;
+            S.cb = __builtin_amdgcn_readlane(cl, b1) | (__builtin_amdgcn_readlane(cl, b2) << 10);
           } else {
             const int b1 = next();
             const u32x4* tp = pd + (e0 + b1) * PackedTile<B>::U32X4 + lane;
@@ -1199,11 +1207,10 @@ __global__ __launch_bounds__(64 * NW, 1) void dnr_kernel(DNArgs a) {
         auto compute = [&](const Slot& S) {
           const int cb = uniform(S.cb);
           if constexpr (B == 16) {
-            const int rl = g < 2 ? (cb & 1023) : ((cb >> 10) & 1023);
-            const u32x4 f = (g < 2 || ((cb >> 20) & 1)) ? S.f[0] : u32x4{0, 0, 0, 0};
+            const int rl = g < 2 ? (cb & 1023) : (cb >> 10);
             const uint32_t pa = lbase + ((uint32_t)((rl * 2 + (g & 1)) ^ i) << 4);
 #pragma unroll
-            for (int q = 0; q < MT; ++q) acc[o][q][0] = mfma_bf16(f, lds16(dn_smem, pa + q * SROWB), acc[o][q][0]);
+            for (int q = 0; q < MT; ++q) acc[o][q][0] = mfma_bf16(S.f[0], lds16(dn_smem, pa + q * SROWB), acc[o][q][0]);
           } else {
             const uint32_t pa = lbase + ((uint32_t)((cb * (B / 8) + g) ^ i) << 4);
 #pragma unroll
@@ -1214,15 +1221,24 @@ __global__ __launch_bounds__(64 * NW, 1) void dnr_kernel(DNArgs a) {
             }
           }
         };
-        const int np = B == 16 ? (n + 1) >> 1 : n;
+        const int np = B == 16 ? n >> 1 : n;
         Slot S[D];
+        if (B != 16 || np > 0) {
 #pragma unroll
-        for (int k = 0; k < D - 1; ++k) fetch(S[k]);
+          for (int k = 0; k < D - 1; ++k) fetch(S[k]);
+        }
         for (int p = 0; p < np; p += D) {
 #pragma unroll
           for (int k = 0; k < D; ++k) {
             fetch(S[(k + D - 1) % D]);
             if (k == 0 || p + k < np) compute(S[k]);
+          }
+        }
+        if constexpr (B == 16) {
+          if (n & 1) {
+            const uint32_t pa = lbase + ((uint32_t)((ocb * 2 + (g >> 1)) ^ i) << 4) + (uint32_t)((g & 1) << 3);
+#pragma unroll
+            for (int q = 0; q < MT; ++q) acc[o][q][0] = mfma_bf16_k16(odd, lds8(dn_smem, pa + q * SROWB), acc[o][q][0]);
           }
         }
       }

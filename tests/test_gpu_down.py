@@ -68,3 +68,29 @@ def test_looped_state(gpu, case):
         xn = x / torch.sqrt(x.pow(2).mean(-1, keepdim=True) + 1e-5) * T.to_gpu(sc).double()
         x = x + (torch.nn.functional.silu(xn @ wg.T + bt[0].double()) * (xn @ wu.T + bt[1].double())) @ wd.T + bt[2].double()
     assert (out.double() - x).norm() <= 6e-3 * x.norm()
+
+
+# the ring kernel's forms at B = 16 (64 x 16, 32 x 8 with 1024 and 2048 columns, 16 x 4) and at B = 32
+@pytest.mark.parametrize("case", [(16, 4099, 31, 132, 127), (16, 3001, 30, 131, 9), (16, 1500, 30, 131, 65),
+                                  (16, 150, 7, 129, 33), (32, 3001, 30, 65, 33), (32, 150, 9, 66, 5)])
+def test_infinite_inputs_stay_infinite(gpu, case):
+    """An infinite input reaches the rows whose live tiles read its block as an infinity of the weight's
+    sign, in runs of odd and even length, and no other value."""
+    from looped_blockell import kernels
+    B, N, R, C, K = case
+    rng = np.random.default_rng(N)
+    vals, col = T.bell_weight(rng, R, C, K, B)
+    col[rng.random(col.shape) < 0.1] = -1
+    v, c = T.gpu_weight((vals, col))
+    x = T.to_gpu_bf16(T.act(rng, N, C * B))
+    w = _dense(v, c, C)
+    ref = x.double() @ w.T
+    for t in range(min(N, C)):                              # token t: infinite in input block t
+        f = t * B + (t * 5) % B
+        ref[t] = torch.where(w[:, f] != 0, torch.sign(w[:, f]) * float("inf"), ref[t] - x[t, f].double() * w[:, f])
+        x[t, f] = float("inf")
+    y = kernels.block_ell_matmul(x, v, c, None).double()
+    assert not torch.isnan(y).any()
+    assert torch.equal(torch.isinf(y), torch.isinf(ref)) and torch.equal(y[torch.isinf(ref)], ref[torch.isinf(ref)])
+    ok = torch.isfinite(ref)
+    assert (y[ok] - ref[ok]).norm() <= 6e-3 * ref[ok].norm()
