@@ -1621,17 +1621,26 @@ static size_t gu_lds(int R_ff, int K, int mt) {
   return (size_t)16 * mt * (8192 / mt) + (((size_t)R_ff * K * 2 + 15) & ~(size_t)15);
 }
 
-// Row slices per token block for the gate/up kernels (one workgroup of NW waves fills a CU): the split
-// with the least rounds of 256 workgroups times the rows a wave walks in each (two more for the panel
-// fill).  About 256 workgroups whatever the token count leaves a last round of a few: 4099 x 512, d_ff
-// 2048 at density 1, B = 16 (65 token blocks), 65 us in four slices of two rounds, 40 in three of one.
-// Above 4 slices the count is a multiple of 8, so that one slice's workgroups share an XCD.
-static int gu_slices(int64_t ntb, int R_ff, int NW) {
+// Row slices per token block for the gate/up kernels (one workgroup fills a CU): the split with the least
+// rounds of 256 workgroups times the rows of a workgroup, plus its panel fill in rows (`fill`: 32 where a
+// row is a single product, 16 for gate and up, 12 where they are exported too).  Rows count one by one and
+// not in whole passes of the waves: they share the CU's LDS reads, so a short pass costs what it holds.
+// About 256 workgroups whatever the token count would leave a last round of a few: 4099 x 512, d_ff 2048 at
+// density 1, B = 16 (65 token blocks), 65 us in four slices of two rounds, 40 in three of one.  Time over
+// that of the best of 1 to 32 slices, mean of 150 shapes of both tile sizes (700 to 24000 tokens, d_model
+// 256 to 2048): 1.01 so, 1.04 in whole passes, 1.16 with about 256 workgroups.  B = 32, 1024, d_ff 4096 at
+// 0.25, us a forward with about 256 / so: 1100 tokens 32.2 / 28.1, 4200 84 / 70, 6000 96 / 79, 17000 210 /
+// 193 (two slices).  One slice that runs the 12-wave kernel (wide_one) counts six sevenths: 9000 x 512, d_ff
+// 2048 at 0.25 49 with it, 54 in three slices; 24000 85, 88 in two.
+// Not met: exports of rows 4096 wide and more run up to 1.2 times faster in three or four slices (their
+// stores), which single rounds of 200 to 256 token blocks do not get.
+// Up to three slices may spread over the XCDs; above 4 the count is a multiple of 8, so that one slice's
+// workgroups share an XCD.
+static int gu_slices(int64_t ntb, int R_ff, int fill, bool wide_one = false) {
   int best = 1;
   int64_t cost = 0;
   for (int H = 1; H <= R_ff; H = H < 4 ? H + 1 : (H / 8 + 1) * 8) {
-    const int rows = (R_ff + H - 1) / H;
-    const int64_t c = (ntb * H + 255) / 256 * ((rows + NW - 1) / NW + 2);
+    const int64_t c = (ntb * H + 255) / 256 * ((R_ff + H - 1) / H + fill) * (H == 1 && wide_one ? 6 : 7);
     if (H == 1 || c < cost) {
       cost = c;
       best = H;
@@ -1692,7 +1701,6 @@ int launch_gu(int B, bool norm, const GUArgs& a0, hipStream_t st) {
   if (mt == 0) return -2;
   GUArgs a = a0;
   const int64_t ntb = (a.N + 16 * mt - 1) / (16 * mt);
-  a.H = gu_slices(ntb, a.R_ff, 8);
   const bool inter = a.gpre || a.uout;
   // gate and up passing the same column-index buffer share their topology (the reference
   // layer initialises both from the same seed)
@@ -1701,13 +1709,14 @@ int launch_gu(int B, bool norm, const GUArgs& a0, hipStream_t st) {
   // biases (interleaved runs: headline forward 0.1455 -> 0.1434 ms, looped launches at L = 8
   // 1.305 -> 1.283 ms with the normalising kernel; with a shared topology 8 waves measured as
   // fast or faster, 0.1378 against 0.1381-0.1429 ms)
-  if (B == 32 && mt == 4 && a.H == 1 && !inter && !shared && !a.bg && !a.bu)
+  const bool w12 = B == 32 && mt == 4 && !inter && !shared && !a.bg && !a.bu;
+  a.H = gu_slices(ntb, a.R_ff, inter ? 12 : 16, w12);
+  if (w12 && a.H == 1)
     return norm ? launch_gu_w12<32, 4, true>(a, st) : launch_gu_w12<32, 4, false>(a, st);
   // B = 16: 16 waves for every topology, bias and export combination (at most 128 VGPRs; against 8
   // waves: reference-default layer forward 0.2615 -> 0.2408 ms, 3000 x 1024 with biases 103 -> 90 us,
   // 3000 x 2048 190 -> 143).  The normalising fill of 2048-wide rows would spill: 8 waves there.
   if (B == 16 && !(mt == 2 && norm)) {
-    a.H = gu_slices(ntb, a.R_ff, 16);
     const int sel = (shared ? 2 : 0) | ((a.bg || a.bu) ? 1 : 0);
 #define LBK_GU16(MM, NO, IN)                                                     \
   switch (sel) {                                                                 \
@@ -1767,7 +1776,7 @@ static int launch_lin_g(int B, const GUArgs& a0, hipStream_t st) {
   a.Ku = a.Kg;
   const int mt = gu_mt(a.d_model);
   if (mt == 0) return -2;
-  a.H = gu_slices((a.N + 16 * mt - 1) / (16 * mt), a.R_ff, LIN_WAVES);
+  a.H = gu_slices((a.N + 16 * mt - 1) / (16 * mt), a.R_ff, 2 * LIN_WAVES);
 #define LBK_LIN(BB, MM)                                                                     \
   if (B == BB && mt == MM)                                                                  \
     return a.bg ? launch_lin_t<BB, MM, true, GELU>(a, st) : launch_lin_t<BB, MM, false, GELU>(a, st);
