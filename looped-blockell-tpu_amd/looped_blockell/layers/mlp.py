@@ -192,9 +192,11 @@ class MLPBlock(nn.Module):
         return (self.w_gate.kernel_values(), cg, self.w_up.kernel_values(), cu, self.w_down.kernel_values(), cd)
 
     def _fp32_values(self):
-        """Whether the projections' values are fp32 and rounded to bf16 without more ado."""
-        return all(lin.values.dtype == torch.float32 and type(lin).kernel_values is BlockELLLinear.kernel_values
-                   and "kernel_values" not in lin.__dict__ for lin in (self.w_gate, self.w_up, self.w_down))
+        """Whether the projections' values are fp32 and rounded to bf16 without more ado: no replaced
+        ``swiglu_weights`` or ``kernel_values`` to ask for them."""
+        return (type(self).swiglu_weights is MLPBlock.swiglu_weights and "swiglu_weights" not in self.__dict__
+                and all(lin.values.dtype == torch.float32 and type(lin).kernel_values is BlockELLLinear.kernel_values
+                        and "kernel_values" not in lin.__dict__ for lin in (self.w_gate, self.w_up, self.w_down)))
 
     def _swiglu_grad(self, x2, bg, bu, bd):
         """The differentiable forward: fp32 values go to the kernels as they are, rounded there."""

@@ -110,3 +110,42 @@ def test_looped_forward_on_two_streams(gpu):
                 a = m(x)
             torch.cuda.current_stream().wait_stream(s)
             assert torch.equal(a, m(x))
+
+
+def _recorded_training(monkeypatch):
+    """Record the calls that MLPBlock makes for a forward with gradients (CPU stand-ins)."""
+    calls = []
+    monkeypatch.setattr(kernels, "swiglu_train", lambda x, vg, *a, **k: calls.append(("train", vg, a, k)) or x * 1.0)
+    monkeypatch.setattr(kernels, "swiglu", lambda x, vg, *a, **k: calls.append(("bf16", vg, a, k)) or x * 1.0)
+    monkeypatch.setattr(kernels, "looped_swiglu_train",
+                        lambda h, s, vg, *a, **k: calls.append(("looped", vg, a, k)) or h * 1.0)
+    return calls
+
+
+@pytest.mark.parametrize("where", ["subclass", "instance"])
+def test_training_forward_uses_an_overridden_swiglu_weights(monkeypatch, where):
+    """A replaced ``swiglu_weights`` (a fake quantiser, say) decides the weights of a training forward."""
+    from looped_blockell.layers import LoopedSwiGLU, MLPBlock
+    from looped_blockell.layers import norms
+    calls = _recorded_training(monkeypatch)
+
+    def doubled(self):
+        w = MLPBlock.swiglu_weights(self)
+        return (2 * w[0], *w[1:])
+
+    class Doubled(MLPBlock):
+        swiglu_weights = doubled
+
+    kw = dict(use_swiglu=True, tile_size=16, density=0.5)
+    if where == "subclass":
+        m = Doubled(64, 128, **kw)
+    else:
+        m = MLPBlock(64, 128, **kw)
+        m.swiglu_weights = lambda: doubled(m)
+    m(torch.zeros(3, 64, dtype=torch.bfloat16))
+    assert calls[-1][0] == "bf16" and torch.equal(calls[-1][1], 2 * m.w_gate.values.to(torch.bfloat16))
+    monkeypatch.setattr(norms.RMSNorm, "forward", lambda self, x: x)
+    loop = LoopedSwiGLU(64, 128, 2, tile_size=16, density=0.5)
+    loop.mlp = m
+    loop(torch.zeros(3, 64, dtype=torch.bfloat16))
+    assert calls[-1][0] == "bf16" and torch.equal(calls[-1][1], 2 * m.w_gate.values.to(torch.bfloat16))
