@@ -58,9 +58,7 @@ class TernaryMLPBlock(nn.Module):
 
     def prepared(self):
         """The cached prepared weights, rebuilt when any weight buffer's version changes."""
-        return self._prepared_for(self.w_gate.triple(), self.w_up.triple(), self.w_down.triple())
-
-    def _prepared_for(self, *triples):
+        triples = (self.w_gate.triple(), self.w_up.triple(), self.w_down.triple())
         key = [f for w in triples for t in w for f in (t.data_ptr(), t._version)]
         if self._prepared is None or self._prepared[0] != key:
             with torch.inference_mode(False):
@@ -90,7 +88,6 @@ class TernaryMLPBlock(nn.Module):
         lead, d = x.shape[:-1], x.shape[-1]
         x2 = x.reshape(-1, d).to(torch.bfloat16).contiguous()
         xq, sx = kernels.quantize_act_int8(x2)
-        g, u, dn = self.w_gate.triple(), self.w_up.triple(), self.w_down.triple()
-        out = kernels.ternary_swiglu_fwd_prepared(xq, sx, self._prepared_for(g, u, dn), g, u, dn,
-                                                  x2 if add_residual else None)
+        out = kernels.ternary_swiglu_fwd_prepared(xq, sx, self.prepared(), self.w_gate.triple(), self.w_up.triple(),
+                                                  self.w_down.triple(), x2 if add_residual else None)
         return out.reshape(*lead, d)

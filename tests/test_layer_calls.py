@@ -149,3 +149,25 @@ def test_training_forward_uses_an_overridden_swiglu_weights(monkeypatch, where):
     loop.mlp = m
     loop(torch.zeros(3, 64, dtype=torch.bfloat16))
     assert calls[-1][0] == "bf16" and torch.equal(calls[-1][1], 2 * m.w_gate.values.to(torch.bfloat16))
+
+
+def test_ternary_forward_uses_an_overridden_prepared(monkeypatch):
+    """A replaced ``prepared`` decides the weights of a ternary forward."""
+    from looped_blockell.layers import TernaryBlockELLWeight, TernaryMLPBlock
+    seen = []
+    monkeypatch.setattr(kernels, "quantize_act_int8", lambda x: (x, x))
+    monkeypatch.setattr(kernels, "ternary_prepare", lambda *t: "built")
+    monkeypatch.setattr(kernels, "ternary_swiglu_fwd_prepared", lambda xq, sx, prep, *a: seen.append(prep) or xq)
+
+    def weight(R, K):
+        return TernaryBlockELLWeight(torch.zeros(R, K, 16, 1, dtype=torch.int32), torch.ones(R, K),
+                                     torch.zeros(R, K, dtype=torch.int32))
+
+    class Own(TernaryMLPBlock):
+        def prepared(self):
+            return "own"
+
+    x = torch.zeros(3, 32)
+    for cls, want in ((TernaryMLPBlock, "built"), (Own, "own")):
+        cls(weight(4, 1), weight(4, 1), weight(2, 1))(x)
+        assert seen[-1] == want
