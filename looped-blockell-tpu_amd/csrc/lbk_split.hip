@@ -1632,15 +1632,18 @@ static size_t gu_lds(int R_ff, int K, int mt) {
 // 0.25, us a forward with about 256 / so: 1100 tokens 32.2 / 28.1, 4200 84 / 70, 6000 96 / 79, 17000 210 /
 // 193 (two slices).  One slice that runs the 12-wave kernel (wide_one) counts six sevenths: 9000 x 512, d_ff
 // 2048 at 0.25 49 with it, 54 in three slices; 24000 85, 88 in two.
-// Not met: exports of rows 4096 wide and more run up to 1.2 times faster in three or four slices (their
-// stores), which single rounds of 200 to 256 token blocks do not get.
+// Exports slow down where a slice is wider than 2048 columns (rows_wide of them; not at 512, d_ff 2048), so
+// those columns count up to double: 14000 x 1024, d_ff 4096 at B = 32, 235 us in one slice, 228 in two, 198
+// in three; 6900 x 2048, d_ff 7168 241 / 208 / 211; 16384 x 768, d_ff 3072 174 / 151 / 151.
 // Up to three slices may spread over the XCDs; above 4 the count is a multiple of 8, so that one slice's
 // workgroups share an XCD.
-static int gu_slices(int64_t ntb, int R_ff, int fill, bool wide_one = false) {
+static int gu_slices(int64_t ntb, int R_ff, int fill, bool wide_one = false, int rows_wide = 0) {
   int best = 1;
   int64_t cost = 0;
   for (int H = 1; H <= R_ff; H = H < 4 ? H + 1 : (H / 8 + 1) * 8) {
-    const int64_t c = (ntb * H + 255) / 256 * ((R_ff + H - 1) / H + fill) * (H == 1 && wide_one ? 6 : 7);
+    int64_t rows = (R_ff + H - 1) / H;
+    if (rows_wide && rows > rows_wide) rows += rows * (rows - rows_wide) / (2 * rows_wide);
+    const int64_t c = (ntb * H + 255) / 256 * (rows + fill) * (H == 1 && wide_one ? 6 : 7);
     if (H == 1 || c < cost) {
       cost = c;
       best = H;
@@ -1710,7 +1713,7 @@ int launch_gu(int B, bool norm, const GUArgs& a0, hipStream_t st) {
   // 1.305 -> 1.283 ms with the normalising kernel; with a shared topology 8 waves measured as
   // fast or faster, 0.1378 against 0.1381-0.1429 ms)
   const bool w12 = B == 32 && mt == 4 && !inter && !shared && !a.bg && !a.bu;
-  a.H = gu_slices(ntb, a.R_ff, inter ? 12 : 16, w12);
+  a.H = gu_slices(ntb, a.R_ff, inter ? 12 : 16, w12, inter ? 2048 / B : 0);
   if (w12 && a.H == 1)
     return norm ? launch_gu_w12<32, 4, true>(a, st) : launch_gu_w12<32, 4, false>(a, st);
   // B = 16: 16 waves for every topology, bias and export combination (at most 128 VGPRs; against 8
