@@ -1859,28 +1859,57 @@ static int launch_dnr(const DNArgs& a, hipStream_t st) {
   return a.Kd > 64 ? launch_dnr_k<B, MT, NW, OPW, COLS, 2>(a, st) : launch_dnr_k<B, MT, NW, OPW, COLS, 1>(a, st);
 }
 
-// The ring kernel's form for a token count and row count (-2: the kernels with 512-column stages are
-// faster).  Workgroups of 64 tokens while they fill about half the CUs or more, then 32 tokens and 8
-// rows (1024-column stages, two workgroups a CU, above 256 of them), then 16 tokens and 4 rows.  us a
-// forward or looped forward, in the order 64 x 16 (B = 16) or 64 x 8 rows (B = 32) / 32 x 8 with 2048
-// columns / with 1024 / 16 x 4 / the two-slot kernel before it:
-//   B = 16  4099 x 512 K 128: 61 / 79 / 70 / 94 / 105     2048 x 512 x4 training: 529 / 491 / 499 / 521 / 531
-//           5000 x 256 x8: 330 / 356 / 308 / 394 / 433    300 x 512 x8: 239 / 181 / 194 / 167 / 210
-//   B = 32  3000 x 1024: 50 / 55 / 58 / 58 / 61           2338 x 512 x7: 247 / 213 / 220 / 222 / 245
-//           700 x 1024: 35 / 26 / 29 / 24 / 31            1313 x 512 x8: 269 / 221 / 231 / 213 / 253
-// At B = 32 whole rounds of 64 tokens and 16 rows stay with dnf_kernel and dn_kernel (16384 x 1024:
-// 166 us, 181 here), and at B = 16 those whose rows have few slots in a stage (3000 x 2048 at 0.1:
-// 144, 147 here).
-template <int B>
-static int launch_dn_ring(const DNArgs& a, int64_t w16, hipStream_t st) {
-  const int64_t w8 = (a.N + 63) / 64 * ((a.R_m + 7) / 8), w2 = (a.N + 31) / 32 * ((a.R_m + 7) / 8);
-  if (B == 16 && w16 >= 256 && (int64_t)a.Kd * 1024 < 8 * a.d_ff) return -2;
-  if (B == 16 && w16 >= 128) return launch_dnr<16, 4, 16, 1, 1024>(a, st);
-  if (B == 32 && w16 >= 200) return -2;
-  if (B == 32 && w8 >= 160) return launch_dnr<32, 4, 8, 1, 1024>(a, st);
-  if (w2 > 256) return launch_dnr<B, 2, 8, 1, 1024>(a, st);
-  if (w2 >= 128) return launch_dnr<B, 2, 8, 1, 2048>(a, st);
-  return launch_dnr<B, 1, 4, 1, 2048>(a, st);
+// The down kernel's form for a token count, row count, width and slots a row (-2: the kernels with
+// 512-column stages).  A workgroup fills a CU or, with 64 KB of LDS and at most 128 VGPRs (the 16 x 4 form
+// and, at B = 16, the 32 x 8 form with 1024-column stages), half of one, and a token block's workgroups
+// share an XCD, so what counts is the rounds of the XCD with the most token blocks.
+// B = 16: the smallest workgroups that take one round; past those 64 x 16 rows, or the kernels with
+// 512-column stages where rows have few slots in a stage (3000 x 2048 at 0.1: 144, 147 us here).
+// B = 32: the least rounds times a round's time, as fitted to 260 products (480 to 8192 wide, 100 to 16384
+// tokens): a + b per stage + c per slot, us.  The time over the best form's, mean and largest: 1.003 and
+// 1.09 so, 1.03 and 1.50 with limits on workgroup counts alone; at B = 16 1.009 and 1.24 (a 5 us product),
+// and 1.02 and 1.53.  5162 x 3072 -> 768, 24 slots: 30.5 us in 64 x 8 rows (33 workgroups on two of the
+// XCDs), 23.2 in 32 x 8; 2147 x 4096 -> 1024, 32 slots: 28.7 in 32 x 8, 21.7 in 64 x 8.
+static int64_t dn_rounds(const DNArgs& a, int tokens, int rows, int per_xcd) {
+  const int64_t ntb = (a.N + tokens - 1) / tokens;
+  return ((ntb + 7) / 8 * ((a.R_m + rows - 1) / rows) + per_xcd - 1) / per_xcd;
+}
+
+static int launch_dn16(const DNArgs& a, hipStream_t st) {
+  if (dn_rounds(a, 16, 4, 64) == 1) return launch_dnr<16, 1, 4, 1, 2048>(a, st);
+  if (dn_rounds(a, 32, 8, 32) == 1) return launch_dnr<16, 2, 8, 1, 2048>(a, st);
+  if (dn_rounds(a, 32, 8, 64) == 1) return launch_dnr<16, 2, 8, 1, 1024>(a, st);
+  if ((a.N + 63) / 64 * ((a.R_m + 15) / 16) >= 256 && (int64_t)a.Kd * 1024 < 8 * a.d_ff) return -2;
+  return launch_dnr<16, 4, 16, 1, 1024>(a, st);
+}
+
+static int launch_dn32(const DNArgs& a, hipStream_t st) {
+  struct Form { int tokens, rows, per_xcd, cols; float a, b, c; };
+  constexpr Form forms[5] = {{64, 8, 32, 1024, 0.8f, 3.2f, 0.18f},
+                             {32, 8, 32, 1024, 0.6f, 2.0f, 0.134f},
+                             {32, 8, 32, 2048, 0.2f, 3.35f, 0.132f},
+                             {16, 4, 64, 2048, 0.1f, 2.25f, 0.1f},
+                             // dnf_kernel and dn_kernel, from 200 workgroups on
+                             {64, 16, 32, 512, 1.5f, 1.45f, 0.32f}};
+  const bool many = (a.N + 63) / 64 * ((a.R_m + 15) / 16) >= 200;
+  int best = 0;
+  float cost = 0.f;
+  for (int f = 0; f < (many ? 5 : 4); ++f) {
+    const Form& F = forms[f];
+    const float c = (float)dn_rounds(a, F.tokens, F.rows, F.per_xcd) *
+                    (F.a + F.b * (float)((a.d_ff + F.cols - 1) / F.cols) + F.c * (float)a.Kd);
+    if (f == 0 || c < cost) {
+      cost = c;
+      best = f;
+    }
+  }
+  switch (best) {
+    case 0: return launch_dnr<32, 4, 8, 1, 1024>(a, st);
+    case 1: return launch_dnr<32, 2, 8, 1, 1024>(a, st);
+    case 2: return launch_dnr<32, 2, 8, 1, 2048>(a, st);
+    case 3: return launch_dnr<32, 1, 4, 1, 2048>(a, st);
+    default: return -2;
+  }
 }
 
 int launch_dn(int B, const DNArgs& a, hipStream_t st) {
@@ -1890,7 +1919,7 @@ int launch_dn(int B, const DNArgs& a, hipStream_t st) {
   const bool plain = !a.state && !a.tdepth && !a.inj_e && a.out && a.Kd <= 64;
   const int64_t w16 = (a.N + 63) / 64 * ((a.R_m + 15) / 16);   // 64-token workgroups of 16 rows
   if (!a.tdepth && !a.inj_e) {
-    const int rc = B == 16 ? launch_dn_ring<16>(a, w16, st) : B == 32 ? launch_dn_ring<32>(a, w16, st) : -2;
+    const int rc = B == 16 ? launch_dn16(a, st) : B == 32 ? launch_dn32(a, st) : -2;
     if (rc != -2) return rc;
   } else if (w16 < 256) {
     // the looped core's state update, with too few workgroups of 64 tokens and 16 rows: smaller ones
