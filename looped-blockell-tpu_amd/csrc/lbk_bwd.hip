@@ -962,43 +962,52 @@ static int launch_dxf(const TProdArgs& a0, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// staged dx when every output block fits the waves' accumulators (OPW * B / 16 <= 8) and the
-// sources' widths are whole stages of 16-byte chunks
-static int launch_dx(int B, const TProdArgs& a0, hipStream_t st) {
-  if (a0.nsrc < 1 || a0.nsrc > 2) return -2;
-  for (int s = 0; s < a0.nsrc; ++s)
-    if (a0.src[s].lda % B) return -2;
-  // With fewer 64-token blocks than CUs, the output blocks are split over nsl workgroups per
-  // token block so that each wave owns one (each workgroup stages all the activation columns).
+// dx at B = 16: the form with the least rounds of its workgroups times a round's time, as fitted to 180
+// products (100 to 15000 tokens, 256 to 8192 wide): a + b per stage + c per list entry, us.  A workgroup
+// fills a CU and a token block's workgroups share an XCD, so the XCD with the most token blocks counts:
+// smallest workgroups while they take one round, then fewer passes over the activations.  The time over the
+// best form's, mean and largest: 1.003 and 1.19 so; with 32 x 8 below 256 workgroups of 64 x 16, 1.12 and
+// 1.86.  us in 32 x 8 / 64 x 16 / 64 x 32: 989 x 512 from 1792, 10 entries, 9.8 / 14.9 / 23; 4911 x 768 from
+// 2688, 14 entries, 39.6 / 21.4 / 27.8; 14792 x 1024 from 4096, 128 entries, 303 / 171 / 155 (170 in 64 x 64).
+static int launch_dx16(const TProdArgs& a0, hipStream_t st) {
+  struct Form { int tokens, blocks, cols; float a, b, c; };
+  constexpr Form forms[3] = {{32, 8, dx16_cols(1, 2), 0.8f, 3.05f, 0.13f},
+                             {64, 16, dx16_cols(1, 4), 1.1f, 4.1f, 0.21f},
+                             {64, 32, dx16_cols(2, 4), 0.9f, 3.8f, 0.24f}};
   TProdArgs a = a0;
-  const int64_t ntb = (a.N + 63) / 64;
-  a.nsl = ntb >= 256 ? 1 : (a.C + 15) / 16;
-  const int cs = (a.C + a.nsl - 1) / a.nsl;        // output blocks per slice
+  int best = 0;
+  float cost = 0.f;
+  for (int f = 0; f < 3; ++f) {
+    const Form& F = forms[f];
+    const int64_t ntb = (a.N + F.tokens - 1) / F.tokens, nsl = (a.C + F.blocks - 1) / F.blocks;
+    float round = F.a;
+    for (int s = 0; s < a.nsrc; ++s)
+      round += F.b * (float)((a.src[s].lda + F.cols - 1) / F.cols) + F.c * (float)a.src[s].cap / (float)a.C;
+    const float c = (float)(((ntb + 7) / 8 * nsl + 31) / 32) * round;
+    if (f == 0 || c < cost) {
+      cost = c;
+      best = f;
+      a.nsl = (int)nsl;
+    }
+  }
+  if (best == 0) return launch_dx16_t<1, 2, 8>(a, st);
+  return best == 1 ? launch_dx16_t<1, 4, 16>(a, st) : launch_dx16_t<2, 4, 16>(a, st);
+}
+
+// dx through LDS when the sources' widths are whole column blocks
+static int launch_dx(int B, const TProdArgs& a, hipStream_t st) {
+  if (a.nsrc < 1 || a.nsrc > 2) return -2;
+  for (int s = 0; s < a.nsrc; ++s)
+    if (a.src[s].lda % B) return -2;
   // B = 32: the deep-ring kernel (headline backward 0.710 -> 0.688 ms; 64 / 1024 / 4096 tokens
   // 0.109 / 0.131 / 0.213 -> 0.105 / 0.127 / 0.199 ms)
-  if (B == 32) return launch_dxf<32>(a0, st);
-  if (B == 16) {
-    // 64-token blocks with 16 waves where those fill the CUs; else 32-token blocks and 8 waves, one
-    // output block each, whose panel reads and staging spread over four times the CUs (us a step,
-    // 2000 x 512, d_ff 2048 / looped x4 of 2048 x 512 / 1000 x 1024, d_ff 4096: 164 / 603 / 206 with
-    // 64 tokens and 16 waves, 156 / 563 / 191 so, 161 / 590 / 203 with 64 tokens and 8 waves, 176 /
-    // 653 / 216 with 32 and 4; the eight-byte single-entry kernel before it 189 / 786 / 238)
-    if (ntb * ((a.C + 15) / 16) < 256) {
-      a.nsl = (a.C + 7) / 8;
-      return launch_dx16_t<1, 2, 8>(a, st);
-    }
-    const int opw = (cs + 15) / 16;
-    if (opw <= 1) return launch_dx16_t<1, 4, 16>(a, st);
-    if (opw <= 2) return launch_dx16_t<2, 4, 16>(a, st);
-    if (opw <= 4) return launch_dx16_t<4, 4, 16>(a, st);
-  }
-  // B = 16 with more output blocks than the staged kernel's accumulators hold (N >= 16321 tokens
-  // and more than 64 output blocks): the deep-ring kernel, one output block per wave, in place of
-  // the per-entry kernel (1024 x 8192 product backward at 16384 tokens 1.275 -> 0.658 ms).  Where
-  // the staged kernel fits it stays: the deep ring stages the activations once per 16 output
-  // blocks and was slower there (SwiGLU backward at d_model 1024 0.823 -> 0.886 ms)
-  if (B == 16) return launch_dxf<16>(a0, st);
-  return -2;
+  if (B == 32) return launch_dxf<32>(a, st);
+  // B = 16 at 16321 tokens and more with more than 64 output blocks: the deep-ring kernel (1024 x 8192
+  // product backward at 16384 tokens 1.275 ms in the per-entry kernel, 0.658 so).  With fewer output
+  // blocks it stages the activations once per 16 of them and is slower (SwiGLU backward at d_model 1024
+  // 0.823 ms, 0.886 so)
+  if (B == 16 && (a.N + 63) / 64 >= 256 && a.C > 64) return launch_dxf<16>(a, st);
+  return B == 16 ? launch_dx16(a, st) : -2;
 }
 
 int launch_tprod(int B, int mode, const TProdArgs& a, hipStream_t st) {
