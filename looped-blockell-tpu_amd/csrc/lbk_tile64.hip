@@ -271,6 +271,11 @@ int launch_t64(int mode, const RowblockLaunch& a, hipStream_t st) {
       ((mode == 1 || a.gelu) && ((a.aux0 && bad(a.aux0, 7)) || (a.aux1 && bad(a.aux1, 7)) || a.ldaux % 4)) ||
       (mode == 2 && a.resid && (bad(a.resid, 7) || a.ldr % 4)) || a.ldx > (1 << 22))
     return -2;
+  // one slot a row: a single step has nothing to overlap, and the row-block kernel, without the trip
+  // through LDS, is faster (us here / there, products of 3000 tokens: 512 -> 2048 10.1 / 7.6, 256 -> 896 6.7 /
+  // 4.8; 10000 x 2048 -> 512 9.6 / 7.1; with two slots 11.0 / 11.6, 7.7 / 7.0, 10.3 / 10.6).  Gate/up of one slot
+  // each stays: within 1 us up to 700 tokens, 3 to 20 us faster from 5000.
+  if (mode != 1 && !a.gelu && a.K0 <= 1 && a.R <= 65535) return -2;
   // the largest token block that leaves two workgroups per CU (2048 tokens, 2048 -> 8192 at 0.5: 159
   // us with 256 tokens two steps deep, 165 and 194 with 128 and 64; three and four steps deep, with
   // fewer workgroups resident, 175 to 236)
