@@ -36,7 +36,7 @@ class LoopedSwiGLU(nn.Module):
         h2 = h.reshape(-1, d).to(torch.bfloat16).contiguous()
         if torch.is_grad_enabled() and (h.requires_grad or any(p.requires_grad for p in self.parameters())):
             if (self.L >= 1 and h2.shape[0] > 0 and d == self.mlp.d_model and _plain(self.norm, RMSNorm)
-                    and _plain(self.mlp, MLPBlock) and self.mlp._fp32_values()):
+                    and _plain(self.mlp, MLPBlock) and self.mlp.use_swiglu and self.mlp._fp32_values()):
                 cg, cu, cd = self.mlp.swiglu_columns()
                 bg, bu, bd = self.mlp.swiglu_biases()
                 m = self.mlp

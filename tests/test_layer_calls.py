@@ -171,3 +171,15 @@ def test_ternary_forward_uses_an_overridden_prepared(monkeypatch):
     for cls, want in ((TernaryMLPBlock, "built"), (Own, "own")):
         cls(weight(4, 1), weight(4, 1), weight(2, 1))(x)
         assert seen[-1] == want
+
+
+def test_looped_training_with_another_mlp(monkeypatch):
+    """A looped block whose MLP was replaced by a GELU one trains through that module's own calls."""
+    from looped_blockell.layers import LoopedSwiGLU, MLPBlock, norms
+    _recorded_training(monkeypatch)
+    monkeypatch.setattr(norms.RMSNorm, "forward", lambda self, x: x)
+    monkeypatch.setattr(MLPBlock, "_gelu", lambda self, x: x + 1)
+    loop = LoopedSwiGLU(64, 128, 3, tile_size=16, density=0.5)
+    loop.mlp = MLPBlock(64, 128, tile_size=16)
+    out = loop(torch.ones(3, 64, dtype=torch.bfloat16))
+    assert (out == 15).all()                  # h <- h + (h + 1), three times from 1
