@@ -124,3 +124,61 @@ def test_swiglu_backward_two_sources(gpu, N):
     for res in (False, True):
         dx = ops.block_ell_swiglu_bwd_ex(dy, x, gp, uo, h, *g, *u, *dn, res)[0]
         assert _close(dx, ref + (dy.double() if res else 0))
+
+
+# slot lists past one 64-entry window: gate ending within the first window with up running on into the
+# second (40 a side), gate itself crossing it (70 a side); rows without a live gate or up slot
+@pytest.mark.parametrize("K", [40, 70])
+@pytest.mark.parametrize("N", [70, 520])
+def test_gate_up_over_windows(gpu, K, N):
+    from looped_blockell import kernels
+    d, ff = 72 * 64, 5 * 64
+    rng = np.random.default_rng(N + K)
+    g = _weight(rng, 5, 72, K, dead=0.1, dead_row=1)
+    u = _weight(rng, 5, 72, K, dead=0.1, dead_row=2)
+    dn = _weight(rng, 72, 5, 3, dead=0.1)
+    x = T.to_gpu_bf16(T.act(rng, N, d))
+    wg, wu, wd = (_dense(*w, C) for w, C in ((g, 72), (u, 72), (dn, 5)))
+    G, U = x.double() @ wg.T, x.double() @ wu.T
+    out, h, gp, uo = kernels.ops().block_ell_swiglu_fwd_with_intermediate(x, *g, *u, *dn, False)
+    H = torch.nn.functional.silu(G) * U
+    for got, want in ((gp, G), (uo, U), (h, H), (out, H @ wd.T)):
+        assert _close(got, want)
+    for got, want in ((gp, G), (uo, U)):               # per block row
+        e = (got.double() - want).reshape(N, 5, 64).norm(dim=(0, 2))
+        assert (e <= REL * want.reshape(N, 5, 64).norm(dim=(0, 2)) + 1e-9).all()
+
+
+@pytest.mark.parametrize("N", [70, 520])
+def test_two_source_lists_over_windows(gpu, N):
+    """dx lists of about 45 gate and 45 up entries: the boundary of the two sources lies within the first
+    64-entry window and up crosses into the second; one input block that no gate slot reads."""
+    from looped_blockell import kernels
+    d, ff = 3 * 64, 135 * 64
+    rng = np.random.default_rng(N)
+    vg, cg = T.bell_weight(rng, 135, 3, 1, 64)
+    cg[cg == 1] = -1
+    g, u, dn = T.gpu_weight((vg, cg)), _weight(rng, 135, 3, 1, dead=0.05), _weight(rng, 3, 135, 30, dead=0.1)
+    x, dy = T.to_gpu_bf16(T.act(rng, N, d)), T.to_gpu_bf16(T.act(rng, N, d))
+    ops = kernels.ops()
+    _, h, gp, uo = ops.block_ell_swiglu_fwd_with_intermediate(x, *g, *u, *dn, True)
+    wg, wu, wd = (_dense(*w, C) for w, C in ((g, 3), (u, 3), (dn, 135)))
+    G, U, dh = gp.double(), uo.double(), dy.double() @ wd
+    s = torch.sigmoid(G)
+    ref = (dh * U * (s + G * s * (1 - s))) @ wg + (dh * G * s) @ wu
+    dx = ops.block_ell_swiglu_bwd_ex(dy, x, gp, uo, h, *g, *u, *dn, False)[0]
+    for c in range(3):
+        assert _close(dx[:, 64 * c:64 * c + 64], ref[:, 64 * c:64 * c + 64]), c
+
+
+@pytest.mark.parametrize("case", [(1, 3, 2), (300, 14, 4), (3000, 14, 4), (10, 40, 32)])
+def test_one_slot_products(gpu, case):
+    """Products of one slot a row take the row-block kernel, with and without a live slot."""
+    from looped_blockell import kernels
+    N, R, C = case
+    rng = np.random.default_rng(N)
+    v, c = _weight(rng, R, C, 1, dead=0.1, dead_row=R - 1)
+    x, b = T.to_gpu_bf16(T.act(rng, N, C * 64)), T.to_gpu(rng.standard_normal(R * 64).astype(np.float32))
+    ref = x.double() @ _dense(v, c, C).T + b.double()
+    y = kernels.block_ell_matmul(x, v, c, b)
+    assert _close(y, ref) and torch.equal(y[:, -64:], b[-64:].to(torch.bfloat16).expand(N, 64))
