@@ -278,7 +278,6 @@ __device__ __forceinline__ int kdiv(const TProdSrc& S, int e) {
   return (int)((__umulhi((uint32_t)e, S.kmul) + (uint32_t)e) >> S.ksh);
 }
 
-// GELU: the epilogue is dg = dh gelu'(g), with no up stream
 // sum over the 16 lanes of a DPP row (every lane gets it): rotations by 8, 4, 2 and 1
 __device__ __forceinline__ float row_sum16(float v) {
 #define LBK_ROR(n) \
@@ -288,6 +287,7 @@ __device__ __forceinline__ float row_sum16(float v) {
   return v;
 }
 
+// GELU: the epilogue is dg = dh gelu'(g), with no up stream
 template <int B, int MT, int NW, bool GELU>
 __global__ __launch_bounds__(64 * NW, 1) void dh_panel_kernel(TProdArgs a) {
   constexpr int NT = 64 * NW;
@@ -577,12 +577,12 @@ static int launch_dh_panel(int B, const TProdArgs& a, hipStream_t st) {
 // t64_dx_kernel of lbk_tile64.hip.)
 constexpr int DX_COLS = 512;                         // activation columns per stage (dxf_kernel)
 
-// dx16_kernel<OPW, MT, NW>: dx at B = 16 (wave w of NW owns output blocks sl + nsl (w + NW o) of
-// 16 MT tokens).  A step of a wave is one list entry and little work, so the kernel is bound by the latency of its tile
-// loads: entries go in pairs (one 16x16x32 MFMA per token tile, lanes g < 2 with entry 2p, the
-// others with 2p + 1, 16 bytes a lane; an odd run's last entry is a 16x16x16 MFMA, as a zero tile in
-// the missing half would turn an infinite gradient into NaN) through a four-pair ring, as in the dh panel kernel, and a
-// stage holds 512 to 2048 activation columns (64 or 128 KB of LDS, the next stage in registers
+// dx16_kernel<OPW, MT, NW>: dx at B = 16 (wave w of NW owns output blocks sl + nsl (w + NW o) of 16 MT
+// tokens).  A step of a wave is one list entry and little work, so the kernel is bound by the latency of
+// its tile loads: entries go in pairs (one 16x16x32 MFMA per token tile, lanes g < 2 with entry 2p, the
+// others with 2p + 1, 16 bytes a lane) through a four-pair ring, as in the dh panel kernel; an odd run's
+// last entry is a 16x16x16 MFMA, as a zero tile in the missing half would turn an infinite gradient into
+// NaN.  A stage holds 512 to 2048 activation columns (64 or 128 KB of LDS, the next stage in registers
 // meanwhile), so that a block's run within a stage is long enough to fill the ring.
 constexpr int dx16_cols(int OPW, int MT) { return MT == 2 ? 2048 : OPW == 1 ? 1024 : 512; }
 template <int OPW, int MT, int NW>
@@ -764,13 +764,13 @@ static int launch_dx16_t(const TProdArgs& a0, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// dxf_kernel<B, D>: dx at B = 32 (and at B = 16 past the staged kernel's widths) with one output
-// block per wave (16 waves; the output blocks are dealt to nsl workgroups per 64-token block,
-// which share an XCD) and a D-slot ring of tiles that
-// runs over the wave's whole list -- the sorted entries of source 0, then of source 1 -- across
-// the 512-column stages of both sources, so D tile loads stay in flight.  A stage change is a workgroup barrier taken inline when the next entry lies in a
-// later stage; every wave passes all of them.  The list entries a pass fetches are read one pass
-// ahead (lane j of a window holds entry j of the pass), so no load waits on a list read.
+// dxf_kernel<B, D>: dx at B = 32 with one output block per wave (16 waves; the output blocks are dealt to
+// nsl workgroups per 64-token block, which share an XCD) and a D-slot ring of tiles that runs over the
+// wave's whole list -- the sorted entries of source 0, then of source 1 -- across the 512-column stages
+// of both sources, so D tile loads stay in flight.  A stage change is a workgroup barrier taken inline
+// when the next entry lies in a later stage; every wave passes all of them.  The list entries a pass
+// fetches are read one pass ahead (lane j of a window holds entry j of the pass), so no load waits on a
+// list read.
 constexpr int DXF_WAVES = 16;
 constexpr int DXF_RING = 4;
 template <int B, int D>
@@ -782,8 +782,7 @@ __global__ __launch_bounds__(64 * DXF_WAVES, 1) void dxf_kernel(TProdArgs a) {
   constexpr int SROWB = COLS * 2;
   constexpr int SBYTES = 64 * SROWB;
   constexpr int PER_T = SBYTES / 16 / NT;
-  // B = 32: one 32-deep k-step per tile; B = 16: the 16x16x16 form (8-byte fragments)
-  static_assert(B == 32 || B == 16, "tile size");
+  static_assert(B == 32, "one 32-deep k-step per tile");
   extern __shared__ __attribute__((aligned(16))) unsigned char stg[];   // two stages
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = uniform(tid >> 6);
@@ -851,9 +850,8 @@ __global__ __launch_bounds__(64 * DXF_WAVES, 1) void dxf_kernel(TProdArgs a) {
 
   struct Slot {
     u32x4 av[CW];
-    u32x2 a16;   // B = 16: the 16x16x16 fragment (tile row i, k = 4g .. 4g + 3)
-    int st;      // stage (-1: past the list)
-    int cb;      // column block within the stage
+    int st;   // stage (-1: past the list)
+    int cb;   // column block within the stage
   };
   // slot S <- entry j of the list (its value e read from the window)
   auto fetch = [&](Slot& S, int j, int e) {
@@ -862,13 +860,9 @@ __global__ __launch_bounds__(64 * DXF_WAVES, 1) void dxf_kernel(TProdArgs a) {
     // r = e / K by multiply and shift (a division by a run-time value is a long sequence)
     const int r = live ? kdiv(s1 ? S1 : S0, e) : 0;
     const int64_t tile = live ? e : 0;              // past the list: tile 0 of source 0, unused
-    if constexpr (B == 16) {
-      S.a16 = *reinterpret_cast<const u32x2*>((live && s1 ? S1.w : S0.w) + tile * B * B + i * B + 4 * g);
-    } else {
-      const uint16_t* tp = (live && s1 ? S1.w : S0.w) + tile * B * B + 8 * g;
+    const uint16_t* tp = (live && s1 ? S1.w : S0.w) + tile * B * B + 8 * g;
 #pragma unroll
-      for (int m = 0; m < CW; ++m) S.av[m] = ld16(tp + op_row<CW>(i, m) * B);
-    }
+    for (int m = 0; m < CW; ++m) S.av[m] = ld16(tp + op_row<CW>(i, m) * B);
     S.st = live ? (s1 ? ns0 : 0) + r / G : -1;
     S.cb = r - (r / G) * G;
   };
@@ -879,14 +873,6 @@ __global__ __launch_bounds__(64 * DXF_WAVES, 1) void dxf_kernel(TProdArgs a) {
 #pragma unroll
     for (int m = 0; m < CW; ++m) acc[q][m] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto compute = [&](const Slot& S, const unsigned char* sb) {
-    if constexpr (B == 16) {
-      // rows 16q + i, k = 4g .. 4g + 3 of the block: 16-byte chunk 2 cb + g / 2, its half g & 1
-      const uint32_t pa = lbase + ((uint32_t)(((S.cb * 2 + (g >> 1)) ^ i) << 4) | (uint32_t)((g & 1) << 3));
-#pragma unroll
-      for (int q = 0; q < MT; ++q)
-        acc[q][0] = mfma_bf16_k16(S.a16, *reinterpret_cast<const u32x2*>(sb + pa + q * SROWB), acc[q][0]);
-      return;
-    }
     const uint32_t pa = lbase + (((S.cb * (B / 8) + g) ^ i) << 4);
 #pragma unroll
     for (int q = 0; q < MT; ++q) {
@@ -968,7 +954,8 @@ static int launch_dxf(const TProdArgs& a0, hipStream_t st) {
 // smallest workgroups while they take one round, then fewer passes over the activations.  The time over the
 // best form's, mean and largest: 1.003 and 1.19 so; with 32 x 8 below 256 workgroups of 64 x 16, 1.12 and
 // 1.86.  us in 32 x 8 / 64 x 16 / 64 x 32: 989 x 512 from 1792, 10 entries, 9.8 / 14.9 / 23; 4911 x 768 from
-// 2688, 14 entries, 39.6 / 21.4 / 27.8; 14792 x 1024 from 4096, 128 entries, 303 / 171 / 155 (170 in 64 x 64).
+// 2688, 14 entries, 39.6 / 21.4 / 27.8; 14792 x 1024 from 4096, 128 entries, 303 / 171 / 155 (170 in 64 x 64);
+// 16384 x 2048 from 1024, 16 entries, 173 / 68 / 70 (110 through the deep ring of dxf_kernel).
 static int launch_dx16(const TProdArgs& a0, hipStream_t st) {
   struct Form { int tokens, blocks, cols; float a, b, c; };
   constexpr Form forms[3] = {{32, 8, dx16_cols(1, 2), 0.8f, 3.05f, 0.13f},
@@ -1002,11 +989,6 @@ static int launch_dx(int B, const TProdArgs& a, hipStream_t st) {
   // B = 32: the deep-ring kernel (headline backward 0.710 -> 0.688 ms; 64 / 1024 / 4096 tokens
   // 0.109 / 0.131 / 0.213 -> 0.105 / 0.127 / 0.199 ms)
   if (B == 32) return launch_dxf<32>(a, st);
-  // B = 16 at 16321 tokens and more with more than 64 output blocks: the deep-ring kernel (1024 x 8192
-  // product backward at 16384 tokens 1.275 ms in the per-entry kernel, 0.658 so).  With fewer output
-  // blocks it stages the activations once per 16 of them and is slower (SwiGLU backward at d_model 1024
-  // 0.823 ms, 0.886 so)
-  if (B == 16 && (a.N + 63) / 64 >= 256 && a.C > 64) return launch_dxf<16>(a, st);
   return B == 16 ? launch_dx16(a, st) : -2;
 }
 
