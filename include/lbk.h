@@ -631,7 +631,9 @@ int lbk_gelu_bwd_train(const uint16_t* grad_out, const uint16_t* x, const uint16
  * rounds the fp32 tiles as lbk_swiglu_fwd_train does and exports per application l, each
  * [L, N, .] bf16: states (the norm's input), normed (its result), h, gate_pre, up_out.  The backward
  * returns dh, the norm scale's gradient, fp32 tile gradients and (each optional) bias gradients,
- * summed over the applications in a fixed order.  The reference differentiates its scan
+ * summed over the applications in a fixed order.  Its workspace holds dg and du of as many
+ * applications as fit 2 GiB (at least one) and the partial sums of one pass over their tokens: up to
+ * about 3.7 GB at 16384 rows, d_model 1024, d_ff 4096.  The reference differentiates its scan
  * (looped_blockell/looping/looped_model.py:342-350).
  */
 size_t lbk_looped_fwd_train_workspace_bytes(int64_t N, int32_t d_model, const lbk_bell* gate,

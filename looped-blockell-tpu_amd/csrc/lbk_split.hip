@@ -3,8 +3,8 @@
 // gu_kernel<B, MT, NORM, INTER>: a workgroup owns 16*MT tokens.  Their input
 // rows sit in LDS as an XOR-swizzled panel (optionally RMSNorm-ed on the way in
 // from an fp32 state), next to a table of the gate/up column indices.  Eight
-// waves (two per SIMD; gu_kernel_w12, for distinct gate/up topologies with no exports and no
-// biases, runs twelve with a shallower ring at B = 32 and sixteen at B = 16) each stream their
+// waves (two per SIMD; gu_kernel_w12 runs twelve with a shallower ring at B = 32, for distinct
+// gate/up topologies with no exports and no biases, and sixteen at B = 16) each stream their
 // own d_ff block rows (r = w, w+8, ...):
 // gate and up tiles are consumed in (gate k, up k) pairs from a GU_RING-deep
 // register ring that runs across row boundaries.  The weight tile is the A
@@ -29,7 +29,7 @@
 // epilogue adds the residual, or carries an fp32 state for the looped block.
 //
 // dnr_kernel: the down kernel where those leave CUs idle, and at B = 16: smaller workgroups, wider
-// stages and a ring (its own comment).
+// stages and a ring (its own comment); launch_dn16 and launch_dn32 choose.
 //
 // dnf_kernel<B, D>: the plain forward's down kernel at B = 32 on 64-token blocks: the same
 // workgroup and stages, but each wave streams its row through a D-slot ring across the stages
@@ -585,12 +585,12 @@ __global__ __launch_bounds__(512, 1) void gu_kernel(GUArgs a) {
   gu_tile<B, MT, NORM, INTER, SHARED, false, BIAS>(a, tb, r_lo, nrs, smem, (int)threadIdx.x);
 }
 
-// gate/up with distinct gate/up topologies, without exported pre-activations or biases, one row
-// slice, with 12 waves and a 2-deep ring (B = 32): at most 168 VGPRs fit three waves per SIMD, and
-// the extra waves hide more of the panel-read and weight-load latency than the shallower ring gives
-// up.  B = 16, with a quarter of the accumulators and 8-byte fragments, runs 16 waves (forward at
-// d_model 1024, d_ff 4096, 25 %, 16384 tokens: 0.2490 ms with 12 waves, 0.2467 with 16).
-// (B = 16 also takes shared topologies, biases, exports and row slices here)
+// The same with more waves and a shallower ring.  B = 32: 12 waves and a 2-deep ring for distinct
+// gate/up topologies, without exported pre-activations or biases, in one row slice: at most 168 VGPRs
+// fit three waves per SIMD, and the extra waves hide more of the panel-read and weight-load latency
+// than the shallower ring gives up.  B = 16, with a quarter of the accumulators and 8-byte fragments:
+// 16 waves (forward at d_model 1024, d_ff 4096, 25 %, 16384 tokens: 0.2490 ms with 12 waves, 0.2467
+// with 16), for every topology, bias, export and slice count.
 template <int B, int MT, bool NORM, bool SHARED = false, bool BIAS = false, bool INTER = false, int NW = 12, int RING = 2>
 __global__ __launch_bounds__(64 * NW, 1) void gu_kernel_w12(GUArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];

@@ -4,11 +4,12 @@ The MLP half of the reference's core block applied L times:
 ``h <- h + MLPBlock(RMSNorm(h))`` (reference ``looped_blockell/layers/transformer_block.py:83-84``,
 the core loop ``looped_blockell/looping/looped_model.py:293-350`` and the MLP path of
 ``csrc/loop/persistent_core.cu:315-335``), one operator call
-(``titan::looped_swiglu``): the weights are packed once, then a gate/up and a down launch per
-application with the carried state in fp32 (``titan::looped_swiglu_persistent`` runs all L in
-one launch).  With gradients required it is one
-operator too (``titan::looped_swiglu_train``), or the applications one by one through the
-differentiable RMSNorm and SwiGLU where those modules' own calls have to be made.
+(``titan::looped_swiglu_bias``): the weights are rounded and packed in the call, then a gate/up and
+a down launch per application with the carried state in fp32 (``titan::looped_swiglu_persistent``
+runs all L in one launch).  With gradients required it is one operator too
+(``titan::looped_swiglu_train``; its backward holds the gradients of up to 2 GiB of applications at a
+time, see ``lbk_looped_bwd_train``), or the applications one by one through the differentiable
+RMSNorm and SwiGLU where those modules' own calls have to be made.
 """
 
 from __future__ import annotations

@@ -46,7 +46,7 @@ def _tensors(lin):
     try:
         b = lin._buffers
         return lin._parameters["values"], b["col_indices"], b["alive_mask"]
-    except KeyError:                                     # parametrized or replaced by plain attributes
+    except KeyError:                                     # replaced by plain attributes (weight norm)
         return lin.values, lin.col_indices, lin.alive_mask
 
 
