@@ -17,9 +17,6 @@ def looped(monkeypatch):
         return h * vg.flatten()[0]
 
     monkeypatch.setattr(kernels, "looped_swiglu_bias", looped_bias)
-    monkeypatch.setattr(kernels, "looped_swiglu_prepacked",
-                        lambda h, scale, packed, *w, **kw: looped_bias(h, scale, *w, **kw), raising=False)
-    monkeypatch.setattr(kernels, "swiglu_prepack", lambda *w: torch.zeros(1, dtype=torch.uint8))
     return LoopedSwiGLU(64, 128, 2, tile_size=16, density=0.5), seen
 
 
